@@ -63,9 +63,10 @@ BYTES_PER_CELL = {
     "fcg_Ap": 4 + 8 + 12 + 16,                       # w, p, L -> p', q
     "fcg_update": 32 + 16,                           # p', q, x64, r64 -> x64, r64
     "redist": (12 + 16 + 16) / 3,                    # ϕ, ϕini (+ ϕ⁰ in stages 2, 3) -> ϕ', per stage
-    # single-reduction CG step on coarse level l (per cell of that level):
-    # r, w, s, iD, p, x, L -> p, s', x, r', w'
-    "cg1_l1": 36 + 20, "cg1_l2": 36 + 20, "cg1_l3": 36 + 20,
+    # single-reduction CG on coarse level l (per cell of that level): one step
+    # r, w, s, iD, p, x, L -> p, s', x, r', w' on level 1; on the levels that
+    # solve in one launch r, iD, L, x -> x, once
+    "cg1_l1": 36 + 20, "cg1_l2": 24 + 4, "cg1_l3": 24 + 4,
 }
 # coarse level of a class (its cells are (N >> level)^3); 0 for the fine-level classes
 LEVEL = {"cg1_l1": 1, "cg1_l2": 2, "cg1_l3": 3}

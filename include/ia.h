@@ -57,7 +57,8 @@ enum ia_limiter {
  *            reference counterpart.  Read at ia_create, for tuning sweeps:
  *            IA_FCG_CIT=a,b,... (coarse iterations on levels 1, 2, ...),
  *            IA_FCG_SMOOTH=n (n fine pcg! iterations instead of Chebyshev),
- *            IA_CG1_NB=a,b,... (coarse CG workgroup sizes on levels 1, 2, ...).
+ *            IA_CG1_NB=a,b,... (one launch per coarse CG iteration, with these
+ *            workgroup sizes on levels 1, 2, ...).
  * PCG:       inproject!(a, b::Poisson, dt) (flow.jl:337-341): psolver! (flow.jl:300-326),
  *            Jacobi-preconditioned CG on the single (finest) level until the
  *            absolute Σr² <= 50eps(T) or 2000 iterations, as the reference runs it
@@ -274,9 +275,10 @@ int ia_learned_grad(ia_ctx *c, const float *feat, const float *dout, float *gw);
 /* Kernel-class timing with HIP events on the context's stream (no reference
  * counterpart; used by the benchmark to measure one kernel's launches inside
  * a timed region).  Enabling resets the record; MG classes time level 0 only,
- * the CG1 classes the coarse level they name, with one event pair around each
- * run of back-to-back step launches (launches counts the launches, total_ms
- * the bracketed time, gaps between those launches included). */
+ * the CG1 classes the coarse level they name: one record per solve where it
+ * is one launch, else one event pair around each run of back-to-back step
+ * launches (launches counts the launches, total_ms the bracketed time, gaps
+ * between those launches included). */
 enum ia_prof_class {
     IA_PROF_VOF = 0,          /* cVOF sweep (face pass + cell pass, one record per sweep) */
     IA_PROF_MOMENTUM = 1,     /* CMOM/SynDRoM sweep (face pass + cell pass, one record per sweep) */
@@ -291,7 +293,7 @@ enum ia_prof_class {
     IA_PROF_PCG_LAST = 10,    /* the flexible CG's fine smoother fused with its dots: two Chebyshev steps
                                  (default), or the last finest-level pcg! update (IA_FCG_SMOOTH set) */
     IA_PROF_REDIST = 11,      /* one level-set reinitialisation stage (computeL! + update + BCf!) */
-    IA_PROF_CG1_L1 = 12,      /* single-reduction CG step of the FCG preconditioner, coarse level 1 */
+    IA_PROF_CG1_L1 = 12,      /* single-reduction CG (a whole solve or its steps) of the FCG preconditioner, coarse level 1 */
     IA_PROF_CG1_L2 = 13,      /* ... level 2 */
     IA_PROF_CG1_L3 = 14,      /* ... level 3 */
     IA_PROF_NCLASS = 15

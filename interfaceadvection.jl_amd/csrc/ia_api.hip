@@ -6,6 +6,7 @@
 // and fill flags).
 #include "ia.h"
 #include "ia_poisson.h"
+#include "ia_cgp.h"
 #include "ia_learned.h"
 
 #include <hip/hip_runtime.h>
@@ -66,6 +67,8 @@ struct Level {
     void *r2 = nullptr, *w = nullptr, *w2 = nullptr;  // single-reduction CG: r, w pairs (levels >= 1)
     CTiling wt;      // the single-reduction CG step's tiling on one-cell-per-thread levels (wnb threads)
     int wnb = NT;
+    const CgpVariant *cgp = nullptr;  // the one-launch coarse CG's variant for this level, or nullptr
+    CgpBox cgp_box{};
     bool own = false;
 };
 
@@ -106,6 +109,9 @@ struct ia_ctx {
     // PLAIN), and fcg_coarse_its(level cells) in the flexible CG's preconditioner
     // (IA_FCG_CIT=a,b,... overrides levels 1, 2, ...; the last value repeats)
     int cit_wl[MAXLEV], cit_fcg[MAXLEV];
+    unsigned long long *cgp_hw = nullptr, *cgp_pw = nullptr;  // the one-launch coarse CG's words
+    unsigned cgp_tag = 1;  // next unused tag of those words
+    bool cgp_off = false;  // one launch per iteration instead (IA_CG1_NB set, or workgroups did not run together)
     int cg1_nb[MAXLEV];  // workgroup size of the coarse CG step per level (one cell per thread)
     struct Cnn {
         bool ready = false;
@@ -501,6 +507,7 @@ template <class T> struct Impl {
                 HIPCHK(c, hipFuncSetAttribute((const void *)k_mg_tail<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               (int)c->tail_lds));
         }
+        if (int r = cgp_setup(c)) return r;
         c->part_n = 5 * maxblk + 64;
         HIPCHK(c, hipMalloc(&c->part, c->part_n * sizeof(double)));
         HIPCHK(c, hipMalloc(&c->fpart, (maxblk + FILL_R2) * sizeof(FillPart)));
@@ -524,6 +531,44 @@ template <class T> struct Impl {
         return IA_OK;
     }
 
+    // the levels that the flexible CG's preconditioner solves with k_cgp: those above the tail whose boxes fit, on a
+    // device that holds twice the workgroups at once (two contexts may run there together)
+    static int cgp_setup(ia_ctx *c) {
+        if (sizeof(T) != 4 || c->cgp_off || c->P.poisson_mode == IA_POISSON_REFERENCE ||
+            c->P.poisson_mode == IA_POISSON_PCG || c->P.poisson_mode == IA_POISSON_PLAIN)
+            return IA_OK;
+        int ncu = 0, nv = 0;
+        HIPCHK(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->dev));
+        const CgpVariant *vs = cgp_variants(nv);
+        size_t words = 0;
+        for (int l = 1; l < c->tail_level && l < c->nlev; ++l) {
+            Level &lv = c->lev[l];
+            int n[3];
+            for (int a = 0; a < 3; ++a) n[a] = a < lv.g.D ? lv.g.Ng[a] - 2 : 1;
+            // everyone reads every sum up to CGP_ONE workgroups; more of them only where the level needs it
+            for (int maxwg : {CGP_ONE, CGP_MAXWG})
+                for (int q = 0; q < nv && !lv.cgp; ++q) {
+                    if (vs[q].D != lv.g.D || (maxwg > CGP_ONE && vs[q].NB < 1024)) continue;
+                    if (!cgp_boxes(n, vs[q], maxwg, lv.cgp_box)) continue;
+                    int per = 0;
+                    HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void *)vs[q].k, vs[q].NB,
+                                                                           cgp_lds(lv)));
+                    if ((long)per * ncu < (maxwg > CGP_ONE ? 1L : 2L) * lv.cgp_box.nwg) continue;
+                    lv.cgp = &vs[q];
+                }
+            if (lv.cgp)
+                words = std::max(words, (size_t)2 * lv.cgp_box.nwg * 2 * lv.g.D * lv.cgp_box.amax);
+        }
+        if (words) {
+            if (int r = alloc_zero(c, (void **)&c->cgp_hw, words * sizeof(unsigned long long))) return r;
+            if (int r = alloc_zero(c, (void **)&c->cgp_pw, 2 * CGP_PW * sizeof(unsigned long long))) return r;
+        }
+        return IA_OK;
+    }
+    static size_t cgp_lds(const Level &l) {
+        const CgpBox &b = l.cgp_box;
+        return sizeof(float) * (b.b[0] + 2) * (b.b[1] + 2) * (l.g.D > 2 ? b.b[2] + 2 : 1);
+    }
     // ----------------------------------------------------------------- MG
     static int mg_update(ia_ctx *c) {
         for (int l = 0; l < c->nlev; ++l) {
@@ -609,15 +654,36 @@ template <class T> struct Impl {
     // pre_done: Jacobi! + increment! of level l were fused into the caller's
     // residual load.  then_pcg: a pcg! on level l follows, so its first
     // statement is fused into the final prolongate! + increment!.
-    // the flexible CG preconditioner's coarse solve: single-reduction CG, one
-    // launch per iteration (k_cg1_init, k_cg1_step).  The final r may sit in
-    // r2; nothing reads a coarse r after its solve (restrict! rewrites it).
+    // the flexible CG preconditioner's coarse solve: single-reduction CG, in
+    // one launch (k_cgp) where the level's boxes fit, else one launch per
+    // iteration (k_cg1_init, k_cg1_step).  The final r may sit in r2 or
+    // nowhere; nothing reads a coarse r after its solve (restrict! rewrites it).
     static void pcg1(ia_ctx *c, Level &l, int it) {
+        int lv = (int)(&l - c->lev), pc = lv >= 1 && lv <= 3 ? IA_PROF_CG1_L1 + lv - 1 : -1;
+        if (l.cgp && !c->cgp_off) {
+            CgpArgs a;
+            a.g = l.g;
+            a.box = l.cgp_box;
+            a.L = P<float>(l.L);
+            a.iD = P<float>(l.iD);
+            a.r = P<float>(l.r);
+            a.x = P<float>(l.x);
+            a.hw = c->cgp_hw;
+            a.pw = c->cgp_pw;
+            a.tag = c->cgp_tag;
+            c->cgp_tag += (unsigned)it + 1;
+            a.it = it;
+            a.halt = cur_halt;
+            a.fail = &c->fst->fail;
+            if (pc >= 0) prof_begin(c, pc);
+            hipLaunchKernelGGL(l.cgp->k, dim3((unsigned)a.box.nwg), dim3((unsigned)l.cgp->NB), cgp_lds(l), c->s, a);
+            if (pc >= 0) prof_end(c, pc);
+            return;
+        }
         LevV<T> v = view(l);
         dim3 B = cb(l);
         T *r[2] = {P<T>(l.r), P<T>(l.r2)}, *w[2] = {P<T>(l.w), P<T>(l.w2)}, *s[2] = {P<T>(l.z), P<T>(l.z2)};
         hipLaunchKernelGGL(k_cg1_init<T>, B, dim3(NT), 0, c->s, v, w[0], c->pst, pp(c, PP_A));
-        int lv = (int)(&l - c->lev), pc = lv >= 1 && lv <= 3 ? IA_PROF_CG1_L1 + lv - 1 : -1;
         if (pc >= 0) prof_begin(c, pc);
         for (int q = 1; q <= it; ++q) {
             int a = (q - 1) & 1;
@@ -947,6 +1013,7 @@ template <class T> struct Impl {
                 it++;
                 rr = st.rr;
                 rel = sqrt(rr) / zn;
+                if (st.fail) c->cgp_off = true;  // workgroups of a k_cgp launch did not run together
                 if (st.halt) {
                     // the queued iteration (if any) returned at once; confirm with
                     // the true FP64 residual and restart from it if it drifted
@@ -1690,9 +1757,10 @@ int ia_create(const ia_params *p, ia_ctx **out) {
         c->cit_fcg[l] = fcg_coarse_its(n, l);
         c->cg1_nb[l] = p->D == 3 ? cg1_workgroup(n) : NT;
     }
-    // IA_CG1_NB=a,b,...: the coarse CG step's workgroup size on levels 1, 2, ...
+    // IA_CG1_NB=a,b,...: one launch per coarse CG iteration, with this workgroup size on levels 1, 2, ...
     // (128, 256, 512 or 1024; used where a level has one cell per thread)
     if (const char *nv = getenv("IA_CG1_NB"); nv && *nv) {
+        c->cgp_off = true;
         int l = 1;
         const char *q = nv;
         while (*q && l < MAXLEV) {
@@ -1756,7 +1824,7 @@ void ia_destroy(ia_ctx *c) {
     void *bufs[] = {c->fb[0], c->fb[1], c->fb[2], c->fb[3], c->u, c->u0, c->ru, c->ru2, c->ruf, c->F, c->p, c->sig,
                     c->st_buf, c->st_fb,
                     c->L, c->al, c->nh, c->cb, c->fpart, c->part, c->st, c->pst, c->fst, c->pp, c->dsc, c->x64, c->r64, c->z64,
-                    c->pa64, c->pb64, c->q64, c->vface, c->mface};
+                    c->pa64, c->pb64, c->q64, c->vface, c->mface, c->cgp_hw, c->cgp_pw};
     for (void *b : bufs)
         if (b && !is_attached(c, b)) (void)hipFree(b);
     for (int l = 0; l < c->nlev; ++l) {

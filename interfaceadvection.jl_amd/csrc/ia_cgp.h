@@ -1,0 +1,439 @@
+// ia_cgp.h -- the single-reduction CG of a coarse level in one launch.
+#pragma once
+#include "ia_poisson.h"
+
+namespace ia {
+
+// ---------------------------------------------------------------------------
+// All iterations of the single-reduction CG (k_cg1_init, k_cg1_step: the same
+// recurrence, the same operations per cell) in one launch of at most CGP_MAXWG
+// workgroups that are resident together.  Each workgroup owns a box of cells
+// whose r, w, s, p, x, iD and L stay in registers; u = r·iD of the box and of
+// its one-cell halo is in LDS.  The halo cells' r and s follow the owners'
+// recurrence, so an iteration needs from outside only the neighbours' new w
+// and everyone's partial sums, once.
+//
+// Both travel as 64-bit words of 32 data bits and a 32-bit tag that names the
+// launch and the iteration, written and read as single relaxed agent-scope
+// atomics: a word whose tag fits is the value itself, so no fence and no
+// ordering between words is needed.  Two slots alternate.  A workgroup writes
+// a slot again two iterations later, after it has read every workgroup's
+// partial of the iteration between, which each of them publishes only after
+// it has read the slot's words.
+//
+// Measured against one launch per iteration, µs per iteration of 64: 64^3 3.84 against 6.6-7.5, 32^3 2.25 against
+// 4.6, 60x44x36 2.9 against 5.4, 192x128 2.0 against 4.5, 96x64 1.8 against 4.3.  What is left is about 1 µs from
+// one workgroup's store to another's load (past the L2s of the eight XCDs) and as much for the operator, the
+// recurrence and the sums.
+//
+// A workgroup that waits longer than CGP_WAIT (another program's work kept
+// some workgroups off the device) writes the x it has, raises *fail and ends,
+// so the launch always ends; x is then a less exact solution.
+// ---------------------------------------------------------------------------
+constexpr int CGP_MAXWG = 256;
+constexpr int CGP_ONE = 64;   // up to so many workgroups everyone reads every partial sum
+constexpr int CGP_GROUP = 16; // above, the sums of groups of this many, which the group's first workgroup forms
+// cycles/64 before the first look for the sums: a look takes about 1100 cycles and disturbs the words' way, so the
+// first one should find them (64 workgroups, 32^3: 3.0 µs an iteration without, 2.5 with 6, 2.25 with 12, 2.3 with 18)
+constexpr int CGP_NAP = 12;
+constexpr long CGP_WAIT = 100000000;  // ticks of the 100 MHz counter: 1 s
+struct CgpBox {
+    int k[3], b[3];  // boxes per axis, cells per box and axis (the last box may have fewer, at least 2)
+    int nwg, amax;   // workgroups, the largest face of a box
+};
+struct CgpArgs {
+    Grid g;
+    CgpBox box;
+    const float *L, *iD, *r;
+    float *x;
+    unsigned long long *hw;  // 2 slots of nwg * 2D * amax words: w of the cells at a box's faces
+    unsigned long long *pw;  // 2 slots of CGP_PW words: the partial sums, then the groups' sums
+    unsigned tag;            // of iteration 0
+    int it;
+    const int *halt;
+    int *fail;
+};
+// a slot of partial sums: CGP_COPY copies of 4 words of CGP_ONE workgroups (or groups), then
+// 4 words of CGP_MAXWG workgroups of a group
+constexpr int CGP_COPY = 16;
+constexpr int CGP_P1 = CGP_COPY * 4 * CGP_ONE;
+constexpr int CGP_PW = CGP_P1 + 4 * CGP_MAXWG;
+typedef unsigned long long cgp_word;
+__device__ inline void cgp_put(cgp_word *p, unsigned v, unsigned tag) {
+    __hip_atomic_store(p, ((cgp_word)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline cgp_word cgp_get(const cgp_word *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+
+// NB threads; a thread owns a column of C cells along the last axis (so two of a cell's neighbours are mostly its own
+// registers); the halo cells are those of wavefronts 1.. (HC each), while wavefront 0 waits for the sums.
+template <int D, int NB, int C, int HC>
+__global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
+    HALT_IF(a)
+    extern __shared__ __align__(16) float cgp_u[];
+    constexpr bool XL = NB * C >= 4096;  // x in LDS: the registers of a 1024-thread workgroup do not hold it
+    __shared__ float xl[XL ? NB * C : 1];
+    __shared__ double shp[2][NB / 64], sht[2];
+    __shared__ int dead;
+    const Grid &g = a.g;
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+    // this workgroup's box: first cell lo (ghost-inclusive), sides n
+    int bi[3], lo[3], n[3];
+    {
+        int q = blockIdx.x;
+        bi[0] = q % a.box.k[0];
+        q /= a.box.k[0];
+        bi[1] = q % a.box.k[1];
+        bi[2] = q / a.box.k[1];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        lo[d] = d < D ? 1 + bi[d] * a.box.b[d] : 0;
+        n[d] = d < D ? min(a.box.b[d], g.Ng[d] - 1 - lo[d]) : 1;
+    }
+    const int t1 = a.box.b[0] + 2, t2 = t1 * (a.box.b[1] + 2);  // strides of the u tile
+    const int tz = D > 2 ? t2 : t1;                            // along a column
+    const long sz = g.st[D - 1];
+    if (tid == 0) dead = 0;
+    // own cells: lateral position (x, y), first cell z0 of the column, cnt of them
+    const int nl = D > 2 ? n[0] * n[1] : n[0];
+    const int col = tid % nl, x0 = col % n[0], y0 = D > 2 ? col / n[0] : 0, z0 = (tid / nl) * C;
+    const int cnt = max(0, min(C, n[D - 1] - z0));
+    const int ti = (x0 + 1) + (D > 2 ? t1 * (y0 + 1) : 0) + tz * (z0 + 1);
+    const long I0 = (long)(lo[0] + x0) + (D > 2 ? g.st[1] * (lo[1] + y0) : 0) + sz * (lo[D - 1] + z0);
+    // words of the column's w in the slot: its side face along x (and y), cell k at + k*stride; the faces of its ends
+    const int fb = (int)blockIdx.x * 2 * D;
+    int px = -1, py = -1, pl = -1, ph = -1;
+    const int sx = D > 2 ? n[1] : 1, sy = n[0];
+    if (cnt > 0) {
+        if (x0 == 0 || x0 == n[0] - 1) px = (fb + (x0 ? 1 : 0)) * a.box.amax + (D > 2 ? y0 + n[1] * z0 : z0);
+        if (D > 2 && (y0 == 0 || y0 == n[1] - 1)) py = (fb + 2 + (y0 ? 1 : 0)) * a.box.amax + x0 + n[0] * z0;
+        if (z0 == 0) pl = (fb + 2 * (D - 1)) * a.box.amax + col;
+        if (z0 + cnt == n[D - 1]) ph = (fb + 2 * (D - 1) + 1) * a.box.amax + col;
+    }
+    float r[C], s[C], w[C], p[C], x[XL ? 1 : C], id[C], u[C], dg[C], lx[C], lxp[C], ly[C], lyp[C], lz[C + 1];
+#pragma unroll
+    for (int k = 0; k <= C; ++k) lz[k] = cnt > 0 && k <= cnt ? a.L[g.ns * (D - 1) + I0 + k * sz] : 0.f;
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        if (!XL) x[XL ? 0 : k] = 0.f;
+        r[k] = s[k] = w[k] = p[k] = id[k] = u[k] = dg[k] = lx[k] = lxp[k] = ly[k] = lyp[k] = 0.f;
+        if (k < cnt) {
+            long I = I0 + k * sz;
+            r[k] = a.r[I];
+            id[k] = a.iD[I];
+            if (XL) xl[k * NB + tid] = a.x[I];
+            else x[XL ? 0 : k] = a.x[I];
+            lx[k] = a.L[I];
+            lxp[k] = a.L[I + 1];
+            dg[k] -= (lx[k] + lxp[k]);
+            if (D > 2) {
+                ly[k] = a.L[g.ns + I];
+                lyp[k] = a.L[g.ns + I + g.st[1]];
+                dg[k] -= (ly[k] + lyp[k]);
+            }
+            dg[k] -= (lz[k] + lz[k + 1]);
+        }
+    }
+    // halo cells of the box's faces (2d + side); none across a wall (u = 0 there, L = 0)
+    bool hon[HC];
+    int hti[HC], hwo[HC];  // place in the tile, word of the cell's w in the slot
+    float hr[HC], hs[HC], hid[HC], hv[HC];
+    {
+        const int area[3] = {n[1] * n[2], n[0] * n[2], n[0] * n[1]};
+        const int hc = 2 * area[0] + 2 * area[1] + (D > 2 ? 2 * area[2] : 0);
+#pragma unroll
+        for (int k = 0; k < HC; ++k) {
+            int h = tid - 64 + k * (NB - 64);
+            hon[k] = false;
+            hti[k] = hwo[k] = 0;
+            hr[k] = hs[k] = hid[k] = hv[k] = 0.f;
+            if (tid >= 64 && h < hc) {
+                int d = 0;
+                if (h >= 2 * area[0]) {
+                    h -= 2 * area[0];
+                    d = 1;
+                    if (D > 2 && h >= 2 * area[1]) {
+                        h -= 2 * area[1];
+                        d = 2;
+                    }
+                }
+                const int ar = d == 0 ? area[0] : d == 1 ? area[1] : area[2];
+                const int side = h >= ar;
+                h -= side * ar;
+                // element h of the face: the two other coordinates in x-y-z order
+                const int m = d == 0 ? n[1] : n[0], e0 = h % m, e1 = h / m;
+                const int qd = side ? (d == 0 ? n[0] : d == 1 ? n[1] : n[2]) : -1;
+                const int q[3] = {d == 0 ? qd : e0, d == 1 ? qd : (d == 0 ? e0 : e1), d == 2 ? qd : e1};
+                hti[k] = (q[0] + 1) + t1 * (q[1] + 1) + (D > 2 ? t2 * (q[2] + 1) : 0);
+                int P[3] = {lo[0] + q[0], lo[1] + q[1], D > 2 ? lo[2] + q[2] : 0}, c[3] = {bi[0], bi[1], bi[2]};
+                bool wall = false;
+#pragma unroll
+                for (int b = 0; b < D; ++b)
+                    if (b == d) {
+                        wall = !g.per[b] && (P[b] == 0 || P[b] == g.Ng[b] - 1);
+                        P[b] = P[b] == 0 ? g.Ng[b] - 2 : P[b] == g.Ng[b] - 1 ? 1 : P[b];
+                        c[b] += side ? 1 : -1;
+                        c[b] = c[b] < 0 ? a.box.k[b] - 1 : c[b] == a.box.k[b] ? 0 : c[b];
+                    }
+                if (wall) {
+                    cgp_u[hti[k]] = 0.f;
+                } else {
+                    hon[k] = true;
+                    long J = (long)P[0] + g.st[1] * P[1] + (D > 2 ? g.st[2] * P[2] : 0);
+                    hr[k] = a.r[J];
+                    hid[k] = a.iD[J];
+                    // the neighbour's facing side holds the same cells in the same order
+                    hwo[k] = ((c[0] + a.box.k[0] * (c[1] + a.box.k[1] * c[2])) * 2 * D + 2 * d + 1 - side) * a.box.amax + h;
+                }
+            }
+        }
+    }
+    const long hslot = (long)a.box.nwg * 2 * D * a.box.amax;
+    const int nwg = a.box.nwg, ngrp = (nwg + CGP_GROUP - 1) / CGP_GROUP;
+    const bool two = nwg > CGP_ONE;
+    auto half_of = [](double va, double vb, int j) {  // word j of a pair of sums
+        double v = j < 2 ? va : vb;
+        return (unsigned)((j & 1) ? __double2hiint(v) : __double2loint(v));
+    };
+    auto tile = [&]() {  // u of the box and its halo
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+            if (k < cnt) {
+                u[k] = r[k] * id[k];
+                cgp_u[ti + k * tz] = u[k];
+            }
+#pragma unroll
+        for (int k = 0; k < HC; ++k)
+            if (hon[k]) cgp_u[hti[k]] = hr[k] * hid[k];
+    };
+    auto apply = [&](unsigned tag) {  // w = A u, published at the box's faces; the partials of r·u and u·w
+        cgp_word *hw = a.hw + (tag & 1 ? hslot : 0);
+        double gd = 0, dd = 0;
+        if (cnt > 0) {
+            const float ulo = cgp_u[ti - tz], uhi = cgp_u[ti + cnt * tz];
+#pragma unroll
+            for (int k = 0; k < C; ++k)
+                if (k < cnt) {
+                    const int t = ti + k * tz;
+                    float sl = 0, su = 0;
+                    sl += cgp_u[t - 1] * lx[k];
+                    su += cgp_u[t + 1] * lxp[k];
+                    if (D > 2) {
+                        sl += cgp_u[t - t1] * ly[k];
+                        su += cgp_u[t + t1] * lyp[k];
+                    }
+                    const float um = k > 0 ? u[k > 0 ? k - 1 : 0] : ulo;
+                    float up = uhi;
+                    if (k + 1 < C) {
+                        float un = u[k + 1 < C ? k + 1 : k];
+                        up = k + 1 < cnt ? un : uhi;
+                    }
+                    sl += um * lz[k];
+                    su += up * lz[k + 1];
+                    w[k] = (u[k] * dg[k] + sl) + su;
+                }
+            if (px >= 0) {
+#pragma unroll
+                for (int k = 0; k < C; ++k)
+                    if (k < cnt) cgp_put(hw + px + k * sx, __float_as_uint(w[k]), tag);
+            }
+            if (D > 2 && py >= 0) {
+#pragma unroll
+                for (int k = 0; k < C; ++k)
+                    if (k < cnt) cgp_put(hw + py + k * sy, __float_as_uint(w[k]), tag);
+            }
+            if (pl >= 0) cgp_put(hw + pl, __float_as_uint(w[0]), tag);
+            if (ph >= 0) {
+#pragma unroll
+                for (int k = 0; k < C; ++k)
+                    if (k == cnt - 1) cgp_put(hw + ph, __float_as_uint(w[k]), tag);
+            }
+#pragma unroll
+            for (int k = 0; k < C; ++k)
+                if (k < cnt) {  // the products are exact
+                    gd = __builtin_fma((double)r[k], (double)u[k], gd);
+                    dd = __builtin_fma((double)u[k], (double)w[k], dd);
+                }
+        }
+        gd = wave_sum(gd);
+        dd = wave_sum(dd);
+        if (lane == 0) {
+            shp[0][wv] = gd;
+            shp[1][wv] = dd;
+        }
+        __syncthreads();
+        if (wv == 0) {
+            double va = 0, vb = 0;
+#pragma unroll
+            for (int q = 0; q < NB / 64; ++q) va += shp[0][q];
+#pragma unroll
+            for (int q = 0; q < NB / 64; ++q) vb += shp[1][q];
+            cgp_word *pw = a.pw + (tag & 1 ? CGP_PW : 0) + CGP_P1;
+            if (lane < 4) cgp_put(pw + lane * CGP_MAXWG + blockIdx.x, half_of(va, vb, lane), tag);
+        }
+    };
+    // the sums of m pairs (m <= 64) by this wavefront; false: not there in time
+    auto gather = [&](const cgp_word *w4, int st, int m, unsigned tag, double &va, double &vb) {
+        cgp_word v[4];
+        const long t0 = wall_clock64();
+        for (int spin = 0;; ++spin) {
+            bool ok = true;
+            if (lane < m) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = cgp_get(w4 + j * st + lane);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ok = ok && (unsigned)(v[j] >> 32) == tag;
+            }
+            if (__all(ok)) break;
+            if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
+        }
+        va = lane < m ? __hiloint2double((int)(unsigned)v[1], (int)(unsigned)v[0]) : 0.0;
+        vb = lane < m ? __hiloint2double((int)(unsigned)v[3], (int)(unsigned)v[2]) : 0.0;
+        va = wave_sum(va);
+        vb = wave_sum(vb);
+        return true;
+    };
+    // the halo cells' w
+    auto halo = [&](const cgp_word *hw, unsigned tag) {
+        cgp_word h[HC];
+        const long t0 = wall_clock64();
+        for (int spin = 0;; ++spin) {
+            bool ok = true;
+#pragma unroll
+            for (int k = 0; k < HC; ++k)
+                if (hon[k]) h[k] = cgp_get(hw + hwo[k]);
+#pragma unroll
+            for (int k = 0; k < HC; ++k)
+                if (hon[k]) ok = ok && (unsigned)(h[k] >> 32) == tag;
+            if (__all(ok)) break;
+            if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
+        }
+#pragma unroll
+        for (int k = 0; k < HC; ++k) hv[k] = hon[k] ? __uint_as_float((unsigned)h[k]) : 0.f;
+        return true;
+    };
+    tile();
+    __syncthreads();
+    apply(a.tag);
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        p[k] = u[k];
+        s[k] = w[k];
+    }
+    float rho = 0, al = 0;
+    for (int q = 1; q <= a.it; ++q) {
+        const unsigned tag = a.tag + q - 1;
+        cgp_word *pw = a.pw + (tag & 1 ? CGP_PW : 0);
+        bool ok = true;
+        if (wv == 0) {
+            double sa = 0, sb = 0;
+            __builtin_amdgcn_s_sleep(CGP_NAP);
+            if (two) {
+                if (blockIdx.x % CGP_GROUP == 0) {
+                    ok = gather(pw + CGP_P1 + blockIdx.x, CGP_MAXWG, min(CGP_GROUP, nwg - (int)blockIdx.x), tag, sa, sb);
+                    if (ok) cgp_put(pw + lane * CGP_ONE + blockIdx.x / CGP_GROUP, half_of(sa, sb, lane & 3), tag);
+                }
+                if (ok) ok = gather(pw + (blockIdx.x % CGP_COPY) * 4 * CGP_ONE, CGP_ONE, ngrp, tag, sa, sb);
+            } else {
+                ok = gather(pw + CGP_P1, CGP_MAXWG, nwg, tag, sa, sb);
+            }
+            if (lane == 0) {
+                sht[0] = sa;
+                sht[1] = sb;
+            }
+        } else {
+            ok = halo(a.hw + (tag & 1 ? hslot : 0), tag);
+        }
+        if (!ok) dead = 1;
+        __syncthreads();
+        if (dead) {
+            if (tid == 0) *a.fail = 1;
+            break;
+        }
+        const float gam = (float)sht[0], del = (float)sht[1];
+        if (fabs(gam) < 10 * eps_of<float>()) break;
+        float beta = 0;
+        if (q == 1) {
+            al = gam / del;
+        } else {
+            beta = gam / rho;
+            al = gam / (del - (beta * gam) / al);
+        }
+        rho = gam;
+        const bool stop = q == a.it || fabs((double)al) < 1e-2;
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+            if (k < cnt) {
+                if (q > 1) {
+                    p[k] = u[k] + beta * p[k];
+                    s[k] = w[k] + beta * s[k];
+                }
+                if (XL) xl[k * NB + tid] += al * p[k];
+                else x[XL ? 0 : k] = x[XL ? 0 : k] + al * p[k];
+                r[k] = r[k] - al * s[k];
+            }
+        if (stop) break;
+#pragma unroll
+        for (int k = 0; k < HC; ++k)
+            if (hon[k]) {
+                hs[k] = q > 1 ? hv[k] + beta * hs[k] : hv[k];
+                hr[k] = hr[k] - al * hs[k];
+            }
+        tile();
+        __syncthreads();
+        apply(tag + 1);
+    }
+#pragma unroll
+    for (int k = 0; k < C; ++k)
+        if (k < cnt) a.x[I0 + k * sz] = XL ? xl[k * NB + tid] : x[XL ? 0 : k];
+}
+
+// The variants: threads and cells per thread, the fewest first, as more cells per workgroup cost more than more
+// workgroups up to CGP_ONE (32^3: 2.25 µs with 2 cells on 256 threads, 2.7 with 4 on 512, 2.8 with 4 on 1024).
+struct CgpVariant {
+    int D, NB, C, HC;
+    void (*k)(CgpArgs);
+};
+inline const CgpVariant *cgp_variants(int &n) {
+    static const CgpVariant v[] = {{2, 256, 1, 1, k_cgp<2, 256, 1, 1>}, {2, 256, 2, 1, k_cgp<2, 256, 2, 1>},
+                                   {2, 512, 4, 1, k_cgp<2, 512, 4, 1>}, {2, 1024, 4, 1, k_cgp<2, 1024, 4, 1>},
+                                   {3, 256, 1, 2, k_cgp<3, 256, 1, 2>}, {3, 256, 2, 3, k_cgp<3, 256, 2, 3>},
+                                   {3, 512, 4, 3, k_cgp<3, 512, 4, 3>}, {3, 1024, 4, 2, k_cgp<3, 1024, 4, 2>}};
+    n = 8;
+    return v;
+}
+// boxes of a level of n cells per axis for a variant, at most maxwg of them; false: none fits
+inline bool cgp_boxes(const int *n, const CgpVariant &v, int maxwg, CgpBox &o) {
+    long best = -1;
+    for (int k2 = 1; k2 <= (v.D > 2 ? n[2] : 1) && k2 <= maxwg; ++k2)
+        for (int k1 = 1; k1 <= n[1] && k1 * k2 <= maxwg; ++k1)
+            for (int k0 = 1; k0 <= n[0] && (long)k0 * k1 * k2 <= maxwg; ++k0) {
+                const int k[3] = {k0, k1, k2};
+                int b[3] = {1, 1, 1};
+                bool ok = true;
+                for (int d = 0; d < v.D; ++d) {
+                    b[d] = (n[d] + k[d] - 1) / k[d];
+                    ok = ok && n[d] - (k[d] - 1) * b[d] >= 2;  // a box's two faces along an axis are different cells
+                }
+                if (!ok) continue;
+                const long lat = (long)b[0] * (v.D > 2 ? b[1] : 1), thr = lat * ((b[v.D - 1] + v.C - 1) / v.C);
+                const long f0 = (long)b[1] * b[2], f1 = (long)b[0] * b[2], f2 = v.D > 2 ? (long)b[0] * b[1] : 0;
+                const long h = 2 * (f0 + f1 + f2);
+                if (thr > v.NB || h > (long)(v.NB - 64) * v.HC) continue;
+                const long cost = (long)b[0] * b[1] * b[2] + h + (long)k0 * k1 * k2;
+                if (best >= 0 && cost >= best) continue;
+                best = cost;
+                for (int d = 0; d < 3; ++d) {
+                    o.k[d] = k[d];
+                    o.b[d] = b[d];
+                }
+                o.nwg = k0 * k1 * k2;
+                o.amax = (int)(f0 > f1 ? (f0 > f2 ? f0 : f2) : (f1 > f2 ? f1 : f2));
+            }
+    return best >= 0;
+}
+
+}  // namespace ia

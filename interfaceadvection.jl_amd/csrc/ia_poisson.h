@@ -57,8 +57,9 @@ struct PcgState {
 struct FcgState {
     double sload, wr, beta, pq, alpha;
     double rr;      // ‖r‖² after the last accepted update
-    int halt, pad;  // set when the recursive residual met the tolerance:
+    int halt;       // set when the recursive residual met the tolerance:
                     // every solver kernel queued after that returns at once
+    int fail;       // set when workgroups of a k_cgp launch did not run together
 };
 
 // every block of a consumer sums the producer's per-block partials itself

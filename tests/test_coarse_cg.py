@@ -1,0 +1,75 @@
+"""The coarse CG in one launch (ia_cgp.h) against one launch per iteration
+(IA_CG1_NB set), which evaluates the same recurrence: whole projections to
+1e-6 from the same inputs, on grids whose coarse levels meet every edge of
+the boxes: levels that the boxes do not divide, sides of 2 cells, sides that
+halve to odd ones, walls and periodic axes (a box that is its own neighbour
+among them), and a level of so many workgroups that their sums are formed in
+groups.  Per cell both do the same operations in the same order; their dot
+products add in another order in FP64 before they are rounded to FP32, which
+changes a rounding of 2^-24 about once in 2^29 sums.  The bar allows such
+changes to reach the result at the size of the solve's tolerance."""
+import ctypes as C
+import os
+
+import numpy as np
+import pytest
+
+from __graft_entry__ import load_package
+from test_gpu_parity import say
+
+pytestmark = pytest.mark.gpu
+
+ia = load_package()
+
+
+def projected(dims, perdir, launched):
+    old = os.environ.get("IA_CG1_NB")
+    if launched:
+        os.environ["IA_CG1_NB"] = "256"
+    try:
+        s = ia.TwoPhaseSimulation(dims, (0.0,) * len(dims), float(dims[-1]), T=np.float32, poisson="refined", perdir=perdir)
+    finally:
+        if launched:
+            del os.environ["IA_CG1_NB"]
+            if old is not None:
+                os.environ["IA_CG1_NB"] = old
+    rng = np.random.default_rng(11)
+    D = len(dims)
+    x = np.meshgrid(*[np.arange(n + 2) / n for n in dims], indexing="ij")
+    f = 0.5 + 0.5 * np.tanh(20 * np.sin(2 * np.pi * x[0]) * np.cos(2 * np.pi * x[D - 1]))
+    s.intf.f = f
+    u = 0.1 * rng.standard_normal(tuple(n + 2 for n in dims) + (D,))
+    for a in range(D):  # no flow through walls
+        if a + 1 not in perdir:
+            for q in (0, 1, -1):
+                u[tuple(q if b == a else slice(None) for b in range(D)) + (a,)] = 0
+        else:
+            ix = [slice(None)] * D
+            ix[a] = -1
+            lo = [slice(None)] * D
+            lo[a] = 1
+            u[tuple(ix)] = u[tuple(lo)]
+    s.flow.u = u
+    s._call("ia_update_L", 0)
+    s._call("ia_mg_update")
+    st = ia.IASolveStats()
+    s._call("ia_project", 1.0, C.byref(st))
+    out = s.flow.u.astype(np.float64), s.flow.p.astype(np.float64), st.iters, st.rel
+    s.close()
+    return out
+
+
+@pytest.mark.parametrize("dims,perdir", [
+    ((256, 200), ()), ((200, 136), (1, 2)), ((2048, 16), (2,)), ((16, 2048), (1,)),
+    ((64, 64, 64), ()), ((120, 88, 72), (1, 2)), ((100, 60, 84), (3,)), ((512, 16, 16), (1, 2, 3)),
+    ((16, 256, 32), ()), ((160, 160, 96), (2,)),
+])
+def test_one_launch_equals_one_launch_per_iteration(dims, perdir):
+    say("coarse CG in one launch", dims, perdir)
+    u, p, it, rel = projected(dims, perdir, False)
+    ul, pl, itl, rell = projected(dims, perdir, True)
+    print(f"iterations {it} / {itl}, rel {rel:.3e} / {rell:.3e}, max|Δu| {np.abs(u - ul).max():.2e}, "
+          f"max|Δp| {np.abs(p - pl).max():.2e} of {np.abs(pl).max():.2e}")
+    assert 0 < rel <= 1e-6 and abs(it - itl) <= 1
+    assert np.abs(u - ul).max() <= 1e-5 * np.abs(ul).max()
+    assert np.abs(p - pl).max() <= 1e-4 * np.abs(pl).max()
