@@ -140,6 +140,8 @@ struct ia_ctx {
     int att_fi = -1, att_f0i = -1;
     int tail_level = 99; // first level handled by the one-workgroup tail kernel
     size_t tail_lds = 0; // its dynamic LDS bytes
+    // the column kernels that hold the tail: 512 threads of 4 cells, 512 of 8, 1024 of 4 (FP32; else k_mg_tail)
+    bool tail_cols[3] = {false, false, false};
     hipEvent_t e0 = nullptr, e1 = nullptr;
     struct ProfClass {
         bool on = false;
@@ -506,6 +508,15 @@ template <class T> struct Impl {
             if (c->tail_lds > 0)
                 HIPCHK(c, hipFuncSetAttribute((const void *)k_mg_tail<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               (int)c->tail_lds));
+            if (sizeof(T) == 4 && c->tail_lds > 0) {
+                const int ntf[3] = {512, 512, 1024}, cm[3] = {4, 8, 4};
+                for (int q = 0; q < 3; ++q) {
+                    c->tail_cols[q] = tail_cols_fit(gs, c->tail_level, c->nlev, ntf[q], cm[q]);
+                    if (c->tail_cols[q])
+                        HIPCHK(c, hipFuncSetAttribute((const void *)tail_cols_kernel(q),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)c->tail_lds));
+                }
+            }
         }
         if (int r = cgp_setup(c)) return r;
         c->part_n = 5 * maxblk + 64;
@@ -650,6 +661,19 @@ template <class T> struct Impl {
             if (i < it && !pair) hipLaunchKernelGGL(k_pcg_eps<T>, B, dim3(NT), 0, c->s, v, c->pst, su, se, pp(c, PP_C));
         }
     }
+    static void (*tail_cols_kernel(int q))(TailArgs<float>) {
+        return q == 0 ? k_mg_tail_cols<512, 4> : q == 1 ? k_mg_tail_cols<512, 8> : k_mg_tail_cols<1024, 4>;
+    }
+    static void launch_tail(ia_ctx *c, const TailArgs<T> &a, bool many) {
+        if constexpr (sizeof(T) == 4) {
+            const int q = c->tail_cols[0] ? 0 : c->tail_cols[1] && (many || !c->tail_cols[2]) ? 1 : 2;
+            if (c->tail_cols[q]) {
+                hipLaunchKernelGGL(tail_cols_kernel(q), dim3(1), dim3(q < 2 ? 512 : 1024), c->tail_lds, c->s, a);
+                return;
+            }
+        }
+        hipLaunchKernelGGL(k_mg_tail<T>, dim3(1), dim3(NT1), c->tail_lds, c->s, a);
+    }
     // Vcycle!(ml; l); the levels from c->tail_level down run in one workgroup.
     // pre_done: Jacobi! + increment! of level l were fused into the caller's
     // residual load.  then_pcg: a pcg! on level l follows, so its first
@@ -744,7 +768,7 @@ template <class T> struct Impl {
             a.nlev = c->nlev;
             for (int q = 0; q < MAXLEV; ++q) a.cit[q] = cit[q];
             a.halt = cur_halt;
-            hipLaunchKernelGGL(k_mg_tail<T>, dim3(1), dim3(NT1), c->tail_lds, c->s, a);
+            launch_tail(c, a, cit == c->cit_fcg);
         } else {
             if (rec) vcycle(c, l + 1, cit, false, true, true);
             if (cit == c->cit_fcg) pcg1(c, co, cit[l + 1]);

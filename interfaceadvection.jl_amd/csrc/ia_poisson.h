@@ -1726,7 +1726,7 @@ __host__ __device__ inline int fcg_coarse_its(long n, int l) {
 // 256 threads, 6.5 with 1024), else 256 (32³: 4.4 µs, against 4.7 with 512
 // and 4.5 with 128)
 inline int cg1_workgroup(long n) { return n > 100000 ? 512 : NT; }
-constexpr size_t TAIL_LDS_MAX = 152 * 1024;  // of the 160 KiB of LDS per CU
+constexpr size_t TAIL_LDS_MAX = 152 * 1024 + 512;  // of the 160 KiB of LDS per CU
 template <class T> struct TailLev {
     Grid g;
     const T *L, *Dg, *iD;
@@ -1820,7 +1820,7 @@ __device__ inline void scoord(const int n[3], int c, int q[3]) {
     SLOOP_OWN(S, __VA_ARGS__) \
     __syncthreads();
 
-template <int D, class T> __device__ void stail_increment(const SLev<T> &l) {
+template <int D, class T> __device__ __forceinline__ void stail_increment(const SLev<T> &l) {
     SLOOP(l, {
         l.r[c] = l.r[c] - smult<D>(l, l.e, c, q);
         l.x[c] = l.x[c] + l.e[c];
@@ -1834,7 +1834,7 @@ template <int D, class T> __device__ void stail_increment(const SLev<T> &l) {
 // global-memory kernels, term for term.  On exit x and r are written back,
 // past a barrier, so the caller may read any cell's x.
 constexpr int TAIL_KC = 4;  // 4096-cell levels over NT1 threads
-template <int D, class T> __device__ void stail_pcg(const SLev<T> &l, int it, double *sh, int &par) {
+template <int D, class T> __device__ __forceinline__ void stail_pcg(const SLev<T> &l, int it, double *sh, int &par) {
     int cc[TAIL_KC], q[TAIL_KC][3];
     bool on[TAIL_KC];
     T x[TAIL_KC], r[TAIL_KC], z[TAIL_KC], e[TAIL_KC], iD[TAIL_KC];
@@ -1925,7 +1925,7 @@ __device__ inline void wave_lds_order() {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-template <int D, class T> __device__ void stail_pcg_wave(const SLev<T> &l, int it) {
+template <int D, class T> __device__ __forceinline__ void stail_pcg_wave(const SLev<T> &l, int it) {
     const int c = threadIdx.x;
     const bool on = c < l.ncell;
     int q[3] = {0, 0, 0};
@@ -1981,26 +1981,28 @@ template <int D, class T> __device__ void stail_pcg_wave(const SLev<T> &l, int i
     }
 }
 // pcg! on a tail level; returns past a workgroup barrier
-template <int D, class T> __device__ void stail_solve(const SLev<T> &l, int it, double *sh, int &par) {
+template <int D, class T> __device__ __forceinline__ void stail_solve(const SLev<T> &l, int it, double *sh, int &par) {
     if (l.ncell <= 64) {
         if (threadIdx.x < 64) stail_pcg_wave<D>(l, it);
         __syncthreads();
-    } else {
-        stail_pcg<D>(l, it, sh, par);
+        return;
     }
+    stail_pcg<D>(l, it, sh, par);
 }
+// LDS values of a level of n cells: its arrays, with room to align the last one
+__device__ __host__ inline int tail_lev_words(int D, int n) { return (n * (D + 5) + 7) & ~3; }
 // LDS bytes the levels l0..nlev-1 need
 template <class T> inline size_t tail_lds_bytes(const Grid *gs, int l0, int nlev) {
     size_t b = 0;
     for (int l = l0; l < nlev; ++l) {
         size_t n = 1;
         for (int a = 0; a < gs[l].D; ++a) n *= (size_t)(gs[l].Ng[a] - 2);
-        b += n * (gs[l].D + 5) * sizeof(T);
+        b += tail_lev_words(gs[l].D, (int)n) * sizeof(T);
     }
     return b;
 }
 // the LDS view of tail level l (levels a.l0 .. l-1 are stored before it)
-template <class T> __device__ inline SLev<T> slev(const TailArgs<T> &a, int l, T *smem) {
+template <class T> __device__ __forceinline__ SLev<T> slev(const TailArgs<T> &a, int l, T *smem) {
     T *base = smem;
     for (int m = a.l0; m < l; ++m) base += (long)a.lv[m].n * (a.lv[m].g.D + 5);
     const TailLev<T> &G = a.lv[l];
@@ -2020,7 +2022,7 @@ template <class T> __device__ inline SLev<T> slev(const TailArgs<T> &a, int l, T
     s.z = base + 4L * s.ncell;
     return s;
 }
-template <int D, class T> __device__ void tail_run(const TailArgs<T> &a, T *smem, double *sh) {
+template <int D, class T> __device__ __forceinline__ void tail_run(const TailArgs<T> &a, T *smem, double *sh) {
     int par = 0;
     for (int l = a.l0; l < a.nlev; ++l) {
         const TailLev<T> &G = a.lv[l];
@@ -2055,10 +2057,12 @@ template <int D, class T> __device__ void tail_run(const TailArgs<T> &a, T *smem
             cs.x[c] = T(0);
         })
     }
-    // ascend: pcg!(l+1), prolongate!, increment!(l)
-    for (int l = last - 1; l >= a.l0; --l) {
-        SLev<T> f = slev(a, l, smem), cs = slev(a, l + 1, smem);
-        stail_solve<D>(cs, a.cit[l + 1], sh, par);
+    // ascend: pcg!(l), then prolongate! and increment! on the level above
+    for (int l = last;; --l) {
+        SLev<T> cs = slev(a, l, smem);
+        stail_solve<D>(cs, a.cit[l], sh, par);
+        if (l == a.l0) break;
+        SLev<T> f = slev(a, l - 1, smem);
         SLOOP(f, {
             int k0 = q[0] / 2, k1 = f.D > 1 ? q[1] / 2 : 0, k2 = f.D > 2 ? q[2] / 2 : 0;
             f.e[c] = cs.x[k0 + cs.n[0] * (k1 + cs.n[1] * k2)];
@@ -2066,13 +2070,480 @@ template <int D, class T> __device__ void tail_run(const TailArgs<T> &a, T *smem
         stail_increment<D>(f);
     }
     SLev<T> s = slev(a, a.l0, smem);
-    stail_solve<D>(s, a.cit[a.l0], sh, par);
     // the top level's solution back to global memory (interior)
     const TailLev<T> &G = a.lv[a.l0];
     SLOOP(s, {
         long I = (long)(q[0] + 1) + G.g.st[1] * (s.D > 1 ? q[1] + 1 : 0) + G.g.st[2] * (s.D > 2 ? q[2] + 1 : 0);
         G.x[I] = s.x[c];
     })
+}
+// ---------------------------------------------------------------------------
+// The tail in FP32 with the cells in columns: a thread owns C cells along the
+// last axis, so two of a cell's neighbours are mostly its own registers; the
+// face coefficients, iD, x and r of a solve stay in registers; ϵ goes through
+// LDS column by column, so a thread reads each of its four side neighbours'
+// columns in one access.  Levels whose columns fit 64 lanes are solved, and
+// everything below them done, by wavefront 0 alone without a barrier.  The
+// prolonged ϵ is formed at a cell's neighbours from the coarse x instead of
+// being stored first.
+//
+// The sums are exact to FP64 and rounded to FP32, so their order does not
+// show (a single wavefront's by two matrix products with ones, half of
+// wave_sum's latency); per cell the operations are tail_run's, term for term.
+//
+// What bounds an iteration is the chain of two sums, three barriers and two
+// divisions, 0.9 µs on 512 threads and more with more wavefronts, and on 4096
+// cells the arithmetic of one CU besides.  µs per iteration, k_mg_tail ->
+// here: 16^3 2.7 -> 1.7, 8^3 1.6 -> 0.86, 4^3 0.52 -> 0.35, 48x32 1.75 ->
+// 1.02, 96 cells 1.5 -> 0.39; a whole tail with the flexible CG's counts:
+// 16^3 273 -> 177, 48x32 245 -> 137, 64x64 364 -> 237 (with 6 iterations a
+// level 78 -> 52).
+// ---------------------------------------------------------------------------
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+// the sum over a fully active wavefront, in every lane: the first product adds lanes i, i+16, i+32, i+48, the lane
+// adds its four rows of the result, and the second product adds the four groups of rows
+__device__ inline double wave_sum_mm(double v) {
+    const f64x4 z = {0, 0, 0, 0};
+    f64x4 d = __builtin_amdgcn_mfma_f64_16x16x4f64(v, 1.0, z, 0, 0, 0);
+    d = __builtin_amdgcn_mfma_f64_16x16x4f64((d[0] + d[1]) + (d[2] + d[3]), 1.0, z, 0, 0, 0);
+    return d[0];
+}
+__device__ inline int small_div(int c, int n) { return (int)(((float)c + 0.5f) * (1.0f / (float)n)); }  // c < 2^16
+struct FLev {  // a level in LDS, interior cells x fastest; e: 2*ncell floats, columns of C cells
+    int n0, n1, n2, nl, nz, ncell;  // nl: cells across the columns, nz along them
+    bool p0, p1, pz;                // periodic: x, y (3D), the columns' axis
+    float *L, *iD, *x, *r, *e;
+};
+template <int D> __device__ __forceinline__ FLev flev(const TailArgs<float> &a, int l, float *smem) {
+    float *base = smem;
+    for (int m = a.l0; m < l; ++m) base += tail_lev_words(D, a.lv[m].n);
+    const Grid &g = a.lv[l].g;
+    FLev s;
+    s.n0 = g.Ng[0] - 2;
+    s.n1 = g.Ng[1] - 2;
+    s.n2 = D > 2 ? g.Ng[2] - 2 : 1;
+    s.nl = D > 2 ? s.n0 * s.n1 : s.n0;
+    s.nz = D > 2 ? s.n2 : s.n1;
+    s.ncell = a.lv[l].n;
+    s.p0 = g.per[0];
+    s.p1 = D > 2 && g.per[1];
+    s.pz = g.per[D - 1];
+    s.L = base;
+    s.iD = base + D * s.ncell;
+    s.x = s.iD + s.ncell;
+    s.r = s.x + s.ncell;
+    s.e = base + (((D + 3) * s.ncell + 3) & ~3);  // 16-byte aligned
+    return s;
+}
+// cells per column of a level solved by wavefront 0, or 0: the level is the workgroup's
+__device__ __host__ inline int tail_wave_cols(int nl, int nz, int CM) {
+    for (int C = 1; C <= CM; C *= 2)
+        if (nl * ((nz + C - 1) / C) <= 64 && ((nz + C - 1) / C) * C <= 2 * nz) return C;
+    return 0;
+}
+template <int D, int C, bool WAVE> struct FCols {
+    int cnt, col, z0, base, x0, y0;   // cells, lateral index, first of them, its cell index
+    int e0, xm, xp, ym, yp, elo, ehi; // place in e, offsets of the side columns, places of the cells at the ends
+    float iD[C], dg[C], lx[C], lxp[C], ly[C], lyp[C], lz[C + 1];
+    __device__ __forceinline__ void init(const FLev &l) {
+        const int tid = threadIdx.x, chunk = small_div(tid, l.nl);
+        col = tid - chunk * l.nl;
+        z0 = chunk * C;
+        cnt = max(0, min(C, l.nz - z0));
+        base = col + l.nl * z0;
+        y0 = D > 2 ? small_div(col, l.n0) : 0;
+        x0 = col - y0 * l.n0;
+        e0 = tid * C;
+        // behind a wall the cell's own column, where L is 0
+        xm = (x0 > 0 ? -1 : l.p0 ? l.n0 - 1 : 0) * C;
+        xp = (x0 < l.n0 - 1 ? 1 : l.p0 ? 1 - l.n0 : 0) * C;
+        ym = D > 2 ? (y0 > 0 ? -l.n0 : l.p1 ? (l.n1 - 1) * l.n0 : 0) * C : 0;
+        yp = D > 2 ? (y0 < l.n1 - 1 ? l.n0 : l.p1 ? (1 - l.n1) * l.n0 : 0) * C : 0;
+        const int ztop = l.nz - 1;
+        elo = z0 > 0 ? e0 - l.nl * C + C - 1 : l.pz ? ((ztop / C) * l.nl + col) * C + ztop % C : e0;
+        ehi = z0 + cnt < l.nz ? e0 + l.nl * C : l.pz ? col * C : e0;
+#pragma unroll
+        for (int k = 0; k <= C; ++k) {
+            lz[k] = 0.f;
+            if (cnt > 0 && k <= cnt) {
+                const bool top = k == cnt && z0 + cnt == l.nz;
+                if (!top) lz[k] = l.L[(D - 1) * l.ncell + base + k * l.nl];
+                else if (l.pz) lz[k] = l.L[(D - 1) * l.ncell + col];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            iD[k] = dg[k] = lx[k] = lxp[k] = ly[k] = lyp[k] = 0.f;
+            if (k < cnt) {
+                const int c = base + k * l.nl;
+                iD[k] = l.iD[c];
+                lx[k] = l.L[c];
+                if (xp) lxp[k] = l.L[c + xp / C];
+                dg[k] -= (lx[k] + lxp[k]);
+                if (D > 2) {
+                    ly[k] = l.L[l.ncell + c];
+                    if (yp) lyp[k] = l.L[l.ncell + c + yp / C];
+                    dg[k] -= (ly[k] + lyp[k]);
+                }
+                dg[k] -= (lz[k] + lz[k + 1]);
+            }
+        }
+    }
+    __device__ __forceinline__ static void rd(const float *p, float v[C]) {
+        if constexpr (C == 1) v[0] = p[0];
+        else if constexpr (C == 2) {
+            float2 q = *(const float2 *)p;
+            v[0] = q.x;
+            v[1] = q.y;
+        } else {
+#pragma unroll
+            for (int j = 0; j < C; j += 4) {
+                float4 q = *(const float4 *)(p + j);
+                v[j] = q.x;
+                v[j + 1] = q.y;
+                v[j + 2] = q.z;
+                v[j + 3] = q.w;
+            }
+        }
+    }
+    __device__ __forceinline__ static void wr(float *p, const float v[C]) {
+        if constexpr (C == 1) p[0] = v[0];
+        else if constexpr (C == 2) *(float2 *)p = make_float2(v[0], v[1]);
+        else {
+#pragma unroll
+            for (int j = 0; j < C; j += 4) *(float4 *)(p + j) = make_float4(v[j], v[j + 1], v[j + 2], v[j + 3]);
+        }
+    }
+    // mult() given the side columns, the cells beyond the ends and the own cells
+    __device__ __forceinline__ void mult(const float e[C], const float a[C], const float b[C], const float c[C],
+                                         const float d[C], float lo, float hi, float z[C]) const {
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            float up = hi;
+            if (k + 1 < C) {
+                float un = e[k + 1 < C ? k + 1 : k];
+                up = k + 1 < cnt ? un : hi;
+            }
+            float sl = a[k] * lx[k], su = b[k] * lxp[k];
+            if (D > 2) {
+                sl += c[k] * ly[k];
+                su += d[k] * lyp[k];
+            }
+            sl += (k > 0 ? e[k > 0 ? k - 1 : 0] : lo) * lz[k];
+            su += up * lz[k + 1];
+            z[k] = (e[k] * dg[k] + sl) + su;
+        }
+    }
+    // A·ϵ from LDS (cells past the column's end give finite values that nothing reads)
+    __device__ __forceinline__ void mult_lds(const float *ev, const float e[C], float z[C]) const {
+        float a[C], b[C], c[C], d[C];
+        rd(ev + e0 + xm, a);
+        rd(ev + e0 + xp, b);
+        if (D > 2) {
+            rd(ev + e0 + ym, c);
+            rd(ev + e0 + yp, d);
+        }
+        mult(e, a, b, c, d, ev[elo], ev[ehi], z);
+    }
+};
+template <bool WAVE> __device__ __forceinline__ void fsync() {
+    if (WAVE) wave_lds_order();
+    else __syncthreads();
+}
+// one level of the way down: Jacobi! and increment! on r (in registers), r and x to LDS
+template <int D, int C, bool WAVE>
+__device__ __forceinline__ void f_down(const FLev &l, const FCols<D, C, WAVE> &q, float r[C]) {
+    float e[C], z[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) e[k] = k < q.cnt ? r[k] * q.iD[k] : 0.f;
+    if (q.cnt > 0) q.wr(l.e + q.e0, e);
+    fsync<WAVE>();
+    if (q.cnt > 0) {
+        q.mult_lds(l.e, e, z);
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+            if (k < q.cnt) {
+                const int c = q.base + k * l.nl;
+                l.r[c] = r[k] - z[k];
+                l.x[c] = 0.f + e[k];
+            }
+    }
+    fsync<WAVE>();
+}
+// restrict!: the column's r from the finer level's
+template <int D, int C, bool WAVE>
+__device__ __forceinline__ void f_restrict(const FLev &f, const FCols<D, C, WAVE> &q, float r[C]) {
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        r[k] = 0.f;
+        if (k < q.cnt) {
+            float s = 0;
+            if (D > 2) {
+                const float *p = f.r + 2 * q.x0 + f.n0 * (2 * q.y0 + f.n1 * (2 * (q.z0 + k)));
+                const int s1 = f.n0, s2 = f.n0 * f.n1;
+                s += p[0];
+                s += p[1];
+                s += p[s1];
+                s += p[s1 + 1];
+                s += p[s2];
+                s += p[s2 + 1];
+                s += p[s2 + s1];
+                s += p[s2 + s1 + 1];
+            } else {
+                const float *p = f.r + 2 * q.x0 + f.n0 * (2 * (q.z0 + k));
+                s += p[0];
+                s += p[1];
+                s += p[f.n0];
+                s += p[f.n0 + 1];
+            }
+            r[k] = s;
+        }
+    }
+}
+// one level of the way up: with `prolong` prolongate! and increment! of the coarser x on r and x from LDS, else r given
+// and x = 0; then pcg!, and x to LDS
+template <int D, int C, bool WAVE, int NTF>
+__device__ __forceinline__ void f_up(const FLev &l, const FCols<D, C, WAVE> &q, const FLev &co, bool prolong, float r[C],
+                                     int it, double *sh, int &par) {
+    float x[C], e[C], z[C];
+    if (prolong) {
+        // coarse x at the cell's and its neighbours' parents
+        const float *xc = co.x;
+        const int m0 = co.n0, m01 = D > 2 ? co.n0 * co.n1 : co.n0;
+        auto at = [&](int cx, int cy, int cz) { return xc[(cx >> 1) + (D > 2 ? m0 * (cy >> 1) : 0) + m01 * (cz >> 1)]; };
+        float a[C], b[C], c[C], d[C];
+        const int wx = q.xm / C, ex = q.xp / C, wy = D > 2 ? small_div(abs(q.ym) / C, l.n0) * (q.ym < 0 ? -1 : 1) : 0,
+                  ey = D > 2 ? small_div(abs(q.yp) / C, l.n0) * (q.yp < 0 ? -1 : 1) : 0;
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+            x[k] = r[k] = e[k] = a[k] = b[k] = c[k] = d[k] = 0.f;
+            if (k < q.cnt) {
+                const int cz = q.z0 + k, cc = q.base + k * l.nl;
+                x[k] = l.x[cc];
+                r[k] = l.r[cc];
+                e[k] = at(q.x0, q.y0, cz);
+                a[k] = at(q.x0 + wx, q.y0, cz);
+                b[k] = at(q.x0 + ex, q.y0, cz);
+                if (D > 2) {
+                    c[k] = at(q.x0, q.y0 + wy, cz);
+                    d[k] = at(q.x0, q.y0 + ey, cz);
+                }
+            }
+        }
+        float lo = 0, hi = 0;
+        if (q.cnt > 0) {
+            lo = at(q.x0, q.y0, q.z0 > 0 ? q.z0 - 1 : l.pz ? l.nz - 1 : 0);
+            hi = at(q.x0, q.y0, q.z0 + q.cnt < l.nz ? q.z0 + q.cnt : l.pz ? 0 : l.nz - 1);
+        }
+        q.mult(e, a, b, c, d, lo, hi, z);
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+            if (k < q.cnt) {
+                r[k] = r[k] - z[k];
+                x[k] = x[k] + e[k];
+            }
+    } else {
+#pragma unroll
+        for (int k = 0; k < C; ++k) x[k] = 0.f;
+    }
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int nw = (l.nl * ((l.nz + C - 1) / C) + 63) >> 6;  // wavefronts with cells
+    // the workgroup's sum (alternating between the halves of sh as bsum1024), or the wavefront's
+    auto sum = [&](double v) -> double {
+        if (WAVE) return wave_sum_mm(v);
+        constexpr int NW = NTF / 64;
+        double *h = sh + par * 16;
+        par ^= 1;
+        if (wv < nw) v = NW <= 4 ? wave_sum_mm(v) : wave_sum(v);  // the matrix products' rate is too low for more
+        if (lane == 0) h[wv] = wv < nw ? v : 0.0;
+        __syncthreads();
+        double t[NW];
+#pragma unroll
+        for (int j = 0; j < NW; ++j) t[j] = h[j];
+#pragma unroll
+        for (int m = NW / 2; m > 0; m /= 2)
+#pragma unroll
+            for (int j = 0; j < m; ++j) t[j] += t[j + m];
+        return t[0];
+    };
+    double v = 0;
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        e[k] = z[k] = 0.f;
+        if (k < q.cnt) {
+            e[k] = z[k] = r[k] * q.iD[k];
+            v = __builtin_fma((double)r[k], (double)z[k], v);
+        }
+    }
+    if (q.cnt > 0) q.wr(l.e + q.e0, e);
+    float rho = (float)sum(v);
+    if (!(fabs(rho) < 10 * eps_of<float>())) {
+        if (WAVE) wave_lds_order();
+        for (int i = 1; i <= it; ++i) {
+            v = 0;
+            if (q.cnt > 0) {
+                q.mult_lds(l.e, e, z);
+#pragma unroll
+                for (int k = 0; k < C; ++k)
+                    if (k < q.cnt) v = __builtin_fma((double)z[k], (double)e[k], v);
+            }
+            const float alpha = rho / (float)sum(v);
+            const bool last = i == it || fabs((double)alpha) < 1e-2;
+            v = 0;
+#pragma unroll
+            for (int k = 0; k < C; ++k)
+                if (k < q.cnt) {
+                    x[k] += alpha * e[k];
+                    r[k] = r[k] - alpha * z[k];
+                    z[k] = r[k] * q.iD[k];
+                    v = __builtin_fma((double)r[k], (double)z[k], v);
+                }
+            if (last) break;
+            const float rho2 = (float)sum(v);
+            if (fabs(rho2) < 10 * eps_of<float>()) break;
+            const float beta = rho2 / rho;
+            if (WAVE) wave_lds_order();
+#pragma unroll
+            for (int k = 0; k < C; ++k)
+                if (k < q.cnt) e[k] = beta * e[k] + z[k];
+            if (q.cnt > 0) q.wr(l.e + q.e0, e);
+            fsync<WAVE>();
+            rho = rho2;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < C; ++k)
+        if (k < q.cnt) l.x[q.base + k * l.nl] = x[k];
+    fsync<WAVE>();
+}
+// a level by wavefront 0: up (o the coarser level), or down (o the finer level unless F_TOP; F_BOTTOM: solved at once)
+enum { F_UP = 1, F_TOP = 2, F_BOTTOM = 4 };
+template <int D, int C, int NTF>
+__device__ __forceinline__ void f_wave(const FLev &l, const FLev &o, int mode, int it) {
+    FCols<D, C, true> q;
+    int par = 0;
+    float r[C];
+    q.init(l);
+    if (mode & F_UP) {
+        f_up<D, C, true, NTF>(l, q, o, true, r, it, nullptr, par);
+        return;
+    }
+    if (mode & F_TOP) {
+#pragma unroll
+        for (int k = 0; k < C; ++k) r[k] = k < q.cnt ? l.r[q.base + k * l.nl] : 0.f;
+    } else {
+        f_restrict(o, q, r);
+    }
+    if (mode & F_BOTTOM) f_up<D, C, true, NTF>(l, q, o, false, r, it, nullptr, par);
+    else f_down(l, q, r);
+}
+template <int D, int NTF, int CM>
+__device__ __forceinline__ void f_wave_any(const FLev &l, const FLev &o, int mode, int it) {
+    const int C = tail_wave_cols(l.nl, l.nz, CM);
+    if (C == 1) f_wave<D, 1, NTF>(l, o, mode, it);
+    else if (C == 2) f_wave<D, 2, NTF>(l, o, mode, it);
+    else if (C == 4) f_wave<D, 4, NTF>(l, o, mode, it);
+    else if constexpr (CM > 4) f_wave<D, CM, NTF>(l, o, mode, it);
+}
+// whether every level's columns fit the workgroup or wavefront 0
+inline bool tail_cols_fit(const Grid *gs, int l0, int nlev, int ntf, int cm) {
+    for (int l = l0; l < nlev; ++l) {
+        const Grid &g = gs[l];
+        const int n0 = g.Ng[0] - 2, nl = g.D > 2 ? n0 * (g.Ng[1] - 2) : n0, nz = g.Ng[g.D - 1] - 2;
+        if (tail_wave_cols(nl, nz, cm)) continue;
+        const int ch = (nz + cm - 1) / cm;
+        if (nl * ch > ntf || ch * cm > 2 * nz) return false;
+    }
+    return true;
+}
+template <int D, int NTF, int CM> __device__ __forceinline__ void ftail_run(const TailArgs<float> &a, float *smem, double *sh) {
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    // constants of every level and the top level's r: 64 cells of one level a wavefront and turn
+    {
+        int t = wv;
+        for (int l = a.l0; l < a.nlev; ++l) {
+            const TailLev<float> &G = a.lv[l];
+            const FLev s = flev<D>(a, l, smem);
+            const int nt = (s.ncell + 63) >> 6;
+#pragma unroll 4
+            for (; t < nt; t += NTF / 64) {
+                const int c = t * 64 + lane;
+                if (c < s.ncell) {
+                    const int r1 = small_div(c, s.n0), x = c - r1 * s.n0, z = D > 2 ? small_div(r1, s.n1) : 0, y = r1 - z * s.n1;
+                    const long I = (long)(x + 1) + G.g.st[1] * (y + 1) + (D > 2 ? G.g.st[2] * (z + 1) : 0);
+#pragma unroll
+                    for (int d = 0; d < D; ++d) s.L[d * s.ncell + c] = G.L[d * G.g.ns + I];
+                    s.iD[c] = G.iD[I];
+                    if (l == a.l0) s.r[c] = G.r[I];
+                }
+            }
+            t -= nt;
+        }
+    }
+    __syncthreads();
+    const int last = a.nlev - 1;
+    int par = 0, lw = a.l0;  // lw: the first level of wavefront 0
+    for (; lw <= last; ++lw) {
+        const FLev s = flev<D>(a, lw, smem);
+        if (tail_wave_cols(s.nl, s.nz, CM)) break;
+    }
+    // down
+    for (int l = a.l0; l < lw; ++l) {
+        const FLev s = flev<D>(a, l, smem);
+        FCols<D, CM, false> q;
+        float r[CM];
+        q.init(s);
+        if (l == a.l0) {
+#pragma unroll
+            for (int k = 0; k < CM; ++k) r[k] = k < q.cnt ? s.r[q.base + k * s.nl] : 0.f;
+        } else {
+            const FLev f = flev<D>(a, l - 1, smem);
+            f_restrict(f, q, r);
+        }
+        if (l == last) f_up<D, CM, false, NTF>(s, q, s, false, r, a.cit[l], sh, par);
+        else f_down(s, q, r);
+    }
+    // the levels of wavefront 0, down and up
+    if (lw <= last) {
+        if (wv == 0) {
+            for (int l = lw; l <= last; ++l) {
+                const FLev s = flev<D>(a, l, smem), f = flev<D>(a, l > a.l0 ? l - 1 : l, smem);
+                f_wave_any<D, NTF, CM>(s, f, (l == a.l0 ? F_TOP : 0) | (l == last ? F_BOTTOM : 0), a.cit[l]);
+            }
+            for (int l = last - 1; l >= lw; --l) {
+                const FLev s = flev<D>(a, l, smem), co = flev<D>(a, l + 1, smem);
+                f_wave_any<D, NTF, CM>(s, co, F_UP, a.cit[l]);
+            }
+        }
+        __syncthreads();
+    }
+    // up
+    for (int l = min(lw, last) - 1; l >= a.l0; --l) {
+        const FLev s = flev<D>(a, l, smem), co = flev<D>(a, l + 1, smem);
+        FCols<D, CM, false> q;
+        float r[CM];
+        q.init(s);
+        f_up<D, CM, false, NTF>(s, q, co, true, r, a.cit[l], sh, par);
+    }
+    // the top level's solution back to global memory (interior)
+    const TailLev<float> &G = a.lv[a.l0];
+    const FLev s = flev<D>(a, a.l0, smem);
+    for (int c = tid; c < s.ncell; c += NTF) {
+        const int r1 = small_div(c, s.n0), x = c - r1 * s.n0, z = D > 2 ? small_div(r1, s.n1) : 0, y = r1 - z * s.n1;
+        G.x[(long)(x + 1) + G.g.st[1] * (y + 1) + (D > 2 ? G.g.st[2] * (z + 1) : 0)] = s.x[c];
+    }
+}
+// NTF threads of at most CM cells each.  512 threads of 4 cells where they hold the levels (a barrier costs by the
+// wavefront: 48x32 1.02 µs an iteration, 1.3 on 1024 threads); else 512 of 8 (16^3 1.67, 1024 of 4 1.76) if the
+// iterations are many, as its setup takes 4 µs more, else 1024 of 4.
+template <int NTF, int CM> __global__ void __launch_bounds__(NTF) k_mg_tail_cols(TailArgs<float> a) {
+    HALT_IF(a)
+    __shared__ double sh[32];
+    if (threadIdx.x < 32) sh[threadIdx.x] = 0.0;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    float *smem = (float *)smem_raw;
+    if (a.lv[a.l0].g.D == 3) ftail_run<3, NTF, CM>(a, smem, sh);
+    else ftail_run<2, NTF, CM>(a, smem, sh);
 }
 template <class T> __global__ void __launch_bounds__(NT1) k_mg_tail(TailArgs<T> a) {
     HALT_IF(a)
