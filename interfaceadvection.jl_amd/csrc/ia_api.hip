@@ -223,6 +223,7 @@ CTiling ctiling(const Grid &g, bool narrow = false) {
     CTiling t;
     int n0 = g.Ng[0] - 2, n1 = g.D > 1 ? g.Ng[1] - 2 : 1, n2 = g.D > 2 ? g.Ng[2] - 2 : 1;
     t.nx = TX;
+    t.rev = 0;
     t.nt[0] = (n0 + TX - 1) / TX;
     t.nt[1] = (n1 + TY - 1) / TY;
     long base = (long)t.nt[0] * t.nt[1];
@@ -595,11 +596,12 @@ template <class T> struct Impl {
         LAUNCHCHK(c);
         return IA_OK;
     }
-    static LevV<T> view(Level &l) {
+    static LevV<T> view(Level &l, int rev = 0) {
         LevV<T> v;
         v.halt = cur_halt;
         v.g = l.g;
         v.t = l.ct;
+        v.t.rev = rev;
         v.L = P<T>(l.L);
         v.Dg = P<T>(l.Dg);
         v.iD = P<T>(l.iD);
@@ -716,6 +718,7 @@ template <class T> struct Impl {
             if (l.ct.zb == 1) {
                 LevV<T> vw = v;
                 vw.t = l.wt;
+                vw.t.rev = 0;
                 long nin = q == 1 ? l.ct.nblk : l.wt.nblk;
                 dim3 W((unsigned)l.wt.nblk);
                 if (l.g.D == 2)
@@ -733,7 +736,9 @@ template <class T> struct Impl {
                     hipLaunchKernelGGL((k_cg1_step1<3, T>), W, dim3(NT), 0, c->s, vw, b, c->pst, q, it, pin, nin,
                                        pout);
             } else {
-                hipLaunchKernelGGL(k_cg1_step<T>, B, dim3(NT), 0, c->s, v, b, c->pst, q, it, pin, pout);
+                LevV<T> vr = v;
+                vr.t.rev = q & 1;
+                hipLaunchKernelGGL(k_cg1_step<T>, B, dim3(NT), 0, c->s, vr, b, c->pst, q, it, pin, pout);
             }
         }
         if (pc >= 0) prof_end(c, pc, it);
@@ -741,7 +746,7 @@ template <class T> struct Impl {
     // e_done: Jacobi!'s ϵ = r·iD on level l was written by the restrict! that
     // produced its r, so only increment! remains.
     static void vcycle(ia_ctx *c, int l, const int *cit, bool pre_done = false, bool then_pcg = false,
-                       bool e_done = false) {
+                       bool e_done = false, int rev = 0) {
         Level &fl = c->lev[l], &co = c->lev[l + 1];
         if (!pre_done) {
             if (e_done) increment(c, fl);
@@ -777,7 +782,7 @@ template <class T> struct Impl {
         if (then_pcg) {
             bool f0 = l == 0;
             if (f0) prof_begin(c, IA_PROF_PROLONG_INC);
-            hipLaunchKernelGGL(k_mg_prolong_inc_init<T>, cb(fl), dim3(NT), 0, c->s, view(fl), co.g, P<T>(co.x),
+            hipLaunchKernelGGL(k_mg_prolong_inc_init<T>, cb(fl), dim3(NT), 0, c->s, view(fl, rev), co.g, P<T>(co.x),
                                pp(c, PP_A));
             if (f0) prof_end(c, IA_PROF_PROLONG_INC);
         } else {
@@ -898,11 +903,12 @@ template <class T> struct Impl {
         return IA_OK;
     }
     // FP64 flexible CG preconditioned by the FP32 V-cycle (REFINED / LEARNED)
-    static FcgV<T> fview(ia_ctx *c, int par = 0) {
+    static FcgV<T> fview(ia_ctx *c, int par = 0, int rev = 0) {
         Level &l0 = c->lev[0];
         FcgV<T> f;
         f.g = l0.g;
         f.t = l0.ct;
+        f.t.rev = rev;
         f.L = P<T>(l0.L);
         f.iD = P<T>(l0.iD);
         f.z = c->z64;
@@ -930,17 +936,18 @@ template <class T> struct Impl {
     // buffer `rbuf` (the true residual after a restart, else the last update).
     static void fcg_body(ia_ctx *c, int first, int par, int rbuf) {
         Level &l0 = c->lev[0];
-        FcgV<T> f = fview(c, par);
+        // the finest level's five kernels alternate their direction (par alternates too, and so does the next one)
+        FcgV<T> f = fview(c, par, par), fr = fview(c, par, !par);
         dim3 B = cb(l0);
         prof_begin(c, IA_PROF_LOAD_INC);
-        hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0), pp(c, rbuf));
+        hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0, par), pp(c, rbuf));
         prof_end(c, IA_PROF_LOAD_INC);
         if (c->fine_cheb) {
-            vcycle(c, 0, c->cit_fcg, true, true);
+            vcycle(c, 0, c->cit_fcg, true, true, false, !par);
             double c0, ca, cb;
             cheb2_coeffs(c0, ca, cb);
             prof_begin(c, IA_PROF_PCG_LAST);
-            hipLaunchKernelGGL(k_cheb2_dots<T>, B, dim3(NT), 0, c->s, view(l0), f, (T)c0, (T)ca, (T)cb, pp(c, PP_FD),
+            hipLaunchKernelGGL(k_cheb2_dots<T>, B, dim3(NT), 0, c->s, view(l0, par), f, (T)c0, (T)ca, (T)cb, pp(c, PP_FD),
                                first);
             prof_end(c, IA_PROF_PCG_LAST);
         } else if (c->smooth_it > 0) {
@@ -951,7 +958,7 @@ template <class T> struct Impl {
             hipLaunchKernelGGL(k_fcg_dots<T>, B, dim3(NT), 0, c->s, f, pp(c, PP_FD), first);
         }
         prof_begin(c, IA_PROF_FCG_AP);
-        hipLaunchKernelGGL(k_fcg_Ap<T>, B, dim3(NT), 0, c->s, f, pp(c, PP_FD), pp(c, PP_FAP), first);
+        hipLaunchKernelGGL(k_fcg_Ap<T>, B, dim3(NT), 0, c->s, fr, pp(c, PP_FD), pp(c, PP_FAP), first);
         prof_end(c, IA_PROF_FCG_AP);
         prof_begin(c, IA_PROF_FCG_UPDATE);
         hipLaunchKernelGGL(k_fcg_update<T>, B, dim3(NT), 0, c->s, f, pp(c, PP_FAP), pp(c, PP_FU));

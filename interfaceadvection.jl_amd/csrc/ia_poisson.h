@@ -23,9 +23,16 @@ struct CTiling {
     int zb;
     long nblk;
     int nx;
+    int rev;  // 1: the workgroups take the tiles in the opposite order (rev_block)
 };
+// The workgroup's place in the traversal: kernels that follow one another on
+// the finest level run through it in alternating directions, so that each
+// starts on what the previous one touched last (the part of it that the
+// 256 MB memory-side cache still holds).  Partial sums are stored by this
+// number, so a sum's order does not depend on the direction.
+__device__ inline long rev_block(const CTiling &t) { return t.rev ? t.nblk - 1 - (long)blockIdx.x : (long)blockIdx.x; }
 __device__ inline bool thread_col(const Grid &g, const CTiling &t, int p[3], int &zlo, int &zhi) {
-    long b = swizzle_block((long)blockIdx.x, t.nblk);
+    long b = swizzle_block(rev_block(t), t.nblk);
     long bx = b % t.nt[0];
     long r = b / t.nt[0];
     long by = r % t.nt[1];
@@ -80,9 +87,9 @@ __device__ inline double block_total(const double *part, long n, int K = 1, int 
     __syncthreads();  // before another block_total of this kernel rewrites sht
     return s;
 }
-__device__ inline void block_partial(double v, double *part, int K = 1, int k = 0) {
+__device__ inline void block_partial(double v, const CTiling &t, double *part, int K = 1, int k = 0) {
     double s = block_sum(v);
-    if (threadIdx.x == 0) part[K * blockIdx.x + k] = s;
+    if (threadIdx.x == 0) part[K * rev_block(t) + k] = s;
 }
 
 template <class T> struct LevV {
@@ -266,7 +273,7 @@ __device__ inline int per_img(const Grid &g, int a, int q) {
 template <class V, class R, class LF, class CF, class PF, class BF>
 __device__ inline void tiled7(const Grid &g, const CTiling &t, LF load, CF comb, PF pre, BF body) {
     __shared__ V tile[2][TY + 2][TX + 2];
-    long b = swizzle_block((long)blockIdx.x, t.nblk);
+    long b = swizzle_block(rev_block(t), t.nblk);
     long bx = b % t.nt[0], rr = b / t.nt[0];
     long by = rr % t.nt[1], bz = rr / t.nt[1];
     int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
@@ -445,7 +452,7 @@ __global__ void __launch_bounds__(NT) k_mg_resid(LevV<T> l, double *part) {
         l.r[I] = rr;
         v += (double)rr;
     })
-    block_partial(v, part);
+    block_partial(v, l.t, part);
 }
 // residual! part 2: r -= mean when |mean| > 2eps (sub), fused with partial r·r
 template <class T>
@@ -466,7 +473,7 @@ __global__ void __launch_bounds__(NT) k_mg_center_l2(LevV<T> l, const double *pa
         }
         v += (double)rr * (double)rr;
     })
-    block_partial(v, part);
+    block_partial(v, l.t, part);
 }
 // Jacobi!: ϵ = r·iD
 template <class T>
@@ -616,7 +623,7 @@ __global__ void __launch_bounds__(NT) k_mg_prolong_inc_init(LevV<T> l, Grid gc, 
     HALT_IF(l)
     double v = 0;
     DISPATCH_D(l.g, prolong_inc_init_d<D>(l, gc, xc, v);)
-    block_partial(v, partA);
+    block_partial(v, l.t, partA);
 }
 // pcg! (WaterLily):  z = ϵ = r·iD ; partial r·z  (-> ρ₀)
 template <class T>
@@ -629,7 +636,7 @@ __global__ void __launch_bounds__(NT) k_pcg_init(LevV<T> l, double *partA) {
         l.e[I] = zz;
         v += (double)l.r[I] * (double)zz;
     })
-    block_partial(v, partA);
+    block_partial(v, l.t, partA);
 }
 template <int D, class T> __device__ inline void pcg_Ae_d(const LevV<T> &l, double &v) {
     const T *__restrict__ e = l.e;
@@ -672,7 +679,7 @@ __global__ void __launch_bounds__(NT) k_pcg_Ae(LevV<T> l, PcgState *S, int sin, 
     if (st.done) return;
     double v = 0;
     DISPATCH_D(l.g, pcg_Ae_d<D>(l, v);)
-    block_partial(v, partB);
+    block_partial(v, l.t, partB);
 }
 // α = ρ/(z·ϵ); x += αϵ; r -= αz; z = r·iD; partial r·z; stop when i == itmax or |α| < 1e-2
 template <class T>
@@ -708,7 +715,7 @@ __global__ void __launch_bounds__(NT) k_pcg_update(LevV<T> l, PcgState *S, int s
                      v += (double)rr * (double)zz;
                  });
     }
-    block_partial(v, partC);
+    block_partial(v, l.t, partC);
 }
 // k_pcg_eps fused with the next k_pcg_Ae: β from ρ₂ = r·z, then ϵ' = βϵ + z
 // formed on the fly at the cell and its neighbours, z' = Aϵ'; ϵ' and z' go
@@ -752,7 +759,7 @@ __global__ void __launch_bounds__(NT) k_pcg_epsAe(LevV<T> l, T *e2, T *z2, PcgSt
     if (!go) return;
     double v = 0;
     DISPATCH_D(l.g, eps_ae_d<D>(l, beta, e2, z2, v);)
-    block_partial(v, partB);
+    block_partial(v, l.t, partB);
 }
 // ρ₂ = r·z; exit when stop or |ρ₂| < 10eps; β = ρ₂/ρ; ϵ = βϵ + z
 template <class T>
@@ -824,8 +831,8 @@ __global__ void __launch_bounds__(NT) k_cg1_init(LevV<T> l, T *w, PcgState *S, d
                      d += (double)st.c * (double)ww;
                  });
     })
-    block_partial(g, part, 2, 0);
-    block_partial(d, part, 2, 1);
+    block_partial(g, l.t, part, 2, 0);
+    block_partial(d, l.t, part, 2, 1);
 }
 template <class T>
 __global__ void __launch_bounds__(NT) k_cg1_step(LevV<T> l, Cg1V<T> b, PcgState *S, int q, int it,
@@ -911,8 +918,8 @@ __global__ void __launch_bounds__(NT) k_cg1_step(LevV<T> l, Cg1V<T> b, PcgState 
                 g += (double)rr * (double)c;
                 d += (double)c * (double)ww;
             });
-        block_partial(g, pout, 2, 0);
-        block_partial(d, pout, 2, 1);
+        block_partial(g, l.t, pout, 2, 0);
+        block_partial(d, l.t, pout, 2, 1);
         return;
     }
     DISPATCH_D(l.g, {
@@ -933,8 +940,8 @@ __global__ void __launch_bounds__(NT) k_cg1_step(LevV<T> l, Cg1V<T> b, PcgState 
                      d += (double)sv.c * (double)ww;
                  });
     })
-    block_partial(g, pout, 2, 0);
-    block_partial(d, pout, 2, 1);
+    block_partial(g, l.t, pout, 2, 0);
+    block_partial(d, l.t, pout, 2, 1);
 }
 
 // two block sums in one pass (same per-thread order and tree as two calls of
@@ -1134,7 +1141,7 @@ template <class T>
 __global__ void __launch_bounds__(NT) k_ps_Ae(LevV<T> l, double *partB) {
     double v = 0;
     DISPATCH_D(l.g, pcg_Ae_d<D>(l, v);)
-    block_partial(v, partB);
+    block_partial(v, l.t, partB);
 }
 // α = ρ/(z·ϵ); x += αϵ; r -= αz; z = r·iD; partials r·z and r·r
 template <class T>
@@ -1151,8 +1158,8 @@ __global__ void __launch_bounds__(NT) k_ps_update(LevV<T> l, const double *rho, 
         vz += (double)rr * (double)zz;
         vr += (double)rr * (double)rr;
     })
-    block_partial(vz, partC, 2, 0);
-    block_partial(vr, partC, 2, 1);
+    block_partial(vz, l.t, partC, 2, 0);
+    block_partial(vr, l.t, partC, 2, 1);
 }
 // ρ₂ = r·z, β = ρ₂/ρ, ϵ = βϵ + z, ρ ← ρ₂ (into the other slot)
 template <class T>
@@ -1283,7 +1290,7 @@ __global__ void __launch_bounds__(NT) k_fcg_init(FcgV<T> f, const T *u, const T 
         f.x[I] = (double)pT[I] * dtw;
         v += s;
     })
-    block_partial(v, part);
+    block_partial(v, f.t, part);
 }
 // z -= mean(z) ; partial ‖z‖²
 template <class T>
@@ -1295,7 +1302,7 @@ __global__ void __launch_bounds__(NT) k_fcg_center_z(FcgV<T> f, const double *pa
         f.z[I] = q;
         v += q * q;
     })
-    block_partial(v, part);
+    block_partial(v, f.t, part);
 }
 // r = z - A x ; partial Σr
 template <class T>
@@ -1321,7 +1328,7 @@ __global__ void __launch_bounds__(NT) k_fcg_resid(FcgV<T> f, double *part) {
                 r[I] = rr;
                 v += rr;
             });
-        block_partial(v, part);
+        block_partial(v, f.t, part);
         return;
     }
     COL_LOOP(f, {
@@ -1329,7 +1336,7 @@ __global__ void __launch_bounds__(NT) k_fcg_resid(FcgV<T> f, double *part) {
         f.r[I] = rr;
         v += rr;
     })
-    block_partial(v, part);
+    block_partial(v, f.t, part);
 }
 // r -= mean(r) ; partial ‖r‖²
 template <class T>
@@ -1341,7 +1348,7 @@ __global__ void __launch_bounds__(NT) k_fcg_center_r(FcgV<T> f, const double *pa
         f.r[I] = q;
         v += q * q;
     })
-    block_partial(v, part);
+    block_partial(v, f.t, part);
 }
 // preconditioner input r/s (s = ‖r‖/√n, so WaterLily's absolute pcg! exit
 // thresholds see a unit-RMS residual), x = 0
@@ -1436,8 +1443,8 @@ __global__ void __launch_bounds__(NT) k_pcg_last_dots(LevV<T> l, FcgV<T> f, PcgS
                      if (!first) b += ww * w.q;
                  });
     }
-    block_partial(a, part, 2, 0);
-    block_partial(b, part, 2, 1);
+    block_partial(a, l.t, part, 2, 0);
+    block_partial(b, l.t, part, 2, 1);
 }
 // coefficients of the fine smoother below: Chebyshev on [λmin, λmax] =
 // [0.5, 2] (D⁻¹A has its spectrum in (0, 2]; the smoother damps the upper
@@ -1509,8 +1516,8 @@ __global__ void __launch_bounds__(NT) k_cheb2_dots(LevV<T> l, FcgV<T> f, T c0, T
                      });
         })
     }
-    block_partial(a, part, 2, 0);
-    block_partial(b, part, 2, 1);
+    block_partial(a, l.t, part, 2, 0);
+    block_partial(b, l.t, part, 2, 1);
 }
 // partials of w·r and w·q (w = s·x_T)
 template <class T>
@@ -1523,8 +1530,8 @@ __global__ void __launch_bounds__(NT) k_fcg_dots(FcgV<T> f, double *part, int fi
         a += w * f.r[I];
         if (!first) b += w * f.q[I];
     })
-    block_partial(a, part, 2, 0);
-    block_partial(b, part, 2, 1);
+    block_partial(a, f.t, part, 2, 0);
+    block_partial(b, f.t, part, 2, 1);
 }
 // p' = s·w + βp at the cell and its neighbours; q = A p' (FP64)
 template <int D, class T>
@@ -1600,7 +1607,7 @@ __global__ void __launch_bounds__(NT) k_fcg_Ap(FcgV<T> f, const double *part_dot
             v += pc * qq;
         })
     }
-    block_partial(v, part);
+    block_partial(v, f.t, part);
 }
 // α = ρ/(p·q); x += αp ; r -= αq ; partial ‖r‖²
 template <class T>
@@ -1630,7 +1637,7 @@ __global__ void __launch_bounds__(NT) k_fcg_update(FcgV<T> f, const double *part
                      v += rr * rr;
                  });
     }
-    block_partial(v, part);
+    block_partial(v, f.t, part);
 }
 // convergence test of the recursive residual on the device, so the host can
 // queue the next iteration before it reads this one's result
