@@ -132,6 +132,7 @@ struct ia_ctx {
     int ls_ini = -1;          // pool buffer holding ϕini of the LevelSet (valid until f is next advected)
     bool ls_valid = false;
     const int *halt = nullptr;   // the flexible CG's stop flag while a pipelined solve runs
+    StepOut *hst = nullptr;      // pinned: what the last kernel of a step hands back
     FcgState *pin = nullptr;     // pinned host copies of the solver state (two slots)
     hipEvent_t it_ev[2] = {nullptr, nullptr};
     // caller-owned device buffers adopted by ia_attach_field (nullptr: the
@@ -522,13 +523,15 @@ template <class T> struct Impl {
         if (int r = cgp_setup(c)) return r;
         c->part_n = 5 * maxblk + 64;
         HIPCHK(c, hipMalloc(&c->part, c->part_n * sizeof(double)));
-        HIPCHK(c, hipMalloc(&c->fpart, (maxblk + FILL_R2) * sizeof(FillPart)));
+        HIPCHK(c, hipMalloc(&c->fpart, 3 * (maxblk + FILL_R2) * sizeof(FillPart)));
         HIPCHK(c, hipMalloc(&c->st, sizeof(StepState)));
         HIPCHK(c, hipMalloc(&c->pst, PCG_SLOTS * sizeof(PcgState)));
         HIPCHK(c, hipMemsetAsync(c->pst, 0, PCG_SLOTS * sizeof(PcgState), c->s));
         HIPCHK(c, hipMalloc(&c->fst, sizeof(FcgState)));
         HIPCHK(c, hipMemsetAsync(c->fst, 0, sizeof(FcgState), c->s));
+        HIPCHK(c, hipMemsetAsync(c->st, 0, sizeof(StepState), c->s));
         HIPCHK(c, hipHostMalloc((void **)&c->pin, 2 * sizeof(FcgState)));
+        HIPCHK(c, hipHostMalloc((void **)&c->hst, sizeof(StepOut)));
         for (auto &ev : c->it_ev) HIPCHK(c, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
         {
             long mb = 0;
@@ -1297,17 +1300,29 @@ template <class T> struct Impl {
     }
 
     // ----------------------------------------------------------------- CFL
-    // vol (optional): Σf in FP64, min f and max f over the interior of the current f
-    static int cfl(ia_ctx *c, double *out, double *vol = nullptr) {
-        Grid &g = c->g;
+    static void cfl_launch(ia_ctx *c) {
         const CTiling &ct = c->lev[0].ct;
-        hipLaunchKernelGGL(k_cfl<T>, dim3((unsigned)ct.nblk), dim3(NT), 0, c->s, g, ct, P<T>(c->u),
+        hipLaunchKernelGGL(k_cfl<T>, dim3((unsigned)ct.nblk), dim3(NT), 0, c->s, c->g, ct, P<T>(c->u),
                            P<T>(c->fb[c->fi]), c->part);
-        hipLaunchKernelGGL(k_fin_cfl, dim3(1), dim3(NT), 0, c->s, c->part, ct.nblk, c->dsc + 8);
-        LAUNCHCHK(c);
-        double mx[5];
-        HIPCHK(c, hipMemcpyAsync(mx, c->dsc + 8, 5 * sizeof(double), hipMemcpyDeviceToHost, c->s));
-        HIPCHK(c, hipStreamSynchronize(c->s));
+    }
+    // the fill reports of `nsweep` sweeps made with u1, u2 and, with `cfl`, the CFL partials; `host`: into c->hst
+    static void finish(ia_ctx *c, int nsweep, const void *u1, const void *u2, double rtol, bool cfl, bool host) {
+        const FillPart *src = c->fpart;
+        long n = c->t.nblk;
+        if (nsweep > 0 && n > 8 * NT) {  // more than one block reads quickly
+            FillPart *out = c->fpart + 3 * n;
+            hipLaunchKernelGGL(k_fill_reduce, dim3(FILL_R2, (unsigned)nsweep), dim3(NT), 0, c->s, src, n, out);
+            src = out;
+            n = FILL_R2;
+        }
+        hipLaunchKernelGGL(k_step_finish<T>, dim3(1), dim3(NT), 0, c->s, c->g, src, n, nsweep, P<T>((void *)u1),
+                           P<T>((void *)u2), rtol, c->st, c->part, cfl ? c->lev[0].ct.nblk : 0L, host ? c->hst : nullptr);
+    }
+    // Δt from the values that a finished step left in c->hst; vol (optional):
+    // Σf in FP64, min f and max f over the interior of the current f
+    static void cfl_value(ia_ctx *c, double *out, double *vol = nullptr) {
+        Grid &g = c->g;
+        const double *mx = c->hst->cfl;
         if (vol)
             for (int q = 0; q < 3; ++q) vol[q] = mx[2 + q];
         T nu = (T)c->P.nu, lm = (T)c->P.lambda_mu, lr = (T)c->P.lambda_rho;
@@ -1323,6 +1338,13 @@ template <class T> struct Impl {
         T dtST = c->P.eta != 0 ? (T)std::sqrt((1 + lr) / ((T)(8 * M_PI) * (T)c->P.eta)) : T(1);
         T m = std::min(std::min(std::min(std::min(dtV, dtAdv), dtG), dtVisc), dtST);
         *out = (double)(T(0.8) * m);
+    }
+    static int cfl(ia_ctx *c, double *out) {
+        cfl_launch(c);
+        finish(c, 0, nullptr, nullptr, 0, true, true);
+        LAUNCHCHK(c);
+        HIPCHK(c, hipStreamSynchronize(c->s));
+        cfl_value(c, out);
         return IA_OK;
     }
 
@@ -1416,12 +1438,15 @@ template <class T> struct Impl {
         return IA_OK;
     }
     // ----------------------------------------------------------------- sweeps
-    static void prepare(ia_ctx *c, const void *f, const void *usrc, bool do_ru) {
+    // clear_st: the step's flags; clear_ruf: ρuf = 0
+    static void prepare(ia_ctx *c, const void *f, const void *usrc, bool do_ru, bool clear_st, bool clear_ruf) {
         hipLaunchKernelGGL(k_prepare<T>, blocks(c->t), dim3(NT), 0, c->s, c->g, c->t, P<T>(f), P<T>(usrc), P<T>(c->ru),
-                           c->cb, (T)c->P.lambda_rho, do_ru ? 1 : 0);
+                           c->cb, (T)c->P.lambda_rho, do_ru ? 1 : 0, clear_st ? c->st : nullptr,
+                           clear_ruf ? P<T>(c->ruf) : nullptr, c->g.ns * c->g.D);
     }
+    // slot: where the sweep's fill partials go, in the order of the sweeps (finish)
     static void vof_sweep(ia_ctx *c, const void *fin, void *fout, const void *u1, const void *u2, int d, T dt,
-                          int mode, double rtol, const void *fn, void *fmid) {
+                          int mode, double rtol, const void *fn, void *fmid, int slot) {
         Grid &g = c->g;
         SweepArgs<T> a;
         a.g = g;
@@ -1434,7 +1459,7 @@ template <class T> struct Impl {
         a.ruf = P<T>(c->ruf) + g.ns * d;
         a.fn = P<T>((void *)fn);
         a.fmid = P<T>(fmid);
-        a.part = c->fpart;
+        a.part = c->fpart + slot * c->t.nblk;
         a.d = d;
         a.scheme = c->P.normal_scheme;
         a.mode = mode;
@@ -1449,10 +1474,6 @@ template <class T> struct Impl {
         hipLaunchKernelGGL(k_vof_face<T>, dim3((unsigned)nfb), dim3(NT), 0, c->s, a, P<T>(c->vface));
         hipLaunchKernelGGL(k_vof_update<T>, blocks(c->t), dim3(NT), 0, c->s, a, P<T>(c->vface));
         prof_end(c, IA_PROF_VOF);  // one sweep (its two launches) per record
-        hipLaunchKernelGGL(k_fill_reduce, dim3(FILL_R2), dim3(NT), 0, c->s, c->fpart, c->t.nblk, c->fpart + c->t.nblk);
-        hipLaunchKernelGGL(k_fill_finalize<T>, dim3(1), dim3(NT), 0, c->s, g, c->fpart + c->t.nblk, (long)FILL_R2,
-                           P<T>((void *)u1),
-                           P<T>((void *)u2), rtol, c->st);
     }
     static void momentum(ia_ctx *c, const void *fpre, const void *u1, const void *u2, const void *uold, int d, T dt) {
         Grid &g = c->g;
@@ -1511,7 +1532,7 @@ template <class T> struct Impl {
             int out = outs[op & 1];
             bool last = op == c->g.D - 1;
             vof_sweep(c, c->fb[cur], c->fb[out], u1, u2, d, dt, 0, rtol, last && mid >= 0 ? c->fb[keep] : nullptr,
-                      last && mid >= 0 ? c->fb[mid] : nullptr);
+                      last && mid >= 0 ? c->fb[mid] : nullptr, op);
             momentum(c, c->fb[cur], u1, u2, uold, d, dt);
             cur = out;
         }
@@ -1572,10 +1593,9 @@ template <class T> struct Impl {
         LAUNCHCHK(c);
         return IA_OK;
     }
+    // of a finished step (c->hst, after the stream was waited for)
     static int read_state(ia_ctx *c, ia_step_stats *ss) {
-        StepState h;
-        HIPCHK(c, hipMemcpyAsync(&h, c->st, sizeof h, hipMemcpyDeviceToHost, c->s));
-        HIPCHK(c, hipStreamSynchronize(c->s));
+        const StepState h = c->hst->st;
         if (ss) {
             ss->status = h.status;
             ss->fill_warnings = h.nwarn;
@@ -1591,20 +1611,20 @@ template <class T> struct Impl {
     static int mom_step(ia_ctx *c, double dtd, int step_index, ia_step_stats *ss) {
         Grid &g = c->g;
         T dt = (T)dtd;
-        HIPCHK(c, hipMemsetAsync(c->st, 0, sizeof(StepState), c->s));
         int fn = c->fi;
         void *U0 = c->u, *U1 = c->u0;  // u⁰ ← u: the predictor reads u^n from U0 and writes u^{n+1/2} to U1
         // predictor (w = ½)
         T w = T(0.5);
-        prepare(c, c->fb[fn], U0, true);
+        prepare(c, c->fb[fn], U0, true, true, false);
         int mid = free_fbuf(c, fn, -1, -1);
         int fstar = advect_fq(c, fn, U0, U0, U0, dt, step_index, fn, mid);
         (void)fstar;
+        finish(c, g.D, U0, U0, 100 * epsT(), false, false);
         if (int e = upd(c, U0, U0, c->fb[fn], c->fb[mid], U1, dt, w)) return e;
         if (int e = mg_update(c)) return e;
         if (int e = project(c, U1, (double)(w * dt), ss ? &ss->solve[0] : nullptr)) return e;
         // corrector (w = 1): f⁰ ← f; ρu = u⁰ρ(f); advect f with u^{n+½}
-        prepare(c, c->fb[fn], U0, true);
+        prepare(c, c->fb[fn], U0, true, false, false);
         int fnew = advect_fq(c, fn, U1, U1, U0, dt, step_index, fn, -1);
         if (int e = upd(c, U1, U0, c->fb[fnew], c->fb[fnew], U0, dt, T(1))) return e;
         if (int e = mg_update(c)) return e;
@@ -1614,8 +1634,12 @@ template <class T> struct Impl {
         c->fi = fnew;
         c->f0i = fn;
         if (int e = restore_attached(c)) return e;
+        cfl_launch(c);
+        finish(c, g.D, U1, U1, 100 * epsT(), true, true);
+        LAUNCHCHK(c);
+        HIPCHK(c, hipStreamSynchronize(c->s));
         double cf, vol[3];
-        if (int e = cfl(c, &cf, vol)) return e;
+        cfl_value(c, &cf, vol);
         int st = read_state(c, ss);
         double nx = std::min(cf, 1.2 * (double)dt);
         if (ss) {
@@ -1634,16 +1658,14 @@ template <class T> struct Impl {
         Grid &g = c->g;
         T dt = (T)dtd;
         int keep = fsrc == c->fi ? c->f0i : c->fi;
-        HIPCHK(c, hipMemsetAsync(c->st, 0, sizeof(StepState), c->s));
-        HIPCHK(c, hipMemsetAsync(c->ruf, 0, g.ns * g.D * sizeof(T), c->s));
-        prepare(c, c->fb[fsrc], u1, false);
+        prepare(c, c->fb[fsrc], u1, false, true, true);
         int dirO[3];
         dir_order(g.D, step_index, dirO);
         int cur = fsrc;
         for (int op = 0; op < g.D; ++op) {
             int d = dirO[op];
-            int out = free_fbuf(c, cur, keep, -1);
-            vof_sweep(c, c->fb[cur], c->fb[out], u1, u2, d, dt, 1, 10 * epsT(), nullptr, nullptr);
+            int out = op == g.D - 1 ? fsrc : free_fbuf(c, cur, keep, fsrc);  // ends where it began
+            vof_sweep(c, c->fb[cur], c->fb[out], u1, u2, d, dt, 1, 10 * epsT(), nullptr, nullptr, op);
             cur = out;
         }
         LAUNCHCHK(c);
@@ -1654,9 +1676,12 @@ template <class T> struct Impl {
         double cf, vol[3];
         int fi_save = c->fi;
         c->fi = adv_f ? c->fi : c->f0i;  // the statistics describe the advected field
-        int e = cfl(c, &cf, vol);
+        cfl_launch(c);
         c->fi = fi_save;
-        if (e) return e;
+        finish(c, g.D, u1, u2, 10 * epsT(), true, true);
+        LAUNCHCHK(c);
+        HIPCHK(c, hipStreamSynchronize(c->s));
+        cfl_value(c, &cf, vol);
         int st = read_state(c, ss);
         if (ss) {
             ss->dt_next = dtd;
@@ -1667,15 +1692,14 @@ template <class T> struct Impl {
         return st;
     }
     static int vof_sweep_stage(ia_ctx *c, int d, double dtd, ia_step_stats *ss) {
-        Grid &g = c->g;
-        HIPCHK(c, hipMemsetAsync(c->st, 0, sizeof(StepState), c->s));
-        HIPCHK(c, hipMemsetAsync(c->ruf, 0, g.ns * g.D * sizeof(T), c->s));
-        prepare(c, c->fb[c->fi], c->u0, false);
+        prepare(c, c->fb[c->fi], c->u0, false, true, true);
         int out = free_fbuf(c, c->fi, c->f0i, -1);
-        vof_sweep(c, c->fb[c->fi], c->fb[out], c->u0, c->u, d, (T)dtd, 1, 100 * epsT(), nullptr, nullptr);
+        vof_sweep(c, c->fb[c->fi], c->fb[out], c->u0, c->u, d, (T)dtd, 1, 100 * epsT(), nullptr, nullptr, 0);
+        finish(c, 1, c->u0, c->u, 100 * epsT(), false, true);
         LAUNCHCHK(c);
         c->fi = out;
         if (int e = restore_attached(c)) return e;
+        HIPCHK(c, hipStreamSynchronize(c->s));
         return read_state(c, ss);
     }
     static int visc_stage(ia_ctx *c, int use_f0) {
@@ -1884,6 +1908,7 @@ void ia_destroy(ia_ctx *c) {
     for (hipEvent_t e : c->it_ev)
         if (e) (void)hipEventDestroy(e);
     if (c->pin) (void)hipHostFree(c->pin);
+    if (c->hst) (void)hipHostFree(c->hst);
     if (c->e0) (void)hipEventDestroy(c->e0);
     if (c->e1) (void)hipEventDestroy(c->e1);
     if (c->s) (void)hipStreamDestroy(c->s);

@@ -44,21 +44,6 @@ __device__ inline double block_sum(double v) {
         for (int q = 0; q < NT / 64; ++q) s += sh[q];
     return s;  // valid in thread 0
 }
-__device__ inline double block_max(double v) {
-    __shared__ double sh[NT / 64];
-    for (int o = 32; o > 0; o >>= 1) {
-        double w2 = __shfl_xor(v, o, 64);
-        v = w2 > v ? w2 : v;
-    }
-    int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) sh[w] = v;
-    __syncthreads();
-    double s = sh[0];
-    if (threadIdx.x == 0)
-        for (int q = 1; q < NT / 64; ++q) s = sh[q] > s ? sh[q] : s;
-    return s;
-}
 
 // argmax/argmin partials of a VOF sweep (findmax/findmin, advection.jl:146-147)
 struct FillPart {
@@ -135,15 +120,51 @@ __device__ inline FillPart block_fill_cells(double v, long I, bool ok, bool nan)
         for (int q = 1; q < NT / 64; ++q) fill_combine(r, shw[q]);
     return r;
 }
+// a block's combined FillPart, each wavefront by DPP (order-independent);
+// valid in thread 0
 __device__ inline FillPart block_fill(FillPart v) {
-    __shared__ FillPart sh[NT];
-    sh[threadIdx.x] = v;
+    __shared__ FillPart sh[NT / 64];
+    FillPart p;
+    p.vmax = wave_max_d(v.vmax);
+    p.vmin = wave_min_d(v.vmin);
+    p.imax = wave_min_l(v.vmax == p.vmax ? v.imax : (1L << 60));
+    p.imin = wave_min_l(v.vmin == p.vmin ? v.imin : (1L << 60));
+    p.nan = __ballot(v.nan != 0) != 0;
+    p.pad = 0;
+    __syncthreads();  // before sh is written again
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = p;
     __syncthreads();
-    for (int s = NT / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) fill_combine(sh[threadIdx.x], sh[threadIdx.x + s]);
-        __syncthreads();
+    FillPart r = sh[0];
+    if (threadIdx.x == 0)
+        for (int q = 1; q < NT / 64; ++q) fill_combine(r, sh[q]);
+    return r;
+}
+// a block's two maxima, sum, minimum and maximum; valid in thread 0.  The sum
+// is block_sum's, wavefront by wavefront.
+struct Red5 {
+    double a, b, s, mn, mx;
+};
+__device__ inline Red5 block_red5(Red5 v) {
+    __shared__ Red5 sh[NT / 64];
+    v.a = wave_max_d(v.a);
+    v.b = wave_max_d(v.b);
+    v.s = wave_sum(v.s);
+    v.mn = wave_min_d(v.mn);
+    v.mx = wave_max_d(v.mx);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    Red5 r = sh[0];
+    if (threadIdx.x == 0) {
+        r.s = 0;
+        for (int q = 0; q < NT / 64; ++q) {
+            r.a = fmax(r.a, sh[q].a);
+            r.b = fmax(r.b, sh[q].b);
+            r.s += sh[q].s;
+            r.mn = fmin(r.mn, sh[q].mn);
+            r.mx = fmax(r.mx, sh[q].mx);
+        }
     }
-    return sh[0];
+    return r;
 }
 
 // device-resident state of a step (flags) and of a solve (pcg scalars)
@@ -152,17 +173,29 @@ struct StepState {
     double maxf, minf;
     long imax, imin;
 };
+// what a step hands back to the host: written by its last kernel into pinned
+// host memory (no copies)
+struct StepOut {
+    double cfl[5];  // the two CFL maxima, Σf, min f, max f
+    StepState st;
+};
 struct SolveCtl {
     double rho, alpha, beta, s, r2, dot;
     int done, stop, it, pad;
 };
 
 // ---------------------------------------------------------------------------
-// c̄ = f≥½ (advection.jl:40, flow.jl:172) and ρu = u·ρ(f) (VOFutil.jl:208-211)
+// c̄ = f≥½ (advection.jl:40, flow.jl:172) and ρu = u·ρ(f) (VOFutil.jl:208-211);
+// with `st` the step's flags are cleared, with `zero` the nz values there
+// (instead of two memsets' launches)
 // ---------------------------------------------------------------------------
 template <class T>
 __global__ void __launch_bounds__(NT) k_prepare(Grid g, Tiling t, const T *__restrict__ f, const T *__restrict__ usrc,
-                                                 T *__restrict__ ru, int8_t *__restrict__ cb, T lr, int do_ru) {
+                                                 T *__restrict__ ru, int8_t *__restrict__ cb, T lr, int do_ru,
+                                                 StepState *st, T *__restrict__ zero, long nz) {
+    if (st && blockIdx.x == 0 && threadIdx.x == 0) *st = StepState{0, 0, 0.0, 0.0, 0, 0};
+    if (zero)
+        for (long q = (long)blockIdx.x * NT + threadIdx.x; q < nz; q += (long)gridDim.x * NT) zero[q] = T(0);
     int p[3];
     if (!thread_cell(g, t, p)) return;
     long I = lin(g, p);
@@ -316,24 +349,21 @@ __device__ inline FillPart fill_identity() {
     acc.pad = 0;
     return acc;
 }
-// first stage of the fill reduction: FILL_R2 blocks fold the per-block
-// partials of a sweep (fill_combine is order-independent: ties go to the
-// smallest index)
+// first stage of the fill reduction: FILL_R2 blocks per sweep fold the
+// per-block partials of each of gridDim.y sweeps (fill_combine is
+// order-independent: ties go to the smallest index)
 constexpr int FILL_R2 = 256;
 __global__ void __launch_bounds__(NT) k_fill_reduce(const FillPart *part, long nblk, FillPart *out) {
+    part += nblk * blockIdx.y;
     FillPart acc = fill_identity();
     for (long b = (long)blockIdx.x * NT + threadIdx.x; b < nblk; b += (long)gridDim.x * NT) fill_combine(acc, part[b]);
     FillPart r = block_fill(acc);
-    if (threadIdx.x == 0) out[blockIdx.x] = r;
+    if (threadIdx.x == 0) out[(long)gridDim.x * blockIdx.y + blockIdx.x] = r;
 }
-// reportFillError (advection.jl:145-189) on the reduced partials
+// reportFillError (advection.jl:145-189) on one sweep's partials (thread 0)
 template <class T>
-__global__ void __launch_bounds__(NT) k_fill_finalize(Grid g, const FillPart *part, long nblk, const T *u1,
-                                                      const T *u2, double tol, StepState *st) {
-    FillPart acc = fill_identity();
-    for (long b = threadIdx.x; b < nblk; b += NT) fill_combine(acc, part[b]);
-    FillPart r = block_fill(acc);
-    if (threadIdx.x != 0) return;
+__device__ inline void fill_report(const Grid &g, const FillPart &r, const T *u1, const T *u2, double tol,
+                                   StepState *st) {
     int s = 0;
     if (r.nan) s = 1;
     else {
@@ -362,6 +392,46 @@ __global__ void __launch_bounds__(NT) k_fill_finalize(Grid g, const FillPart *pa
         st->imin = r.imin;
     }
     st->status = worst;
+}
+// The end of a run of sweeps, in one block: the sweeps' fill reports in their
+// order (n partials each; u1, u2 still hold the velocities they were made
+// with), then the CFL partials (ncfl > 0: k_cfl's, five values each), then
+// everything into pinned host memory (out).  One launch where there were two
+// per sweep, one for the CFL and two copies.
+template <class T>
+__global__ void __launch_bounds__(NT) k_step_finish(Grid g, const FillPart *part, long n, int nsweep, const T *u1,
+                                                    const T *u2, double tol, StepState *st, const double *cfl,
+                                                    long ncfl, StepOut *out) {
+    StepState s = *st;
+    for (int w = 0; w < nsweep; ++w) {
+        FillPart acc = fill_identity();
+        for (long b = threadIdx.x; b < n; b += NT) fill_combine(acc, part[n * w + b]);
+        FillPart r = block_fill(acc);
+        if (threadIdx.x == 0) fill_report(g, r, u1, u2, tol, &s);
+    }
+    if (ncfl > 0) {
+        Red5 v{0, 0, 0, 1e300, -1e300};
+        for (long q = threadIdx.x; q < ncfl; q += NT) {
+            const double *o = cfl + 5 * q;
+            v.a = o[0] > v.a ? o[0] : v.a;
+            v.b = o[1] > v.b ? o[1] : v.b;
+            v.s += o[2];
+            v.mn = o[3] < v.mn ? o[3] : v.mn;
+            v.mx = o[4] > v.mx ? o[4] : v.mx;
+        }
+        v = block_red5(v);
+        if (threadIdx.x == 0 && out) {
+            out->cfl[0] = v.a;
+            out->cfl[1] = v.b;
+            out->cfl[2] = v.s;
+            out->cfl[3] = v.mn;
+            out->cfl[4] = v.mx;
+        }
+    }
+    if (threadIdx.x == 0) {
+        *st = s;
+        if (out) out->st = s;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -965,35 +1035,6 @@ __global__ void __launch_bounds__(NT) k_project(Grid g, Tiling t, T *u, const T 
         T un = u[g.ns * i + I] - L[g.ns * i + I] * dx;
         T xv = i == 0 && g.exitx ? u[I + g.st[0]] : T(0);  // exitBC: the exit face is left alone
         write_images<T>(g, u + g.ns * i, p, un, 2, i, ub[i], xv);
-    }
-}
-// the two CFL maxima, Σf (each thread adds its blocks in order, then a fixed
-// tree), min f and max f of the k_cfl partials
-__global__ void __launch_bounds__(NT) k_fin_cfl(const double *part, long nblk, double *out) {
-    double a = 0, b = 0, s = 0, mn = 1e300, mx = -1e300;
-    for (long q = threadIdx.x; q < nblk; q += NT) {
-        const double *o = part + 5 * q;
-        a = o[0] > a ? o[0] : a;
-        b = o[1] > b ? o[1] : b;
-        s += o[2];
-        mn = o[3] < mn ? o[3] : mn;
-        mx = o[4] > mx ? o[4] : mx;
-    }
-    double ma = block_max(a);
-    __syncthreads();
-    double mb = block_max(b);
-    __syncthreads();
-    double ss = block_sum(s);
-    __syncthreads();
-    double mmx = block_max(mx);
-    __syncthreads();
-    double mmn = -block_max(-mn);
-    if (threadIdx.x == 0) {
-        out[0] = ma;
-        out[1] = mb;
-        out[2] = ss;
-        out[3] = mmn;
-        out[4] = mmx;
     }
 }
 // f⁰ = (f⁰ + f)/2 over every cell (flow.jl:74)
