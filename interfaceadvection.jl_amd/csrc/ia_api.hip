@@ -586,15 +586,27 @@ template <class T> struct Impl {
     }
     // ----------------------------------------------------------------- MG
     static int mg_update(ia_ctx *c) {
-        for (int l = 0; l < c->nlev; ++l) {
-            Level &lv = c->lev[l];
-            if (l > 0) {
-                Level &lf = c->lev[l - 1];
-                hipLaunchKernelGGL(k_restrictL<T>, blocks(lv.t), dim3(NT), 0, c->s, lv.g, lv.t, lf.g, P<T>(lf.L),
-                                   P<T>(lv.L));
+        Level &l0 = c->lev[0];
+        hipLaunchKernelGGL(k_set_diag<T>, blocks(l0.t), dim3(NT), 0, c->s, l0.g, l0.t, P<T>(l0.L), P<T>(l0.Dg),
+                           P<T>(l0.iD));
+        int l = 1;
+        for (; l < c->nlev && interior(c->lev[l].g) > MGU_NT; ++l) {
+            Level &lv = c->lev[l], &lf = c->lev[l - 1];
+            hipLaunchKernelGGL(k_coarse_level<T>, blocks(lv.t), dim3(NT), 0, c->s, lv.g, lv.t, lf.g, P<T>(lf.L),
+                               P<T>(lv.L), P<T>(lv.Dg), P<T>(lv.iD));
+        }
+        if (l < c->nlev) {
+            static_assert(sizeof(c->lev) / sizeof(c->lev[0]) <= MGU_LEV, "levels");
+            MguArgs<T> a;
+            for (int q = 0; q < c->nlev; ++q) {
+                a.g[q] = c->lev[q].g;
+                a.L[q] = P<T>(c->lev[q].L);
+                a.Dg[q] = P<T>(c->lev[q].Dg);
+                a.iD[q] = P<T>(c->lev[q].iD);
             }
-            hipLaunchKernelGGL(k_set_diag<T>, blocks(lv.t), dim3(NT), 0, c->s, lv.g, lv.t, P<T>(lv.L), P<T>(lv.Dg),
-                               P<T>(lv.iD));
+            a.l0 = l;
+            a.nlev = c->nlev;
+            hipLaunchKernelGGL(k_coarse_levels<T>, dim3(1), dim3(MGU_NT), 0, c->s, a);
         }
         LAUNCHCHK(c);
         return IA_OK;
