@@ -100,7 +100,7 @@ struct ia_ctx {
     FcgState *fst = nullptr;   // flexible-CG scalars
     double *pp = nullptr;      // partial-sum buffers (PP_N of pp_stride doubles)
     long pp_stride = 0;
-    std::vector<double> hpart; // host copy of a partial-sum buffer
+    double *hpart = nullptr;   // pinned host copy of a partial-sum buffer
     double *dsc = nullptr;   // device scalars
     double *x64 = nullptr, *r64 = nullptr, *z64 = nullptr, *pa64 = nullptr, *pb64 = nullptr, *q64 = nullptr;
     int fine_cheb = 1;   // the finest level's smoother after each preconditioning V-cycle: two Chebyshev steps
@@ -111,6 +111,7 @@ struct ia_ctx {
     int cit_wl[MAXLEV], cit_fcg[MAXLEV];
     unsigned long long *cgp_hw = nullptr, *cgp_pw = nullptr;  // the one-launch coarse CG's words
     unsigned cgp_tag = 1;  // next unused tag of those words
+    bool pcgp = false;     // solver!'s pcg! in one launch (k_pcgp)
     bool cgp_off = false;  // one launch per iteration instead (IA_CG1_NB set, or workgroups did not run together)
     int cg1_nb[MAXLEV];  // workgroup size of the coarse CG step per level (one cell per thread)
     struct Cnn {
@@ -143,7 +144,7 @@ struct ia_ctx {
     size_t tail_lds = 0; // its dynamic LDS bytes
     // the column kernels that hold the tail: 512 threads of 4 cells, 512 of 8, 1024 of 4 (FP32; else k_mg_tail)
     bool tail_cols[3] = {false, false, false};
-    hipEvent_t e0 = nullptr, e1 = nullptr;
+    hipEvent_t ev_solve[2][2] = {};  // around a step's two projections
     struct ProfClass {
         bool on = false;
         int n = 0;         // event pairs
@@ -532,12 +533,14 @@ template <class T> struct Impl {
         HIPCHK(c, hipMemsetAsync(c->st, 0, sizeof(StepState), c->s));
         HIPCHK(c, hipHostMalloc((void **)&c->pin, 2 * sizeof(FcgState)));
         HIPCHK(c, hipHostMalloc((void **)&c->hst, sizeof(StepOut)));
+        memset(c->hst, 0, sizeof(StepOut));
         for (auto &ev : c->it_ev) HIPCHK(c, hipEventCreateWithFlags(&ev, hipEventDisableTiming));
         {
             long mb = 0;
             for (int l = 0; l < c->nlev; ++l) mb = std::max(mb, c->lev[l].ct.nblk);
             c->pp_stride = 2 * mb + 64;
             HIPCHK(c, hipMalloc(&c->pp, PP_N * c->pp_stride * sizeof(double)));
+            HIPCHK(c, hipHostMalloc((void **)&c->hpart, c->pp_stride * sizeof(double)));
             HIPCHK(c, hipMemsetAsync(c->pp, 0, PP_N * c->pp_stride * sizeof(double), c->s));
         }
         HIPCHK(c, hipMalloc(&c->dsc, 64 * sizeof(double)));
@@ -546,17 +549,18 @@ template <class T> struct Impl {
         return IA_OK;
     }
 
-    // the levels that the flexible CG's preconditioner solves with k_cgp: those above the tail whose boxes fit, on a
-    // device that holds twice the workgroups at once (two contexts may run there together)
+    // the levels solved in one launch, by k_cgp (the flexible CG's preconditioner) or k_pcgp (solver!'s pcg!, the
+    // finest level among them): those above the tail whose boxes fit, on a device that holds twice the workgroups at
+    // once (two contexts may run there together)
     static int cgp_setup(ia_ctx *c) {
-        if (sizeof(T) != 4 || c->cgp_off || c->P.poisson_mode == IA_POISSON_REFERENCE ||
-            c->P.poisson_mode == IA_POISSON_PCG || c->P.poisson_mode == IA_POISSON_PLAIN)
-            return IA_OK;
+        // FP64's sums show the order of their terms in the result, which the launches' tiles set
+        if (sizeof(T) != 4 || c->cgp_off || c->P.poisson_mode == IA_POISSON_PCG) return IA_OK;
+        c->pcgp = c->P.poisson_mode == IA_POISSON_REFERENCE || c->P.poisson_mode == IA_POISSON_PLAIN;
         int ncu = 0, nv = 0;
         HIPCHK(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->dev));
         const CgpVariant *vs = cgp_variants(nv);
         size_t words = 0;
-        for (int l = 1; l < c->tail_level && l < c->nlev; ++l) {
+        for (int l = c->pcgp ? 0 : 1; l < c->tail_level && l < c->nlev; ++l) {
             Level &lv = c->lev[l];
             int n[3];
             for (int a = 0; a < 3; ++a) n[a] = a < lv.g.D ? lv.g.Ng[a] - 2 : 1;
@@ -566,8 +570,9 @@ template <class T> struct Impl {
                     if (vs[q].D != lv.g.D || (maxwg > CGP_ONE && vs[q].NB < 1024)) continue;
                     if (!cgp_boxes(n, vs[q], maxwg, lv.cgp_box)) continue;
                     int per = 0;
-                    HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void *)vs[q].k, vs[q].NB,
-                                                                           cgp_lds(lv)));
+                    HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                                  &per, c->pcgp ? (const void *)pcgp_kernel(q) : (const void *)vs[q].k, vs[q].NB,
+                                  cgp_lds(lv)));
                     if ((long)per * ncu < (maxwg > CGP_ONE ? 1L : 2L) * lv.cgp_box.nwg) continue;
                     lv.cgp = &vs[q];
                 }
@@ -580,6 +585,7 @@ template <class T> struct Impl {
         }
         return IA_OK;
     }
+    static bool cgp_failed(const ia_ctx *c) { return *(volatile int *)&c->hst->fail != 0; }
     static size_t cgp_lds(const Level &l) {
         const CgpBox &b = l.cgp_box;
         return sizeof(float) * (b.b[0] + 2) * (b.b[1] + 2) * (l.g.D > 2 ? b.b[2] + 2 : 1);
@@ -641,8 +647,39 @@ template <class T> struct Impl {
     // WaterLily pcg!(p; it).  init_done: ϵ = r·iD and the partials of ρ₀ (PP_A)
     // were produced by the preceding fused prolongate!/increment!.  last: the
     // final update is fused with the FCG dots of the preconditioned residual.
+    // solver!'s pcg! on l in one launch
+    static bool one_launch(const ia_ctx *c, const Level &l) { return c->pcgp && l.cgp && !c->cgp_off; }
+    // r2: also the parts of Σr² (one per workgroup), r, z and the next Jacobi!'s ϵ
+    static void pcg_launch(ia_ctx *c, Level &l, int it, bool prolong, double *r2) {
+        PcgpArgs a;
+        a.g = l.g;
+        a.box = l.cgp_box;
+        a.L = P<float>(l.L);
+        a.iD = P<float>(l.iD);
+        a.x = P<float>(l.x);
+        a.r = P<float>(l.r);
+        a.z = P<float>(l.z);
+        a.e = P<float>(l.e);
+        a.xc = prolong ? P<float>((&l)[1].x) : nullptr;
+        a.gc = prolong ? (&l)[1].g : l.g;
+        a.hw = c->cgp_hw;
+        a.pw = c->cgp_pw;
+        a.tag = c->cgp_tag;
+        c->cgp_tag += 2 * (unsigned)it + 2;
+        a.it = it;
+        a.r2 = r2;
+        a.halt = cur_halt;
+        a.fail = &c->hst->fail;
+        int nv;
+        hipLaunchKernelGGL(pcgp_kernel((int)(l.cgp - cgp_variants(nv))), dim3((unsigned)a.box.nwg),
+                           dim3((unsigned)l.cgp->NB), cgp_lds(l), c->s, a);
+    }
     static void pcg(ia_ctx *c, Level &l, int it = 6, bool init_done = false, const FcgV<T> *last = nullptr,
                     int first = 0) {
+        if (one_launch(c, l)) {
+            pcg_launch(c, l, it, init_done, nullptr);
+            return;
+        }
         LevV<T> v = view(l);
         bool f0 = &l == &c->lev[0];
         dim3 B = cb(l);
@@ -715,7 +752,7 @@ template <class T> struct Impl {
             c->cgp_tag += (unsigned)it + 1;
             a.it = it;
             a.halt = cur_halt;
-            a.fail = &c->fst->fail;
+            a.fail = &c->hst->fail;
             if (pc >= 0) prof_begin(c, pc);
             hipLaunchKernelGGL(l.cgp->k, dim3((unsigned)a.box.nwg), dim3((unsigned)l.cgp->NB), cgp_lds(l), c->s, a);
             if (pc >= 0) prof_end(c, pc);
@@ -794,6 +831,7 @@ template <class T> struct Impl {
             if (cit == c->cit_fcg) pcg1(c, co, cit[l + 1]);
             else pcg(c, co, cit[l + 1], rec);
         }
+        if (then_pcg && one_launch(c, fl)) return;  // the pcg! begins with both
         if (then_pcg) {
             bool f0 = l == 0;
             if (f0) prof_begin(c, IA_PROF_PROLONG_INC);
@@ -807,8 +845,7 @@ template <class T> struct Impl {
     }
     // fixed-order host sum of one partial-sum buffer (K values per block)
     static int host_total(ia_ctx *c, int buf, long nblk, int K, double *out) {
-        c->hpart.resize(K * nblk);
-        HIPCHK(c, hipMemcpyAsync(c->hpart.data(), pp(c, buf), K * nblk * sizeof(double), hipMemcpyDeviceToHost, c->s));
+        HIPCHK(c, hipMemcpyAsync(c->hpart, pp(c, buf), K * nblk * sizeof(double), hipMemcpyDeviceToHost, c->s));
         HIPCHK(c, hipStreamSynchronize(c->s));
         for (int k = 0; k < K; ++k) {
             double s = 0;
@@ -817,27 +854,45 @@ template <class T> struct Impl {
         }
         return IA_OK;
     }
-    // WaterLily solver!(ml; tol, itmx)
-    static int solver(ia_ctx *c, double tol, int itmx, int *iters, double *r2o) {
+    // WaterLily solver!(ml; tol, itmx) on z = div u
+    static int residual(ia_ctx *c, const void *u, double *r2) {
         Level &l0 = c->lev[0];
-        long ncell = interior(l0.g), nb = l0.ct.nblk;
+        hipLaunchKernelGGL(k_div<T>, blocks(c->t), dim3(NT), 0, c->s, c->g, c->t, P<T>((void *)u), P<T>(c->sig));
         hipLaunchKernelGGL(k_mg_resid<T>, cb(l0), dim3(NT), 0, c->s, view(l0), pp(c, PP_MR));
-        hipLaunchKernelGGL(k_mg_center_l2<T>, cb(l0), dim3(NT), 0, c->s, view(l0), pp(c, PP_MR), ncell, 1,
+        hipLaunchKernelGGL(k_mg_center_l2<T>, cb(l0), dim3(NT), 0, c->s, view(l0), pp(c, PP_MR), interior(l0.g), 1,
                            pp(c, PP_ML2));
         LAUNCHCHK(c);
+        if (int e = host_total(c, PP_ML2, l0.ct.nblk, 1, r2)) return e;
+        *r2 = (double)(T)*r2;
+        return IA_OK;
+    }
+    static int solver(ia_ctx *c, const void *u, double tol, int itmx, int *iters, double *r2o) {
+        Level &l0 = c->lev[0];
+        long ncell = interior(l0.g), nb = l0.ct.nblk;
         double r2;
-        if (int e = host_total(c, PP_ML2, nb, 1, &r2)) return e;
-        r2 = (double)(T)r2;
+        if (int e = residual(c, u, &r2)) return e;
         int n = 0;
         while (r2 > tol && n < itmx) {
-            vcycle(c, 0, c->cit_wl, false, true);
-            pcg(c, l0, 6, true);
-            hipLaunchKernelGGL(k_mg_center_l2<T>, cb(l0), dim3(NT), 0, c->s, view(l0), pp(c, PP_MR), ncell, 0,
-                               pp(c, PP_ML2));
-            LAUNCHCHK(c);
-            if (int e = host_total(c, PP_ML2, nb, 1, &r2)) return e;
+            vcycle(c, 0, c->cit_wl, false, true, true);
+            if (one_launch(c, l0)) {
+                pcg_launch(c, l0, 6, true, c->hst->r2);
+                LAUNCHCHK(c);
+                HIPCHK(c, hipStreamSynchronize(c->s));
+                r2 = 0;
+                for (int q = 0; q < l0.cgp_box.nwg; ++q) r2 += c->hst->r2[q];
+            } else {
+                pcg(c, l0, 6, true);
+                hipLaunchKernelGGL(k_mg_center_l2<T>, cb(l0), dim3(NT), 0, c->s, view(l0), pp(c, PP_MR), ncell, 0,
+                                   pp(c, PP_ML2));
+                LAUNCHCHK(c);
+                if (int e = host_total(c, PP_ML2, nb, 1, &r2)) return e;
+            }
             r2 = (double)(T)r2;
             n++;
+            if (cgp_failed(c) && !c->cgp_off) {  // x and r may not fit together: go on from x's own residual
+                c->cgp_off = true;
+                if (int e = residual(c, u, &r2)) return e;
+            }
         }
         hipLaunchKernelGGL(k_mg_perbc<T>, cb(l0), dim3(NT), 0, c->s, view(l0), P<T>(l0.x));
         LAUNCHCHK(c);
@@ -849,11 +904,10 @@ template <class T> struct Impl {
     static int project_ref(ia_ctx *c, void *u, double dtw_d, ia_solve_stats *ss) {
         Grid &g = c->g;
         T dtw = (T)dtw_d;
-        hipLaunchKernelGGL(k_div<T>, blocks(c->t), dim3(NT), 0, c->s, g, c->t, P<T>(u), P<T>(c->sig));
         hipLaunchKernelGGL(k_scale<T>, blocks1(g.ns), dim3(256), 0, c->s, P<T>(c->p), g.ns, dtw);
         int it = 0;
         double r2 = 0;
-        if (int e = solver(c, c->P.poisson_tol, c->P.poisson_itmx, &it, &r2)) return e;
+        if (int e = solver(c, u, c->P.poisson_tol, c->P.poisson_itmx, &it, &r2)) return e;
         hipLaunchKernelGGL(k_project<T>, blocks(c->t), dim3(NT), 0, c->s, g, c->t, P<T>(u), P<T>(c->L), P<T>(c->p),
                            (T)c->P.u_bc[0], (T)c->P.u_bc[1], (T)c->P.u_bc[2]);
         hipLaunchKernelGGL(k_scale<T>, blocks1(g.ns), dim3(256), 0, c->s, P<T>(c->p), g.ns, T(1) / dtw);
@@ -1059,7 +1113,7 @@ template <class T> struct Impl {
                 it++;
                 rr = st.rr;
                 rel = sqrt(rr) / zn;
-                if (st.fail) c->cgp_off = true;  // workgroups of a k_cgp launch did not run together
+                if (cgp_failed(c)) c->cgp_off = true;
                 if (st.halt) {
                     // the queued iteration (if any) returned at once; confirm with
                     // the true FP64 residual and restart from it if it drifted
@@ -1295,20 +1349,27 @@ template <class T> struct Impl {
         HIPCHK(c, hipStreamSynchronize(c->s));
         return IA_OK;
     }
-    static int project(ia_ctx *c, void *u, double dtw, ia_solve_stats *ss) {
-        HIPCHK(c, hipEventRecord(c->e0, c->s));
+    // slot: the pair of events around the solve (solve_ms reads them once the stream was waited for)
+    static int project(ia_ctx *c, void *u, double dtw, ia_solve_stats *ss, int slot) {
+        HIPCHK(c, hipEventRecord(c->ev_solve[slot][0], c->s));
         int e = c->P.poisson_mode == IA_POISSON_REFERENCE ? project_ref(c, u, dtw, ss)
                 : c->P.poisson_mode == IA_POISSON_PCG     ? project_pcg(c, u, dtw, ss)
                                                           : project_refined(c, u, dtw, ss);
         if (e) return e;
-        HIPCHK(c, hipEventRecord(c->e1, c->s));
-        if (ss) {
-            HIPCHK(c, hipEventSynchronize(c->e1));
-            float ms = 0;
-            HIPCHK(c, hipEventElapsedTime(&ms, c->e0, c->e1));
-            ss->ms = ms;
-        }
+        HIPCHK(c, hipEventRecord(c->ev_solve[slot][1], c->s));
         return IA_OK;
+    }
+    static int solve_ms(ia_ctx *c, int slot, ia_solve_stats *ss) {
+        float ms = 0;
+        HIPCHK(c, hipEventElapsedTime(&ms, c->ev_solve[slot][0], c->ev_solve[slot][1]));
+        ss->ms = ms;
+        return IA_OK;
+    }
+    static int project_stage(ia_ctx *c, double dtw, ia_solve_stats *ss) {
+        if (int e = project(c, c->u, dtw, ss, 0)) return e;
+        if (!ss) return IA_OK;
+        HIPCHK(c, hipEventSynchronize(c->ev_solve[0][1]));
+        return solve_ms(c, 0, ss);
     }
 
     // ----------------------------------------------------------------- CFL
@@ -1634,13 +1695,13 @@ template <class T> struct Impl {
         finish(c, g.D, U0, U0, 100 * epsT(), false, false);
         if (int e = upd(c, U0, U0, c->fb[fn], c->fb[mid], U1, dt, w)) return e;
         if (int e = mg_update(c)) return e;
-        if (int e = project(c, U1, (double)(w * dt), ss ? &ss->solve[0] : nullptr)) return e;
+        if (int e = project(c, U1, (double)(w * dt), ss ? &ss->solve[0] : nullptr, 0)) return e;
         // corrector (w = 1): f⁰ ← f; ρu = u⁰ρ(f); advect f with u^{n+½}
         prepare(c, c->fb[fn], U0, true, false, false);
         int fnew = advect_fq(c, fn, U1, U1, U0, dt, step_index, fn, -1);
         if (int e = upd(c, U1, U0, c->fb[fnew], c->fb[fnew], U0, dt, T(1))) return e;
         if (int e = mg_update(c)) return e;
-        if (int e = project(c, U0, (double)dt, ss ? &ss->solve[1] : nullptr)) return e;
+        if (int e = project(c, U0, (double)dt, ss ? &ss->solve[1] : nullptr, 1)) return e;
         c->u = U0;
         c->u0 = U1;
         c->fi = fnew;
@@ -1655,6 +1716,8 @@ template <class T> struct Impl {
         int st = read_state(c, ss);
         double nx = std::min(cf, 1.2 * (double)dt);
         if (ss) {
+            for (int q = 0; q < 2; ++q)
+                if (int e = solve_ms(c, q, &ss->solve[q])) return e;
             ss->dt_next = (double)(T)nx;
             ss->vol = vol[0];
             ss->fmin = vol[1];
@@ -1866,7 +1929,8 @@ int ia_create(const ia_params *p, ia_ctx **out) {
     c->g.exitx = p->exit_bc && !(p->perdir & 1);
     c->t = tiling(c->g);
     if (hipSetDevice(c->dev) != hipSuccess || hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreate(&c->e0) != hipSuccess || hipEventCreate(&c->e1) != hipSuccess) {
+        hipEventCreate(&c->ev_solve[0][0]) != hipSuccess || hipEventCreate(&c->ev_solve[0][1]) != hipSuccess ||
+        hipEventCreate(&c->ev_solve[1][0]) != hipSuccess || hipEventCreate(&c->ev_solve[1][1]) != hipSuccess) {
         delete c;
         return IA_ERR_HIP;
     }
@@ -1921,8 +1985,10 @@ void ia_destroy(ia_ctx *c) {
         if (e) (void)hipEventDestroy(e);
     if (c->pin) (void)hipHostFree(c->pin);
     if (c->hst) (void)hipHostFree(c->hst);
-    if (c->e0) (void)hipEventDestroy(c->e0);
-    if (c->e1) (void)hipEventDestroy(c->e1);
+    if (c->hpart) (void)hipHostFree(c->hpart);
+    for (auto &pr : c->ev_solve)
+        for (hipEvent_t e : pr)
+            if (e) (void)hipEventDestroy(e);
     if (c->s) (void)hipStreamDestroy(c->s);
     delete c;
 }
@@ -2045,7 +2111,7 @@ int ia_mg_update(ia_ctx *c) {
 }
 int ia_project(ia_ctx *c, double dt_w, ia_solve_stats *stats) {
     if (stats) memset(stats, 0, sizeof *stats);
-    return dispatch(c, [&](auto impl) { return decltype(impl)::project(c, c->u, dt_w, stats); });
+    return dispatch(c, [&](auto impl) { return decltype(impl)::project_stage(c, dt_w, stats); });
 }
 int ia_synchronize(ia_ctx *c) {
     if (!c) return IA_ERR_BADARG;

@@ -36,7 +36,7 @@ constexpr int CGP_GROUP = 16; // above, the sums of groups of this many, which t
 // cycles/64 before the first look for the sums: a look takes about 1100 cycles and disturbs the words' way, so the
 // first one should find them (64 workgroups, 32^3: 3.0 µs an iteration without, 2.5 with 6, 2.25 with 12, 2.3 with 18)
 constexpr int CGP_NAP = 12;
-constexpr long CGP_WAIT = 100000000;  // ticks of the 100 MHz counter: 1 s
+constexpr long CGP_WAIT = 2000000;  // ticks of the 100 MHz counter: 20 ms
 struct CgpBox {
     int k[3], b[3];  // boxes per axis, cells per box and axis (the last box may have fewer, at least 2)
     int nwg, amax;   // workgroups, the largest face of a box
@@ -391,6 +391,390 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
         if (k < cnt) a.x[I0 + k * sz] = XL ? xl[k * NB + tid] : x[XL ? 0 : k];
 }
 
+// ---------------------------------------------------------------------------
+// WaterLily's pcg! on a level in one launch, on the same boxes and words: two
+// sums an iteration, so two exchanges, the first with the face values of
+// z = A ϵ; the halo cells' r and ϵ follow the owners' recurrence.  With xc it
+// begins with the prolongate! and increment! before it (the coarse x's parents
+// at the cell and its neighbours, on the halo cells too), and on the finest
+// level (r2 set) it ends with what solver! does next: r, z, the next Jacobi!'s
+// ϵ and the workgroups' parts of Σr², in host memory.  x and r are written
+// only after the last exchange, which every workgroup reaches only when all
+// have read their halo, so they are updated in place.
+//
+// 6 iterations on 256x256 (64 workgroups) and on 128x128 were 18 and 13
+// launches of 2.7-3.0 µs, each 4 µs of the host's time, which set the pace.
+// ---------------------------------------------------------------------------
+struct PcgpArgs {
+    Grid g;
+    CgpBox box;
+    const float *L, *iD;
+    float *x, *r, *z, *e;
+    const float *xc;  // the coarser level's x, or nullptr
+    Grid gc;
+    cgp_word *hw, *pw;
+    unsigned tag;
+    int it;
+    double *r2;
+    const int *halt;
+    int *fail;
+};
+// the prolonged x at cell P
+template <int D> __device__ inline float cgp_parent(const PcgpArgs &a, const int P[3]) {
+    return a.xc[(long)((P[0] + 3) / 2 - 1) + a.gc.st[1] * ((P[1] + 3) / 2 - 1) +
+                (D > 2 ? a.gc.st[2] * ((P[2] + 3) / 2 - 1) : 0)];
+}
+template <int D> __device__ inline float cgp_mult_parent(const PcgpArgs &a, const int P[3], long I) {
+    return mgmult_fc<D>(a.g, P, I, a.L, [&](const int *q) { return cgp_parent<D>(a, q); });
+}
+template <int D, int NB, int C, int HC>
+__global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
+    HALT_IF(a)
+    extern __shared__ __align__(16) float cgp_u[];
+    constexpr bool XL = NB * C >= 4096;  // x in LDS, as k_cgp
+    __shared__ float xl[XL ? NB * C : 1];
+    __shared__ double shp[NB / 64], sht;
+    __shared__ int dead;
+    const Grid &g = a.g;
+    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+    // this workgroup's box: first cell lo (ghost-inclusive), sides n
+    int bi[3], lo[3], n[3];
+    {
+        int q = blockIdx.x;
+        bi[0] = q % a.box.k[0];
+        q /= a.box.k[0];
+        bi[1] = q % a.box.k[1];
+        bi[2] = q / a.box.k[1];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        lo[d] = d < D ? 1 + bi[d] * a.box.b[d] : 0;
+        n[d] = d < D ? min(a.box.b[d], g.Ng[d] - 1 - lo[d]) : 1;
+    }
+    const int t1 = a.box.b[0] + 2, t2 = t1 * (a.box.b[1] + 2);  // strides of the u tile
+    const int tz = D > 2 ? t2 : t1;                            // along a column
+    const long sz = g.st[D - 1];
+    if (tid == 0) dead = 0;
+    // own cells: lateral position (x, y), first cell z0 of the column, cnt of them
+    const int nl = D > 2 ? n[0] * n[1] : n[0];
+    const int col = tid % nl, x0 = col % n[0], y0 = D > 2 ? col / n[0] : 0, z0 = (tid / nl) * C;
+    const int cnt = max(0, min(C, n[D - 1] - z0));
+    const int ti = (x0 + 1) + (D > 2 ? t1 * (y0 + 1) : 0) + tz * (z0 + 1);
+    const long I0 = (long)(lo[0] + x0) + (D > 2 ? g.st[1] * (lo[1] + y0) : 0) + sz * (lo[D - 1] + z0);
+    // words of the column's w in the slot: its side face along x (and y), cell k at + k*stride; the faces of its ends
+    const int fb = (int)blockIdx.x * 2 * D;
+    int px = -1, py = -1, pl = -1, ph = -1;
+    const int sx = D > 2 ? n[1] : 1, sy = n[0];
+    if (cnt > 0) {
+        if (x0 == 0 || x0 == n[0] - 1) px = (fb + (x0 ? 1 : 0)) * a.box.amax + (D > 2 ? y0 + n[1] * z0 : z0);
+        if (D > 2 && (y0 == 0 || y0 == n[1] - 1)) py = (fb + 2 + (y0 ? 1 : 0)) * a.box.amax + x0 + n[0] * z0;
+        if (z0 == 0) pl = (fb + 2 * (D - 1)) * a.box.amax + col;
+        if (z0 + cnt == n[D - 1]) ph = (fb + 2 * (D - 1) + 1) * a.box.amax + col;
+    }
+    float r[C], w[C], x[XL ? 1 : C], id[C], u[C], dg[C], lx[C], lxp[C], ly[C], lyp[C], lz[C + 1];
+#pragma unroll
+    for (int k = 0; k <= C; ++k) lz[k] = cnt > 0 && k <= cnt ? a.L[g.ns * (D - 1) + I0 + k * sz] : 0.f;
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+        if (!XL) x[XL ? 0 : k] = 0.f;
+        r[k] = w[k] = id[k] = u[k] = dg[k] = lx[k] = lxp[k] = ly[k] = lyp[k] = 0.f;
+        if (k < cnt) {
+            long I = I0 + k * sz;
+            r[k] = a.r[I];
+            id[k] = a.iD[I];
+            if (XL) xl[k * NB + tid] = a.x[I];
+            else x[XL ? 0 : k] = a.x[I];
+            lx[k] = a.L[I];
+            lxp[k] = a.L[I + 1];
+            dg[k] -= (lx[k] + lxp[k]);
+            if (D > 2) {
+                ly[k] = a.L[g.ns + I];
+                lyp[k] = a.L[g.ns + I + g.st[1]];
+                dg[k] -= (ly[k] + lyp[k]);
+            }
+            dg[k] -= (lz[k] + lz[k + 1]);
+            if (a.xc) {  // prolongate! and increment!
+                const int P[3] = {lo[0] + x0, D > 2 ? lo[1] + y0 : lo[1] + z0 + k, D > 2 ? lo[2] + z0 + k : 0};
+                const float ec = cgp_parent<D>(a, P);
+                r[k] = r[k] - cgp_mult_parent<D>(a, P, I);
+                if (XL) xl[k * NB + tid] += ec;
+                else x[XL ? 0 : k] = x[XL ? 0 : k] + ec;
+            }
+        }
+    }
+    // halo cells of the box's faces (2d + side); none across a wall (u = 0 there, L = 0)
+    bool hon[HC];
+    int hti[HC], hwo[HC];  // place in the tile, word of the cell's w in the slot
+    float hr[HC], hu[HC], hid[HC], hv[HC];
+    {
+        const int area[3] = {n[1] * n[2], n[0] * n[2], n[0] * n[1]};
+        const int hc = 2 * area[0] + 2 * area[1] + (D > 2 ? 2 * area[2] : 0);
+#pragma unroll
+        for (int k = 0; k < HC; ++k) {
+            int h = tid - 64 + k * (NB - 64);
+            hon[k] = false;
+            hti[k] = hwo[k] = 0;
+            hr[k] = hu[k] = hid[k] = hv[k] = 0.f;
+            if (tid >= 64 && h < hc) {
+                int d = 0;
+                if (h >= 2 * area[0]) {
+                    h -= 2 * area[0];
+                    d = 1;
+                    if (D > 2 && h >= 2 * area[1]) {
+                        h -= 2 * area[1];
+                        d = 2;
+                    }
+                }
+                const int ar = d == 0 ? area[0] : d == 1 ? area[1] : area[2];
+                const int side = h >= ar;
+                h -= side * ar;
+                // element h of the face: the two other coordinates in x-y-z order
+                const int m = d == 0 ? n[1] : n[0], e0 = h % m, e1 = h / m;
+                const int qd = side ? (d == 0 ? n[0] : d == 1 ? n[1] : n[2]) : -1;
+                const int q[3] = {d == 0 ? qd : e0, d == 1 ? qd : (d == 0 ? e0 : e1), d == 2 ? qd : e1};
+                hti[k] = (q[0] + 1) + t1 * (q[1] + 1) + (D > 2 ? t2 * (q[2] + 1) : 0);
+                int P[3] = {lo[0] + q[0], lo[1] + q[1], D > 2 ? lo[2] + q[2] : 0}, c[3] = {bi[0], bi[1], bi[2]};
+                bool wall = false;
+#pragma unroll
+                for (int b = 0; b < D; ++b)
+                    if (b == d) {
+                        wall = !g.per[b] && (P[b] == 0 || P[b] == g.Ng[b] - 1);
+                        P[b] = P[b] == 0 ? g.Ng[b] - 2 : P[b] == g.Ng[b] - 1 ? 1 : P[b];
+                        c[b] += side ? 1 : -1;
+                        c[b] = c[b] < 0 ? a.box.k[b] - 1 : c[b] == a.box.k[b] ? 0 : c[b];
+                    }
+                if (wall) {
+                    cgp_u[hti[k]] = 0.f;
+                } else {
+                    hon[k] = true;
+                    long J = (long)P[0] + g.st[1] * P[1] + (D > 2 ? g.st[2] * P[2] : 0);
+                    hr[k] = a.r[J];
+                    hid[k] = a.iD[J];
+                    if (a.xc) hr[k] = hr[k] - cgp_mult_parent<D>(a, P, J);
+                    // the neighbour's facing side holds the same cells in the same order
+                    hwo[k] = ((c[0] + a.box.k[0] * (c[1] + a.box.k[1] * c[2])) * 2 * D + 2 * d + 1 - side) * a.box.amax + h;
+                }
+            }
+        }
+    }
+    const long hslot = (long)a.box.nwg * 2 * D * a.box.amax;
+    const int nwg = a.box.nwg, ngrp = (nwg + CGP_GROUP - 1) / CGP_GROUP;
+    const bool two = nwg > CGP_ONE;
+    auto half_of = [](double v, int j) { return (unsigned)((j & 1) ? __double2hiint(v) : __double2loint(v)); };
+    auto tile = [&]() {  // ϵ of the box and its halo
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+            if (k < cnt) cgp_u[ti + k * tz] = u[k];
+#pragma unroll
+        for (int k = 0; k < HC; ++k)
+            if (hon[k]) cgp_u[hti[k]] = hu[k];
+    };
+    auto publish = [&](unsigned tag, double v) {  // this workgroup's part of a sum
+        v = wave_sum(v);
+        if (lane == 0) shp[wv] = v;
+        __syncthreads();
+        if (wv == 0) {
+            double t = 0;
+#pragma unroll
+            for (int q = 0; q < NB / 64; ++q) t += shp[q];
+            cgp_word *pw = a.pw + (tag & 1 ? CGP_PW : 0) + CGP_P1;
+            if (lane < 2) cgp_put(pw + lane * CGP_MAXWG + blockIdx.x, half_of(t, lane), tag);
+        }
+    };
+    // the sum of m parts (m <= 64) by this wavefront; false: not there in time
+    auto gather = [&](const cgp_word *w2, int st, int m, unsigned tag, double &v) {
+        cgp_word q[2];
+        const long t0 = wall_clock64();
+        for (int spin = 0;; ++spin) {
+            bool ok = true;
+            if (lane < m) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) q[j] = cgp_get(w2 + j * st + lane);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) ok = ok && (unsigned)(q[j] >> 32) == tag;
+            }
+            if (__all(ok)) break;
+            if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
+        }
+        v = wave_sum(lane < m ? __hiloint2double((int)(unsigned)q[1], (int)(unsigned)q[0]) : 0.0);
+        return true;
+    };
+    // the halo cells' z = A ϵ
+    auto halo = [&](const cgp_word *hw, unsigned tag) {
+        cgp_word h[HC];
+        const long t0 = wall_clock64();
+        for (int spin = 0;; ++spin) {
+            bool ok = true;
+#pragma unroll
+            for (int k = 0; k < HC; ++k)
+                if (hon[k]) h[k] = cgp_get(hw + hwo[k]);
+#pragma unroll
+            for (int k = 0; k < HC; ++k)
+                if (hon[k]) ok = ok && (unsigned)(h[k] >> 32) == tag;
+            if (__all(ok)) break;
+            if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
+        }
+#pragma unroll
+        for (int k = 0; k < HC; ++k) hv[k] = hon[k] ? __uint_as_float((unsigned)h[k]) : 0.f;
+        return true;
+    };
+    // the total of a published sum, in FP32 (and the halo with it); false: gave up
+    auto total = [&](unsigned tag, const cgp_word *hw, float &out) {
+        cgp_word *pw = a.pw + (tag & 1 ? CGP_PW : 0);
+        bool ok = true;
+        if (wv == 0) {
+            double v = 0;
+            __builtin_amdgcn_s_sleep(CGP_NAP);
+            if (two) {
+                if (blockIdx.x % CGP_GROUP == 0) {
+                    ok = gather(pw + CGP_P1 + blockIdx.x, CGP_MAXWG, min(CGP_GROUP, nwg - (int)blockIdx.x), tag, v);
+                    if (ok && (lane & 2) == 0)
+                        cgp_put(pw + lane * CGP_ONE + blockIdx.x / CGP_GROUP, half_of(v, lane), tag);
+                }
+                if (ok) ok = gather(pw + (blockIdx.x % CGP_COPY) * 4 * CGP_ONE, CGP_ONE, ngrp, tag, v);
+            } else {
+                ok = gather(pw + CGP_P1, CGP_MAXWG, nwg, tag, v);
+            }
+            if (lane == 0) sht = v;
+        } else if (hw) {
+            ok = halo(hw, tag);
+        }
+        if (!ok) dead = 1;
+        __syncthreads();
+        out = (float)sht;
+        return dead == 0;
+    };
+    // z = ϵ = r·iD, ρ = r·z
+    double v = 0;
+#pragma unroll
+    for (int k = 0; k < C; ++k)
+        if (k < cnt) {
+            u[k] = r[k] * id[k];
+            v = __builtin_fma((double)r[k], (double)u[k], v);  // the products are exact
+        }
+#pragma unroll
+    for (int k = 0; k < HC; ++k)
+        if (hon[k]) hu[k] = hr[k] * hid[k];
+    tile();
+    publish(a.tag, v);
+    float rho = 0;
+    bool ok = total(a.tag, nullptr, rho);
+    bool done = !ok || fabs(rho) < 10 * eps_of<float>();
+    const bool zset = !done;
+    for (int i = 1; i <= a.it && !done; ++i) {
+        // z = A ϵ, published at the box's faces; z·ϵ (total's barrier came after the tile's last write)
+        const unsigned ta = a.tag + 2 * i - 1, tb = ta + 1;
+        cgp_word *hw = a.hw + (i & 1 ? hslot : 0);
+        v = 0;
+        if (cnt > 0) {
+            const float ulo = cgp_u[ti - tz], uhi = cgp_u[ti + cnt * tz];
+#pragma unroll
+            for (int k = 0; k < C; ++k)
+                if (k < cnt) {
+                    const int t = ti + k * tz;
+                    float sl = 0, su = 0;
+                    sl += cgp_u[t - 1] * lx[k];
+                    su += cgp_u[t + 1] * lxp[k];
+                    if (D > 2) {
+                        sl += cgp_u[t - t1] * ly[k];
+                        su += cgp_u[t + t1] * lyp[k];
+                    }
+                    const float um = k > 0 ? u[k > 0 ? k - 1 : 0] : ulo;
+                    float up = uhi;
+                    if (k + 1 < C) {
+                        float un = u[k + 1 < C ? k + 1 : k];
+                        up = k + 1 < cnt ? un : uhi;
+                    }
+                    sl += um * lz[k];
+                    su += up * lz[k + 1];
+                    w[k] = (u[k] * dg[k] + sl) + su;
+                }
+            if (px >= 0) {
+#pragma unroll
+                for (int k = 0; k < C; ++k)
+                    if (k < cnt) cgp_put(hw + px + k * sx, __float_as_uint(w[k]), ta);
+            }
+            if (D > 2 && py >= 0) {
+#pragma unroll
+                for (int k = 0; k < C; ++k)
+                    if (k < cnt) cgp_put(hw + py + k * sy, __float_as_uint(w[k]), ta);
+            }
+            if (pl >= 0) cgp_put(hw + pl, __float_as_uint(w[0]), ta);
+            if (ph >= 0) {
+#pragma unroll
+                for (int k = 0; k < C; ++k)
+                    if (k == cnt - 1) cgp_put(hw + ph, __float_as_uint(w[k]), ta);
+            }
+#pragma unroll
+            for (int k = 0; k < C; ++k)
+                if (k < cnt) v = __builtin_fma((double)w[k], (double)u[k], v);
+        }
+        publish(ta, v);
+        float ze;
+        if (!total(ta, hw, ze)) {
+            ok = false;
+            break;
+        }
+        const float alpha = rho / ze;
+        v = 0;
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+            if (k < cnt) {
+                if (XL) xl[k * NB + tid] += alpha * u[k];
+                else x[XL ? 0 : k] = x[XL ? 0 : k] + alpha * u[k];
+                r[k] = r[k] - alpha * w[k];
+                w[k] = r[k] * id[k];
+                v = __builtin_fma((double)r[k], (double)w[k], v);
+            }
+        if (i == a.it || fabs((double)alpha) < 1e-2) break;
+        publish(tb, v);
+        float rho2;
+        if (!total(tb, nullptr, rho2)) {
+            ok = false;
+            break;
+        }
+        if (fabs(rho2) < 10 * eps_of<float>()) break;
+        const float beta = rho2 / rho;
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+            if (k < cnt) u[k] = beta * u[k] + w[k];
+#pragma unroll
+        for (int k = 0; k < HC; ++k)
+            if (hon[k]) {
+                hr[k] = hr[k] - alpha * hv[k];
+                hu[k] = beta * hu[k] + hr[k] * hid[k];
+            }
+        tile();
+        __syncthreads();
+        rho = rho2;
+    }
+    if (!ok && tid == 0) *a.fail = 1;
+    v = 0;
+#pragma unroll
+    for (int k = 0; k < C; ++k)
+        if (k < cnt) {
+            const long I = I0 + k * sz;
+            a.x[I] = XL ? xl[k * NB + tid] : x[XL ? 0 : k];
+            if (a.r2) {
+                a.r[I] = r[k];
+                const float zz = r[k] * id[k];
+                if (zset) a.z[I] = zz;
+                a.e[I] = zz;
+                v = __builtin_fma((double)r[k], (double)r[k], v);
+            }
+        }
+    if (a.r2) {
+        v = wave_sum(v);
+        __syncthreads();
+        if (lane == 0) shp[wv] = v;
+        __syncthreads();
+        if (tid == 0) {
+            double t = 0;
+            for (int q = 0; q < NB / 64; ++q) t += shp[q];
+            a.r2[blockIdx.x] = t;
+        }
+    }
+}
 // The variants: threads and cells per thread, the fewest first, as more cells per workgroup cost more than more
 // workgroups up to CGP_ONE (32^3: 2.25 µs with 2 cells on 256 threads, 2.7 with 4 on 512, 2.8 with 4 on 1024).
 struct CgpVariant {
@@ -404,6 +788,14 @@ inline const CgpVariant *cgp_variants(int &n) {
                                    {3, 512, 4, 3, k_cgp<3, 512, 4, 3>}, {3, 1024, 4, 2, k_cgp<3, 1024, 4, 2>}};
     n = 8;
     return v;
+}
+// pcg! in one launch: the variant of cgp_variants with the same number
+typedef void (*PcgpKernel)(PcgpArgs);
+inline PcgpKernel pcgp_kernel(int q) {
+    static const PcgpKernel k[] = {k_pcgp<2, 256, 1, 1>, k_pcgp<2, 256, 2, 1>, k_pcgp<2, 512, 4, 1>,
+                                   k_pcgp<2, 1024, 4, 1>, k_pcgp<3, 256, 1, 2>, k_pcgp<3, 256, 2, 3>,
+                                   k_pcgp<3, 512, 4, 3>, k_pcgp<3, 1024, 4, 2>};
+    return k[q];
 }
 // boxes of a level of n cells per axis for a variant, at most maxwg of them; false: none fits
 inline bool cgp_boxes(const int *n, const CgpVariant &v, int maxwg, CgpBox &o) {

@@ -178,6 +178,9 @@ struct StepState {
 struct StepOut {
     double cfl[5];  // the two CFL maxima, Σf, min f, max f
     StepState st;
+    int fail;       // workgroups of a one-launch coarse solve did not run together
+    int pad;
+    double r2[256]; // the parts of Σr² of a one-launch pcg!
 };
 struct SolveCtl {
     double rho, alpha, beta, s, r2, dot;

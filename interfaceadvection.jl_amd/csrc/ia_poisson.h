@@ -64,9 +64,8 @@ struct PcgState {
 struct FcgState {
     double sload, wr, beta, pq, alpha;
     double rr;      // ‖r‖² after the last accepted update
-    int halt;       // set when the recursive residual met the tolerance:
+    int halt, pad;  // set when the recursive residual met the tolerance:
                     // every solver kernel queued after that returns at once
-    int fail;       // set when workgroups of a k_cgp launch did not run together
 };
 
 // every block of a consumer sums the producer's per-block partials itself
@@ -454,7 +453,8 @@ __global__ void __launch_bounds__(NT) k_mg_resid(LevV<T> l, double *part) {
     })
     block_partial(v, l.t, part);
 }
-// residual! part 2: r -= mean when |mean| > 2eps (sub), fused with partial r·r
+// residual! part 2: r -= mean when |mean| > 2eps (sub), fused with partial
+// r·r and with Jacobi!'s ϵ = r·iD of the V-cycle that may follow
 template <class T>
 __global__ void __launch_bounds__(NT) k_mg_center_l2(LevV<T> l, const double *part_in, long ncell, int sub,
                                                      double *part) {
@@ -471,6 +471,7 @@ __global__ void __launch_bounds__(NT) k_mg_center_l2(LevV<T> l, const double *pa
             rr = rr - m;
             l.r[I] = rr;
         }
+        l.e[I] = rr * l.iD[I];
         v += (double)rr * (double)rr;
     })
     block_partial(v, l.t, part);

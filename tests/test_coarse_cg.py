@@ -1,4 +1,4 @@
-"""The coarse CG in one launch (ia_cgp.h) against one launch per iteration
+"""The coarse CG and pcg! in one launch (ia_cgp.h) against one launch per iteration
 (IA_CG1_NB set), which evaluates the same recurrence: whole projections to
 1e-6 from the same inputs, on grids whose coarse levels meet every edge of
 the boxes: levels that the boxes do not divide, sides of 2 cells, sides that
@@ -22,12 +22,12 @@ pytestmark = pytest.mark.gpu
 ia = load_package()
 
 
-def projected(dims, perdir, launched):
+def projected(dims, perdir, launched, **kw):
     old = os.environ.get("IA_CG1_NB")
     if launched:
         os.environ["IA_CG1_NB"] = "256"
     try:
-        s = ia.TwoPhaseSimulation(dims, (0.0,) * len(dims), float(dims[-1]), T=np.float32, poisson="refined", perdir=perdir)
+        s = ia.TwoPhaseSimulation(dims, (0.0,) * len(dims), float(dims[-1]), T=np.float32, perdir=perdir, **kw)
     finally:
         if launched:
             del os.environ["IA_CG1_NB"]
@@ -54,7 +54,7 @@ def projected(dims, perdir, launched):
     s._call("ia_mg_update")
     st = ia.IASolveStats()
     s._call("ia_project", 1.0, C.byref(st))
-    out = s.flow.u.astype(np.float64), s.flow.p.astype(np.float64), st.iters, st.rel
+    out = s.flow.u.astype(np.float64), s.flow.p.astype(np.float64), st.iters, st.rel, s.flow.σ.astype(np.float64), st.r2
     s.close()
     return out
 
@@ -66,10 +66,31 @@ def projected(dims, perdir, launched):
 ])
 def test_one_launch_equals_one_launch_per_iteration(dims, perdir):
     say("coarse CG in one launch", dims, perdir)
-    u, p, it, rel = projected(dims, perdir, False)
-    ul, pl, itl, rell = projected(dims, perdir, True)
+    u, p, it, rel, _, _ = projected(dims, perdir, False, poisson="refined")
+    ul, pl, itl, rell, _, _ = projected(dims, perdir, True, poisson="refined")
     print(f"iterations {it} / {itl}, rel {rel:.3e} / {rell:.3e}, max|Δu| {np.abs(u - ul).max():.2e}, "
           f"max|Δp| {np.abs(p - pl).max():.2e} of {np.abs(pl).max():.2e}")
     assert 0 < rel <= 1e-6 and abs(it - itl) <= 1
     assert np.abs(u - ul).max() <= 1e-5 * np.abs(ul).max()
     assert np.abs(p - pl).max() <= 1e-4 * np.abs(pl).max()
+
+
+@pytest.mark.parametrize("dims,perdir", [
+    ((64, 64), (1, 2)), ((256, 200), ()), ((1000, 24), (2,)), ((512, 512), ()), ((1024, 640), (1,)),
+    ((48, 32, 40), ()), ((100, 60, 84), (1, 3)), ((64, 64, 64), ()), ((96, 96, 96), (2,)),
+])
+def test_default_solver_in_one_launch(dims, perdir):
+    """pcg! on the finest and the coarse levels in one launch each against its
+    launches, over three V-cycles of the default solver that it does not end
+    earlier: u, p, the scratch that Flow.σ holds afterwards, and Σr² (FP64
+    parts of FP32 values) to the bars above."""
+    say("pcg! in one launch", dims, perdir)
+    kw = dict(poisson="reference", poisson_tol=1e-12, poisson_itmx=3)
+    u, p, it, _, z, r2 = projected(dims, perdir, False, **kw)
+    ul, pl, itl, _, zl, r2l = projected(dims, perdir, True, **kw)
+    print(f"Σr² {r2:.6e} / {r2l:.6e}, max|Δu| {np.abs(u - ul).max():.2e}, max|Δp| {np.abs(p - pl).max():.2e}")
+    assert it == itl == 3
+    assert abs(r2 - r2l) <= 1e-4 * r2l
+    assert np.abs(u - ul).max() <= 1e-5 * np.abs(ul).max()
+    assert np.abs(p - pl).max() <= 1e-4 * np.abs(pl).max()
+    assert np.abs(z - zl).max() <= 1e-4 * np.abs(zl).max()
