@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(NT) k_prepare(Grid g, Tiling t, const T *__res
     if (!thread_cell(g, t, p)) return;
     long I = lin(g, p);
     int8_t c = f[I] < T(0.5) ? 0 : 1;
-    write_images<int8_t>(g, cb, p, c, 0, 0, 0);
+    write_row<int8_t>(g, cb, p, I, c);
     if (do_ru)
         for (int d = 0; d < g.D; ++d) {
             long o = g.ns * d;
@@ -336,8 +336,8 @@ __global__ void __launch_bounds__(NT) k_vof_update(SweepArgs<T> a, const T *__re
         fv = (double)fnew;
         fi = I;
         T fc = fnew < a.ctol ? T(0) : (fnew > 1 - a.ctol ? T(1) : fnew);
-        write_images<T>(g, a.fout, p, fc, 0, 0, T(0));
-        if (a.fmid) write_images<T>(g, a.fmid, p, (fc + a.fn[I]) / 2, 0, 0, T(0));
+        write_row<T>(g, a.fout, p, I, fc);
+        if (a.fmid) write_row<T>(g, a.fmid, p, I, (fc + a.fn[I]) / 2);
     }
     FillPart r = block_fill_cells(fv, fi, fok, fnan);
     if (threadIdx.x == 0) a.part[blockIdx.x] = r;
@@ -942,8 +942,8 @@ __global__ void __launch_bounds__(NT) k_visc_update(UpdArgs<T> a) {
     for (int i = 0; i < D; ++i) {
         // exitBC: updateU!'s axpy! (flow.jl:251) is the only update of the exit face
         T xv = i == 0 && g.exitx ? a.v.u[I + g.st[0]] + (a.dt * wT) * a.g[0] : T(0);
-        write_images<T>(g, a.uout + g.ns * i, p, un[i], 2, i, a.v.ubc[i], xv);
-        write_images<T>(g, a.L + g.ns * i, p, T(1) / rh[i], 1, i, T(0));
+        write_row_u<T>(g, a.uout + g.ns * i, p, I, un[i], true, i, a.v.ubc[i], xv);
+        write_row_u<T>(g, a.L + g.ns * i, p, I, T(1) / rh[i], false, i, T(0));
     }
 }
 // viscSurfTenρu! alone (stage entry point): Flow.f = visc
@@ -965,7 +965,7 @@ __global__ void __launch_bounds__(NT) k_update_L(Grid g, Tiling t, const T *f, T
     if (!thread_cell(g, t, p)) return;
     long I = lin(g, p);
     for (int i = 0; i < g.D; ++i)
-        write_images<T>(g, L + g.ns * i, p, T(1) / linp((f[I] + f[I - g.st[i]]) / 2, lr), 1, i, T(0));
+        write_row_u<T>(g, L + g.ns * i, p, I, T(1) / linp((f[I] + f[I - g.st[i]]) / 2, lr), false, i, T(0));
 }
 
 // z = div(u); (flow.jl:345)
@@ -1088,7 +1088,7 @@ __global__ void __launch_bounds__(NT) k_project(Grid g, Tiling t, T *u, const T 
         T dx = x[I] - xper(g, x, q[0], q[1], q[2]);
         T un = u[g.ns * i + I] - L[g.ns * i + I] * dx;
         T xv = i == 0 && g.exitx ? u[I + g.st[0]] : T(0);  // exitBC: the exit face is left alone
-        write_images<T>(g, u + g.ns * i, p, un, 2, i, ub[i], xv);
+        write_row_u<T>(g, u + g.ns * i, p, I, un, true, i, ub[i], xv);
     }
 }
 // f⁰ = (f⁰ + f)/2 over every cell (flow.jl:74)
