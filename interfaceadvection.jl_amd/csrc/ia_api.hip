@@ -17,6 +17,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <mutex>
 #include <vector>
@@ -111,6 +112,7 @@ struct ia_ctx {
     int cit_wl[MAXLEV], cit_fcg[MAXLEV];
     unsigned long long *cgp_hw = nullptr, *cgp_pw = nullptr;  // the one-launch coarse CG's words
     unsigned cgp_tag = 1;  // next unused tag of those words
+    int xcd = 0;           // where launches of few workgroups run: contexts take the XCDs in turn
     bool pcgp = false;     // solver!'s pcg! in one launch (k_pcgp)
     bool cgp_off = false;  // one launch per iteration instead (IA_CG1_NB set, or workgroups did not run together)
     int cg1_nb[MAXLEV];  // workgroup size of the coarse CG step per level (one cell per thread)
@@ -572,9 +574,12 @@ template <class T> struct Impl {
                     int per = 0;
                     HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(
                                   &per, c->pcgp ? (const void *)pcgp_kernel(q) : (const void *)vs[q].k, vs[q].NB,
-                                  cgp_lds(lv)));
+                                  cgp_lds(lv, vs[q].C)));
                     if ((long)per * ncu < (maxwg > CGP_ONE ? 1L : 2L) * lv.cgp_box.nwg) continue;
                     lv.cgp = &vs[q];
+                    // on one XCD where there is room for two such launches
+                    const bool near = maxwg <= CGP_ONE && vs[q].NB < 1024 && per * CGP_XCU >= 2 * lv.cgp_box.nwg;
+                    lv.cgp_box.spread = near ? CGP_XCDS : 1;
                 }
             if (lv.cgp)
                 words = std::max(words, (size_t)2 * lv.cgp_box.nwg * 2 * lv.g.D * lv.cgp_box.amax);
@@ -586,9 +591,10 @@ template <class T> struct Impl {
         return IA_OK;
     }
     static bool cgp_failed(const ia_ctx *c) { return *(volatile int *)&c->hst->fail != 0; }
-    static size_t cgp_lds(const Level &l) {
+    static size_t cgp_lds(const Level &l, int C) {
         const CgpBox &b = l.cgp_box;
-        return sizeof(float) * (b.b[0] + 2) * (b.b[1] + 2) * (l.g.D > 2 ? b.b[2] + 2 : 1);
+        const int t1 = b.b[0] + 2, t2 = t1 * (b.b[1] + 2), tz = l.g.D > 2 ? t2 : t1;
+        return 2 * sizeof(float) * (t2 * (l.g.D > 2 ? b.b[2] + 2 : 1) + (C - 1) * tz + 1);  // the tiles of u and w
     }
     // ----------------------------------------------------------------- MG
     static int mg_update(ia_ctx *c) {
@@ -664,6 +670,8 @@ template <class T> struct Impl {
         a.gc = prolong ? (&l)[1].g : l.g;
         a.hw = c->cgp_hw;
         a.pw = c->cgp_pw;
+        a.spread = a.box.spread;
+        a.xcd = a.spread > 1 ? c->xcd : 0;
         a.tag = c->cgp_tag;
         c->cgp_tag += 2 * (unsigned)it + 2;
         a.it = it;
@@ -671,8 +679,8 @@ template <class T> struct Impl {
         a.halt = cur_halt;
         a.fail = &c->hst->fail;
         int nv;
-        hipLaunchKernelGGL(pcgp_kernel((int)(l.cgp - cgp_variants(nv))), dim3((unsigned)a.box.nwg),
-                           dim3((unsigned)l.cgp->NB), cgp_lds(l), c->s, a);
+        hipLaunchKernelGGL(pcgp_kernel((int)(l.cgp - cgp_variants(nv))), dim3((unsigned)(a.box.nwg * a.spread)),
+                           dim3((unsigned)l.cgp->NB), cgp_lds(l, l.cgp->C), c->s, a);
     }
     static void pcg(ia_ctx *c, Level &l, int it = 6, bool init_done = false, const FcgV<T> *last = nullptr,
                     int first = 0) {
@@ -748,13 +756,16 @@ template <class T> struct Impl {
             a.x = P<float>(l.x);
             a.hw = c->cgp_hw;
             a.pw = c->cgp_pw;
+            a.spread = a.box.spread;
+            a.xcd = a.spread > 1 ? c->xcd : 0;
             a.tag = c->cgp_tag;
             c->cgp_tag += (unsigned)it + 1;
             a.it = it;
             a.halt = cur_halt;
             a.fail = &c->hst->fail;
             if (pc >= 0) prof_begin(c, pc);
-            hipLaunchKernelGGL(l.cgp->k, dim3((unsigned)a.box.nwg), dim3((unsigned)l.cgp->NB), cgp_lds(l), c->s, a);
+            hipLaunchKernelGGL(l.cgp->k, dim3((unsigned)(a.box.nwg * a.spread)), dim3((unsigned)l.cgp->NB),
+                               cgp_lds(l, l.cgp->C), c->s, a);
             if (pc >= 0) prof_end(c, pc);
             return;
         }
@@ -1875,6 +1886,8 @@ int ia_create(const ia_params *p, ia_ctx **out) {
     if (c->P.poisson_rtol <= 0) c->P.poisson_rtol = 1e-6;
     if (c->P.poisson_max_outer <= 0) c->P.poisson_max_outer = 100;
     c->dev = p->device;
+    static std::atomic<unsigned> created{0};
+    c->xcd = (int)(created++ % CGP_XCDS);
     c->es = p->dtype == IA_F64 ? 8 : 4;
     if (const char *sv = getenv("IA_FCG_SMOOTH"); sv && *sv) {
         c->smooth_it = std::max(0, std::min(CIT_MAX, atoi(sv)));

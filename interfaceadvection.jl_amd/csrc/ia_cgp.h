@@ -21,25 +21,34 @@ namespace ia {
 // partial of the iteration between, which each of them publishes only after
 // it has read the slot's words.
 //
-// Measured against one launch per iteration, µs per iteration of 64: 64^3 3.84 against 6.6-7.5, 32^3 2.25 against
-// 4.6, 60x44x36 2.9 against 5.4, 192x128 2.0 against 4.5, 96x64 1.8 against 4.3.  What is left is about 1 µs from
-// one workgroup's store to another's load (past the L2s of the eight XCDs) and as much for the operator, the
-// recurrence and the sums.
+// Up to CGP_ONE workgroups of the smaller kind run on one XCD if they fit there: of CGP_XCDS times as many only every
+// CGP_XCDS'th takes part, and they say where they run with the first sum.  All on one, the words need only reach its L2:
+// store to load 0.5 µs instead of 0.8 past the L2s of the eight XCDs (0.47 against 1.27 with 64 workgroups reading
+// everyone's).  Each context has an XCD of its own in turn, so that contexts do not wait for one another's places.
+//
+// Measured, µs per iteration of 64, one launch per iteration / here: 64^3 6.6-7.5 / 2.7, 60x44x36 5.4 / 2.2, 32^3 4.6 /
+// 1.55, 192x128 4.5 / 1.3, 96x64 4.3 / 1.2.  What is left is the exchange and as much again for the operator, the
+// recurrence and the two sums, a chain of some 2000 cycles in which a wavefront mostly waits for itself: nothing in it
+// stands behind a branch, faces are published through a tile, and a workgroup's words of a sum lie together.
 //
 // A workgroup that waits longer than CGP_WAIT (another program's work kept
 // some workgroups off the device) writes the x it has, raises *fail and ends,
 // so the launch always ends; x is then a less exact solution.
 // ---------------------------------------------------------------------------
 constexpr int CGP_MAXWG = 256;
+constexpr int CGP_XCDS = 8;   // workgroups go to the XCDs in turn, so those of every eighth number share one
+constexpr int CGP_XCU = 32;   // compute units of an XCD
 constexpr int CGP_ONE = 64;   // up to so many workgroups everyone reads every partial sum
 constexpr int CGP_GROUP = 16; // above, the sums of groups of this many, which the group's first workgroup forms
-// cycles/64 before the first look for the sums: a look takes about 1100 cycles and disturbs the words' way, so the
-// first one should find them (64 workgroups, 32^3: 3.0 µs an iteration without, 2.5 with 6, 2.25 with 12, 2.3 with 18)
+// cycles/64 before the first look for the sums past the L2s: a look takes about 1100 cycles and disturbs the words' way,
+// so the first one should find them (64 workgroups, 32^3: 3.0 µs an iteration without, 2.5 with 6, 2.25 with 12, 2.3
+// with 18); within one L2 waiting first gains nothing
 constexpr int CGP_NAP = 12;
 constexpr long CGP_WAIT = 2000000;  // ticks of the 100 MHz counter: 20 ms
 struct CgpBox {
     int k[3], b[3];  // boxes per axis, cells per box and axis (the last box may have fewer, at least 2)
     int nwg, amax;   // workgroups, the largest face of a box
+    int spread;      // CGP_XCDS: they fit on one XCD, else 1
 };
 struct CgpArgs {
     Grid g;
@@ -50,39 +59,85 @@ struct CgpArgs {
     unsigned long long *pw;  // 2 slots of CGP_PW words: the partial sums, then the groups' sums
     unsigned tag;            // of iteration 0
     int it;
+    int spread, xcd;  // of spread workgroups one takes part, those of blockIdx.x % spread == xcd
     const int *halt;
     int *fail;
 };
-// a slot of partial sums: CGP_COPY copies of 4 words of CGP_ONE workgroups (or groups), then
-// 4 words of CGP_MAXWG workgroups of a group
+// a slot of partial sums: 4 words for each workgroup of a group in CGP_COPY copies, then 4 words for each workgroup
 constexpr int CGP_COPY = 16;
 constexpr int CGP_P1 = CGP_COPY * 4 * CGP_ONE;
-constexpr int CGP_PW = CGP_P1 + 4 * CGP_MAXWG;
+constexpr int CGP_PW = CGP_P1 + 5 * CGP_MAXWG;  // the fifth: the XCD (a launch's first sum, if it asked for one)
 typedef unsigned long long cgp_word;
-__device__ inline void cgp_put(cgp_word *p, unsigned v, unsigned tag) {
-    __hip_atomic_store(p, ((cgp_word)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+constexpr int CGP_SC0 = 1, CGP_VOLATILE = (int)0x80000000u;  // of a buffer load's last argument
+// near: all workgroups run on one XCD, so a word need only reach its L2: a store of workgroup scope goes there, and a
+// load with sc0 set reads from there (an atomic load of workgroup scope may be served by the compute unit's own cache:
+// it is compiled without sc0).  Should a load ever take an old word, its tag shows it.
+__device__ inline void cgp_put(cgp_word *p, unsigned v, unsigned tag, bool near) {
+    const cgp_word q = ((cgp_word)tag << 32) | v;
+    if (near) __hip_atomic_store(p, q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else __hip_atomic_store(p, q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ inline cgp_word cgp_get(const cgp_word *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// word i of p (the same for the wavefront)
+__device__ inline cgp_word cgp_get(const cgp_word *p, int i, bool near) {
+    if (!near) return __hip_atomic_load(p + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    typedef unsigned v2 __attribute__((ext_vector_type(2)));
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, 0x7ffffff8, 0x00027000);
+    const v2 q = __builtin_amdgcn_raw_buffer_load_b64(rs, i * (int)sizeof(cgp_word), 0, CGP_SC0 | CGP_VOLATILE);
+    return ((cgp_word)q[1] << 32) | q[0];
 }
-
-
+// words i to i + N - 1 (i a multiple of N = 2 or 4)
+template <int N> __device__ inline void cgp_getn(const cgp_word *p, int i, cgp_word (&v)[N], bool near) {
+    if (near) {
+        typedef unsigned v4 __attribute__((ext_vector_type(4)));
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, 0x7ffffff8, 0x00027000);
+#pragma unroll
+        for (int j = 0; j < N; j += 2) {
+            const v4 q = __builtin_amdgcn_raw_buffer_load_b128(rs, (i + j) * (int)sizeof(cgp_word), 0,
+                                                               CGP_SC0 | CGP_VOLATILE);
+            v[j] = ((cgp_word)q[1] << 32) | q[0];
+            v[j + 1] = ((cgp_word)q[3] << 32) | q[2];
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) v[j] = __hip_atomic_load(p + i + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+// the XCD this wavefront runs on (HW_REG_XCC_ID)
+__device__ inline unsigned cgp_xcd() { return __builtin_amdgcn_s_getreg(20 | (3 << 11)); }
+// whether the nwg (<= CGP_ONE) workgroups said that they run on this wavefront's XCD; w: their words of that, written
+// with those of the sum just gathered.  Every workgroup comes to the same answer.
+__device__ inline bool cgp_near(const cgp_word *w, int nwg, unsigned tag) {
+    const int lane = threadIdx.x & 63;
+    const long t0 = wall_clock64();
+    for (;;) {
+        bool here = true, same = true;
+        for (int q = lane; q < nwg; q += 64) {
+            const cgp_word v = cgp_get(w, q, false);
+            here = here && (unsigned)(v >> 32) == tag;
+            same = same && (unsigned)v == cgp_xcd();
+        }
+        if (__all(here)) return __all(same);
+        if (wall_clock64() - t0 > CGP_WAIT) return false;
+    }
+}
 // NB threads; a thread owns a column of C cells along the last axis (so two of a cell's neighbours are mostly its own
 // registers); the halo cells are those of wavefronts 1.. (HC each), while wavefront 0 waits for the sums.
 template <int D, int NB, int C, int HC>
 __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     HALT_IF(a)
+    if ((int)blockIdx.x % a.spread != a.xcd) return;
+    const int wg = (int)blockIdx.x / a.spread;
     extern __shared__ __align__(16) float cgp_u[];
     constexpr bool XL = NB * C >= 4096;  // x in LDS: the registers of a 1024-thread workgroup do not hold it
     __shared__ float xl[XL ? NB * C : 1];
     __shared__ double shp[2][NB / 64], sht[2];
-    __shared__ int dead;
+    __shared__ int dead, nears;
     const Grid &g = a.g;
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
     // this workgroup's box: first cell lo (ghost-inclusive), sides n
     int bi[3], lo[3], n[3];
     {
-        int q = blockIdx.x;
+        int q = wg;
         bi[0] = q % a.box.k[0];
         q /= a.box.k[0];
         bi[1] = q % a.box.k[1];
@@ -96,29 +151,28 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     const int t1 = a.box.b[0] + 2, t2 = t1 * (a.box.b[1] + 2);  // strides of the u tile
     const int tz = D > 2 ? t2 : t1;                            // along a column
     const long sz = g.st[D - 1];
+    // every thread works on all C cells of its column: those past its cnt are all zeros, read the tile's spare planes
+    // and write its last word, so no load or store waits behind a branch
+    const int dump = t1 * (a.box.b[1] + 2) * (D > 2 ? a.box.b[2] + 2 : 1) + (C - 1) * tz;
+    for (int q = tid; q <= dump; q += NB) cgp_u[q] = 0.f;
     if (tid == 0) dead = 0;
+    __syncthreads();
     // own cells: lateral position (x, y), first cell z0 of the column, cnt of them
     const int nl = D > 2 ? n[0] * n[1] : n[0];
     const int col = tid % nl, x0 = col % n[0], y0 = D > 2 ? col / n[0] : 0, z0 = (tid / nl) * C;
     const int cnt = max(0, min(C, n[D - 1] - z0));
-    const int ti = (x0 + 1) + (D > 2 ? t1 * (y0 + 1) : 0) + tz * (z0 + 1);
+    const int ti = (x0 + 1) + (D > 2 ? t1 * (y0 + 1) : 0) + tz * (cnt > 0 ? z0 + 1 : 1);
+    int tw[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) tw[k] = k < cnt ? ti + k * tz : dump;
     const long I0 = (long)(lo[0] + x0) + (D > 2 ? g.st[1] * (lo[1] + y0) : 0) + sz * (lo[D - 1] + z0);
-    // words of the column's w in the slot: its side face along x (and y), cell k at + k*stride; the faces of its ends
-    const int fb = (int)blockIdx.x * 2 * D;
-    int px = -1, py = -1, pl = -1, ph = -1;
-    const int sx = D > 2 ? n[1] : 1, sy = n[0];
-    if (cnt > 0) {
-        if (x0 == 0 || x0 == n[0] - 1) px = (fb + (x0 ? 1 : 0)) * a.box.amax + (D > 2 ? y0 + n[1] * z0 : z0);
-        if (D > 2 && (y0 == 0 || y0 == n[1] - 1)) py = (fb + 2 + (y0 ? 1 : 0)) * a.box.amax + x0 + n[0] * z0;
-        if (z0 == 0) pl = (fb + 2 * (D - 1)) * a.box.amax + col;
-        if (z0 + cnt == n[D - 1]) ph = (fb + 2 * (D - 1) + 1) * a.box.amax + col;
-    }
     float r[C], s[C], w[C], p[C], x[XL ? 1 : C], id[C], u[C], dg[C], lx[C], lxp[C], ly[C], lyp[C], lz[C + 1];
 #pragma unroll
     for (int k = 0; k <= C; ++k) lz[k] = cnt > 0 && k <= cnt ? a.L[g.ns * (D - 1) + I0 + k * sz] : 0.f;
 #pragma unroll
     for (int k = 0; k < C; ++k) {
-        if (!XL) x[XL ? 0 : k] = 0.f;
+        if (XL) xl[k * NB + tid] = 0.f;
+        else x[XL ? 0 : k] = 0.f;
         r[k] = s[k] = w[k] = p[k] = id[k] = u[k] = dg[k] = lx[k] = lxp[k] = ly[k] = lyp[k] = 0.f;
         if (k < cnt) {
             long I = I0 + k * sz;
@@ -138,8 +192,11 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
         }
     }
     // halo cells of the box's faces (2d + side); none across a wall (u = 0 there, L = 0)
-    bool hon[HC];
+    // the same threads publish the cells on this side of the faces
+    bool hon[HC], fon[HC];
     int hti[HC], hwo[HC];  // place in the tile, word of the cell's w in the slot
+    int fti[HC], fwo[HC];
+    float *const cgp_w = cgp_u + dump + 1;  // a tile of w
     float hr[HC], hs[HC], hid[HC], hv[HC];
     {
         const int area[3] = {n[1] * n[2], n[0] * n[2], n[0] * n[1]};
@@ -147,8 +204,9 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
 #pragma unroll
         for (int k = 0; k < HC; ++k) {
             int h = tid - 64 + k * (NB - 64);
-            hon[k] = false;
-            hti[k] = hwo[k] = 0;
+            hon[k] = fon[k] = false;
+            hti[k] = fti[k] = dump;
+            hwo[k] = fwo[k] = 0;
             hr[k] = hs[k] = hid[k] = hv[k] = 0.f;
             if (tid >= 64 && h < hc) {
                 int d = 0;
@@ -167,7 +225,10 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
                 const int m = d == 0 ? n[1] : n[0], e0 = h % m, e1 = h / m;
                 const int qd = side ? (d == 0 ? n[0] : d == 1 ? n[1] : n[2]) : -1;
                 const int q[3] = {d == 0 ? qd : e0, d == 1 ? qd : (d == 0 ? e0 : e1), d == 2 ? qd : e1};
-                hti[k] = (q[0] + 1) + t1 * (q[1] + 1) + (D > 2 ? t2 * (q[2] + 1) : 0);
+                const int tq = (q[0] + 1) + t1 * (q[1] + 1) + (D > 2 ? t2 * (q[2] + 1) : 0);
+                fon[k] = true;
+                fti[k] = tq + (side ? -1 : 1) * (d == 0 ? 1 : d == 1 ? t1 : t2);
+                fwo[k] = (wg * 2 * D + 2 * d + side) * a.box.amax + h;
                 int P[3] = {lo[0] + q[0], lo[1] + q[1], D > 2 ? lo[2] + q[2] : 0}, c[3] = {bi[0], bi[1], bi[2]};
                 bool wall = false;
 #pragma unroll
@@ -178,10 +239,9 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
                         c[b] += side ? 1 : -1;
                         c[b] = c[b] < 0 ? a.box.k[b] - 1 : c[b] == a.box.k[b] ? 0 : c[b];
                     }
-                if (wall) {
-                    cgp_u[hti[k]] = 0.f;
-                } else {
+                if (!wall) {
                     hon[k] = true;
+                    hti[k] = tq;
                     long J = (long)P[0] + g.st[1] * P[1] + (D > 2 ? g.st[2] * P[2] : 0);
                     hr[k] = a.r[J];
                     hid[k] = a.iD[J];
@@ -194,72 +254,78 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     const long hslot = (long)a.box.nwg * 2 * D * a.box.amax;
     const int nwg = a.box.nwg, ngrp = (nwg + CGP_GROUP - 1) / CGP_GROUP;
     const bool two = nwg > CGP_ONE;
+    constexpr bool FAR = NB >= 1024;  // too large for one XCD
+    bool near = false;                // known once the first sum is
     auto half_of = [](double va, double vb, int j) {  // word j of a pair of sums
         double v = j < 2 ? va : vb;
         return (unsigned)((j & 1) ? __double2hiint(v) : __double2loint(v));
     };
+    auto faces = [&](unsigned tag) {  // w of the box's faces, from its tile
+        cgp_word *hw = a.hw + (tag & 1 ? hslot : 0);
+        float f[HC];
+#pragma unroll
+        for (int k = 0; k < HC; ++k) f[k] = cgp_w[fti[k]];
+        if (near) {
+#pragma unroll
+            for (int k = 0; k < HC; ++k)
+                if (fon[k]) cgp_put(hw + fwo[k], __float_as_uint(f[k]), tag, true);
+        } else {
+#pragma unroll
+            for (int k = 0; k < HC; ++k)
+                if (fon[k]) cgp_put(hw + fwo[k], __float_as_uint(f[k]), tag, false);
+        }
+    };
     auto tile = [&]() {  // u of the box and its halo
 #pragma unroll
-        for (int k = 0; k < C; ++k)
-            if (k < cnt) {
-                u[k] = r[k] * id[k];
-                cgp_u[ti + k * tz] = u[k];
-            }
+        for (int k = 0; k < C; ++k) {
+            u[k] = r[k] * id[k];
+            cgp_u[tw[k]] = u[k];
+        }
 #pragma unroll
-        for (int k = 0; k < HC; ++k)
-            if (hon[k]) cgp_u[hti[k]] = hr[k] * hid[k];
+        for (int k = 0; k < HC; ++k) cgp_u[hti[k]] = hr[k] * hid[k];
     };
     auto apply = [&](unsigned tag) {  // w = A u, published at the box's faces; the partials of r·u and u·w
-        cgp_word *hw = a.hw + (tag & 1 ? hslot : 0);
         double gd = 0, dd = 0;
-        if (cnt > 0) {
+        {
             const float ulo = cgp_u[ti - tz], uhi = cgp_u[ti + cnt * tz];
+            float um[C], up[C], vm[D > 2 ? C : 1], vp[D > 2 ? C : 1];
 #pragma unroll
-            for (int k = 0; k < C; ++k)
-                if (k < cnt) {
-                    const int t = ti + k * tz;
-                    float sl = 0, su = 0;
-                    sl += cgp_u[t - 1] * lx[k];
-                    su += cgp_u[t + 1] * lxp[k];
-                    if (D > 2) {
-                        sl += cgp_u[t - t1] * ly[k];
-                        su += cgp_u[t + t1] * lyp[k];
-                    }
-                    const float um = k > 0 ? u[k > 0 ? k - 1 : 0] : ulo;
-                    float up = uhi;
-                    if (k + 1 < C) {
-                        float un = u[k + 1 < C ? k + 1 : k];
-                        up = k + 1 < cnt ? un : uhi;
-                    }
-                    sl += um * lz[k];
-                    su += up * lz[k + 1];
-                    w[k] = (u[k] * dg[k] + sl) + su;
+            for (int k = 0; k < C; ++k) {
+                const int t = ti + k * tz;
+                um[k] = cgp_u[t - 1];
+                up[k] = cgp_u[t + 1];
+                if (D > 2) {
+                    vm[D > 2 ? k : 0] = cgp_u[t - t1];
+                    vp[D > 2 ? k : 0] = cgp_u[t + t1];
                 }
-            if (px >= 0) {
-#pragma unroll
-                for (int k = 0; k < C; ++k)
-                    if (k < cnt) cgp_put(hw + px + k * sx, __float_as_uint(w[k]), tag);
-            }
-            if (D > 2 && py >= 0) {
-#pragma unroll
-                for (int k = 0; k < C; ++k)
-                    if (k < cnt) cgp_put(hw + py + k * sy, __float_as_uint(w[k]), tag);
-            }
-            if (pl >= 0) cgp_put(hw + pl, __float_as_uint(w[0]), tag);
-            if (ph >= 0) {
-#pragma unroll
-                for (int k = 0; k < C; ++k)
-                    if (k == cnt - 1) cgp_put(hw + ph, __float_as_uint(w[k]), tag);
             }
 #pragma unroll
-            for (int k = 0; k < C; ++k)
-                if (k < cnt) {  // the products are exact
-                    gd = __builtin_fma((double)r[k], (double)u[k], gd);
-                    dd = __builtin_fma((double)u[k], (double)w[k], dd);
+            for (int k = 0; k < C; ++k) {
+                float sl = 0, su = 0;
+                sl += um[k] * lx[k];
+                su += up[k] * lxp[k];
+                if (D > 2) {
+                    sl += vm[D > 2 ? k : 0] * ly[k];
+                    su += vp[D > 2 ? k : 0] * lyp[k];
                 }
+                float hi = uhi;
+                if (k + 1 < C) {
+                    const float un = u[k + 1 < C ? k + 1 : k];
+                    hi = k + 1 < cnt ? un : uhi;
+                }
+                sl += (k > 0 ? u[k > 0 ? k - 1 : 0] : ulo) * lz[k];
+                su += hi * lz[k + 1];
+                w[k] = (u[k] * dg[k] + sl) + su;
+            }
+#pragma unroll
+            for (int k = 0; k < C; ++k) cgp_w[tw[k]] = w[k];
+#pragma unroll
+            for (int k = 0; k < C; ++k) {  // the products are exact
+                gd = __builtin_fma((double)r[k], (double)u[k], gd);
+                dd = __builtin_fma((double)u[k], (double)w[k], dd);
+            }
         }
-        gd = wave_sum(gd);
-        dd = wave_sum(dd);
+        wave_sum2(gd, dd);
         if (lane == 0) {
             shp[0][wv] = gd;
             shp[1][wv] = dd;
@@ -272,18 +338,19 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
 #pragma unroll
             for (int q = 0; q < NB / 64; ++q) vb += shp[1][q];
             cgp_word *pw = a.pw + (tag & 1 ? CGP_PW : 0) + CGP_P1;
-            if (lane < 4) cgp_put(pw + lane * CGP_MAXWG + blockIdx.x, half_of(va, vb, lane), tag);
+            if (lane < 4) cgp_put(pw + 4 * wg + lane, half_of(va, vb, lane), tag, near);
+            if (a.spread > 1 && tag == a.tag && lane == 4) cgp_put(pw + 4 * CGP_MAXWG + wg, cgp_xcd(), tag, near);
         }
+        faces(tag);
     };
-    // the sums of m pairs (m <= 64) by this wavefront; false: not there in time
-    auto gather = [&](const cgp_word *w4, int st, int m, unsigned tag, double &va, double &vb) {
+    // the sums of m pairs (m <= 64) of four words each by this wavefront; false: not there in time
+    auto gather = [&](const cgp_word *w4, int m, unsigned tag, double &va, double &vb) {
         cgp_word v[4];
         const long t0 = wall_clock64();
         for (int spin = 0;; ++spin) {
             bool ok = true;
             if (lane < m) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = cgp_get(w4 + j * st + lane);
+                cgp_getn(w4, 4 * lane, v, near);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) ok = ok && (unsigned)(v[j] >> 32) == tag;
             }
@@ -292,8 +359,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
         }
         va = lane < m ? __hiloint2double((int)(unsigned)v[1], (int)(unsigned)v[0]) : 0.0;
         vb = lane < m ? __hiloint2double((int)(unsigned)v[3], (int)(unsigned)v[2]) : 0.0;
-        va = wave_sum(va);
-        vb = wave_sum(vb);
+        wave_sum2(va, vb);
         return true;
     };
     // the halo cells' w
@@ -304,10 +370,10 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
             bool ok = true;
 #pragma unroll
             for (int k = 0; k < HC; ++k)
-                if (hon[k]) h[k] = cgp_get(hw + hwo[k]);
+                h[k] = cgp_get(hw, hwo[k], near);
 #pragma unroll
             for (int k = 0; k < HC; ++k)
-                if (hon[k]) ok = ok && (unsigned)(h[k] >> 32) == tag;
+                ok = ok && (!hon[k] || (unsigned)(h[k] >> 32) == tag);
             if (__all(ok)) break;
             if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
         }
@@ -325,27 +391,33 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     }
     float rho = 0, al = 0;
     for (int q = 1; q <= a.it; ++q) {
+        const double irho = inverse((double)rho), ial = inverse((double)al);
         const unsigned tag = a.tag + q - 1;
-        cgp_word *pw = a.pw + (tag & 1 ? CGP_PW : 0);
+        cgp_word *pw = a.pw + (tag & 1 ? CGP_PW : 0), *hw = a.hw + (tag & 1 ? hslot : 0);
         bool ok = true;
         if (wv == 0) {
             double sa = 0, sb = 0;
-            __builtin_amdgcn_s_sleep(CGP_NAP);
+            if (!near) __builtin_amdgcn_s_sleep(CGP_NAP);
             if (two) {
-                if (blockIdx.x % CGP_GROUP == 0) {
-                    ok = gather(pw + CGP_P1 + blockIdx.x, CGP_MAXWG, min(CGP_GROUP, nwg - (int)blockIdx.x), tag, sa, sb);
-                    if (ok) cgp_put(pw + lane * CGP_ONE + blockIdx.x / CGP_GROUP, half_of(sa, sb, lane & 3), tag);
+                if (wg % CGP_GROUP == 0) {
+                    ok = gather(pw + CGP_P1 + 4 * wg, min(CGP_GROUP, nwg - wg), tag, sa, sb);
+                    if (ok)  // a copy for each of the group's workgroups
+                        cgp_put(pw + 4 * ((lane >> 2) * CGP_ONE + wg / CGP_GROUP) + (lane & 3),
+                                half_of(sa, sb, lane & 3), tag, near);
                 }
-                if (ok) ok = gather(pw + (blockIdx.x % CGP_COPY) * 4 * CGP_ONE, CGP_ONE, ngrp, tag, sa, sb);
+                if (ok) ok = gather(pw + (wg % CGP_COPY) * 4 * CGP_ONE, ngrp, tag, sa, sb);
             } else {
-                ok = gather(pw + CGP_P1, CGP_MAXWG, nwg, tag, sa, sb);
+                ok = gather(pw + CGP_P1, nwg, tag, sa, sb);
             }
+            const bool nr =
+                near || (a.spread > 1 && q == 1 && ok && cgp_near(pw + CGP_P1 + 4 * CGP_MAXWG, nwg, tag));
             if (lane == 0) {
                 sht[0] = sa;
                 sht[1] = sb;
+                nears = nr;
             }
         } else {
-            ok = halo(a.hw + (tag & 1 ? hslot : 0), tag);
+            ok = halo(hw, tag);
         }
         if (!ok) dead = 1;
         __syncthreads();
@@ -353,35 +425,34 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
             if (tid == 0) *a.fail = 1;
             break;
         }
+        near = !FAR && nears != 0;
         const float gam = (float)sht[0], del = (float)sht[1];
         if (fabs(gam) < 10 * eps_of<float>()) break;
         float beta = 0;
         if (q == 1) {
             al = gam / del;
         } else {
-            beta = gam / rho;
-            al = gam / (del - (beta * gam) / al);
+            beta = quotient(gam, irho);
+            al = quotient(gam, inverse((double)(del - quotient(beta * gam, ial))));
         }
         rho = gam;
         const bool stop = q == a.it || fabs((double)al) < 1e-2;
 #pragma unroll
-        for (int k = 0; k < C; ++k)
-            if (k < cnt) {
-                if (q > 1) {
-                    p[k] = u[k] + beta * p[k];
-                    s[k] = w[k] + beta * s[k];
-                }
-                if (XL) xl[k * NB + tid] += al * p[k];
-                else x[XL ? 0 : k] = x[XL ? 0 : k] + al * p[k];
-                r[k] = r[k] - al * s[k];
+        for (int k = 0; k < C; ++k) {
+            if (q > 1) {
+                p[k] = u[k] + beta * p[k];
+                s[k] = w[k] + beta * s[k];
             }
+            if (XL) xl[k * NB + tid] += al * p[k];
+            else x[XL ? 0 : k] = x[XL ? 0 : k] + al * p[k];
+            r[k] = r[k] - al * s[k];
+        }
         if (stop) break;
 #pragma unroll
-        for (int k = 0; k < HC; ++k)
-            if (hon[k]) {
-                hs[k] = q > 1 ? hv[k] + beta * hs[k] : hv[k];
-                hr[k] = hr[k] - al * hs[k];
-            }
+        for (int k = 0; k < HC; ++k) {
+            hs[k] = q > 1 ? hv[k] + beta * hs[k] : hv[k];
+            hr[k] = hr[k] - al * hs[k];
+        }
         tile();
         __syncthreads();
         apply(tag + 1);
@@ -403,7 +474,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
 // have read their halo, so they are updated in place.
 //
 // 6 iterations on 256x256 (64 workgroups) and on 128x128 were 18 and 13
-// launches of 2.7-3.0 µs, each 4 µs of the host's time, which set the pace.
+// launches of 2.7-3.0 µs, each 4 µs of the host's time, which set the pace; now 15.5 and 11.2 µs.
 // ---------------------------------------------------------------------------
 struct PcgpArgs {
     Grid g;
@@ -416,6 +487,7 @@ struct PcgpArgs {
     unsigned tag;
     int it;
     double *r2;
+    int spread, xcd;  // of spread workgroups one takes part, those of wg % spread == xcd
     const int *halt;
     int *fail;
 };
@@ -430,17 +502,19 @@ template <int D> __device__ inline float cgp_mult_parent(const PcgpArgs &a, cons
 template <int D, int NB, int C, int HC>
 __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     HALT_IF(a)
+    if ((int)blockIdx.x % a.spread != a.xcd) return;
+    const int wg = (int)blockIdx.x / a.spread;
     extern __shared__ __align__(16) float cgp_u[];
     constexpr bool XL = NB * C >= 4096;  // x in LDS, as k_cgp
     __shared__ float xl[XL ? NB * C : 1];
     __shared__ double shp[NB / 64], sht;
-    __shared__ int dead;
+    __shared__ int dead, nears;
     const Grid &g = a.g;
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
     // this workgroup's box: first cell lo (ghost-inclusive), sides n
     int bi[3], lo[3], n[3];
     {
-        int q = blockIdx.x;
+        int q = wg;
         bi[0] = q % a.box.k[0];
         q /= a.box.k[0];
         bi[1] = q % a.box.k[1];
@@ -454,29 +528,28 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     const int t1 = a.box.b[0] + 2, t2 = t1 * (a.box.b[1] + 2);  // strides of the u tile
     const int tz = D > 2 ? t2 : t1;                            // along a column
     const long sz = g.st[D - 1];
+    // every thread works on all C cells of its column: those past its cnt are all zeros, read the tile's spare planes
+    // and write its last word, so no load or store waits behind a branch
+    const int dump = t1 * (a.box.b[1] + 2) * (D > 2 ? a.box.b[2] + 2 : 1) + (C - 1) * tz;
+    for (int q = tid; q <= dump; q += NB) cgp_u[q] = 0.f;
     if (tid == 0) dead = 0;
+    __syncthreads();
     // own cells: lateral position (x, y), first cell z0 of the column, cnt of them
     const int nl = D > 2 ? n[0] * n[1] : n[0];
     const int col = tid % nl, x0 = col % n[0], y0 = D > 2 ? col / n[0] : 0, z0 = (tid / nl) * C;
     const int cnt = max(0, min(C, n[D - 1] - z0));
-    const int ti = (x0 + 1) + (D > 2 ? t1 * (y0 + 1) : 0) + tz * (z0 + 1);
+    const int ti = (x0 + 1) + (D > 2 ? t1 * (y0 + 1) : 0) + tz * (cnt > 0 ? z0 + 1 : 1);
+    int tw[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) tw[k] = k < cnt ? ti + k * tz : dump;
     const long I0 = (long)(lo[0] + x0) + (D > 2 ? g.st[1] * (lo[1] + y0) : 0) + sz * (lo[D - 1] + z0);
-    // words of the column's w in the slot: its side face along x (and y), cell k at + k*stride; the faces of its ends
-    const int fb = (int)blockIdx.x * 2 * D;
-    int px = -1, py = -1, pl = -1, ph = -1;
-    const int sx = D > 2 ? n[1] : 1, sy = n[0];
-    if (cnt > 0) {
-        if (x0 == 0 || x0 == n[0] - 1) px = (fb + (x0 ? 1 : 0)) * a.box.amax + (D > 2 ? y0 + n[1] * z0 : z0);
-        if (D > 2 && (y0 == 0 || y0 == n[1] - 1)) py = (fb + 2 + (y0 ? 1 : 0)) * a.box.amax + x0 + n[0] * z0;
-        if (z0 == 0) pl = (fb + 2 * (D - 1)) * a.box.amax + col;
-        if (z0 + cnt == n[D - 1]) ph = (fb + 2 * (D - 1) + 1) * a.box.amax + col;
-    }
     float r[C], w[C], x[XL ? 1 : C], id[C], u[C], dg[C], lx[C], lxp[C], ly[C], lyp[C], lz[C + 1];
 #pragma unroll
     for (int k = 0; k <= C; ++k) lz[k] = cnt > 0 && k <= cnt ? a.L[g.ns * (D - 1) + I0 + k * sz] : 0.f;
 #pragma unroll
     for (int k = 0; k < C; ++k) {
-        if (!XL) x[XL ? 0 : k] = 0.f;
+        if (XL) xl[k * NB + tid] = 0.f;
+        else x[XL ? 0 : k] = 0.f;
         r[k] = w[k] = id[k] = u[k] = dg[k] = lx[k] = lxp[k] = ly[k] = lyp[k] = 0.f;
         if (k < cnt) {
             long I = I0 + k * sz;
@@ -503,8 +576,11 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
         }
     }
     // halo cells of the box's faces (2d + side); none across a wall (u = 0 there, L = 0)
-    bool hon[HC];
+    // the same threads publish the cells on this side of the faces
+    bool hon[HC], fon[HC];
     int hti[HC], hwo[HC];  // place in the tile, word of the cell's w in the slot
+    int fti[HC], fwo[HC];
+    float *const cgp_w = cgp_u + dump + 1;  // a tile of w
     float hr[HC], hu[HC], hid[HC], hv[HC];
     {
         const int area[3] = {n[1] * n[2], n[0] * n[2], n[0] * n[1]};
@@ -512,8 +588,9 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
 #pragma unroll
         for (int k = 0; k < HC; ++k) {
             int h = tid - 64 + k * (NB - 64);
-            hon[k] = false;
-            hti[k] = hwo[k] = 0;
+            hon[k] = fon[k] = false;
+            hti[k] = fti[k] = dump;
+            hwo[k] = fwo[k] = 0;
             hr[k] = hu[k] = hid[k] = hv[k] = 0.f;
             if (tid >= 64 && h < hc) {
                 int d = 0;
@@ -532,7 +609,10 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
                 const int m = d == 0 ? n[1] : n[0], e0 = h % m, e1 = h / m;
                 const int qd = side ? (d == 0 ? n[0] : d == 1 ? n[1] : n[2]) : -1;
                 const int q[3] = {d == 0 ? qd : e0, d == 1 ? qd : (d == 0 ? e0 : e1), d == 2 ? qd : e1};
-                hti[k] = (q[0] + 1) + t1 * (q[1] + 1) + (D > 2 ? t2 * (q[2] + 1) : 0);
+                const int tq = (q[0] + 1) + t1 * (q[1] + 1) + (D > 2 ? t2 * (q[2] + 1) : 0);
+                fon[k] = true;
+                fti[k] = tq + (side ? -1 : 1) * (d == 0 ? 1 : d == 1 ? t1 : t2);
+                fwo[k] = (wg * 2 * D + 2 * d + side) * a.box.amax + h;
                 int P[3] = {lo[0] + q[0], lo[1] + q[1], D > 2 ? lo[2] + q[2] : 0}, c[3] = {bi[0], bi[1], bi[2]};
                 bool wall = false;
 #pragma unroll
@@ -543,10 +623,9 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
                         c[b] += side ? 1 : -1;
                         c[b] = c[b] < 0 ? a.box.k[b] - 1 : c[b] == a.box.k[b] ? 0 : c[b];
                     }
-                if (wall) {
-                    cgp_u[hti[k]] = 0.f;
-                } else {
+                if (!wall) {
                     hon[k] = true;
+                    hti[k] = tq;
                     long J = (long)P[0] + g.st[1] * P[1] + (D > 2 ? g.st[2] * P[2] : 0);
                     hr[k] = a.r[J];
                     hid[k] = a.iD[J];
@@ -560,17 +639,32 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     const long hslot = (long)a.box.nwg * 2 * D * a.box.amax;
     const int nwg = a.box.nwg, ngrp = (nwg + CGP_GROUP - 1) / CGP_GROUP;
     const bool two = nwg > CGP_ONE;
+    constexpr bool FAR = NB >= 1024;  // too large for one XCD
+    bool near = false;                // known once the first sum is
     auto half_of = [](double v, int j) { return (unsigned)((j & 1) ? __double2hiint(v) : __double2loint(v)); };
+    auto faces = [&](unsigned tag) {  // w of the box's faces, from its tile
+        cgp_word *hw = a.hw + (tag & 1 ? hslot : 0);
+        float f[HC];
+#pragma unroll
+        for (int k = 0; k < HC; ++k) f[k] = cgp_w[fti[k]];
+        if (near) {
+#pragma unroll
+            for (int k = 0; k < HC; ++k)
+                if (fon[k]) cgp_put(hw + fwo[k], __float_as_uint(f[k]), tag, true);
+        } else {
+#pragma unroll
+            for (int k = 0; k < HC; ++k)
+                if (fon[k]) cgp_put(hw + fwo[k], __float_as_uint(f[k]), tag, false);
+        }
+    };
     auto tile = [&]() {  // ϵ of the box and its halo
 #pragma unroll
-        for (int k = 0; k < C; ++k)
-            if (k < cnt) cgp_u[ti + k * tz] = u[k];
+        for (int k = 0; k < C; ++k) cgp_u[tw[k]] = u[k];
 #pragma unroll
-        for (int k = 0; k < HC; ++k)
-            if (hon[k]) cgp_u[hti[k]] = hu[k];
+        for (int k = 0; k < HC; ++k) cgp_u[hti[k]] = hu[k];
     };
     auto publish = [&](unsigned tag, double v) {  // this workgroup's part of a sum
-        v = wave_sum(v);
+        v = wave_sum1(v);
         if (lane == 0) shp[wv] = v;
         __syncthreads();
         if (wv == 0) {
@@ -578,25 +672,24 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
 #pragma unroll
             for (int q = 0; q < NB / 64; ++q) t += shp[q];
             cgp_word *pw = a.pw + (tag & 1 ? CGP_PW : 0) + CGP_P1;
-            if (lane < 2) cgp_put(pw + lane * CGP_MAXWG + blockIdx.x, half_of(t, lane), tag);
+            if (lane < 2) cgp_put(pw + 2 * wg + lane, half_of(t, lane), tag, near);
+            if (a.spread > 1 && tag == a.tag && lane == 4) cgp_put(pw + 4 * CGP_MAXWG + wg, cgp_xcd(), tag, near);
         }
     };
-    // the sum of m parts (m <= 64) by this wavefront; false: not there in time
-    auto gather = [&](const cgp_word *w2, int st, int m, unsigned tag, double &v) {
+    // the sum of m parts (m <= 64) of two words each by this wavefront; false: not there in time
+    auto gather = [&](const cgp_word *w2, int m, unsigned tag, double &v) {
         cgp_word q[2];
         const long t0 = wall_clock64();
         for (int spin = 0;; ++spin) {
             bool ok = true;
             if (lane < m) {
-#pragma unroll
-                for (int j = 0; j < 2; ++j) q[j] = cgp_get(w2 + j * st + lane);
-#pragma unroll
-                for (int j = 0; j < 2; ++j) ok = ok && (unsigned)(q[j] >> 32) == tag;
+                cgp_getn(w2, 2 * lane, q, near);
+                ok = (unsigned)(q[0] >> 32) == tag && (unsigned)(q[1] >> 32) == tag;
             }
             if (__all(ok)) break;
             if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
         }
-        v = wave_sum(lane < m ? __hiloint2double((int)(unsigned)q[1], (int)(unsigned)q[0]) : 0.0);
+        v = wave_sum1(lane < m ? __hiloint2double((int)(unsigned)q[1], (int)(unsigned)q[0]) : 0.0);
         return true;
     };
     // the halo cells' z = A ϵ
@@ -607,10 +700,10 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
             bool ok = true;
 #pragma unroll
             for (int k = 0; k < HC; ++k)
-                if (hon[k]) h[k] = cgp_get(hw + hwo[k]);
+                h[k] = cgp_get(hw, hwo[k], near);
 #pragma unroll
             for (int k = 0; k < HC; ++k)
-                if (hon[k]) ok = ok && (unsigned)(h[k] >> 32) == tag;
+                ok = ok && (!hon[k] || (unsigned)(h[k] >> 32) == tag);
             if (__all(ok)) break;
             if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
         }
@@ -624,37 +717,42 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
         bool ok = true;
         if (wv == 0) {
             double v = 0;
-            __builtin_amdgcn_s_sleep(CGP_NAP);
+            if (!near) __builtin_amdgcn_s_sleep(CGP_NAP);
             if (two) {
-                if (blockIdx.x % CGP_GROUP == 0) {
-                    ok = gather(pw + CGP_P1 + blockIdx.x, CGP_MAXWG, min(CGP_GROUP, nwg - (int)blockIdx.x), tag, v);
-                    if (ok && (lane & 2) == 0)
-                        cgp_put(pw + lane * CGP_ONE + blockIdx.x / CGP_GROUP, half_of(v, lane), tag);
+                if (wg % CGP_GROUP == 0) {
+                    ok = gather(pw + CGP_P1 + 2 * wg, min(CGP_GROUP, nwg - wg), tag, v);
+                    if (ok && lane < 2 * CGP_COPY)  // a copy for each of the group's workgroups
+                        cgp_put(pw + 2 * ((lane >> 1) * CGP_ONE + wg / CGP_GROUP) + (lane & 1), half_of(v, lane & 1),
+                                tag, near);
                 }
-                if (ok) ok = gather(pw + (blockIdx.x % CGP_COPY) * 4 * CGP_ONE, CGP_ONE, ngrp, tag, v);
+                if (ok) ok = gather(pw + (wg % CGP_COPY) * 2 * CGP_ONE, ngrp, tag, v);
             } else {
-                ok = gather(pw + CGP_P1, CGP_MAXWG, nwg, tag, v);
+                ok = gather(pw + CGP_P1, nwg, tag, v);
             }
-            if (lane == 0) sht = v;
+            const bool nr =
+                near || (a.spread > 1 && tag == a.tag && ok && cgp_near(pw + CGP_P1 + 4 * CGP_MAXWG, nwg, tag));
+            if (lane == 0) {
+                sht = v;
+                nears = nr;
+            }
         } else if (hw) {
             ok = halo(hw, tag);
         }
         if (!ok) dead = 1;
         __syncthreads();
         out = (float)sht;
+        near = !FAR && nears != 0;
         return dead == 0;
     };
     // z = ϵ = r·iD, ρ = r·z
     double v = 0;
 #pragma unroll
-    for (int k = 0; k < C; ++k)
-        if (k < cnt) {
-            u[k] = r[k] * id[k];
-            v = __builtin_fma((double)r[k], (double)u[k], v);  // the products are exact
-        }
+    for (int k = 0; k < C; ++k) {
+        u[k] = r[k] * id[k];
+        v = __builtin_fma((double)r[k], (double)u[k], v);  // the products are exact
+    }
 #pragma unroll
-    for (int k = 0; k < HC; ++k)
-        if (hon[k]) hu[k] = hr[k] * hid[k];
+    for (int k = 0; k < HC; ++k) hu[k] = hr[k] * hid[k];
     tile();
     publish(a.tag, v);
     float rho = 0;
@@ -664,52 +762,47 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     for (int i = 1; i <= a.it && !done; ++i) {
         // z = A ϵ, published at the box's faces; z·ϵ (total's barrier came after the tile's last write)
         const unsigned ta = a.tag + 2 * i - 1, tb = ta + 1;
-        cgp_word *hw = a.hw + (i & 1 ? hslot : 0);
+        const cgp_word *hw = a.hw + (ta & 1 ? hslot : 0);
         v = 0;
-        if (cnt > 0) {
+        {
             const float ulo = cgp_u[ti - tz], uhi = cgp_u[ti + cnt * tz];
+            float um[C], up[C], vm[D > 2 ? C : 1], vp[D > 2 ? C : 1];
 #pragma unroll
-            for (int k = 0; k < C; ++k)
-                if (k < cnt) {
-                    const int t = ti + k * tz;
-                    float sl = 0, su = 0;
-                    sl += cgp_u[t - 1] * lx[k];
-                    su += cgp_u[t + 1] * lxp[k];
-                    if (D > 2) {
-                        sl += cgp_u[t - t1] * ly[k];
-                        su += cgp_u[t + t1] * lyp[k];
-                    }
-                    const float um = k > 0 ? u[k > 0 ? k - 1 : 0] : ulo;
-                    float up = uhi;
-                    if (k + 1 < C) {
-                        float un = u[k + 1 < C ? k + 1 : k];
-                        up = k + 1 < cnt ? un : uhi;
-                    }
-                    sl += um * lz[k];
-                    su += up * lz[k + 1];
-                    w[k] = (u[k] * dg[k] + sl) + su;
+            for (int k = 0; k < C; ++k) {
+                const int t = ti + k * tz;
+                um[k] = cgp_u[t - 1];
+                up[k] = cgp_u[t + 1];
+                if (D > 2) {
+                    vm[D > 2 ? k : 0] = cgp_u[t - t1];
+                    vp[D > 2 ? k : 0] = cgp_u[t + t1];
                 }
-            if (px >= 0) {
-#pragma unroll
-                for (int k = 0; k < C; ++k)
-                    if (k < cnt) cgp_put(hw + px + k * sx, __float_as_uint(w[k]), ta);
             }
-            if (D > 2 && py >= 0) {
 #pragma unroll
-                for (int k = 0; k < C; ++k)
-                    if (k < cnt) cgp_put(hw + py + k * sy, __float_as_uint(w[k]), ta);
+            for (int k = 0; k < C; ++k) {
+                float sl = 0, su = 0;
+                sl += um[k] * lx[k];
+                su += up[k] * lxp[k];
+                if (D > 2) {
+                    sl += vm[D > 2 ? k : 0] * ly[k];
+                    su += vp[D > 2 ? k : 0] * lyp[k];
+                }
+                float hi = uhi;
+                if (k + 1 < C) {
+                    const float un = u[k + 1 < C ? k + 1 : k];
+                    hi = k + 1 < cnt ? un : uhi;
+                }
+                sl += (k > 0 ? u[k > 0 ? k - 1 : 0] : ulo) * lz[k];
+                su += hi * lz[k + 1];
+                w[k] = (u[k] * dg[k] + sl) + su;
             }
-            if (pl >= 0) cgp_put(hw + pl, __float_as_uint(w[0]), ta);
-            if (ph >= 0) {
 #pragma unroll
-                for (int k = 0; k < C; ++k)
-                    if (k == cnt - 1) cgp_put(hw + ph, __float_as_uint(w[k]), ta);
-            }
+            for (int k = 0; k < C; ++k) cgp_w[tw[k]] = w[k];
 #pragma unroll
             for (int k = 0; k < C; ++k)
-                if (k < cnt) v = __builtin_fma((double)w[k], (double)u[k], v);
+                v = __builtin_fma((double)w[k], (double)u[k], v);
         }
         publish(ta, v);
+        faces(ta);
         float ze;
         if (!total(ta, hw, ze)) {
             ok = false;
@@ -718,14 +811,13 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
         const float alpha = rho / ze;
         v = 0;
 #pragma unroll
-        for (int k = 0; k < C; ++k)
-            if (k < cnt) {
-                if (XL) xl[k * NB + tid] += alpha * u[k];
-                else x[XL ? 0 : k] = x[XL ? 0 : k] + alpha * u[k];
-                r[k] = r[k] - alpha * w[k];
-                w[k] = r[k] * id[k];
-                v = __builtin_fma((double)r[k], (double)w[k], v);
-            }
+        for (int k = 0; k < C; ++k) {
+            if (XL) xl[k * NB + tid] += alpha * u[k];
+            else x[XL ? 0 : k] = x[XL ? 0 : k] + alpha * u[k];
+            r[k] = r[k] - alpha * w[k];
+            w[k] = r[k] * id[k];
+            v = __builtin_fma((double)r[k], (double)w[k], v);
+        }
         if (i == a.it || fabs((double)alpha) < 1e-2) break;
         publish(tb, v);
         float rho2;
@@ -736,14 +828,12 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
         if (fabs(rho2) < 10 * eps_of<float>()) break;
         const float beta = rho2 / rho;
 #pragma unroll
-        for (int k = 0; k < C; ++k)
-            if (k < cnt) u[k] = beta * u[k] + w[k];
+        for (int k = 0; k < C; ++k) u[k] = beta * u[k] + w[k];
 #pragma unroll
-        for (int k = 0; k < HC; ++k)
-            if (hon[k]) {
-                hr[k] = hr[k] - alpha * hv[k];
-                hu[k] = beta * hu[k] + hr[k] * hid[k];
-            }
+        for (int k = 0; k < HC; ++k) {
+            hr[k] = hr[k] - alpha * hv[k];
+            hu[k] = beta * hu[k] + hr[k] * hid[k];
+        }
         tile();
         __syncthreads();
         rho = rho2;
@@ -764,19 +854,19 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
             }
         }
     if (a.r2) {
-        v = wave_sum(v);
+        v = wave_sum1(v);
         __syncthreads();
         if (lane == 0) shp[wv] = v;
         __syncthreads();
         if (tid == 0) {
             double t = 0;
             for (int q = 0; q < NB / 64; ++q) t += shp[q];
-            a.r2[blockIdx.x] = t;
+            a.r2[wg] = t;
         }
     }
 }
 // The variants: threads and cells per thread, the fewest first, as more cells per workgroup cost more than more
-// workgroups up to CGP_ONE (32^3: 2.25 µs with 2 cells on 256 threads, 2.7 with 4 on 512, 2.8 with 4 on 1024).
+// workgroups up to CGP_ONE (32^3: 1.9 µs with 2 cells on 256 threads, 2.4 with 4 on 512).
 struct CgpVariant {
     int D, NB, C, HC;
     void (*k)(CgpArgs);

@@ -2130,9 +2130,45 @@ template <int D, class T> __device__ __forceinline__ void tail_run(const TailArg
 // cells the arithmetic of one CU besides.  µs per iteration, k_mg_tail ->
 // here: 16^3 2.7 -> 1.7, 8^3 1.6 -> 0.86, 4^3 0.52 -> 0.35, 48x32 1.75 ->
 // 1.02, 96 cells 1.5 -> 0.39; a whole tail with the flexible CG's counts:
-// 16^3 273 -> 177, 48x32 245 -> 137, 64x64 364 -> 237 (with 6 iterations a
+// 16^3 273 -> 170, 48x32 245 -> 134, 64x64 364 -> 237 (with 6 iterations a
 // level 78 -> 52).
 // ---------------------------------------------------------------------------
+// the sums of a and of b over the wavefront, in every lane: the halves of the two are exchanged, so that one reduction
+// over 32 lanes does both
+__device__ inline void wave_sum2(double &a, double &b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    double v = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    v += dpp_d<0xB1>(v);
+    v += dpp_d<0x4E>(v);
+    v += dpp_d<0x141>(v);
+    v += dpp_d<0x140>(v);
+    a = lane_d(v, 0) + lane_d(v, 16);
+    b = lane_d(v, 32) + lane_d(v, 48);
+}
+// the sum of a over the wavefront, in every lane: the rows of 16 as wave_sum, then rows and halves exchanged
+__device__ inline double wave_sum1(double v) {
+    v += dpp_d<0xB1>(v);
+    v += dpp_d<0x4E>(v);
+    v += dpp_d<0x141>(v);
+    v += dpp_d<0x140>(v);
+    auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v), __double2loint(v), false, false);
+    auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v), __double2hiint(v), false, false);
+    v = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    lo = __builtin_amdgcn_permlane32_swap(__double2loint(v), __double2loint(v), false, false);
+    hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v), __double2hiint(v), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+// 1/y to about 2^-52.  A quotient of two 24-bit numbers is never within 2^-49 of itself of the middle between two such
+// numbers, so x * inverse(y) rounds to FP32's x/y; most of a division's latency (130 cycles, of which an iteration
+// had three in a row) can pass before x is known.
+__device__ inline double inverse(double y) {
+    double q = __builtin_amdgcn_rcp(y);
+    double e = __builtin_fma(-y, q, 1.0);
+    double z = __builtin_fma(q, __builtin_fma(e, e, e), q);  // the estimate's error cubed
+    return e == e ? z : q;                                   // y = 0 or infinite
+}
+__device__ inline float quotient(float x, double inv) { return (float)((double)x * inv); }
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 // the sum over a fully active wavefront, in every lane: the first product adds lanes i, i+16, i+32, i+48, the lane
 // adds its four rows of the result, and the second product adds the four groups of rows
@@ -2388,7 +2424,7 @@ __device__ __forceinline__ void f_up(const FLev &l, const FCols<D, C, WAVE> &q, 
         constexpr int NW = NTF / 64;
         double *h = sh + par * 16;
         par ^= 1;
-        if (wv < nw) v = NW <= 4 ? wave_sum_mm(v) : wave_sum(v);  // the matrix products' rate is too low for more
+        if (wv < nw) v = NW <= 4 ? wave_sum_mm(v) : wave_sum1(v);  // the matrix products' rate is too low for more
         if (lane == 0) h[wv] = wv < nw ? v : 0.0;
         __syncthreads();
         double t[NW];
@@ -2415,31 +2451,33 @@ __device__ __forceinline__ void f_up(const FLev &l, const FCols<D, C, WAVE> &q, 
         if (WAVE) wave_lds_order();
         for (int i = 1; i <= it; ++i) {
             v = 0;
+            double irho = 0;
             if (q.cnt > 0) {
                 q.mult_lds(l.e, e, z);
+                irho = inverse((double)rho);
 #pragma unroll
-                for (int k = 0; k < C; ++k)
-                    if (k < q.cnt) v = __builtin_fma((double)z[k], (double)e[k], v);
+                for (int k = 0; k < C; ++k) {  // cells past the column's end have ϵ = iD = 0
+                    z[k] = k < q.cnt ? z[k] : 0.f;
+                    v = __builtin_fma((double)z[k], (double)e[k], v);
+                }
             }
             const float alpha = rho / (float)sum(v);
             const bool last = i == it || fabs((double)alpha) < 1e-2;
             v = 0;
 #pragma unroll
-            for (int k = 0; k < C; ++k)
-                if (k < q.cnt) {
-                    x[k] += alpha * e[k];
-                    r[k] = r[k] - alpha * z[k];
-                    z[k] = r[k] * q.iD[k];
-                    v = __builtin_fma((double)r[k], (double)z[k], v);
-                }
+            for (int k = 0; k < C; ++k) {
+                x[k] += alpha * e[k];
+                r[k] = r[k] - alpha * z[k];
+                z[k] = r[k] * q.iD[k];
+                v = __builtin_fma((double)r[k], (double)z[k], v);
+            }
             if (last) break;
             const float rho2 = (float)sum(v);
             if (fabs(rho2) < 10 * eps_of<float>()) break;
-            const float beta = rho2 / rho;
+            const float beta = quotient(rho2, irho);
             if (WAVE) wave_lds_order();
 #pragma unroll
-            for (int k = 0; k < C; ++k)
-                if (k < q.cnt) e[k] = beta * e[k] + z[k];
+            for (int k = 0; k < C; ++k) e[k] = beta * e[k] + z[k];
             if (q.cnt > 0) q.wr(l.e + q.e0, e);
             fsync<WAVE>();
             rho = rho2;

@@ -94,3 +94,14 @@ def test_default_solver_in_one_launch(dims, perdir):
     assert np.abs(u - ul).max() <= 1e-5 * np.abs(ul).max()
     assert np.abs(p - pl).max() <= 1e-4 * np.abs(pl).max()
     assert np.abs(z - zl).max() <= 1e-4 * np.abs(zl).max()
+
+
+@pytest.mark.parametrize("poisson", ["refined", "reference"])
+def test_contexts_take_the_xcds_in_turn(poisson):
+    """Nine contexts, one after the other: wherever a launch runs, the same bits."""
+    dims = (192, 136)
+    say("one launch on each XCD", dims, poisson)
+    ref = projected(dims, (), False, poisson=poisson)
+    for _ in range(8):
+        got = projected(dims, (), False, poisson=poisson)
+        assert got[2] == ref[2] and all(np.array_equal(a, b) for a, b in zip((got[0], got[1]), (ref[0], ref[1])))
