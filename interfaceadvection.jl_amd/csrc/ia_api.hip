@@ -569,12 +569,15 @@ template <class T> struct Impl {
             // everyone reads every sum up to CGP_ONE workgroups; more of them only where the level needs it
             for (int maxwg : {CGP_ONE, CGP_MAXWG})
                 for (int q = 0; q < nv && !lv.cgp; ++q) {
-                    if (vs[q].D != lv.g.D || (maxwg > CGP_ONE && vs[q].NB < 1024)) continue;
-                    if (!cgp_boxes(n, vs[q], maxwg, lv.cgp_box)) continue;
+                    const int cells = vs[q].NB * vs[q].C;
+                    if (vs[q].D != lv.g.D || (maxwg > CGP_ONE ? cells < 4096 : cells > 4096)) continue;
+                    const void *k = c->pcgp ? (const void *)pcgp_kernel(q) : (const void *)vs[q].k;
+                    if (!k || !cgp_boxes(n, vs[q], maxwg, lv.cgp_box)) continue;
+                    const size_t lds = cgp_lds(lv, vs[q]);
+                    if (lds > 64 * 1024)
+                        HIPCHK(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                     int per = 0;
-                    HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                                  &per, c->pcgp ? (const void *)pcgp_kernel(q) : (const void *)vs[q].k, vs[q].NB,
-                                  cgp_lds(lv, vs[q].C)));
+                    HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, vs[q].NB, lds));
                     if ((long)per * ncu < (maxwg > CGP_ONE ? 1L : 2L) * lv.cgp_box.nwg) continue;
                     lv.cgp = &vs[q];
                     // on one XCD where there is room for two such launches
@@ -591,10 +594,8 @@ template <class T> struct Impl {
         return IA_OK;
     }
     static bool cgp_failed(const ia_ctx *c) { return *(volatile int *)&c->hst->fail != 0; }
-    static size_t cgp_lds(const Level &l, int C) {
-        const CgpBox &b = l.cgp_box;
-        const int t1 = b.b[0] + 2, t2 = t1 * (b.b[1] + 2), tz = l.g.D > 2 ? t2 : t1;
-        return 2 * sizeof(float) * (t2 * (l.g.D > 2 ? b.b[2] + 2 : 1) + (C - 1) * tz + 1);  // the tiles of u and w
+    static size_t cgp_lds(const Level &l, const CgpVariant &v) {
+        return sizeof(float) * cgp_words(v.D, v.NB, v.C, l.cgp_box.b);
     }
     // ----------------------------------------------------------------- MG
     static int mg_update(ia_ctx *c) {
@@ -680,7 +681,7 @@ template <class T> struct Impl {
         a.fail = &c->hst->fail;
         int nv;
         hipLaunchKernelGGL(pcgp_kernel((int)(l.cgp - cgp_variants(nv))), dim3((unsigned)(a.box.nwg * a.spread)),
-                           dim3((unsigned)l.cgp->NB), cgp_lds(l, l.cgp->C), c->s, a);
+                           dim3((unsigned)l.cgp->NB), cgp_lds(l, *l.cgp), c->s, a);
     }
     static void pcg(ia_ctx *c, Level &l, int it = 6, bool init_done = false, const FcgV<T> *last = nullptr,
                     int first = 0) {
@@ -765,7 +766,7 @@ template <class T> struct Impl {
             a.fail = &c->hst->fail;
             if (pc >= 0) prof_begin(c, pc);
             hipLaunchKernelGGL(l.cgp->k, dim3((unsigned)(a.box.nwg * a.spread)), dim3((unsigned)l.cgp->NB),
-                               cgp_lds(l, l.cgp->C), c->s, a);
+                               cgp_lds(l, *l.cgp), c->s, a);
             if (pc >= 0) prof_end(c, pc);
             return;
         }

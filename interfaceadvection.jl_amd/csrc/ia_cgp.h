@@ -26,8 +26,12 @@ namespace ia {
 // store to load 0.5 µs instead of 0.8 past the L2s of the eight XCDs (0.47 against 1.27 with 64 workgroups reading
 // everyone's).  Each context has an XCD of its own in turn, so that contexts do not wait for one another's places.
 //
-// Measured, µs per iteration of 64, one launch per iteration / here: 64^3 6.6-7.5 / 2.7, 60x44x36 5.4 / 2.2, 32^3 4.6 /
-// 1.55, 192x128 4.5 / 1.3, 96x64 4.3 / 1.2.  What is left is the exchange and as much again for the operator, the
+// Levels of up to 2M cells take every CU's registers and LDS (BIG: 16 cells of a thread, x, p, s and a tile in 155 KB):
+// an iteration reads nothing from memory but the faces.
+//
+// Measured, µs per iteration of 64, one launch per iteration / here: 128^3 22-24 / 9.0 (6 iterations 145 / 83), 64^3
+// 6.6-7.5 / 3.0, 60x44x36 5.4 / 2.2, 32^3 4.6 / 1.55, 192x128 4.5 / 1.3, 96x64 4.3 / 1.2.  What is left on the small
+// ones is the exchange and as much again for the operator, the
 // recurrence and the two sums, a chain of some 2000 cycles in which a wavefront mostly waits for itself: nothing in it
 // stands behind a branch, faces are published through a tile, and a workgroup's words of a sum lie together.
 //
@@ -45,6 +49,7 @@ constexpr int CGP_GROUP = 16; // above, the sums of groups of this many, which t
 // with 18); within one L2 waiting first gains nothing
 constexpr int CGP_NAP = 12;
 constexpr long CGP_WAIT = 2000000;  // ticks of the 100 MHz counter: 20 ms
+constexpr long CGP_LDS = 158 * 1024;  // of the 160 KiB of a CU
 struct CgpBox {
     int k[3], b[3];  // boxes per axis, cells per box and axis (the last box may have fewer, at least 2)
     int nwg, amax;   // workgroups, the largest face of a box
@@ -120,6 +125,22 @@ __device__ inline bool cgp_near(const cgp_word *w, int nwg, unsigned tag) {
         if (wall_clock64() - t0 > CGP_WAIT) return false;
     }
 }
+// planes past the end of a box of b cells along the columns that columns of C cells reach
+__host__ __device__ inline int cgp_spare(int b, int C) { return (b + C - 1) / C * C - b; }
+// BIG's tile has a column's cells side by side, read and written four at a time: a column of b cells starts at word 4,
+// the halo cells at 3 and 4 + b; an odd number of fours from column to column spreads them over the banks
+__host__ __device__ inline int cgp_zstride(int b, int C) { return 4 * (((5 + b + cgp_spare(b, C) + 3) / 4) | 1); }
+// words of LDS of a box: the tiles of u and w, or BIG's tile and x, p and s
+__host__ __device__ inline int cgp_tile(int D, int NB, int C, const int *b) {
+    const int t1 = b[0] + 2, t2 = t1 * (b[1] + 2);
+    if (NB * C > 4096) return t2 * cgp_zstride(b[2], C) + 4;
+    return D > 2 ? t2 * (b[2] + 2 + cgp_spare(b[2], C)) + 1 : t1 * (b[1] + 2 + cgp_spare(b[1], C)) + 1;
+}
+__host__ __device__ inline int cgp_words(int D, int NB, int C, const int *b) {
+    const int t = cgp_tile(D, NB, C, b);
+    return NB * C > 4096 ? t + 3 * NB * C : 2 * t;
+}
+
 // NB threads; a thread owns a column of C cells along the last axis (so two of a cell's neighbours are mostly its own
 // registers); the halo cells are those of wavefronts 1.. (HC each), while wavefront 0 waits for the sums.
 template <int D, int NB, int C, int HC>
@@ -129,7 +150,9 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     const int wg = (int)blockIdx.x / a.spread;
     extern __shared__ __align__(16) float cgp_u[];
     constexpr bool XL = NB * C >= 4096;  // x in LDS: the registers of a 1024-thread workgroup do not hold it
-    __shared__ float xl[XL ? NB * C : 1];
+    constexpr bool BIG = NB * C > 4096;  // p and s in LDS too, u and the diagonal formed again, w in u's tile
+    constexpr int CR = BIG ? 1 : C;
+    __shared__ float xs[XL && !BIG ? NB * C : 1];
     __shared__ double shp[2][NB / 64], sht[2];
     __shared__ int dead, nears;
     const Grid &g = a.g;
@@ -148,12 +171,18 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
         lo[d] = d < D ? 1 + bi[d] * a.box.b[d] : 0;
         n[d] = d < D ? min(a.box.b[d], g.Ng[d] - 1 - lo[d]) : 1;
     }
-    const int t1 = a.box.b[0] + 2, t2 = t1 * (a.box.b[1] + 2);  // strides of the u tile
-    const int tz = D > 2 ? t2 : t1;                            // along a column
+    // strides of the u tile, along a column last
+    const int zs = BIG ? cgp_zstride(a.box.b[2], C) : 1, t0 = BIG ? zs : 1, t1 = t0 * (a.box.b[0] + 2);
+    const int tz = BIG ? 1 : D > 2 ? t1 * (a.box.b[1] + 2) : t1;
+    auto at = [&](int x, int y, int z) {
+        return t0 * (x + 1) + t1 * (y + 1) + (D > 2 ? tz * (z + 1) : 0) + (BIG ? 3 : 0);
+    };
     const long sz = g.st[D - 1];
     // every thread works on all C cells of its column: those past its cnt are all zeros, read the tile's spare planes
     // and write its last word, so no load or store waits behind a branch
-    const int dump = t1 * (a.box.b[1] + 2) * (D > 2 ? a.box.b[2] + 2 : 1) + (C - 1) * tz;
+    const int dump = cgp_tile(D, NB, C, a.box.b) - (BIG ? 4 : 1);
+    float *const xl = BIG ? cgp_u + dump + 4 : xs;  // cell k at k * NB + tid; BIG: four cells together
+    float4 *const x4 = (float4 *)xl, *const p4 = x4 + NB * C / 4, *const s4 = p4 + NB * C / 4;
     for (int q = tid; q <= dump; q += NB) cgp_u[q] = 0.f;
     if (tid == 0) dead = 0;
     __syncthreads();
@@ -161,42 +190,52 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     const int nl = D > 2 ? n[0] * n[1] : n[0];
     const int col = tid % nl, x0 = col % n[0], y0 = D > 2 ? col / n[0] : 0, z0 = (tid / nl) * C;
     const int cnt = max(0, min(C, n[D - 1] - z0));
-    const int ti = (x0 + 1) + (D > 2 ? t1 * (y0 + 1) : 0) + tz * (cnt > 0 ? z0 + 1 : 1);
-    int tw[C];
-#pragma unroll
-    for (int k = 0; k < C; ++k) tw[k] = k < cnt ? ti + k * tz : dump;
+    const int ti = D > 2 ? at(x0, y0, cnt > 0 ? z0 : 0) : at(x0, cnt > 0 ? z0 : 0, 0);
+    auto tw = [&](int t, int k) { return k < cnt ? t + k * tz : dump; };
+    // the column's place in the tile; BIG: anew at each use, or the cells' places would be kept in registers
+    auto place = [&]() {
+        int t = ti;
+        if (BIG) asm volatile("" : "+v"(t));
+        return t;
+    };
     const long I0 = (long)(lo[0] + x0) + (D > 2 ? g.st[1] * (lo[1] + y0) : 0) + sz * (lo[D - 1] + z0);
-    float r[C], s[C], w[C], p[C], x[XL ? 1 : C], id[C], u[C], dg[C], lx[C], lxp[C], ly[C], lyp[C], lz[C + 1];
+    float r[C], s[CR], w[C], p[CR], x[XL ? 1 : C], id[C], u[CR], dg[CR], lx[C], lxp[C], ly[C], lyp[C], lz[C + 1];
 #pragma unroll
     for (int k = 0; k <= C; ++k) lz[k] = cnt > 0 && k <= cnt ? a.L[g.ns * (D - 1) + I0 + k * sz] : 0.f;
 #pragma unroll
     for (int k = 0; k < C; ++k) {
-        if (XL) xl[k * NB + tid] = 0.f;
-        else x[XL ? 0 : k] = 0.f;
-        r[k] = s[k] = w[k] = p[k] = id[k] = u[k] = dg[k] = lx[k] = lxp[k] = ly[k] = lyp[k] = 0.f;
+        float xk = 0.f;
+        r[k] = w[k] = id[k] = lx[k] = lxp[k] = ly[k] = lyp[k] = 0.f;
         if (k < cnt) {
             long I = I0 + k * sz;
             r[k] = a.r[I];
             id[k] = a.iD[I];
-            if (XL) xl[k * NB + tid] = a.x[I];
-            else x[XL ? 0 : k] = a.x[I];
+            xk = a.x[I];
             lx[k] = a.L[I];
             lxp[k] = a.L[I + 1];
-            dg[k] -= (lx[k] + lxp[k]);
             if (D > 2) {
                 ly[k] = a.L[g.ns + I];
                 lyp[k] = a.L[g.ns + I + g.st[1]];
-                dg[k] -= (ly[k] + lyp[k]);
             }
-            dg[k] -= (lz[k] + lz[k + 1]);
         }
+        if (BIG) xl[4 * (k / 4 * NB + tid) + k % 4] = xk;
+        else if (XL) xl[k * NB + tid] = xk;
+        else x[XL ? 0 : k] = xk;
     }
+    auto diag = [&](int k) {
+        float d = 0.f - (lx[k] + lxp[k]);
+        if (D > 2) d -= (ly[k] + lyp[k]);
+        return d - (lz[k] + lz[k + 1]);
+    };
+#pragma unroll
+    for (int k = 0; k < CR; ++k) dg[k] = BIG ? 0.f : diag(k);
+    auto U = [&](int k) { return BIG ? r[k] * id[k] : u[BIG ? 0 : k]; };
     // halo cells of the box's faces (2d + side); none across a wall (u = 0 there, L = 0)
     // the same threads publish the cells on this side of the faces
     bool hon[HC], fon[HC];
     int hti[HC], hwo[HC];  // place in the tile, word of the cell's w in the slot
     int fti[HC], fwo[HC];
-    float *const cgp_w = cgp_u + dump + 1;  // a tile of w
+    float *const cgp_w = BIG ? cgp_u : cgp_u + dump + 1;  // a tile of w
     float hr[HC], hs[HC], hid[HC], hv[HC];
     {
         const int area[3] = {n[1] * n[2], n[0] * n[2], n[0] * n[1]};
@@ -225,9 +264,9 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
                 const int m = d == 0 ? n[1] : n[0], e0 = h % m, e1 = h / m;
                 const int qd = side ? (d == 0 ? n[0] : d == 1 ? n[1] : n[2]) : -1;
                 const int q[3] = {d == 0 ? qd : e0, d == 1 ? qd : (d == 0 ? e0 : e1), d == 2 ? qd : e1};
-                const int tq = (q[0] + 1) + t1 * (q[1] + 1) + (D > 2 ? t2 * (q[2] + 1) : 0);
+                const int tq = at(q[0], q[1], q[2]);
                 fon[k] = true;
-                fti[k] = tq + (side ? -1 : 1) * (d == 0 ? 1 : d == 1 ? t1 : t2);
+                fti[k] = tq + (side ? -1 : 1) * (d == 0 ? t0 : d == 1 ? t1 : tz);
                 fwo[k] = (wg * 2 * D + 2 * d + side) * a.box.amax + h;
                 int P[3] = {lo[0] + q[0], lo[1] + q[1], D > 2 ? lo[2] + q[2] : 0}, c[3] = {bi[0], bi[1], bi[2]};
                 bool wall = false;
@@ -254,8 +293,8 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     const long hslot = (long)a.box.nwg * 2 * D * a.box.amax;
     const int nwg = a.box.nwg, ngrp = (nwg + CGP_GROUP - 1) / CGP_GROUP;
     const bool two = nwg > CGP_ONE;
-    constexpr bool FAR = NB >= 1024;  // too large for one XCD
-    bool near = false;                // known once the first sum is
+    constexpr bool FAR = NB >= 1024 || BIG;  // too large for one XCD
+    bool near = false;  // known once the first sum is
     auto half_of = [](double va, double vb, int j) {  // word j of a pair of sums
         double v = j < 2 ? va : vb;
         return (unsigned)((j & 1) ? __double2hiint(v) : __double2loint(v));
@@ -275,55 +314,87 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
                 if (fon[k]) cgp_put(hw + fwo[k], __float_as_uint(f[k]), tag, false);
         }
     };
+    auto own = [&](float *tl, const float (&v)[C]) {  // the own cells' values to a tile
+        const int t = place();
+        if (BIG && cnt == C) {
+#pragma unroll
+            for (int k = 0; k < C; k += 4)
+                *(float4 *)(tl + t + k) = make_float4(v[k], v[k + 1 < C ? k + 1 : k], v[k + 2 < C ? k + 2 : k],
+                                                      v[k + 3 < C ? k + 3 : k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < C; ++k) tl[tw(t, k)] = v[k];
+        }
+    };
     auto tile = [&]() {  // u of the box and its halo
+        float uk[C];
 #pragma unroll
         for (int k = 0; k < C; ++k) {
-            u[k] = r[k] * id[k];
-            cgp_u[tw[k]] = u[k];
+            uk[k] = r[k] * id[k];
+            if (!BIG) u[BIG ? 0 : k] = uk[k];
         }
+        own(cgp_u, uk);
 #pragma unroll
         for (int k = 0; k < HC; ++k) cgp_u[hti[k]] = hr[k] * hid[k];
     };
     auto apply = [&](unsigned tag) {  // w = A u, published at the box's faces; the partials of r·u and u·w
         double gd = 0, dd = 0;
         {
-            const float ulo = cgp_u[ti - tz], uhi = cgp_u[ti + cnt * tz];
-            float um[C], up[C], vm[D > 2 ? C : 1], vp[D > 2 ? C : 1];
+            const int tc = place();
+            const float ulo = cgp_u[tc - tz], uhi = cgp_u[tc + cnt * tz];
+            constexpr int G = BIG ? 4 : C;  // cells whose neighbours are read together
+            float um[G], up[G], vm[D > 2 ? G : 1], vp[D > 2 ? G : 1];
+            if (!BIG) {
 #pragma unroll
-            for (int k = 0; k < C; ++k) {
-                const int t = ti + k * tz;
-                um[k] = cgp_u[t - 1];
-                up[k] = cgp_u[t + 1];
-                if (D > 2) {
-                    vm[D > 2 ? k : 0] = cgp_u[t - t1];
-                    vp[D > 2 ? k : 0] = cgp_u[t + t1];
+                for (int k = 0; k < C; ++k) {
+                    const int t = tc + k * tz;
+                    um[k % G] = cgp_u[t - 1];
+                    up[k % G] = cgp_u[t + 1];
+                    if (D > 2) {
+                        vm[D > 2 ? k % G : 0] = cgp_u[t - t1];
+                        vp[D > 2 ? k % G : 0] = cgp_u[t + t1];
+                    }
                 }
             }
 #pragma unroll
             for (int k = 0; k < C; ++k) {
+                if (BIG && k % 4 == 0) {
+                    // no loads of later groups: the registers do not hold them
+                    __builtin_amdgcn_sched_barrier(0);
+                    auto rd = [&](float *v, int t) {
+                        const float4 q = *(const float4 *)(cgp_u + t + k);
+                        v[0] = q.x;
+                        v[BIG ? 1 : 0] = q.y;
+                        v[BIG ? 2 : 0] = q.z;
+                        v[BIG ? 3 : 0] = q.w;
+                    };
+                    rd(um, tc - t0);
+                    rd(up, tc + t0);
+                    rd(vm, tc - t1);
+                    rd(vp, tc + t1);
+                }
                 float sl = 0, su = 0;
-                sl += um[k] * lx[k];
-                su += up[k] * lxp[k];
+                sl += um[k % G] * lx[k];
+                su += up[k % G] * lxp[k];
                 if (D > 2) {
-                    sl += vm[D > 2 ? k : 0] * ly[k];
-                    su += vp[D > 2 ? k : 0] * lyp[k];
+                    sl += vm[D > 2 ? k % G : 0] * ly[k];
+                    su += vp[D > 2 ? k % G : 0] * lyp[k];
                 }
                 float hi = uhi;
                 if (k + 1 < C) {
-                    const float un = u[k + 1 < C ? k + 1 : k];
+                    const float un = U(k + 1 < C ? k + 1 : k);
                     hi = k + 1 < cnt ? un : uhi;
                 }
-                sl += (k > 0 ? u[k > 0 ? k - 1 : 0] : ulo) * lz[k];
+                const float uk = U(k);
+                sl += (k > 0 ? U(k > 0 ? k - 1 : 0) : ulo) * lz[k];
                 su += hi * lz[k + 1];
-                w[k] = (u[k] * dg[k] + sl) + su;
+                w[k] = (uk * (BIG ? diag(k) : dg[BIG ? 0 : k]) + sl) + su;
+                // the products are exact
+                gd = __builtin_fma((double)r[k], (double)uk, gd);
+                dd = __builtin_fma((double)uk, (double)w[k], dd);
             }
-#pragma unroll
-            for (int k = 0; k < C; ++k) cgp_w[tw[k]] = w[k];
-#pragma unroll
-            for (int k = 0; k < C; ++k) {  // the products are exact
-                gd = __builtin_fma((double)r[k], (double)u[k], gd);
-                dd = __builtin_fma((double)u[k], (double)w[k], dd);
-            }
+            if (BIG) __syncthreads();  // everyone has read u
+            own(cgp_w, w);
         }
         wave_sum2(gd, dd);
         if (lane == 0) {
@@ -386,8 +457,13 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     apply(a.tag);
 #pragma unroll
     for (int k = 0; k < C; ++k) {
-        p[k] = u[k];
-        s[k] = w[k];
+        if (BIG) {
+            ((float *)p4)[4 * (k / 4 * NB + tid) + k % 4] = U(k);
+            ((float *)s4)[4 * (k / 4 * NB + tid) + k % 4] = w[k];
+        } else {
+            p[BIG ? 0 : k] = U(k);
+            s[BIG ? 0 : k] = w[k];
+        }
     }
     float rho = 0, al = 0;
     for (int q = 1; q <= a.it; ++q) {
@@ -437,15 +513,31 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
         }
         rho = gam;
         const bool stop = q == a.it || fabs((double)al) < 1e-2;
-#pragma unroll
-        for (int k = 0; k < C; ++k) {
+        auto cell = [&](int k, float &pk, float &sk, float &xk) {
             if (q > 1) {
-                p[k] = u[k] + beta * p[k];
-                s[k] = w[k] + beta * s[k];
+                pk = U(k) + beta * pk;
+                sk = w[k] + beta * sk;
             }
-            if (XL) xl[k * NB + tid] += al * p[k];
-            else x[XL ? 0 : k] = x[XL ? 0 : k] + al * p[k];
-            r[k] = r[k] - al * s[k];
+            xk = xk + al * pk;
+            r[k] = r[k] - al * sk;
+        };
+        if constexpr (BIG) {
+#pragma unroll
+            for (int k = 0; k < C; k += 4) {
+                const int j = k / 4 * NB + tid;
+                __builtin_amdgcn_sched_barrier(0);
+                float4 pk = p4[j], sk = s4[j], xk = x4[j];
+                cell(k, pk.x, sk.x, xk.x);
+                cell(k + 1, pk.y, sk.y, xk.y);
+                cell(k + 2, pk.z, sk.z, xk.z);
+                cell(k + 3, pk.w, sk.w, xk.w);
+                p4[j] = pk;
+                s4[j] = sk;
+                x4[j] = xk;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < C; ++k) cell(k, p[k], s[k], XL ? xl[k * NB + tid] : x[XL ? 0 : k]);
         }
         if (stop) break;
 #pragma unroll
@@ -459,7 +551,8 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     }
 #pragma unroll
     for (int k = 0; k < C; ++k)
-        if (k < cnt) a.x[I0 + k * sz] = XL ? xl[k * NB + tid] : x[XL ? 0 : k];
+        if (k < cnt)
+            a.x[I0 + k * sz] = BIG ? xl[4 * (k / 4 * NB + tid) + k % 4] : XL ? xl[k * NB + tid] : x[XL ? 0 : k];
 }
 
 // ---------------------------------------------------------------------------
@@ -530,7 +623,7 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     const long sz = g.st[D - 1];
     // every thread works on all C cells of its column: those past its cnt are all zeros, read the tile's spare planes
     // and write its last word, so no load or store waits behind a branch
-    const int dump = t1 * (a.box.b[1] + 2) * (D > 2 ? a.box.b[2] + 2 : 1) + (C - 1) * tz;
+    const int dump = t1 * (a.box.b[1] + 2) * (D > 2 ? a.box.b[2] + 2 : 1) + cgp_spare(a.box.b[D - 1], C) * tz;
     for (int q = tid; q <= dump; q += NB) cgp_u[q] = 0.f;
     if (tid == 0) dead = 0;
     __syncthreads();
@@ -640,7 +733,7 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     const int nwg = a.box.nwg, ngrp = (nwg + CGP_GROUP - 1) / CGP_GROUP;
     const bool two = nwg > CGP_ONE;
     constexpr bool FAR = NB >= 1024;  // too large for one XCD
-    bool near = false;                // known once the first sum is
+    bool near = false;  // known once the first sum is
     auto half_of = [](double v, int j) { return (unsigned)((j & 1) ? __double2hiint(v) : __double2loint(v)); };
     auto faces = [&](unsigned tag) {  // w of the box's faces, from its tile
         cgp_word *hw = a.hw + (tag & 1 ? hslot : 0);
@@ -866,7 +959,8 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     }
 }
 // The variants: threads and cells per thread, the fewest first, as more cells per workgroup cost more than more
-// workgroups up to CGP_ONE (32^3: 1.9 µs with 2 cells on 256 threads, 2.4 with 4 on 512).
+// workgroups up to CGP_ONE (32^3: 1.9 µs with 2 cells on 256 threads, 2.4 with 4 on 512).  16 cells on 512 threads hold
+// twice as many as 4 on 1024, whose register limit 8 would exceed (14.5 µs for 128^3, with spills).
 struct CgpVariant {
     int D, NB, C, HC;
     void (*k)(CgpArgs);
@@ -875,8 +969,9 @@ inline const CgpVariant *cgp_variants(int &n) {
     static const CgpVariant v[] = {{2, 256, 1, 1, k_cgp<2, 256, 1, 1>}, {2, 256, 2, 1, k_cgp<2, 256, 2, 1>},
                                    {2, 512, 4, 1, k_cgp<2, 512, 4, 1>}, {2, 1024, 4, 1, k_cgp<2, 1024, 4, 1>},
                                    {3, 256, 1, 2, k_cgp<3, 256, 1, 2>}, {3, 256, 2, 3, k_cgp<3, 256, 2, 3>},
-                                   {3, 512, 4, 3, k_cgp<3, 512, 4, 3>}, {3, 1024, 4, 2, k_cgp<3, 1024, 4, 2>}};
-    n = 8;
+                                   {3, 512, 4, 3, k_cgp<3, 512, 4, 3>}, {3, 1024, 4, 2, k_cgp<3, 1024, 4, 2>},
+                                   {3, 512, 16, 6, k_cgp<3, 512, 16, 6>}};
+    n = 9;
     return v;
 }
 // pcg! in one launch: the variant of cgp_variants with the same number
@@ -884,7 +979,7 @@ typedef void (*PcgpKernel)(PcgpArgs);
 inline PcgpKernel pcgp_kernel(int q) {
     static const PcgpKernel k[] = {k_pcgp<2, 256, 1, 1>, k_pcgp<2, 256, 2, 1>, k_pcgp<2, 512, 4, 1>,
                                    k_pcgp<2, 1024, 4, 1>, k_pcgp<3, 256, 1, 2>, k_pcgp<3, 256, 2, 3>,
-                                   k_pcgp<3, 512, 4, 3>, k_pcgp<3, 1024, 4, 2>};
+                                   k_pcgp<3, 512, 4, 3>, k_pcgp<3, 1024, 4, 2>, nullptr};
     return k[q];
 }
 // boxes of a level of n cells per axis for a variant, at most maxwg of them; false: none fits
@@ -904,6 +999,7 @@ inline bool cgp_boxes(const int *n, const CgpVariant &v, int maxwg, CgpBox &o) {
                 const long lat = (long)b[0] * (v.D > 2 ? b[1] : 1), thr = lat * ((b[v.D - 1] + v.C - 1) / v.C);
                 const long f0 = (long)b[1] * b[2], f1 = (long)b[0] * b[2], f2 = v.D > 2 ? (long)b[0] * b[1] : 0;
                 const long h = 2 * (f0 + f1 + f2);
+                if (cgp_words(v.D, v.NB, v.C, b) * 4L > CGP_LDS) continue;
                 if (thr > v.NB || h > (long)(v.NB - 64) * v.HC) continue;
                 const long cost = (long)b[0] * b[1] * b[2] + h + (long)k0 * k1 * k2;
                 if (best >= 0 && cost >= best) continue;

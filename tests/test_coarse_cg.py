@@ -62,7 +62,7 @@ def projected(dims, perdir, launched, **kw):
 @pytest.mark.parametrize("dims,perdir", [
     ((256, 200), ()), ((200, 136), (1, 2)), ((2048, 16), (2,)), ((16, 2048), (1,)),
     ((64, 64, 64), ()), ((120, 88, 72), (1, 2)), ((100, 60, 84), (3,)), ((512, 16, 16), (1, 2, 3)),
-    ((16, 256, 32), ()), ((160, 160, 96), (2,)),
+    ((16, 256, 32), ()), ((160, 160, 96), (2,)), ((240, 208, 200), (1,)), ((256, 256, 248), (3,)),
 ])
 def test_one_launch_equals_one_launch_per_iteration(dims, perdir):
     say("coarse CG in one launch", dims, perdir)
