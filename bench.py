@@ -56,18 +56,25 @@ BYTES_PER_CELL = {
     "pcg_Ae": 4 + 12 + 4,                            # ϵ, L -> z
     "pcg_update": 20 + 12,                           # x, ϵ, r, z, iD -> x, r, z
     "increment": 4 + 4 + 12 + 4 + 8,                 # r, ϵ, L, x -> r, x
-    "load_inc": 8 + 4 + 12 + 8,                      # r64, iD, L -> r, x
-    "prolong_inc": 4 + 4 + 12 + 4 + 0.5 + 12,        # r, x, L, iD, coarse x -> r, x, ϵ
+    "load_inc": 8 + 4 + 12 + 4,                      # r64, iD, L -> r
+    "prolong_inc": 4 + 12 + 0.5 + 4,                 # r, L, coarse x -> r
     "pcg_last": 4 + 4 + 8 + 8 + 4,                   # x, ϵ, r64, q64 -> x
-    "cheb2_dots": 4 + 12 + 4 + 4 + 4 + 8 + 8 + 4,    # ϵ, L, r, x, iD, r64, q64 -> x
+    "cheb2_dots": 12 + 4 + 4 + 0.5 + 8 + 8 + 4,      # L, r, iD, coarse x, r64, q64 -> x
     "fcg_Ap": 4 + 8 + 12 + 16,                       # w, p, L -> p', q
     "fcg_update": 32 + 16,                           # p', q, x64, r64 -> x64, r64
     "redist": (12 + 16 + 16) / 3,                    # ϕ, ϕini (+ ϕ⁰ in stages 2, 3) -> ϕ', per stage
-    # single-reduction CG on coarse level l (per cell of that level): one step
-    # r, w, s, iD, p, x, L -> p, s', x, r', w' on level 1; on the levels that
-    # solve in one launch r, iD, L, x -> x, once
-    "cg1_l1": 36 + 20, "cg1_l2": 24 + 4, "cg1_l3": 24 + 4,
+    # single-reduction CG on coarse level l (per cell of that level): a whole
+    # solve in one launch r, iD, L, x -> x
+    "cg1_l1": 24 + 4, "cg1_l2": 24 + 4, "cg1_l3": 24 + 4,
 }
+# levels too large for one launch: a step r, w, s, iD, p, x, L -> p, s', x, r', w'
+CG1_STEP, CG1_CELLS = 36 + 20, 2 << 20
+
+
+def bytes_per_cell(k, cells):
+    return CG1_STEP if k.startswith("cg1") and cells > CG1_CELLS else BYTES_PER_CELL[k]
+
+
 # coarse level of a class (its cells are (N >> level)^3); 0 for the fine-level classes
 LEVEL = {"cg1_l1": 1, "cg1_l2": 2, "cg1_l3": 3}
 # kernel classes timed with HIP events in the timed region; the one with the
@@ -271,7 +278,7 @@ def main():
                 avg = ms.value / nl.value
                 kc = (N >> LEVEL.get(k, 0)) ** 3
                 out[k] = dict(launches=nl.value, total_ms=round(ms.value, 3), avg_ms=round(avg, 4),
-                              GBps=round(BYTES_PER_CELL[k] * kc / (avg * 1e-3) / 1e9, 1), cells=kc)
+                              GBps=round(bytes_per_cell(k, kc) * kc / (avg * 1e-3) / 1e9, 1), cells=kc)
         return out
 
     # Every class is timed over the warm-up steps; inside the timed steps only
@@ -330,7 +337,7 @@ def main():
     if dom:
         traffic, traffic_src = pmc_traffic(dom) if (args.case, N) == ("pool", 256) else (None, None)
         avg_ms = timed[dom]["avg_ms"]
-        bpl = BYTES_PER_CELL[dom] * timed[dom]["cells"]
+        bpl = bytes_per_cell(dom, timed[dom]["cells"]) * timed[dom]["cells"]
         achieved = bpl / (avg_ms * 1e-3) / 1e9
         out["roofline"] = {"kernel": dom, "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK,
                            "unit": "GB/s", "frac": round(achieved / HBM_PEAK, 4),

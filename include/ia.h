@@ -287,7 +287,7 @@ enum ia_prof_class {
     IA_PROF_PCG_UPDATE = 4,   /* pcg x,r,z update, finest level */
     IA_PROF_INCREMENT = 5,    /* increment! r -= Aϵ, x += ϵ, finest level (unfused) */
     IA_PROF_LOAD_INC = 6,     /* FCG residual load + Jacobi! + increment!, finest level */
-    IA_PROF_PROLONG_INC = 7,  /* prolongate! + increment! + pcg! ϵ = r·iD, finest level */
+    IA_PROF_PROLONG_INC = 7,  /* prolongate! + increment!, finest level (with pcg! ϵ = r·iD where a pcg! follows) */
     IA_PROF_FCG_AP = 8,       /* FCG p = w + βp, q = A p (FP64) */
     IA_PROF_FCG_UPDATE = 9,   /* FCG x += αp, r -= αq (FP64) */
     IA_PROF_PCG_LAST = 10,    /* the flexible CG's fine smoother fused with its dots: two Chebyshev steps

@@ -847,8 +847,11 @@ template <class T> struct Impl {
         if (then_pcg) {
             bool f0 = l == 0;
             if (f0) prof_begin(c, IA_PROF_PROLONG_INC);
-            hipLaunchKernelGGL(k_mg_prolong_inc_init<T>, cb(fl), dim3(NT), 0, c->s, view(fl, rev), co.g, P<T>(co.x),
-                               pp(c, PP_A));
+            auto k = cit != c->cit_fcg ? k_mg_prolong_inc_init<PRO_PCG, T>
+                     : l > 0           ? k_mg_prolong_inc_init<PRO_CG1, T>
+                     : c->fine_cheb    ? k_mg_prolong_inc_init<PRO_R, T>
+                                       : k_mg_prolong_inc_init<PRO_PCG, T>;
+            hipLaunchKernelGGL(k, cb(fl), dim3(NT), 0, c->s, view(fl, rev), co.g, P<T>(co.x), pp(c, PP_A));
             if (f0) prof_end(c, IA_PROF_PROLONG_INC);
         } else {
             hipLaunchKernelGGL(k_mg_prolong<T>, cb(fl), dim3(NT), 0, c->s, view(fl), co.g, P<T>(co.x));
@@ -1021,15 +1024,16 @@ template <class T> struct Impl {
         FcgV<T> f = fview(c, par, par), fr = fview(c, par, !par);
         dim3 B = cb(l0);
         prof_begin(c, IA_PROF_LOAD_INC);
-        hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0, par), pp(c, rbuf));
+        hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0, par), pp(c, rbuf),
+                           c->fine_cheb ? 0 : 1);
         prof_end(c, IA_PROF_LOAD_INC);
         if (c->fine_cheb) {
             vcycle(c, 0, c->cit_fcg, true, true, false, !par);
             double c0, ca, cb;
             cheb2_coeffs(c0, ca, cb);
             prof_begin(c, IA_PROF_PCG_LAST);
-            hipLaunchKernelGGL(k_cheb2_dots<T>, B, dim3(NT), 0, c->s, view(l0, par), f, (T)c0, (T)ca, (T)cb, pp(c, PP_FD),
-                               first);
+            hipLaunchKernelGGL(k_cheb2_dots<T>, B, dim3(NT), 0, c->s, view(l0, par), c->lev[1].g, P<T>(c->lev[1].x), f,
+                               (T)c0, (T)ca, (T)cb, pp(c, PP_FD), first);
             prof_end(c, IA_PROF_PCG_LAST);
         } else if (c->smooth_it > 0) {
             vcycle(c, 0, c->cit_fcg, true, true);
@@ -1080,7 +1084,7 @@ template <class T> struct Impl {
             // plain multigrid: one V-cycle + pcg!(fine, 6) on the unit-RMS residual, x += s·w
             f = fview(c);
             prof_begin(c, IA_PROF_LOAD_INC);
-            hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0), pp(c, rbuf));
+            hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0), pp(c, rbuf), 1);
             prof_end(c, IA_PROF_LOAD_INC);
             vcycle(c, 0, c->cit_wl, true, true);
             pcg(c, l0, 6, true);

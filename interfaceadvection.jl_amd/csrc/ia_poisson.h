@@ -260,7 +260,9 @@ template <int D, class T> __device__ inline T mul7(const S7<D, T> &s) {
 // plane); the z-neighbours stay in registers.  Periodic axes are resolved by
 // evaluating ghost positions at their periodic image, so the tile holds
 // exactly the values the neighbour-offset stencil would read.
-//   body(p, I, c, xm, xp, ym, yp, zm, zp) runs for every interior cell.
+//   body(p, I, pre, c, xm, xp, ym, yp, zm, zp[, raw]) runs for every interior
+// cell, with what pre(I[, x, y, z]) loaded one plane ahead; raw is what load
+// gave for the cell.
 // ---------------------------------------------------------------------------
 __device__ inline int per_img(const Grid &g, int a, int q) {
     if (g.per[a]) {
@@ -296,6 +298,13 @@ __device__ inline void tiled7(const Grid &g, const CTiling &t, LF load, CF comb,
         else
             return load((long)q0 + g.st[1] * q1 + g.st[2] * q2);
     };
+    auto PV = [&](int z) {
+        const long I = (long)x + g.st[1] * y + g.st[2] * z;
+        if constexpr (std::is_invocable_v<PF, long, int, int, int>)
+            return pre(active ? I : 0, active ? x : 1, active ? y : 1, z);
+        else
+            return pre(active ? I : 0);
+    };
     R rm{}, rc{}, rp{}, rhx{}, rhy{};
     if (inarr) {
         rm = LD(xi, yi, per_img(g, 2, zlo - 1));
@@ -305,8 +314,7 @@ __device__ inline void tiled7(const Grid &g, const CTiling &t, LF load, CF comb,
     if (hx_ok) rhx = LD(hxq, yi, zlo);
     if (hy_ok) rhy = LD(xi, hyq, zlo);
     V em = comb(rm), ec = comb(rc);
-    long I0 = (long)x + g.st[1] * y + g.st[2] * zlo;
-    auto pv = pre(active ? I0 : 0);
+    auto pv = PV(zlo);
     for (int z = zlo; z <= zhi; ++z) {
         int buf = (z - zlo) & 1;
         long I = (long)x + g.st[1] * y + g.st[2] * z;
@@ -317,7 +325,7 @@ __device__ inline void tiled7(const Grid &g, const CTiling &t, LF load, CF comb,
             if (inarr) rn = LD(xi, yi, per_img(g, 2, z + 2));
             if (hx_ok) nhx = LD(hxq, yi, z + 1);
             if (hy_ok) nhy = LD(xi, hyq, z + 1);
-            pvn = pre(active ? I + g.st[2] : 0);
+            pvn = PV(z + 1);
         }
         V ep = comb(rp);
         tile[buf][ty + 1][tx + 1] = ec;
@@ -326,9 +334,14 @@ __device__ inline void tiled7(const Grid &g, const CTiling &t, LF load, CF comb,
         __syncthreads();
         if (active) {
             int p[3] = {x, y, z};
-            body(p, I, pv, ec, tile[buf][ty + 1][tx], tile[buf][ty + 1][tx + 2], tile[buf][ty][tx + 1],
-                 tile[buf][ty + 2][tx + 1], em, ep);
+            const V xm = tile[buf][ty + 1][tx], xp = tile[buf][ty + 1][tx + 2];
+            const V ym = tile[buf][ty][tx + 1], yp = tile[buf][ty + 2][tx + 1];
+            if constexpr (std::is_invocable_v<BF, const int *, long, decltype(pv) &, V, V, V, V, V, V, V, const R &>)
+                body(p, I, pv, ec, xm, xp, ym, yp, em, ep, rc);
+            else
+                body(p, I, pv, ec, xm, xp, ym, yp, em, ep);
         }
+        rc = rp;
         em = ec;
         ec = ep;
         rp = rn;
@@ -557,8 +570,12 @@ __global__ void __launch_bounds__(NT) k_mg_prolong(LevV<T> f, Grid gc, const T *
 // prolongate! + increment! + the first statement of the pcg! that follows:
 // ϵ = coarse x[down(I)] formed on the fly at the cell and its neighbours;
 // r -= Aϵ; x += ϵ; then ϵ = r·iD and partial r·ϵ (-> ρ₀).  pcg!'s z = r·iD
-// is not stored: its first use overwrites it with Aϵ.
-template <int D, class T>
+// is not stored: its first use overwrites it with Aϵ.  MODE: PRO_PCG all of
+// that, PRO_CG1 r and x alone (the single-reduction CG forms its own ϵ),
+// PRO_R r alone (k_cheb2_dots forms x): 36, 28 and 20 bytes a cell, 130 and
+// 71 µs at 256³ for the first and the last.
+enum { PRO_PCG, PRO_CG1, PRO_R };
+template <int MODE, int D, class T>
 __device__ inline void prolong_inc_init_d(const LevV<T> &l, const Grid &gc, const T *__restrict__ xc, double &v) {
     T *__restrict__ r = l.r;
     T *__restrict__ x = l.x;
@@ -581,17 +598,19 @@ __device__ inline void prolong_inc_init_d(const LevV<T> &l, const Grid &gc, cons
                 Pre w;
                 w.l = load_L6<T>(g, I, l.L);
                 w.r = r[I];
-                w.x = x[I];
-                w.d = iD[I];
+                w.x = MODE != PRO_R ? x[I] : T(0);
+                w.d = MODE == PRO_PCG ? iD[I] : T(0);
                 return w;
             },
             [&](const int *, long I, const Pre &pv, T c, T xm, T xp, T ym, T yp, T zm, T zp) {
                 T rr = pv.r - mult7<T>(pv.l, c, xm, xp, ym, yp, zm, zp);
                 r[I] = rr;
-                x[I] = pv.x + c;
-                T zz = rr * pv.d;
-                e[I] = zz;
-                v += (double)rr * (double)zz;
+                if (MODE != PRO_R) x[I] = pv.x + c;
+                if (MODE == PRO_PCG) {
+                    T zz = rr * pv.d;
+                    e[I] = zz;
+                    v += (double)rr * (double)zz;
+                }
             });
         return;
     }
@@ -621,25 +640,27 @@ __device__ inline void prolong_inc_init_d(const LevV<T> &l, const Grid &gc, cons
                 w.s.lp[i] = l.L[g.ns * i + I + g.st[i]];
             }
             w.r = r[I];
-            w.x = x[I];
-            w.d = iD[I];
+            w.x = MODE != PRO_R ? x[I] : T(0);
+            w.d = MODE == PRO_PCG ? iD[I] : T(0);
             return w;
         },
         [&](const int *, long I, const V &w) {
             T rr = w.r - mul7<D>(w.s);
             r[I] = rr;
-            x[I] = w.x + w.s.c;
-            T zz = rr * w.d;
-            e[I] = zz;
-            v += (double)rr * (double)zz;
+            if (MODE != PRO_R) x[I] = w.x + w.s.c;
+            if (MODE == PRO_PCG) {
+                T zz = rr * w.d;
+                e[I] = zz;
+                v += (double)rr * (double)zz;
+            }
         });
 }
-template <class T>
+template <int MODE, class T>
 __global__ void __launch_bounds__(NT) k_mg_prolong_inc_init(LevV<T> l, Grid gc, const T *xc, double *partA) {
     HALT_IF(l)
     double v = 0;
-    DISPATCH_D(l.g, prolong_inc_init_d<D>(l, gc, xc, v);)
-    block_partial(v, l.t, partA);
+    DISPATCH_D(l.g, prolong_inc_init_d<MODE, D>(l, gc, xc, v);)
+    if (MODE == PRO_PCG) block_partial(v, l.t, partA);
 }
 // pcg! (WaterLily):  z = ϵ = r·iD ; partial r·z  (-> ρ₀)
 template <class T>
@@ -835,7 +856,22 @@ __global__ void __launch_bounds__(NT) k_cg1_init(LevV<T> l, T *w, PcgState *S, d
     T *__restrict__ pd = l.e;  // search direction
     T *__restrict__ s = l.z;
     double g = 0, d = 0;
-    DISPATCH_D(l.g, {
+    if (l.g.D == 3 && l.t.zb > 1) {
+        struct Raw {
+            T r, d;
+        };
+        tiled7<T, Raw>(
+            l.g, l.t, [&](long K) { return Raw{r[K], iD[K]}; }, [&](const Raw &q) { return q.r * q.d; },
+            [&](long I) { return load_L6<T>(l.g, I, l.L); },
+            [&](const int *, long I, const L6<T> &lv, T c, T xm, T xp, T ym, T yp, T zm, T zp, const Raw &q) {
+                T ww = mult7<T>(lv, c, xm, xp, ym, yp, zm, zp);
+                pd[I] = c;
+                s[I] = ww;
+                w[I] = ww;
+                g += (double)q.r * (double)c;
+                d += (double)c * (double)ww;
+            });
+    } else DISPATCH_D(l.g, {
         col_pipe(l.g, l.t,
                  [&](const int *q, long I) { return ld7<D>(l.g, q, I, l.L, [&](long K) { return r[K] * iD[K]; }); },
                  [&](const int *, long I, const S7<D, T> &st) {
@@ -1388,22 +1424,32 @@ __global__ void __launch_bounds__(NT) k_fcg_load(FcgV<T> f, const double *part_r
         f.w[I] = T(0);
     })
 }
+// a/s, is = 1/s: correctly rounded from the quotient's remainder (Markstein),
+// in three operations instead of a division's dozen
+__device__ inline double div_by(double a, double s, double is) {
+    const double q = a * is;
+    return __builtin_fma(__builtin_fma(-q, s, a), is, q);
+}
 // k_fcg_load fused with the V-cycle's first Jacobi! + increment! on level 0:
 // ϵ = (r/s)·iD is formed on the fly at the cell and its neighbours, so
-// r_T = r/s - Aϵ and x_T = ϵ are written without storing r/s or ϵ.
+// r_T = r/s - Aϵ and, with keep_x, x_T = ϵ are written without storing r/s or
+// ϵ.  Without it k_cheb2_dots forms x_T's ϵ again (4 bytes a cell less here
+// and there): 122 µs at 256³, 143 with it and two divisions a cell.
 template <int D, class T>
-__device__ inline void load_inc_cell(const FcgV<T> &f, const LevV<T> &l, double s, const int p[3], long I) {
+__device__ inline void load_inc_cell(const FcgV<T> &f, const LevV<T> &l, double s, double is, int keep_x,
+                                     const int p[3], long I) {
     const double *__restrict__ r64 = f.r;
     const T *__restrict__ iD = l.iD;
-    auto ev = [&](long K) { return (T)(r64[K] / s) * iD[K]; };
-    T wr = (T)(r64[I] / s);
+    auto ev = [&](long K) { return (T)div_by(r64[K], s, is) * iD[K]; };
+    T wr = (T)div_by(r64[I], s, is);
     l.r[I] = wr - mgmult_fd<D>(l.g, p, I, l.L, ev);
-    l.x[I] = T(0) + ev(I);
+    if (keep_x) l.x[I] = T(0) + ev(I);
 }
 template <class T>
-__global__ void __launch_bounds__(NT) k_fcg_load_inc(FcgV<T> f, LevV<T> l, const double *part_rr) {
+__global__ void __launch_bounds__(NT) k_fcg_load_inc(FcgV<T> f, LevV<T> l, const double *part_rr, int keep_x) {
     HALT_IF(l)
     double s = sqrt(block_total(part_rr, f.t.nblk) / (double)f.ncell);
+    const double is = 1.0 / s;
     if (blockIdx.x == 0 && threadIdx.x == 0) f.S->sload = s;
     if (l.g.D == 3) {
         const double *__restrict__ r64 = f.r;
@@ -1414,20 +1460,16 @@ __global__ void __launch_bounds__(NT) k_fcg_load_inc(FcgV<T> f, LevV<T> l, const
             double r;
             T d;
         };
-        struct Pre {
-            L6<T> l;
-            double rc;
-        };
         tiled7<T, Raw>(
-            l.g, l.t, [&](long K) { return Raw{r64[K], iD[K]}; }, [&](const Raw &q) { return (T)(q.r / s) * q.d; },
-            [&](long I) { return Pre{load_L6<T>(l.g, I, l.L), r64[I]}; },
-            [&](const int *, long I, const Pre &pv, T c, T xm, T xp, T ym, T yp, T zm, T zp) {
-                T wr = (T)(pv.rc / s);
-                r[I] = wr - mult7<T>(pv.l, c, xm, xp, ym, yp, zm, zp);
-                x[I] = T(0) + c;
+            l.g, l.t, [&](long K) { return Raw{r64[K], iD[K]}; },
+            [&](const Raw &q) { return (T)div_by(q.r, s, is) * q.d; }, [&](long I) { return load_L6<T>(l.g, I, l.L); },
+            [&](const int *, long I, const L6<T> &lv, T c, T xm, T xp, T ym, T yp, T zm, T zp, const Raw &q) {
+                T wr = (T)div_by(q.r, s, is);
+                r[I] = wr - mult7<T>(lv, c, xm, xp, ym, yp, zm, zp);
+                if (keep_x) x[I] = T(0) + c;
             });
     } else {
-        COL_LOOP(f, { load_inc_cell<2>(f, l, s, p, I); })
+        COL_LOOP(f, { load_inc_cell<2>(f, l, s, is, keep_x, p, I); })
     }
 }
 // the last pcg! iteration on level 0 inside the preconditioner, fused with
@@ -1486,35 +1528,44 @@ inline void cheb2_coeffs(double &c0, double &ca, double &cb) {
 }
 // the preconditioner's fine-level smoother: two Chebyshev steps on D⁻¹A for
 // the eigenvalue interval [0.5, 2] (Saad's three-term recurrence; c0 = 1/θ,
-// ca = ρ₁ρ₀, cb = 2ρ₁/δ), fused with the FCG dots.  ϵ = r·iD is on hand from
-// the V-cycle's last prolongate!/increment!, so d₀ = c0·ϵ at every stencil
-// point; r₁ = r - A d₀; d₁ = ca·d₀ + cb·(r₁·iD); x = (x + d₀) + d₁ (the
-// second step's residual update is dead: only x leaves the preconditioner).
-// Then the partials of w·r and w·q with w = s·x.
+// ca = ρ₁ρ₀, cb = 2ρ₁/δ), fused with the FCG dots.  d₀ = c0·(r·iD) is formed
+// at every stencil point, and x, which so far is the first Jacobi!'s ϵ =
+// (r64/s)·iD plus the prolonged coarse x, at the cell: neither is stored before
+// (138 µs at 256³, 161 when they were).  r₁ = r - A d₀; d₁ = ca·d₀ +
+// cb·(r₁·iD); x = (x + d₀) + d₁ (the second step's residual update is dead:
+// only x leaves the preconditioner).  Then the partials of w·r and w·q with w = s·x.
 template <class T>
-__global__ void __launch_bounds__(NT) k_cheb2_dots(LevV<T> l, FcgV<T> f, T c0, T ca, T cb, double *part, int first) {
+__global__ void __launch_bounds__(NT) k_cheb2_dots(LevV<T> l, Grid gc, const T *__restrict__ xc, FcgV<T> f, T c0,
+                                                   T ca, T cb, double *part, int first) {
     HALT_IF(l)
-    double s = f.S->sload;
+    const double s = f.S->sload, is = 1.0 / s;
     double a = 0, b = 0;
     T *__restrict__ x = l.x;
-    const T *__restrict__ e = l.e;
     const T *__restrict__ r = l.r;
     const T *__restrict__ iD = l.iD;
     const double *__restrict__ r64 = f.r;
     const double *__restrict__ q64 = f.q;
     if (l.g.D == 3 && l.t.zb > 1) {
+        struct Raw {
+            T r, d;
+        };
         struct Pre {
             L6<T> l;
-            T r, x, d;
+            T c;
             double r64, q64;
         };
-        tiled7<T, T>(
-            l.g, l.t, [&](long K) { return e[K]; }, [&](T q) { return q * c0; },
-            [&](long I) { return Pre{load_L6<T>(l.g, I, l.L), r[I], x[I], iD[I], r64[I], first ? 0.0 : q64[I]}; },
-            [&](const int *, long I, const Pre &pv, T c, T xm, T xp, T ym, T yp, T zm, T zp) {
-                T r1 = pv.r - mult7<T>(pv.l, c, xm, xp, ym, yp, zm, zp);
-                T d1 = ca * c + cb * (r1 * pv.d);
-                T xn = (pv.x + c) + d1;
+        tiled7<T, Raw>(
+            l.g, l.t, [&](long K) { return Raw{r[K], iD[K]}; }, [&](const Raw &q) { return (q.r * q.d) * c0; },
+            [&](long I, int p0, int p1, int p2) {
+                return Pre{load_L6<T>(l.g, I, l.L),
+                           xc[(long)((p0 + 3) / 2 - 1) + gc.st[1] * ((p1 + 3) / 2 - 1) + gc.st[2] * ((p2 + 3) / 2 - 1)],
+                           r64[I], first ? 0.0 : q64[I]};
+            },
+            [&](const int *, long I, const Pre &pv, T c, T xm, T xp, T ym, T yp, T zm, T zp, const Raw &q) {
+                T r1 = q.r - mult7<T>(pv.l, c, xm, xp, ym, yp, zm, zp);
+                T d1 = ca * c + cb * (r1 * q.d);
+                T x0 = (T(0) + (T)div_by(pv.r64, s, is) * q.d) + pv.c;
+                T xn = (x0 + c) + d1;
                 x[I] = xn;
                 double ww = s * (double)xn;
                 a += ww * pv.r64;
@@ -1524,18 +1575,21 @@ __global__ void __launch_bounds__(NT) k_cheb2_dots(LevV<T> l, FcgV<T> f, T c0, T
         DISPATCH_D(l.g, {
             struct V {
                 S7<D, T> s7;
-                T r, x, d;
+                T r, c, d;
                 double r64, q64;
             };
             col_pipe(l.g, l.t,
                      [&](const int *p, long I) {
-                         return V{ld7<D>(l.g, p, I, l.L, [&](long K) { return e[K] * c0; }), r[I], x[I], iD[I],
-                                  r64[I], first ? 0.0 : q64[I]};
+                         long Kc = (long)((p[0] + 3) / 2 - 1) + gc.st[1] * ((p[1] + 3) / 2 - 1);
+                         if (D > 2) Kc += gc.st[2] * ((p[2] + 3) / 2 - 1);
+                         return V{ld7<D>(l.g, p, I, l.L, [&](long K) { return (r[K] * iD[K]) * c0; }), r[I], xc[Kc],
+                                  iD[I], r64[I], first ? 0.0 : q64[I]};
                      },
                      [&](const int *, long I, const V &v) {
                          T r1 = v.r - mul7<D>(v.s7);
                          T d1 = ca * v.s7.c + cb * (r1 * v.d);
-                         T xn = (v.x + v.s7.c) + d1;
+                         T x0 = (T(0) + (T)div_by(v.r64, s, is) * v.d) + v.c;
+                         T xn = (x0 + v.s7.c) + d1;
                          x[I] = xn;
                          double ww = s * (double)xn;
                          a += ww * v.r64;
