@@ -136,7 +136,7 @@ struct ia_ctx {
     bool ls_valid = false;
     const int *halt = nullptr;   // the flexible CG's stop flag while a pipelined solve runs
     StepOut *hst = nullptr;      // pinned: what the last kernel of a step hands back
-    FcgState *pin = nullptr;     // pinned host copies of the solver state (two slots)
+    FcgState *pin = nullptr;     // pinned: ‖r‖² and halt after an iteration (two slots)
     hipEvent_t it_ev[2] = {nullptr, nullptr};
     // caller-owned device buffers adopted by ia_attach_field (nullptr: the
     // library's own); att_fi/att_f0i: the f-pool slots holding attached f, f⁰
@@ -1016,15 +1016,15 @@ template <class T> struct Impl {
         return host_total(c, PP_FRR, l0.ct.nblk, 1, rr);
     }
     // one flexible-CG iteration: preconditioner (V-cycle + fine smoothing) and
-    // the FP64 Krylov update.  The input residual's partial sums are in
-    // buffer `rbuf` (the true residual after a restart, else the last update).
-    static void fcg_body(ia_ctx *c, int first, int par, int rbuf) {
+    // the FP64 Krylov update.  The input residual's ‖r‖² is in the state
+    // (k_fcg_begin's, then k_fcg_check's).
+    static void fcg_body(ia_ctx *c, int first, int par) {
         Level &l0 = c->lev[0];
         // the finest level's five kernels alternate their direction (par alternates too, and so does the next one)
         FcgV<T> f = fview(c, par, par), fr = fview(c, par, !par);
         dim3 B = cb(l0);
         prof_begin(c, IA_PROF_LOAD_INC);
-        hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0, par), pp(c, rbuf),
+        hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0, par),
                            c->fine_cheb ? 0 : 1);
         prof_end(c, IA_PROF_LOAD_INC);
         if (c->fine_cheb) {
@@ -1042,15 +1042,26 @@ template <class T> struct Impl {
             vcycle(c, 0, c->cit_fcg, true, false);
             hipLaunchKernelGGL(k_fcg_dots<T>, B, dim3(NT), 0, c->s, f, pp(c, PP_FD), first);
         }
+        const bool many = l0.ct.nblk > FCG_MANY;
+        if (many)
+            hipLaunchKernelGGL(k_fcg_sum, dim3(1), dim3(NT), 0, c->s, &c->fst->halt, pp(c, PP_FD), l0.ct.nblk, 2,
+                               &c->fst->wr, &c->fst->wq);
         prof_begin(c, IA_PROF_FCG_AP);
         hipLaunchKernelGGL(k_fcg_Ap<T>, B, dim3(NT), 0, c->s, fr, pp(c, PP_FD), pp(c, PP_FAP), first);
         prof_end(c, IA_PROF_FCG_AP);
+        if (many)
+            hipLaunchKernelGGL(k_fcg_sum, dim3(1), dim3(NT), 0, c->s, &c->fst->halt, pp(c, PP_FAP), l0.ct.nblk, 1,
+                               &c->fst->pq, (double *)nullptr);
         prof_begin(c, IA_PROF_FCG_UPDATE);
         hipLaunchKernelGGL(k_fcg_update<T>, B, dim3(NT), 0, c->s, f, pp(c, PP_FAP), pp(c, PP_FU));
         prof_end(c, IA_PROF_FCG_UPDATE);
     }
-    static int fcg_iteration(ia_ctx *c, int first, int par, int rbuf) {
-        fcg_body(c, first, par, rbuf);
+    static void fcg_begin(ia_ctx *c) {
+        hipLaunchKernelGGL(k_fcg_begin, dim3(1), dim3(NT), 0, c->s, c->fst, pp(c, PP_FRR), c->lev[0].ct.nblk);
+    }
+    static int fcg_iteration(ia_ctx *c, int first, int par) {
+        if (first) fcg_begin(c);
+        fcg_body(c, first, par);
         LAUNCHCHK(c);
         return IA_OK;
     }
@@ -1067,7 +1078,6 @@ template <class T> struct Impl {
         }
         FcgV<T> f = fview(c);
         dim3 B = cb(l0);
-        hipLaunchKernelGGL(k_fcg_halt, dim3(1), dim3(64), 0, c->s, c->fst, 0);
         hipLaunchKernelGGL(k_fcg_init<T>, B, dim3(NT), 0, c->s, f, P<T>(u), P<T>(c->p), dtw, pp(c, PP_FI));
         hipLaunchKernelGGL(k_fcg_center_z<T>, B, dim3(NT), 0, c->s, f, pp(c, PP_FI), pp(c, PP_FZ));
         double zn2 = 0, rr = 0;
@@ -1075,7 +1085,6 @@ template <class T> struct Impl {
         if (int e = true_resid(c, &rr)) return e;
         if (c->P.poisson_mode == IA_POISSON_LEARNED)
             if (int e = cnn_prelude(c, &rr)) return e;
-        int rbuf = PP_FRR;  // buffer holding the partials of ‖r‖²
         double zn = sqrt(zn2);
         double rel = zn > 0 ? sqrt(rr) / zn : 0.0;
         int it = 0;
@@ -1083,15 +1092,15 @@ template <class T> struct Impl {
         while (c->P.poisson_mode == IA_POISSON_PLAIN && rel > c->P.poisson_rtol && it < c->P.poisson_max_outer) {
             // plain multigrid: one V-cycle + pcg!(fine, 6) on the unit-RMS residual, x += s·w
             f = fview(c);
+            fcg_begin(c);
             prof_begin(c, IA_PROF_LOAD_INC);
-            hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0), pp(c, rbuf), 1);
+            hipLaunchKernelGGL(k_fcg_load_inc<T>, B, dim3(NT), 0, c->s, f, view(l0), 1);
             prof_end(c, IA_PROF_LOAD_INC);
             vcycle(c, 0, c->cit_wl, true, true);
             pcg(c, l0, 6, true);
             hipLaunchKernelGGL(k_ir_accum<T>, B, dim3(NT), 0, c->s, f);
             LAUNCHCHK(c);
             if (int e = true_resid(c, &rr)) return e;
-            rbuf = PP_FRR;
             rel = sqrt(rr) / zn;
             it++;
         }
@@ -1108,11 +1117,10 @@ template <class T> struct Impl {
             } hs(&c->fst->halt);
             int queued = 0, qslot = 0, rslot = 0;
             auto enqueue = [&](int first) -> int {
-                if (int e = fcg_iteration(c, first, par, rbuf)) return e;
+                if (int e = fcg_iteration(c, first, par)) return e;
                 par ^= 1;
-                rbuf = PP_FU;
-                hipLaunchKernelGGL(k_fcg_check<T>, dim3(1), dim3(NT), 0, c->s, fview(c), pp(c, PP_FU), zn, rtol);
-                HIPCHK(c, hipMemcpyAsync(&c->pin[qslot], c->fst, sizeof(FcgState), hipMemcpyDeviceToHost, c->s));
+                hipLaunchKernelGGL(k_fcg_check<T>, dim3(1), dim3(NT), 0, c->s, fview(c), pp(c, PP_FU), zn, rtol,
+                                   &c->pin[qslot]);
                 HIPCHK(c, hipEventRecord(c->it_ev[qslot], c->s));
                 qslot ^= 1;
                 queued++;
@@ -1139,8 +1147,6 @@ template <class T> struct Impl {
                     if (int e = true_resid(c, &rr)) return e;
                     rel = sqrt(rr) / zn;
                     if (rel <= rtol || it >= maxo) break;
-                    hipLaunchKernelGGL(k_fcg_halt, dim3(1), dim3(64), 0, c->s, c->fst, 0);
-                    rbuf = PP_FRR;
                     if (int e = enqueue(1)) return e;
                     continue;
                 }

@@ -62,7 +62,7 @@ struct PcgState {
 };
 // scalar state of the flexible CG
 struct FcgState {
-    double sload, wr, beta, pq, alpha;
+    double sload, wr, wq, beta, pq, alpha;
     double rr;      // ‖r‖² after the last accepted update
     int halt, pad;  // set when the recursive residual met the tolerance:
                     // every solver kernel queued after that returns at once
@@ -1308,6 +1308,10 @@ __global__ void __launch_bounds__(NT) k_mg_perbc(LevV<T> l, T *x) {
 // ---------------------------------------------------------------------------
 // FP64 flexible CG (FCG(1)) preconditioned by the FP32 V-cycle
 // ---------------------------------------------------------------------------
+// above so many workgroups a workgroup that summed everyone's partial sums
+// would read about as much for them as for its cells (512³: 16384 of 256 KB
+// each), so one more launch sums them first (Ap 1572 -> 1203 µs)
+constexpr long FCG_MANY = 4096;
 template <class T> struct FcgV {
     Grid g;
     CTiling t;
@@ -1413,27 +1417,17 @@ __global__ void __launch_bounds__(NT) k_fcg_center_r(FcgV<T> f, const double *pa
     })
     block_partial(v, f.t, part);
 }
-// preconditioner input r/s (s = ‖r‖/√n, so WaterLily's absolute pcg! exit
-// thresholds see a unit-RMS residual), x = 0
-template <class T>
-__global__ void __launch_bounds__(NT) k_fcg_load(FcgV<T> f, const double *part_rr) {
-    double s = sqrt(block_total(part_rr, f.t.nblk) / (double)f.ncell);
-    if (blockIdx.x == 0 && threadIdx.x == 0) f.S->sload = s;
-    COL_LOOP(f, {
-        f.wr[I] = (T)(f.r[I] / s);
-        f.w[I] = T(0);
-    })
-}
 // a/s, is = 1/s: correctly rounded from the quotient's remainder (Markstein),
 // in three operations instead of a division's dozen
 __device__ inline double div_by(double a, double s, double is) {
     const double q = a * is;
     return __builtin_fma(__builtin_fma(-q, s, a), is, q);
 }
-// k_fcg_load fused with the V-cycle's first Jacobi! + increment! on level 0:
+// the preconditioner's input r/s fused with the V-cycle's first Jacobi! + increment! on level 0:
 // ϵ = (r/s)·iD is formed on the fly at the cell and its neighbours, so
 // r_T = r/s - Aϵ and, with keep_x, x_T = ϵ are written without storing r/s or
-// ϵ.  Without it k_cheb2_dots forms x_T's ϵ again (4 bytes a cell less here
+// ϵ (s = ‖r‖/√n, so WaterLily's absolute pcg! exit thresholds see a unit-RMS
+// residual).  Without it k_cheb2_dots forms x_T's ϵ again (4 bytes a cell less here
 // and there): 122 µs at 256³, 143 with it and two divisions a cell.
 template <int D, class T>
 __device__ inline void load_inc_cell(const FcgV<T> &f, const LevV<T> &l, double s, double is, int keep_x,
@@ -1446,9 +1440,9 @@ __device__ inline void load_inc_cell(const FcgV<T> &f, const LevV<T> &l, double 
     if (keep_x) l.x[I] = T(0) + ev(I);
 }
 template <class T>
-__global__ void __launch_bounds__(NT) k_fcg_load_inc(FcgV<T> f, LevV<T> l, const double *part_rr, int keep_x) {
+__global__ void __launch_bounds__(NT) k_fcg_load_inc(FcgV<T> f, LevV<T> l, int keep_x) {
     HALT_IF(l)
-    double s = sqrt(block_total(part_rr, f.t.nblk) / (double)f.ncell);
+    double s = sqrt(f.S->rr / (double)f.ncell);
     const double is = 1.0 / s;
     if (blockIdx.x == 0 && threadIdx.x == 0) f.S->sload = s;
     if (l.g.D == 3) {
@@ -1647,8 +1641,9 @@ __device__ inline void fcg_apply(const FcgV<T> &f, const int p[3], long I, doubl
 template <class T>
 __global__ void __launch_bounds__(NT) k_fcg_Ap(FcgV<T> f, const double *part_dots, double *part, int first) {
     if (f.S->halt) return;
-    double wr = block_total(part_dots, f.t.nblk, 2, 0);
-    double wq = first ? 0.0 : block_total(part_dots, f.t.nblk, 2, 1);
+    const bool many = f.t.nblk > FCG_MANY;
+    double wr = many ? f.S->wr : block_total(part_dots, f.t.nblk, 2, 0);
+    double wq = first ? 0.0 : many ? f.S->wq : block_total(part_dots, f.t.nblk, 2, 1);
     FcgState st = *f.S;
     double beta = first ? 0.0 : -wq / st.pq;
     double s = st.sload;
@@ -1694,7 +1689,7 @@ __global__ void __launch_bounds__(NT) k_fcg_Ap(FcgV<T> f, const double *part_dot
 template <class T>
 __global__ void __launch_bounds__(NT) k_fcg_update(FcgV<T> f, const double *part_pq, double *part) {
     if (f.S->halt) return;
-    double pq = block_total(part_pq, f.t.nblk);
+    double pq = f.t.nblk > FCG_MANY ? f.S->pq : block_total(part_pq, f.t.nblk);
     double alpha = f.S->wr / pq;
     __syncthreads();
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -1720,19 +1715,43 @@ __global__ void __launch_bounds__(NT) k_fcg_update(FcgV<T> f, const double *part
     }
     block_partial(v, f.t, part);
 }
-// convergence test of the recursive residual on the device, so the host can
-// queue the next iteration before it reads this one's result
-template <class T>
-__global__ void __launch_bounds__(NT) k_fcg_check(FcgV<T> f, const double *part_rr, double zn, double rtol) {
-    if (f.S->halt) return;
-    double rr = block_total(part_rr, f.t.nblk);
+// the totals of K partial sums per workgroup, in block_total's order
+__global__ void __launch_bounds__(NT) k_fcg_sum(const int *halt, const double *part, long nblk, int K, double *o0,
+                                                double *o1) {
+    if (*halt) return;
+    const double s0 = block_total(part, nblk, K, 0);
+    __syncthreads();
+    const double s1 = K > 1 ? block_total(part, nblk, K, 1) : 0.0;
     if (threadIdx.x == 0) {
-        f.S->rr = rr;
-        if (sqrt(rr) / zn <= rtol) f.S->halt = 1;
+        *o0 = s0;
+        if (K > 1) *o1 = s1;
     }
 }
-__global__ void k_fcg_halt(FcgState *S, int v) {
-    if (threadIdx.x == 0) S->halt = v;
+// ‖r‖² at the start (or restart) of the iterations
+__global__ void __launch_bounds__(NT) k_fcg_begin(FcgState *S, const double *part_rr, long nblk) {
+    const double rr = block_total(part_rr, nblk);
+    if (threadIdx.x == 0) {
+        S->rr = rr;
+        S->halt = 0;
+    }
+}
+// convergence test of the recursive residual on the device, so the host can
+// queue the next iteration before it reads this one's result, which is left
+// in its pinned memory
+template <class T>
+__global__ void __launch_bounds__(NT) k_fcg_check(FcgV<T> f, const double *part_rr, double zn, double rtol,
+                                                  FcgState *host) {
+    int halt = f.S->halt;
+    const double rr = halt ? f.S->rr : block_total(part_rr, f.t.nblk);
+    if (threadIdx.x == 0) {
+        if (!halt) {
+            halt = sqrt(rr) / zn <= rtol;
+            f.S->rr = rr;
+            if (halt) f.S->halt = 1;
+        }
+        host->rr = rr;
+        host->halt = halt;
+    }
 }
 // plain multigrid refinement: x += s·x_T ; r = z - A x is recomputed by the caller
 template <class T>
