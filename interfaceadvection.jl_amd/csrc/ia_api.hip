@@ -79,7 +79,7 @@ struct ia_ctx {
     ia_params P;
     int es = 4;
     Grid g;
-    Tiling t;
+    Tiling t, vt;
     int dev = 0;
     hipStream_t s = nullptr;
     // fields
@@ -219,6 +219,20 @@ Tiling tiling(const Grid &g) {
     t.nt[2] = n2;
     t.tz = 1;
     t.nblk = (long)t.nt[0] * t.nt[1] * t.nt[2];
+    return t;
+}
+// columns of up to 8 cells along z where 2048 workgroups are left: for
+// k_prepare and k_vof_update, whose reduction of the fill report costs a workgroup more than
+// a cell's loads (256³ FP32: 118 µs with one cell, 90 with 8; 200x132x148:
+// 36.8, 32 with 2, 25.4 with 8).  k_vof_face is slower so (37 -> 44 µs there:
+// the wavefronts that cross the interface take longest, and take them all).
+Tiling column_tiling(const Grid &g) {
+    Tiling t = tiling(g);
+    if (g.D < 3) return t;
+    const long base = (long)t.nt[0] * t.nt[1];
+    t.tz = (int)std::max(1L, std::min(8L, base * t.nt[2] / 2048));
+    t.nt[2] = (t.nt[2] + t.tz - 1) / t.tz;
+    t.nblk = base * t.nt[2];
     return t;
 }
 // narrow: a coarse level may take 32-wide rows (only the one-cell-per-thread
@@ -1403,7 +1417,7 @@ template <class T> struct Impl {
     // the fill reports of `nsweep` sweeps made with u1, u2 and, with `cfl`, the CFL partials; `host`: into c->hst
     static void finish(ia_ctx *c, int nsweep, const void *u1, const void *u2, double rtol, bool cfl, bool host) {
         const FillPart *src = c->fpart;
-        long n = c->t.nblk;
+        long n = c->vt.nblk;
         if (nsweep > 0 && n > 8 * NT) {  // more than one block reads quickly
             FillPart *out = c->fpart + 3 * n;
             hipLaunchKernelGGL(k_fill_reduce, dim3(FILL_R2, (unsigned)nsweep), dim3(NT), 0, c->s, src, n, out);
@@ -1533,11 +1547,11 @@ template <class T> struct Impl {
         return IA_OK;
     }
     // ----------------------------------------------------------------- sweeps
-    // clear_st: the step's flags; clear_ruf: ρuf = 0
-    static void prepare(ia_ctx *c, const void *f, const void *usrc, bool do_ru, bool clear_st, bool clear_ruf) {
-        hipLaunchKernelGGL(k_prepare<T>, blocks(c->t), dim3(NT), 0, c->s, c->g, c->t, P<T>(f), P<T>(usrc), P<T>(c->ru),
-                           c->cb, (T)c->P.lambda_rho, do_ru ? 1 : 0, clear_st ? c->st : nullptr,
-                           clear_ruf ? P<T>(c->ruf) : nullptr, c->g.ns * c->g.D);
+    // clear_st: the step's flags; clear_ruf: ρuf = 0, 2: outside the interior (all sweeps follow)
+    static void prepare(ia_ctx *c, const void *f, const void *usrc, bool do_ru, bool clear_st, int clear_ruf) {
+        hipLaunchKernelGGL(k_prepare<T>, blocks(c->vt), dim3(NT), 0, c->s, c->g, c->vt, P<T>(f), P<T>(usrc),
+                           P<T>(c->ru), c->cb, (T)c->P.lambda_rho, do_ru ? 1 : 0, clear_st ? c->st : nullptr,
+                           clear_ruf ? P<T>(c->ruf) : nullptr, clear_ruf == 2 ? 1 : 0);
     }
     // slot: where the sweep's fill partials go, in the order of the sweeps (finish)
     static void vof_sweep(ia_ctx *c, const void *fin, void *fout, const void *u1, const void *u2, int d, T dt,
@@ -1546,6 +1560,7 @@ template <class T> struct Impl {
         SweepArgs<T> a;
         a.g = g;
         a.t = c->t;
+        a.ct = c->vt;
         a.fin = P<T>((void *)fin);
         a.fout = P<T>(fout);
         a.u1 = P<T>((void *)u1) + g.ns * d;
@@ -1554,7 +1569,7 @@ template <class T> struct Impl {
         a.ruf = P<T>(c->ruf) + g.ns * d;
         a.fn = P<T>((void *)fn);
         a.fmid = P<T>(fmid);
-        a.part = c->fpart + slot * c->t.nblk;
+        a.part = c->fpart + slot * c->vt.nblk;
         a.d = d;
         a.scheme = c->P.normal_scheme;
         a.mode = mode;
@@ -1567,7 +1582,7 @@ template <class T> struct Impl {
         prof_begin(c, IA_PROF_VOF);
         long nfb = c->t.nblk + (d == 0 ? top_face_x_blocks(g) : 0);
         hipLaunchKernelGGL(k_vof_face<T>, dim3((unsigned)nfb), dim3(NT), 0, c->s, a, P<T>(c->vface));
-        hipLaunchKernelGGL(k_vof_update<T>, blocks(c->t), dim3(NT), 0, c->s, a, P<T>(c->vface));
+        hipLaunchKernelGGL(k_vof_update<T>, blocks(c->vt), dim3(NT), 0, c->s, a, P<T>(c->vface));
         prof_end(c, IA_PROF_VOF);  // one sweep (its two launches) per record
     }
     static void momentum(ia_ctx *c, const void *fpre, const void *u1, const void *u2, const void *uold, int d, T dt) {
@@ -1710,7 +1725,7 @@ template <class T> struct Impl {
         void *U0 = c->u, *U1 = c->u0;  // u⁰ ← u: the predictor reads u^n from U0 and writes u^{n+1/2} to U1
         // predictor (w = ½)
         T w = T(0.5);
-        prepare(c, c->fb[fn], U0, true, true, false);
+        prepare(c, c->fb[fn], U0, true, true, 0);
         int mid = free_fbuf(c, fn, -1, -1);
         int fstar = advect_fq(c, fn, U0, U0, U0, dt, step_index, fn, mid);
         (void)fstar;
@@ -1719,7 +1734,7 @@ template <class T> struct Impl {
         if (int e = mg_update(c)) return e;
         if (int e = project(c, U1, (double)(w * dt), ss ? &ss->solve[0] : nullptr, 0)) return e;
         // corrector (w = 1): f⁰ ← f; ρu = u⁰ρ(f); advect f with u^{n+½}
-        prepare(c, c->fb[fn], U0, true, false, false);
+        prepare(c, c->fb[fn], U0, true, false, 0);
         int fnew = advect_fq(c, fn, U1, U1, U0, dt, step_index, fn, -1);
         if (int e = upd(c, U1, U0, c->fb[fnew], c->fb[fnew], U0, dt, T(1))) return e;
         if (int e = mg_update(c)) return e;
@@ -1755,7 +1770,7 @@ template <class T> struct Impl {
         Grid &g = c->g;
         T dt = (T)dtd;
         int keep = fsrc == c->fi ? c->f0i : c->fi;
-        prepare(c, c->fb[fsrc], u1, false, true, true);
+        prepare(c, c->fb[fsrc], u1, false, true, 2);
         int dirO[3];
         dir_order(g.D, step_index, dirO);
         int cur = fsrc;
@@ -1789,7 +1804,7 @@ template <class T> struct Impl {
         return st;
     }
     static int vof_sweep_stage(ia_ctx *c, int d, double dtd, ia_step_stats *ss) {
-        prepare(c, c->fb[c->fi], c->u0, false, true, true);
+        prepare(c, c->fb[c->fi], c->u0, false, true, 1);
         int out = free_fbuf(c, c->fi, c->f0i, -1);
         vof_sweep(c, c->fb[c->fi], c->fb[out], c->u0, c->u, d, (T)dtd, 1, 100 * epsT(), nullptr, nullptr, 0);
         finish(c, 1, c->u0, c->u, 100 * epsT(), false, true);
@@ -1952,6 +1967,7 @@ int ia_create(const ia_params *p, ia_ctx **out) {
     grid_init(c->g, p->D, Ng, p->perdir);
     c->g.exitx = p->exit_bc && !(p->perdir & 1);
     c->t = tiling(c->g);
+    c->vt = column_tiling(c->g);
     if (hipSetDevice(c->dev) != hipSuccess || hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&c->ev_solve[0][0]) != hipSuccess || hipEventCreate(&c->ev_solve[0][1]) != hipSuccess ||
         hipEventCreate(&c->ev_solve[1][0]) != hipSuccess || hipEventCreate(&c->ev_solve[1][1]) != hipSuccess) {

@@ -30,18 +30,17 @@ struct CTiling {
 // starts on what the previous one touched last (the part of it that the
 // 256 MB memory-side cache still holds).  Partial sums are stored by this
 // number, so a sum's order does not depend on the direction.
-__device__ inline long rev_block(const CTiling &t) { return t.rev ? t.nblk - 1 - (long)blockIdx.x : (long)blockIdx.x; }
+__device__ inline unsigned rev_block(const CTiling &t) {
+    return t.rev ? (unsigned)t.nblk - 1 - blockIdx.x : blockIdx.x;
+}
 __device__ inline bool thread_col(const Grid &g, const CTiling &t, int p[3], int &zlo, int &zhi) {
-    long b = swizzle_block(rev_block(t), t.nblk);
-    long bx = b % t.nt[0];
-    long r = b / t.nt[0];
-    long by = r % t.nt[1];
-    long bz = r / t.nt[1];
+    int q[3];
+    tile_of(t.nt, swizzle_block(rev_block(t), (unsigned)t.nblk), q);
     int tx = threadIdx.x % t.nx, ty = threadIdx.x / t.nx;
-    p[0] = 1 + (int)bx * t.nx + tx;
-    p[1] = g.D > 1 ? 1 + (int)by * (NT / t.nx) + ty : 0;
+    p[0] = 1 + q[0] * t.nx + tx;
+    p[1] = g.D > 1 ? 1 + q[1] * (NT / t.nx) + ty : 0;
     if (g.D > 2) {
-        zlo = 1 + (int)bz * t.zb;
+        zlo = 1 + q[2] * t.zb;
         zhi = zlo + t.zb - 1;
         if (zhi > g.Ng[2] - 2) zhi = g.Ng[2] - 2;
     } else {
@@ -274,12 +273,11 @@ __device__ inline int per_img(const Grid &g, int a, int q) {
 template <class V, class R, class LF, class CF, class PF, class BF>
 __device__ inline void tiled7(const Grid &g, const CTiling &t, LF load, CF comb, PF pre, BF body) {
     __shared__ V tile[2][TY + 2][TX + 2];
-    long b = swizzle_block(rev_block(t), t.nblk);
-    long bx = b % t.nt[0], rr = b / t.nt[0];
-    long by = rr % t.nt[1], bz = rr / t.nt[1];
+    int tq[3];
+    tile_of(t.nt, swizzle_block(rev_block(t), (unsigned)t.nblk), tq);
     int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-    int x = 1 + (int)bx * TX + tx, y = 1 + (int)by * TY + ty;
-    int zlo = 1 + (int)bz * t.zb, zhi = min(zlo + t.zb - 1, g.Ng[2] - 2);
+    int x = 1 + tq[0] * TX + tx, y = 1 + tq[1] * TY + ty;
+    int zlo = 1 + tq[2] * t.zb, zhi = min(zlo + t.zb - 1, g.Ng[2] - 2);
     bool active = x <= g.Ng[0] - 2 && y <= g.Ng[1] - 2;
     bool inarr = x <= g.Ng[0] - 1 && y <= g.Ng[1] - 1;
     int xi = per_img(g, 0, x), yi = per_img(g, 1, y);
@@ -372,13 +370,12 @@ __global__ void __launch_bounds__(NT) k_ls_stage_tiled(Grid g, CTiling t, const 
                                                        T *out, T dtau, T alpha) {
     constexpr int WX = TX + 4, WY = TY + 4, NW = WX * WY;
     __shared__ T tile[2][WY][WX];
-    long b = swizzle_block((long)blockIdx.x, t.nblk);
-    long bx = b % t.nt[0], rr = b / t.nt[0];
-    long by = rr % t.nt[1], bz = rr / t.nt[1];
+    int tq[3];
+    tile_of(t.nt, swizzle_block(blockIdx.x, (unsigned)t.nblk), tq);
     int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-    int x0 = 1 + (int)bx * TX, y0 = 1 + (int)by * TY;
+    int x0 = 1 + tq[0] * TX, y0 = 1 + tq[1] * TY;
     int x = x0 + tx, y = y0 + ty;
-    int zlo = 1 + (int)bz * t.zb, zhi = min(zlo + t.zb - 1, g.Ng[2] - 2);
+    int zlo = 1 + tq[2] * t.zb, zhi = min(zlo + t.zb - 1, g.Ng[2] - 2);
     bool active = x <= g.Ng[0] - 2 && y <= g.Ng[1] - 2;
     // tile entries k = threadIdx.x + NT*j: positions (x0-2+i, y0-2+j') mapped by
     // ls_img2; entries beyond Ng in x or y are read by no interior cell
@@ -1047,15 +1044,12 @@ __device__ inline void block_total2(const double *part, long n, double &a, doubl
 // workgroup); nin partial pairs come in (k_cg1_init's, then this kernel's).
 template <int NB>
 __device__ inline bool thread_row(const Grid &g, const CTiling &t, int p[3]) {
-    long b = swizzle_block((long)blockIdx.x, t.nblk);
-    long bx = b % t.nt[0];
-    long r = b / t.nt[0];
-    long by = r % t.nt[1];
-    long bz = r / t.nt[1];
+    int q[3];
+    tile_of(t.nt, swizzle_block(blockIdx.x, (unsigned)t.nblk), q);
     int tx = threadIdx.x % t.nx, ty = threadIdx.x / t.nx;
-    p[0] = 1 + (int)bx * t.nx + tx;
-    p[1] = g.D > 1 ? 1 + (int)by * (NB / t.nx) + ty : 0;
-    p[2] = g.D > 2 ? 1 + (int)bz : 0;
+    p[0] = 1 + q[0] * t.nx + tx;
+    p[1] = g.D > 1 ? 1 + q[1] * (NB / t.nx) + ty : 0;
+    p[2] = g.D > 2 ? 1 + q[2] : 0;
     bool ok = p[0] <= g.Ng[0] - 2;
     if (g.D > 1) ok = ok && p[1] <= g.Ng[1] - 2;
     return ok;
