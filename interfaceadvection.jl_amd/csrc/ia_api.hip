@@ -64,7 +64,7 @@ struct Level {
     Tiling t;
     CTiling ct;
     void *L = nullptr, *Dg = nullptr, *iD = nullptr, *x = nullptr, *e = nullptr, *r = nullptr, *z = nullptr;
-    void *e2 = nullptr, *z2 = nullptr;  // second ϵ/z pair of the fused pcg! iterations (levels >= 1)
+    void *e2 = nullptr, *z2 = nullptr;  // second ϵ/z pair of the fused pcg! iterations (on level 0 in FP64 if small)
     void *r2 = nullptr, *w = nullptr, *w2 = nullptr;  // single-reduction CG: r, w pairs (levels >= 1)
     CTiling wt;      // the single-reduction CG step's tiling on one-cell-per-thread levels (wnb threads)
     int wnb = NT;
@@ -482,6 +482,10 @@ template <class T> struct Impl {
         void **l0b[] = {&l0.Dg, &l0.iD, &l0.e, &l0.r};
         for (void **v : l0b)
             if (int r = alloc_zero(c, v, ns * es)) return r;
+        // FP64 pcg! on a small finest level: a launch less per iteration for two more arrays
+        if (es == 8 && interior(g) < (1 << 20))
+            for (void **v : {&l0.e2, &l0.z2})
+                if (int r = alloc_zero(c, v, ns * es)) return r;
         c->nlev = 1;
         long maxblk = c->t.nblk;
         for (;;) {
@@ -707,22 +711,28 @@ template <class T> struct Impl {
         bool f0 = &l == &c->lev[0];
         dim3 B = cb(l);
         if (!init_done) hipLaunchKernelGGL(k_pcg_init<T>, B, dim3(NT), 0, c->s, v, pp(c, PP_A));
-        // levels >= 1 fuse each ϵ update into the next z = Aϵ, alternating
-        // between the (e, z) and (e2, z2) buffer pairs
+        // each ϵ update is fused into the next z = Aϵ, alternating between the
+        // (e, z) and (e2, z2) buffer pairs; on level 0, where z is a field that
+        // is read afterwards, Aϵ goes to z2 and z = r·iD to z each time
         bool pair = l.e2 != nullptr && it > 1;
+        const T *za = pair && f0 ? P<T>(l.z2) : nullptr;
         for (int i = 1; i <= it; ++i) {
             int sa = 3 * (i - 1), su = sa + 1, se = sa + 2;
             int sin = i == 1 ? -1 : sa - 1;
             if (i > 1 && pair) {
                 LevV<T> w = v;
                 w.e = (i % 2 == 0) ? P<T>(l.e2) : P<T>(l.e);
-                w.z = (i % 2 == 0) ? P<T>(l.z2) : P<T>(l.z);
-                hipLaunchKernelGGL(k_pcg_epsAe<T>, B, dim3(NT), 0, c->s, v, w.e, w.z, c->pst, sa - 2, sa, pp(c, PP_C),
-                                   pp(c, PP_B));
+                if (!f0) w.z = (i % 2 == 0) ? P<T>(l.z2) : P<T>(l.z);
+                if (f0) prof_begin(c, IA_PROF_PCG_AE);
+                hipLaunchKernelGGL(k_pcg_epsAe<T>, B, dim3(NT), 0, c->s, v, w.e, f0 ? P<T>(l.z2) : w.z, c->pst, sa - 2,
+                                   sa, pp(c, PP_C), pp(c, PP_B));
+                if (f0) prof_end(c, IA_PROF_PCG_AE);
                 v = w;
             } else {
+                LevV<T> w = v;
+                if (za) w.z = P<T>(l.z2);
                 if (f0) prof_begin(c, IA_PROF_PCG_AE);
-                hipLaunchKernelGGL(k_pcg_Ae<T>, B, dim3(NT), 0, c->s, v, c->pst, sin, sa, pp(c, PP_A), pp(c, PP_B));
+                hipLaunchKernelGGL(k_pcg_Ae<T>, B, dim3(NT), 0, c->s, w, c->pst, sin, sa, pp(c, PP_A), pp(c, PP_B));
                 if (f0) prof_end(c, IA_PROF_PCG_AE);
             }
             if (i == it && last) {
@@ -733,7 +743,8 @@ template <class T> struct Impl {
                 continue;
             }
             if (f0) prof_begin(c, IA_PROF_PCG_UPDATE);
-            hipLaunchKernelGGL(k_pcg_update<T>, B, dim3(NT), 0, c->s, v, c->pst, sa, su, pp(c, PP_B), pp(c, PP_C), i, it);
+            hipLaunchKernelGGL(k_pcg_update<T>, B, dim3(NT), 0, c->s, v, za ? za : v.z, c->pst, sa, su, pp(c, PP_B),
+                               pp(c, PP_C), i, it);
             if (f0) prof_end(c, IA_PROF_PCG_UPDATE);
             if (i < it && !pair) hipLaunchKernelGGL(k_pcg_eps<T>, B, dim3(NT), 0, c->s, v, c->pst, su, se, pp(c, PP_C));
         }
@@ -1652,17 +1663,16 @@ template <class T> struct Impl {
     static int surften(ia_ctx *c, const void *f, void *out, int acc) {
         Grid &g = c->g;
         if (!c->st_fb) {
-            HIPCHK(c, hipMalloc(&c->st_fb, g.ns * sizeof(T)));
-            HIPCHK(c, hipMemsetAsync(c->st_fb, 0, g.ns * sizeof(T), c->s));
+            HIPCHK(c, hipMalloc(&c->st_fb, g.ns * g.D * sizeof(T)));
+            HIPCHK(c, hipMemsetAsync(c->st_fb, 0, g.ns * g.D * sizeof(T), c->s));
         }
-        for (int d = 0; d < g.D; ++d) {
-            hipLaunchKernelGGL(k_st_fbuf<T>, blocks(c->t), dim3(NT), 0, c->s, g, c->t, P<T>((void *)f), P<T>(c->st_fb), d);
-            for (int j = 0; j < g.D; ++j)
-                hipLaunchKernelGGL(k_st_bc<T>, blocks1(g.ns / g.Ng[j]), dim3(NT), 0, c->s, g, P<T>(c->st_fb), d, j);
-            auto ks = g.D == 3 ? k_surften<3, T> : k_surften<2, T>;
-            hipLaunchKernelGGL(ks, blocks(c->t), dim3(NT), 0, c->s, g, c->t, P<T>(c->st_fb), P<T>((void *)f),
-                               (T)c->P.eta, d, P<T>(out), acc);
-        }
+        hipLaunchKernelGGL(k_st_fbuf<T>, blocks(c->t), dim3(NT), 0, c->s, g, c->t, P<T>((void *)f), P<T>(c->st_fb));
+        for (int j = 0; j < g.D; ++j)
+            hipLaunchKernelGGL(k_st_bc<T>, dim3(blocks1(g.ns / g.Ng[j]).x, (unsigned)g.D), dim3(NT), 0, c->s, g,
+                               P<T>(c->st_fb), j);
+        auto ks = g.D == 3 ? k_surften<3, T> : k_surften<2, T>;
+        hipLaunchKernelGGL(ks, dim3((unsigned)c->t.nblk, (unsigned)g.D), dim3(NT), 0, c->s, g, c->t, P<T>(c->st_fb),
+                           P<T>((void *)f), (T)c->P.eta, P<T>(out), acc);
         LAUNCHCHK(c);
         return IA_OK;
     }
@@ -2000,11 +2010,11 @@ void ia_destroy(ia_ctx *c) {
         if (b && !is_attached(c, b)) (void)hipFree(b);
     for (int l = 0; l < c->nlev; ++l) {
         Level &lv = c->lev[l];
-        void *lb[] = {lv.Dg, lv.iD, lv.e, lv.r};
+        void *lb[] = {lv.Dg, lv.iD, lv.e, lv.r, lv.e2, lv.z2};
         for (void *b : lb)
             if (b) (void)hipFree(b);
         if (lv.own) {
-            void *ob[] = {lv.L, lv.x, lv.z, lv.e2, lv.z2, lv.r2, lv.w, lv.w2};
+            void *ob[] = {lv.L, lv.x, lv.z, lv.r2, lv.w, lv.w2};
             for (void *b : ob)
                 if (b) (void)hipFree(b);
         }

@@ -271,6 +271,15 @@ __device__ inline long shell_entry(const Grid &g, long q) {
     return (k & 1 ? n0 - 1 : 0) + (long)(1 + r % n1) * g.st[1] + (long)(z0 + r / n1) * (g.D > 2 ? g.st[2] : 0);
 }
 
+// orders the lanes' exchange through LDS within a wavefront, without a
+// barrier: its LDS accesses complete in program order, and the fences keep the
+// compiler from moving them across one another
+__device__ inline void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------------------
 // scalar helpers with Julia semantics
 // ---------------------------------------------------------------------------

@@ -830,53 +830,57 @@ template <class T> __device__ inline T popinet_height(const Grid &g, const T *f,
     return H;
 }
 template <class T> __device__ inline T root1p5(T a) { return sqrt((a * a) * a); }  // surfaceTension.jl:89
-// getCurvature (surfaceTension.jl:35-80) with getXdir / getXYdir (util.jl:62-63)
-template <int D, class T> __device__ inline T curvature(const Grid &g, const T *f, const int p[3], int i) {
-    int s = i > 0 ? 1 : -1, ai = abs(i);
-    if (D == 2) {
-        int ix = ai == 1 ? -2 * s : s, ax = abs(ix) - 1, sx = ix > 0 ? 1 : -1;
-        T H[3];
-        for (int u = -1; u <= 1; ++u) {
-            int q[3] = {p[0], p[1], p[2]};
-            q[ax] += u * sx;
-            H[u + 1] = popinet_height(g, f, q, i);
-        }
-        T Hx = (H[2] - H[0]) / 2;
-        T Hxx = (H[2] + H[0]) - 2 * H[1];
-        return Hxx / root1p5(1 + Hx * Hx);
+// getCurvature (surfaceTension.jl:35-80) with getXdir / getXYdir (util.jl:62-63):
+// the cell of its k-th height about q along the signed axis i, H[u+1] in 2D,
+// H[u+1][v+1] in 3D
+template <int D> __device__ inline void height_cell(int i, int k, int q[3]) {
+    const int s = i > 0 ? 1 : -1, ai = abs(i);
+    const int ix = D == 2 ? (ai == 1 ? -2 * s : s) : s * (ai % 3 + 1);
+    const int du = (D == 2 ? k - 1 : k / 3 - 1) * (ix > 0 ? 1 : -1), iy = (ai + 1) % 3;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        if (a == abs(ix) - 1) q[a] += du;
+        if (D == 3 && a == iy) q[a] += k % 3 - 1;
     }
-    int ix = s * (ai % 3 + 1), iy = (ai + 1) % 3 + 1;
-    int axx = abs(ix) - 1, sx = ix > 0 ? 1 : -1;
-    T H[3][3], flt = T(0.2);
-    for (int u = -1; u <= 1; ++u)
-        for (int v = -1; v <= 1; ++v) {
-            int q[3] = {p[0], p[1], p[2]};
-            q[axx] += u * sx;
-            q[iy - 1] += v;
-            H[u + 1][v + 1] = popinet_height(g, f, q, i);
-        }
-    T Hx = (H[2][1] - H[0][1]) / 2, Hy = (H[1][2] - H[1][0]) / 2;
-    T Hxx = (((H[2][1] + H[0][1]) - 2 * H[1][1]) + ((H[2][0] + H[0][0]) - 2 * H[1][0]) * flt +
-             ((H[2][2] + H[0][2]) - 2 * H[1][2]) * flt) / (1 + 2 * flt);
-    T Hyy = (((H[1][2] + H[1][0]) - 2 * H[1][1]) + ((H[0][2] + H[0][0]) - 2 * H[0][1]) * flt +
-             ((H[2][2] + H[2][0]) - 2 * H[2][1]) * flt) / (1 + 2 * flt);
-    T Hxy = (((H[2][2] + H[0][0]) - H[2][0]) - H[0][2]) / 4;
-    return ((Hxx * (1 + Hy * Hy) + Hyy * (1 + Hx * Hx)) - ((2 * Hxy) * Hx) * Hy) / root1p5((1 + Hx * Hx) + Hy * Hy);
 }
+template <int D, class T> __device__ inline T curvature(const T (&h)[D == 3 ? 9 : 3]) {
+    if constexpr (D == 2) {
+        T Hx = (h[2] - h[0]) / 2;
+        T Hxx = (h[2] + h[0]) - 2 * h[1];
+        return Hxx / root1p5(1 + Hx * Hx);
+    } else {
+        T H[3][3], flt = T(0.2);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) H[k / 3][k % 3] = h[k];
+        T Hx = (H[2][1] - H[0][1]) / 2, Hy = (H[1][2] - H[1][0]) / 2;
+        T Hxx = (((H[2][1] + H[0][1]) - 2 * H[1][1]) + ((H[2][0] + H[0][0]) - 2 * H[1][0]) * flt +
+                 ((H[2][2] + H[0][2]) - 2 * H[1][2]) * flt) / (1 + 2 * flt);
+        T Hyy = (((H[1][2] + H[1][0]) - 2 * H[1][1]) + ((H[0][2] + H[0][0]) - 2 * H[0][1]) * flt +
+                 ((H[2][2] + H[2][0]) - 2 * H[2][1]) * flt) / (1 + 2 * flt);
+        T Hxy = (((H[2][2] + H[0][0]) - H[2][0]) - H[0][2]) / 4;
+        return ((Hxx * (1 + Hy * Hy) + Hyy * (1 + Hx * Hx)) - ((2 * Hxy) * Hx) * Hy) /
+               root1p5((1 + Hx * Hx) + Hy * Hy);
+    }
+}
+// The forcing's buffer of direction d is component d of a vector, so that one
+// launch serves all directions: in a launch for one of them most wavefronts
+// end at once and the few at the interface leave the chip idle.
 // fbuffer[I] = ϕ(d, I, f) = (f[I] + f[I-δd]) / 2 on the interior
-template <class T> __global__ void __launch_bounds__(NT) k_st_fbuf(Grid g, Tiling t, const T *f, T *fb, int d) {
+template <class T> __global__ void __launch_bounds__(NT) k_st_fbuf(Grid g, Tiling t, const T *f, T *fb) {
     int p[3];
     if (!thread_cell(g, t, p)) return;
     long I = lin(g, p);
-    fb[I] = (f[I] + f[I - g.st[d]]) / 2;
+    for (int d = 0; d < g.D; ++d) fb[g.ns * d + I] = (f[I] + f[I - g.st[d]]) / 2;
 }
 // BCf!(d, fbuffer) on the ghost planes of axis j (VOFutil.jl:76-89), axis by
 // axis as the reference loops; the upper plane of axis d, which BCf!(d, ·)
 // does not write, is set to 0
-template <class T> __global__ void __launch_bounds__(NT) k_st_bc(Grid g, T *fb, int d, int j) {
+template <class T> __global__ void __launch_bounds__(NT) k_st_bc(Grid g, T *fb, int j) {
     long n = g.ns / g.Ng[j];
     long q = (long)blockIdx.x * NT + threadIdx.x;
     if (q >= n) return;
+    const int d = blockIdx.y;
+    fb += g.ns * d;
     int c[3];
     long r = q;
     for (int a = 0; a < 3; ++a) {
@@ -899,22 +903,52 @@ template <class T> __global__ void __launch_bounds__(NT) k_st_bc(Grid g, T *fb, 
     }
 }
 // forcing[I,d] (+)= η κ(I, fbuffer, majorDir) (-∂_d f) at interface cells of
-// fbuffer, 0 elsewhere (surfaceTension.jl:7-19)
+// fbuffer, 0 elsewhere (surfaceTension.jl:7-19).  A height is a walk of
+// dependent loads and a curvature takes nine of them (three in 2D), but few of
+// a wavefront's cells are at the interface: its heights are dealt out to all
+// lanes, one each (48³ FP64: 54 µs a direction with each cell walking its own
+// nine, 26 all three together).
 template <int D, class T>
-__global__ void __launch_bounds__(NT) k_surften(Grid g, Tiling t, const T *fb, const T *f, T eta, int d, T *out,
-                                                int acc) {
+__global__ void __launch_bounds__(NT) k_surften(Grid g, Tiling t, const T *fbv, const T *f, T eta, T *out, int acc) {
+    constexpr int NH = D == 3 ? 9 : 3, PER = 64 / NH;  // heights of a cell, cells at a time
+    __shared__ unsigned char who[NT / 64][64];
     int p[3];
-    if (!thread_cell(g, t, p)) return;
-    long I = lin(g, p);
-    T st = 0;
-    bool hit = contain_if(fb[I]);
+    const int d = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const bool in = thread_cell(g, t, p);
+    const long I = in ? lin(g, p) : 0;
+    const T *fb = fbv + g.ns * d;
+    const bool hit = in && contain_if(fb[I]);
+    int i = 1;  // the major direction
     if (hit) {
         T n[3];
         normal_wy(g, fb, I, n);
         int im = argabsmax(g.D, n);
-        int i = (signbit(n[im]) ? -1 : 1) * (im + 1);
-        st = eta * curvature<D>(g, fb, p, i) * -(f[I] - f[I - g.st[d]]);
+        i = (signbit(n[im]) ? -1 : 1) * (im + 1);
     }
+    const unsigned long long m = __ballot(hit);
+    const int rank = __popcll(m & ((1ull << lane) - 1)), nhit = __popcll(m);
+    if (hit) who[wv][rank] = (unsigned char)lane;
+    wave_lds_order();
+    T H[NH];
+    for (int b = 0; b < nhit; b += PER) {
+        const int s = lane / NH, k = lane % NH;
+        const bool on = s < PER && b + s < nhit;
+        const int src = on ? who[wv][b + s] : lane;
+        int q[3] = {__shfl(p[0], src), __shfl(p[1], src), __shfl(p[2], src)};
+        const int qi = __shfl(i, src);
+        T h = 0;
+        if (on) {
+            height_cell<D>(qi, k, q);
+            h = popinet_height(g, fb, q, qi);
+        }
+#pragma unroll
+        for (int j = 0; j < NH; ++j) {
+            const T v = __shfl(h, ((rank - b) * NH + j) & 63);
+            if (hit && rank >= b && rank < b + PER) H[j] = v;
+        }
+    }
+    if (!in) return;
+    const T st = hit ? eta * curvature<D>(H) * -(f[I] - f[I - g.st[d]]) : T(0);
     long o = g.ns * d + I;
     if (!acc) out[o] = st;
     else if (hit) out[o] = out[o] + st;

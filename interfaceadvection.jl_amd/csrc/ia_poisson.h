@@ -717,7 +717,7 @@ __global__ void __launch_bounds__(NT) k_pcg_Ae(LevV<T> l, PcgState *S, int sin, 
 }
 // α = ρ/(z·ϵ); x += αϵ; r -= αz; z = r·iD; partial r·z; stop when i == itmax or |α| < 1e-2
 template <class T>
-__global__ void __launch_bounds__(NT) k_pcg_update(LevV<T> l, PcgState *S, int sin, int sout, const double *partB,
+__global__ void __launch_bounds__(NT) k_pcg_update(LevV<T> l, const T *za, PcgState *S, int sin, int sout, const double *partB,
                                                    double *partC, int i, int itmax) {
     HALT_IF(l)
     PcgState st = S[sin];
@@ -733,13 +733,13 @@ __global__ void __launch_bounds__(NT) k_pcg_update(LevV<T> l, PcgState *S, int s
     {
         T *__restrict__ x = l.x;
         T *__restrict__ r = l.r;
-        T *__restrict__ z = l.z;
+        T *z = l.z;  // may be za
         const T *__restrict__ e = l.e;
         const T *__restrict__ iD = l.iD;
         struct V {
             T x, e, r, z, d;
         };
-        col_pipe(l.g, l.t, [&](const int *, long I) { return V{x[I], e[I], r[I], z[I], iD[I]}; },
+        col_pipe(l.g, l.t, [&](const int *, long I) { return V{x[I], e[I], r[I], za[I], iD[I]}; },
                  [&](const int *, long I, const V &w) {
                      x[I] = w.x + alpha * w.e;
                      T rr = w.r - alpha * w.z;
@@ -2018,14 +2018,7 @@ template <int D, class T> __device__ __forceinline__ void stail_pcg(const SLev<T
 // pcg!(l; it) on a level of at most 64 cells, by wavefront 0 alone, one
 // cell per lane.  Its sums are the wavefront's butterfly sums plus 0.0: in
 // stail_pcg the other wavefronts' partials would all be 0, so the values are
-// the same.  The lanes exchange ϵ through LDS with no workgroup barrier; a
-// wavefront's LDS accesses complete in program order, and the fences keep
-// the compiler from moving them across one another.
-__device__ inline void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
+// the same.  The lanes exchange ϵ through LDS (wave_lds_order).
 template <int D, class T> __device__ __forceinline__ void stail_pcg_wave(const SLev<T> &l, int it) {
     const int c = threadIdx.x;
     const bool on = c < l.ncell;
