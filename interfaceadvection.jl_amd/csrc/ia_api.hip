@@ -770,7 +770,12 @@ template <class T> struct Impl {
     // one launch (k_cgp) where the level's boxes fit, else one launch per
     // iteration (k_cg1_init, k_cg1_step).  The final r may sit in r2 or
     // nowhere; nothing reads a coarse r after its solve (restrict! rewrites it).
-    static void pcg1(ia_ctx *c, Level &l, int it) {
+    // with `prolong` the launch begins with the prolongate! and increment! that
+    // vcycle leaves to it (folds).
+    static bool folds(const ia_ctx *c, const Level &l) {
+        return l.cgp && !c->cgp_off && l.cgp->NB * l.cgp->C <= 4096;
+    }
+    static void pcg1(ia_ctx *c, Level &l, int it, bool prolong) {
         int lv = (int)(&l - c->lev), pc = lv >= 1 && lv <= 3 ? IA_PROF_CG1_L1 + lv - 1 : -1;
         if (l.cgp && !c->cgp_off) {
             CgpArgs a;
@@ -780,6 +785,8 @@ template <class T> struct Impl {
             a.iD = P<float>(l.iD);
             a.r = P<float>(l.r);
             a.x = P<float>(l.x);
+            a.xc = prolong && folds(c, l) ? P<float>((&l)[1].x) : nullptr;
+            a.gc = a.xc ? (&l)[1].g : l.g;
             a.hw = c->cgp_hw;
             a.pw = c->cgp_pw;
             a.spread = a.box.spread;
@@ -837,13 +844,18 @@ template <class T> struct Impl {
     static void vcycle(ia_ctx *c, int l, const int *cit, bool pre_done = false, bool then_pcg = false,
                        bool e_done = false, int rev = 0) {
         Level &fl = c->lev[l], &co = c->lev[l + 1];
-        if (!pre_done) {
-            if (e_done) increment(c, fl);
-            else jacobi(c, fl);
-        }
         bool rec = l + 2 < c->nlev, co_jacobi = l + 1 < c->tail_level && rec;
-        hipLaunchKernelGGL(k_mg_restrict<T>, cb(co), dim3(NT), 0, c->s, view(co), fl.g, P<T>(fl.r),
-                           co_jacobi ? 1 : 0);
+        if (!pre_done && e_done && interior(fl.g) <= 1 << 18) {
+            auto k = fl.g.D == 3 ? k_mg_inc_restrict<3, T> : k_mg_inc_restrict<2, T>;
+            hipLaunchKernelGGL(k, cb(co), dim3(NT), 0, c->s, view(co), view(fl), co_jacobi ? 1 : 0);
+        } else {
+            if (!pre_done) {
+                if (e_done) increment(c, fl);
+                else jacobi(c, fl);
+            }
+            hipLaunchKernelGGL(k_mg_restrict<T>, cb(co), dim3(NT), 0, c->s, view(co), fl.g, P<T>(fl.r),
+                               co_jacobi ? 1 : 0);
+        }
         if (l + 1 >= c->tail_level) {
             TailArgs<T> a;
             for (int q = 0; q < c->nlev && q < MAXLEV; ++q) {
@@ -865,10 +877,11 @@ template <class T> struct Impl {
             launch_tail(c, a, cit == c->cit_fcg);
         } else {
             if (rec) vcycle(c, l + 1, cit, false, true, true);
-            if (cit == c->cit_fcg) pcg1(c, co, cit[l + 1]);
+            if (cit == c->cit_fcg) pcg1(c, co, cit[l + 1], rec);
             else pcg(c, co, cit[l + 1], rec);
         }
-        if (then_pcg && one_launch(c, fl)) return;  // the pcg! begins with both
+        // the launch of the solve begins with both
+        if (then_pcg && (cit == c->cit_fcg ? l > 0 && folds(c, fl) : one_launch(c, fl))) return;
         if (then_pcg) {
             bool f0 = l == 0;
             if (f0) prof_begin(c, IA_PROF_PROLONG_INC);

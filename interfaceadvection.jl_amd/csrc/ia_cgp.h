@@ -60,6 +60,8 @@ struct CgpArgs {
     CgpBox box;
     const float *L, *iD, *r;
     float *x;
+    const float *xc;  // the coarser level's x, to prolongate! and increment! by first (not BIG), or nullptr
+    Grid gc;
     unsigned long long *hw;  // 2 slots of nwg * 2D * amax words: w of the cells at a box's faces
     unsigned long long *pw;  // 2 slots of CGP_PW words: the partial sums, then the groups' sums
     unsigned tag;            // of iteration 0
@@ -141,6 +143,15 @@ __host__ __device__ inline int cgp_words(int D, int NB, int C, const int *b) {
     return NB * C > 4096 ? t + 3 * NB * C : 2 * t;
 }
 
+// the prolonged x at cell P, A times it
+template <int D, class A> __device__ inline float cgp_parent(const A &a, const int P[3]) {
+    return a.xc[(long)((P[0] + 3) / 2 - 1) + a.gc.st[1] * ((P[1] + 3) / 2 - 1) +
+                (D > 2 ? a.gc.st[2] * ((P[2] + 3) / 2 - 1) : 0)];
+}
+template <int D, class A> __device__ inline float cgp_mult_parent(const A &a, const int P[3], long I) {
+    return mgmult_fc<D>(a.g, P, I, a.L, [&](const int *q) { return cgp_parent<D>(a, q); });
+}
+
 // NB threads; a thread owns a column of C cells along the last axis (so two of a cell's neighbours are mostly its own
 // registers); the halo cells are those of wavefronts 1.. (HC each), while wavefront 0 waits for the sums.
 template <int D, int NB, int C, int HC>
@@ -217,6 +228,11 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
                 ly[k] = a.L[g.ns + I];
                 lyp[k] = a.L[g.ns + I + g.st[1]];
             }
+            if (!BIG && a.xc) {
+                const int P[3] = {lo[0] + x0, D > 2 ? lo[1] + y0 : lo[1] + z0 + k, D > 2 ? lo[2] + z0 + k : 0};
+                r[k] = r[k] - cgp_mult_parent<D>(a, P, I);
+                xk += cgp_parent<D>(a, P);
+            }
         }
         if (BIG) xl[4 * (k / 4 * NB + tid) + k % 4] = xk;
         else if (XL) xl[k * NB + tid] = xk;
@@ -284,6 +300,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
                     long J = (long)P[0] + g.st[1] * P[1] + (D > 2 ? g.st[2] * P[2] : 0);
                     hr[k] = a.r[J];
                     hid[k] = a.iD[J];
+                    if (!BIG && a.xc) hr[k] = hr[k] - cgp_mult_parent<D>(a, P, J);
                     // the neighbour's facing side holds the same cells in the same order
                     hwo[k] = ((c[0] + a.box.k[0] * (c[1] + a.box.k[1] * c[2])) * 2 * D + 2 * d + 1 - side) * a.box.amax + h;
                 }
@@ -584,14 +601,6 @@ struct PcgpArgs {
     const int *halt;
     int *fail;
 };
-// the prolonged x at cell P
-template <int D> __device__ inline float cgp_parent(const PcgpArgs &a, const int P[3]) {
-    return a.xc[(long)((P[0] + 3) / 2 - 1) + a.gc.st[1] * ((P[1] + 3) / 2 - 1) +
-                (D > 2 ? a.gc.st[2] * ((P[2] + 3) / 2 - 1) : 0)];
-}
-template <int D> __device__ inline float cgp_mult_parent(const PcgpArgs &a, const int P[3], long I) {
-    return mgmult_fc<D>(a.g, P, I, a.L, [&](const int *q) { return cgp_parent<D>(a, q); });
-}
 template <int D, int NB, int C, int HC>
 __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     HALT_IF(a)
