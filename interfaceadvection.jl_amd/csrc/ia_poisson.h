@@ -535,24 +535,24 @@ __global__ void __launch_bounds__(NT) k_mg_increment(LevV<T> l) {
     HALT_IF(l)
     DISPATCH_D(l.g, increment_d<D>(l);)
 }
-// restrict!: coarse r = Σ children; coarse x = 0
+// restrict!: coarse r = Σ children (all of them loaded before the sum); coarse x = 0
+template <int D, class T>
+__device__ inline void restrict_cell(const LevV<T> &c, const Grid &gf, const T *__restrict__ rf, int with_e,
+                                     const int p[3], long I) {
+    const T *b = rf + (2 * p[0] - 1) + gf.st[1] * (2 * p[1] - 1) + (D > 2 ? gf.st[2] * (2 * p[2] - 1) : 0);
+    T v[1 << D], s = 0;
+#pragma unroll
+    for (int k = 0; k < 1 << D; ++k) v[k] = b[(k & 1) + gf.st[1] * (k >> 1 & 1) + (D > 2 ? gf.st[2] * (k >> 2) : 0)];
+#pragma unroll
+    for (int k = 0; k < 1 << D; ++k) s += v[k];
+    c.r[I] = s;
+    c.x[I] = T(0);
+    if (with_e) c.e[I] = s * c.iD[I];  // the Jacobi! step that follows on this level
+}
 template <class T>
 __global__ void __launch_bounds__(NT) k_mg_restrict(LevV<T> c, Grid gf, const T *rf, int with_e) {
     HALT_IF(c)
-    COL_LOOP(c, {
-        int lo[3], hi[3];
-        for (int a = 0; a < 3; ++a) {
-            lo[a] = a < c.g.D ? 2 * p[a] - 1 : 0;
-            hi[a] = a < c.g.D ? 2 * p[a] : 0;
-        }
-        T s = 0;
-        for (int c2 = lo[2]; c2 <= hi[2]; ++c2)
-            for (int c1 = lo[1]; c1 <= hi[1]; ++c1)
-                for (int c0 = lo[0]; c0 <= hi[0]; ++c0) s += rf[c0 + gf.st[1] * c1 + gf.st[2] * c2];
-        c.r[I] = s;
-        c.x[I] = T(0);
-        if (with_e) c.e[I] = s * c.iD[I];  // the Jacobi! step that follows on this level
-    })
+    DISPATCH_D(c.g, COL_LOOP(c, { restrict_cell<D>(c, gf, rf, with_e, p, I); }))
 }
 // increment! on a level and restrict! of the result in one launch, a thread per
 // coarse cell: for levels whose launches cost more than their cells (4.2 + 4.1
