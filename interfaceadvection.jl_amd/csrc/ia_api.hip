@@ -599,7 +599,7 @@ template <class T> struct Impl {
                     if ((long)per * ncu < (maxwg > CGP_ONE ? 1L : 2L) * lv.cgp_box.nwg) continue;
                     lv.cgp = &vs[q];
                     // on one XCD where there is room for two such launches
-                    const bool near = maxwg <= CGP_ONE && vs[q].NB < 1024 && per * CGP_XCU >= 2 * lv.cgp_box.nwg;
+                    const bool near = maxwg <= CGP_ONE && cells < 4096 && per * CGP_XCU >= 2 * lv.cgp_box.nwg;
                     lv.cgp_box.spread = near ? CGP_XCDS : 1;
                 }
             if (lv.cgp)

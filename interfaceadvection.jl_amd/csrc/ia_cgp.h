@@ -30,7 +30,7 @@ namespace ia {
 // an iteration reads nothing from memory but the faces.
 //
 // Measured, µs per iteration of 64, one launch per iteration / here: 128^3 22-24 / 9.0 (6 iterations 145 / 83), 64^3
-// 6.6-7.5 / 3.0, 60x44x36 5.4 / 2.2, 32^3 4.6 / 1.55, 192x128 4.5 / 1.3, 96x64 4.3 / 1.2.  What is left on the small
+// 6.6-7.5 / 3.1, 60x44x36 5.4 / 2.2, 32^3 4.6 / 1.55, 192x128 4.5 / 1.3, 96x64 4.3 / 1.2.  What is left on the small
 // ones is the exchange and as much again for the operator, the
 // recurrence and the two sums, a chain of some 2000 cycles in which a wavefront mostly waits for itself: nothing in it
 // stands behind a branch, faces are published through a tile, and a workgroup's words of a sum lie together.
@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     if ((int)blockIdx.x % a.spread != a.xcd) return;
     const int wg = (int)blockIdx.x / a.spread;
     extern __shared__ __align__(16) float cgp_u[];
-    constexpr bool XL = NB * C >= 4096;  // x in LDS: the registers of a 1024-thread workgroup do not hold it
+    constexpr bool XL = NB * C >= 4096;  // x in LDS: the registers do not hold it
     constexpr bool BIG = NB * C > 4096;  // p and s in LDS too, u and the diagonal formed again, w in u's tile
     constexpr int CR = BIG ? 1 : C;
     __shared__ float xs[XL && !BIG ? NB * C : 1];
@@ -310,7 +310,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     const long hslot = (long)a.box.nwg * 2 * D * a.box.amax;
     const int nwg = a.box.nwg, ngrp = (nwg + CGP_GROUP - 1) / CGP_GROUP;
     const bool two = nwg > CGP_ONE;
-    constexpr bool FAR = NB >= 1024 || BIG;  // too large for one XCD
+    constexpr bool FAR = NB * C >= 4096;  // too large for one XCD
     bool near = false;  // known once the first sum is
     auto half_of = [](double va, double vb, int j) {  // word j of a pair of sums
         double v = j < 2 ? va : vb;
@@ -741,7 +741,7 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     const long hslot = (long)a.box.nwg * 2 * D * a.box.amax;
     const int nwg = a.box.nwg, ngrp = (nwg + CGP_GROUP - 1) / CGP_GROUP;
     const bool two = nwg > CGP_ONE;
-    constexpr bool FAR = NB >= 1024;  // too large for one XCD
+    constexpr bool FAR = NB * C >= 4096;  // too large for one XCD
     bool near = false;  // known once the first sum is
     auto half_of = [](double v, int j) { return (unsigned)((j & 1) ? __double2hiint(v) : __double2loint(v)); };
     auto faces = [&](unsigned tag) {  // w of the box's faces, from its tile
@@ -968,8 +968,9 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     }
 }
 // The variants: threads and cells per thread, the fewest first, as more cells per workgroup cost more than more
-// workgroups up to CGP_ONE (32^3: 1.9 µs with 2 cells on 256 threads, 2.4 with 4 on 512).  16 cells on 512 threads hold
-// twice as many as 4 on 1024, whose register limit 8 would exceed (14.5 µs for 128^3, with spills).
+// workgroups up to CGP_ONE (32^3: 1.9 µs with 2 cells on 256 threads, 2.4 with 4 on 512).  8 cells on 512 threads take
+// 3.37 µs at 64^3, 4 on 1024 (at their limit of 128 registers, with spills) 3.77; 16 on 512 hold the largest levels,
+// where 8 on 1024 took 14.5 µs with spills.
 struct CgpVariant {
     int D, NB, C, HC;
     void (*k)(CgpArgs);
@@ -978,7 +979,7 @@ inline const CgpVariant *cgp_variants(int &n) {
     static const CgpVariant v[] = {{2, 256, 1, 1, k_cgp<2, 256, 1, 1>}, {2, 256, 2, 1, k_cgp<2, 256, 2, 1>},
                                    {2, 512, 4, 1, k_cgp<2, 512, 4, 1>}, {2, 1024, 4, 1, k_cgp<2, 1024, 4, 1>},
                                    {3, 256, 1, 2, k_cgp<3, 256, 1, 2>}, {3, 256, 2, 3, k_cgp<3, 256, 2, 3>},
-                                   {3, 512, 4, 3, k_cgp<3, 512, 4, 3>}, {3, 1024, 4, 2, k_cgp<3, 1024, 4, 2>},
+                                   {3, 512, 4, 3, k_cgp<3, 512, 4, 3>}, {3, 512, 8, 4, k_cgp<3, 512, 8, 4>},
                                    {3, 512, 16, 6, k_cgp<3, 512, 16, 6>}};
     n = 9;
     return v;
@@ -988,7 +989,7 @@ typedef void (*PcgpKernel)(PcgpArgs);
 inline PcgpKernel pcgp_kernel(int q) {
     static const PcgpKernel k[] = {k_pcgp<2, 256, 1, 1>, k_pcgp<2, 256, 2, 1>, k_pcgp<2, 512, 4, 1>,
                                    k_pcgp<2, 1024, 4, 1>, k_pcgp<3, 256, 1, 2>, k_pcgp<3, 256, 2, 3>,
-                                   k_pcgp<3, 512, 4, 3>, k_pcgp<3, 1024, 4, 2>, nullptr};
+                                   k_pcgp<3, 512, 4, 3>, k_pcgp<3, 512, 8, 4>, nullptr};
     return k[q];
 }
 // boxes of a level of n cells per axis for a variant, at most maxwg of them; false: none fits
