@@ -272,6 +272,25 @@ int ia_learned_stats(ia_ctx *c, ia_learned_info *s);
 int ia_learned_forward(ia_ctx *c, const float *feat, float *out);
 int ia_learned_grad(ia_ctx *c, const float *feat, const float *dout, float *gw);
 
+/* The pressure solve's CG on the coarse levels (REFERENCE and PLAIN: the
+ * finest level's pcg! too) runs in one launch per solve where the level fits
+ * the device's workgroups at once.  Such a launch needs all of them to run
+ * together; if other work keeps some off the device for 20 ms it gives up, the
+ * solve goes on with one launch per iteration (to the same tolerance, not the
+ * same bits), and so do the next 15 projections, then twice as many after each
+ * further time.  ia_last_error then says so.  No reference counterpart. */
+typedef struct ia_one_launch_info {
+    int levels;            /* bit l: level l is solved in one launch */
+    int near_levels;       /* ... whose workgroups fit one XCD */
+    int rest;              /* projections, the last one included, still to be solved by one launch per iteration */
+    int solves_near;       /* one-launch solves that did run on one XCD */
+    long long solves;      /* one-launch solves queued so far */
+    long long given_up;    /* times one gave up */
+} ia_one_launch_info;
+/* `lose` != 0 (for tests): the next one-launch solve of more than one
+ * workgroup runs without its last one, so that it gives up.  info may be NULL. */
+int ia_one_launch(ia_ctx *c, int lose, ia_one_launch_info *info);
+
 /* Kernel-class timing with HIP events on the context's stream (no reference
  * counterpart; used by the benchmark to measure one kernel's launches inside
  * a timed region).  Enabling resets the record; MG classes time level 0 only,

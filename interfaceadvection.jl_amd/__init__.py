@@ -52,6 +52,11 @@ class IALearnedInfo(C.Structure):
                 ("last_ratio", C.c_double)]
 
 
+class IAOneLaunchInfo(C.Structure):
+    _fields_ = [("levels", C.c_int), ("near_levels", C.c_int), ("rest", C.c_int), ("solves_near", C.c_int),
+                ("solves", C.c_longlong), ("given_up", C.c_longlong)]
+
+
 # parameters of the learned correction: 5 layers x (27 taps x 16 x 16) weights, then 5 x 16 biases
 LEARNED_NPAR = 5 * (27 * 16 * 16 + 16)
 
@@ -86,6 +91,7 @@ def lib():
         "ia_update_L": (C.c_int, [vp, C.c_int]),
         "ia_mg_update": (C.c_int, [vp]),
         "ia_project": (C.c_int, [vp, C.c_double, C.POINTER(IASolveStats)]),
+        "ia_one_launch": (C.c_int, [vp, C.c_int, C.POINTER(IAOneLaunchInfo)]),
         "ia_synchronize": (C.c_int, [vp]),
         "ia_profile_enable": (C.c_int, [vp, C.c_int, C.c_int]),
         "ia_profile_read": (C.c_int, [vp, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_double)]),

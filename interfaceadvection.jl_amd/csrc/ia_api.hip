@@ -114,7 +114,12 @@ struct ia_ctx {
     unsigned cgp_tag = 1;  // next unused tag of those words
     int xcd = 0;           // where launches of few workgroups run: contexts take the XCDs in turn
     bool pcgp = false;     // solver!'s pcg! in one launch (k_pcgp)
-    bool cgp_off = false;  // one launch per iteration instead (IA_CG1_NB set, or workgroups did not run together)
+    bool cgp_off = false;  // one launch per iteration instead (IA_CG1_NB set)
+    int cgp_rest = 0;      // ... for so many projections, this one included, after a launch that gave up
+    int cgp_back = CGP_REST;  // the next such rest
+    bool cgp_lose = false;    // the next one-launch solve runs without its last workgroup (ia_one_launch)
+    int *cgp_stat = nullptr;  // given up; launches that ran on one XCD
+    long cgp_solves = 0, cgp_gave_up = 0;
     int cg1_nb[MAXLEV];  // workgroup size of the coarse CG step per level (one cell per thread)
     struct Cnn {
         bool ready = false;
@@ -606,12 +611,54 @@ template <class T> struct Impl {
                 words = std::max(words, (size_t)2 * lv.cgp_box.nwg * 2 * lv.g.D * lv.cgp_box.amax);
         }
         if (words) {
+            if (int r = alloc_zero(c, (void **)&c->cgp_stat, 2 * sizeof(int))) return r;
             if (int r = alloc_zero(c, (void **)&c->cgp_hw, words * sizeof(unsigned long long))) return r;
             if (int r = alloc_zero(c, (void **)&c->cgp_pw, 2 * CGP_PW * sizeof(unsigned long long))) return r;
         }
         return IA_OK;
     }
+    static bool cgp_on(const ia_ctx *c) { return !c->cgp_off && c->cgp_rest == 0; }
     static bool cgp_failed(const ia_ctx *c) { return *(volatile int *)&c->hst->fail != 0; }
+    // after a one-launch solve that gave up: one launch per iteration for the rest of this projection and some more,
+    // then another try, each time after twice as many (what keeps workgroups off the device may last)
+    static int cgp_give_up(ia_ctx *c) {
+        HIPCHK(c, hipStreamSynchronize(c->s));
+        c->hst->fail = 0;
+        HIPCHK(c, hipMemsetAsync(c->cgp_stat, 0, sizeof(int), c->s));
+        c->cgp_gave_up++;
+        c->cgp_rest = c->cgp_back;
+        c->cgp_back = std::min(2 * c->cgp_back, CGP_REST_MAX);
+        snprintf(c->msg, sizeof c->msg,
+                 "one-launch coarse solve: its workgroups did not run together within 20 ms (%ld times so far); one launch "
+                 "per iteration for %d projections", c->cgp_gave_up, c->cgp_rest);
+        return IA_OK;
+    }
+    // what k_cgp's and k_pcgp's arguments have in common; returns the grid
+    template <class A> static dim3 cgp_args(ia_ctx *c, const Level &l, int it, int tags, A &a) {
+        a.g = l.g;
+        a.box = l.cgp_box;
+        a.L = P<float>(l.L);
+        a.iD = P<float>(l.iD);
+        a.r = P<float>(l.r);
+        a.x = P<float>(l.x);
+        a.hw = c->cgp_hw;
+        a.pw = c->cgp_pw;
+        a.spread = a.box.spread;
+        a.xcd = a.spread > 1 ? c->xcd : 0;
+        a.tag = c->cgp_tag;
+        c->cgp_tag += (unsigned)tags;
+        a.it = it;
+        a.halt = cur_halt;
+        a.fail = &c->hst->fail;
+        a.stat = c->cgp_stat;
+        c->cgp_solves++;
+        int n = a.box.nwg;
+        if (c->cgp_lose && n > 1) {
+            n--;
+            c->cgp_lose = false;
+        }
+        return dim3((unsigned)(n * a.spread));
+    }
     static size_t cgp_lds(const Level &l, const CgpVariant &v) {
         return sizeof(float) * cgp_words(v.D, v.NB, v.C, l.cgp_box.b);
     }
@@ -673,33 +720,19 @@ template <class T> struct Impl {
     // were produced by the preceding fused prolongate!/increment!.  last: the
     // final update is fused with the FCG dots of the preconditioned residual.
     // solver!'s pcg! on l in one launch
-    static bool one_launch(const ia_ctx *c, const Level &l) { return c->pcgp && l.cgp && !c->cgp_off; }
+    static bool one_launch(const ia_ctx *c, const Level &l) { return c->pcgp && l.cgp && cgp_on(c); }
     // r2: also the parts of Σr² (one per workgroup), r, z and the next Jacobi!'s ϵ
     static void pcg_launch(ia_ctx *c, Level &l, int it, bool prolong, double *r2) {
         PcgpArgs a;
-        a.g = l.g;
-        a.box = l.cgp_box;
-        a.L = P<float>(l.L);
-        a.iD = P<float>(l.iD);
-        a.x = P<float>(l.x);
-        a.r = P<float>(l.r);
+        const dim3 grid = cgp_args(c, l, it, 2 * it + 2, a);
         a.z = P<float>(l.z);
         a.e = P<float>(l.e);
         a.xc = prolong ? P<float>((&l)[1].x) : nullptr;
         a.gc = prolong ? (&l)[1].g : l.g;
-        a.hw = c->cgp_hw;
-        a.pw = c->cgp_pw;
-        a.spread = a.box.spread;
-        a.xcd = a.spread > 1 ? c->xcd : 0;
-        a.tag = c->cgp_tag;
-        c->cgp_tag += 2 * (unsigned)it + 2;
-        a.it = it;
         a.r2 = r2;
-        a.halt = cur_halt;
-        a.fail = &c->hst->fail;
         int nv;
-        hipLaunchKernelGGL(pcgp_kernel((int)(l.cgp - cgp_variants(nv))), dim3((unsigned)(a.box.nwg * a.spread)),
-                           dim3((unsigned)l.cgp->NB), cgp_lds(l, *l.cgp), c->s, a);
+        hipLaunchKernelGGL(pcgp_kernel((int)(l.cgp - cgp_variants(nv))), grid, dim3((unsigned)l.cgp->NB),
+                           cgp_lds(l, *l.cgp), c->s, a);
     }
     static void pcg(ia_ctx *c, Level &l, int it = 6, bool init_done = false, const FcgV<T> *last = nullptr,
                     int first = 0) {
@@ -773,32 +806,17 @@ template <class T> struct Impl {
     // with `prolong` the launch begins with the prolongate! and increment! that
     // vcycle leaves to it (folds).
     static bool folds(const ia_ctx *c, const Level &l) {
-        return l.cgp && !c->cgp_off && l.cgp->NB * l.cgp->C <= 4096;
+        return l.cgp && cgp_on(c) && l.cgp->NB * l.cgp->C <= 4096;
     }
     static void pcg1(ia_ctx *c, Level &l, int it, bool prolong) {
         int lv = (int)(&l - c->lev), pc = lv >= 1 && lv <= 3 ? IA_PROF_CG1_L1 + lv - 1 : -1;
-        if (l.cgp && !c->cgp_off) {
+        if (l.cgp && cgp_on(c)) {
             CgpArgs a;
-            a.g = l.g;
-            a.box = l.cgp_box;
-            a.L = P<float>(l.L);
-            a.iD = P<float>(l.iD);
-            a.r = P<float>(l.r);
-            a.x = P<float>(l.x);
+            const dim3 grid = cgp_args(c, l, it, it + 1, a);
             a.xc = prolong && folds(c, l) ? P<float>((&l)[1].x) : nullptr;
             a.gc = a.xc ? (&l)[1].g : l.g;
-            a.hw = c->cgp_hw;
-            a.pw = c->cgp_pw;
-            a.spread = a.box.spread;
-            a.xcd = a.spread > 1 ? c->xcd : 0;
-            a.tag = c->cgp_tag;
-            c->cgp_tag += (unsigned)it + 1;
-            a.it = it;
-            a.halt = cur_halt;
-            a.fail = &c->hst->fail;
             if (pc >= 0) prof_begin(c, pc);
-            hipLaunchKernelGGL(l.cgp->k, dim3((unsigned)(a.box.nwg * a.spread)), dim3((unsigned)l.cgp->NB),
-                               cgp_lds(l, *l.cgp), c->s, a);
+            hipLaunchKernelGGL(l.cgp->k, grid, dim3((unsigned)l.cgp->NB), cgp_lds(l, *l.cgp), c->s, a);
             if (pc >= 0) prof_end(c, pc);
             return;
         }
@@ -942,8 +960,8 @@ template <class T> struct Impl {
             }
             r2 = (double)(T)r2;
             n++;
-            if (cgp_failed(c) && !c->cgp_off) {  // x and r may not fit together: go on from x's own residual
-                c->cgp_off = true;
+            if (cgp_failed(c)) {  // x and r may not fit together: go on from x's own residual
+                if (int e = cgp_give_up(c)) return e;
                 if (int e = residual(c, u, &r2)) return e;
             }
         }
@@ -1175,7 +1193,8 @@ template <class T> struct Impl {
                 it++;
                 rr = st.rr;
                 rel = sqrt(rr) / zn;
-                if (cgp_failed(c)) c->cgp_off = true;
+                if (cgp_failed(c))
+                    if (int e = cgp_give_up(c)) return e;
                 if (st.halt) {
                     // the queued iteration (if any) returned at once; confirm with
                     // the true FP64 residual and restart from it if it drifted
@@ -1412,6 +1431,7 @@ template <class T> struct Impl {
     // slot: the pair of events around the solve (solve_ms reads them once the stream was waited for)
     static int project(ia_ctx *c, void *u, double dtw, ia_solve_stats *ss, int slot) {
         HIPCHK(c, hipEventRecord(c->ev_solve[slot][0], c->s));
+        if (c->cgp_rest > 0) c->cgp_rest--;
         int e = c->P.poisson_mode == IA_POISSON_REFERENCE ? project_ref(c, u, dtw, ss)
                 : c->P.poisson_mode == IA_POISSON_PCG     ? project_pcg(c, u, dtw, ss)
                                                           : project_refined(c, u, dtw, ss);
@@ -2018,7 +2038,7 @@ void ia_destroy(ia_ctx *c) {
     void *bufs[] = {c->fb[0], c->fb[1], c->fb[2], c->fb[3], c->u, c->u0, c->ru, c->ru2, c->ruf, c->F, c->p, c->sig,
                     c->st_buf, c->st_fb,
                     c->L, c->al, c->nh, c->cb, c->fpart, c->part, c->st, c->pst, c->fst, c->pp, c->dsc, c->x64, c->r64, c->z64,
-                    c->pa64, c->pb64, c->q64, c->vface, c->mface, c->cgp_hw, c->cgp_pw};
+                    c->pa64, c->pb64, c->q64, c->vface, c->mface, c->cgp_hw, c->cgp_pw, c->cgp_stat};
     for (void *b : bufs)
         if (b && !is_attached(c, b)) (void)hipFree(b);
     for (int l = 0; l < c->nlev; ++l) {
@@ -2175,6 +2195,26 @@ int ia_mg_update(ia_ctx *c) {
 int ia_project(ia_ctx *c, double dt_w, ia_solve_stats *stats) {
     if (stats) memset(stats, 0, sizeof *stats);
     return dispatch(c, [&](auto impl) { return decltype(impl)::project_stage(c, dt_w, stats); });
+}
+int ia_one_launch(ia_ctx *c, int lose, ia_one_launch_info *o) {
+    if (!c) return IA_ERR_BADARG;
+    if (lose) c->cgp_lose = true;
+    if (!o) return IA_OK;
+    int stat[2] = {0, 0};
+    HIPCHK(c, hipSetDevice(c->dev));
+    HIPCHK(c, hipStreamSynchronize(c->s));
+    if (c->cgp_stat) HIPCHK(c, hipMemcpy(stat, c->cgp_stat, sizeof stat, hipMemcpyDeviceToHost));
+    memset(o, 0, sizeof *o);
+    for (int l = 0; l < c->nlev; ++l)
+        if (c->lev[l].cgp) {
+            o->levels |= 1 << l;
+            if (c->lev[l].cgp_box.spread > 1) o->near_levels |= 1 << l;
+        }
+    o->rest = c->cgp_rest;
+    o->solves = c->cgp_solves;
+    o->solves_near = stat[1];
+    o->given_up = c->cgp_gave_up;
+    return IA_OK;
 }
 int ia_synchronize(ia_ctx *c) {
     if (!c) return IA_ERR_BADARG;

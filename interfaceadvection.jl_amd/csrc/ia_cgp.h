@@ -35,9 +35,10 @@ namespace ia {
 // recurrence and the two sums, a chain of some 2000 cycles in which a wavefront mostly waits for itself: nothing in it
 // stands behind a branch, faces are published through a tile, and a workgroup's words of a sum lie together.
 //
-// A workgroup that waits longer than CGP_WAIT (another program's work kept
-// some workgroups off the device) writes the x it has, raises *fail and ends,
-// so the launch always ends; x is then a less exact solution.
+// A workgroup that waits longer than CGP_WAIT (other work kept some
+// workgroups off the device) writes the x it has, raises *fail and ends, so
+// the launch always ends; x is then a less exact solution.  The host then
+// solves by one launch per iteration for a while (cgp_give_up).
 // ---------------------------------------------------------------------------
 constexpr int CGP_MAXWG = 256;
 constexpr int CGP_XCDS = 8;   // workgroups go to the XCDs in turn, so those of every eighth number share one
@@ -49,6 +50,7 @@ constexpr int CGP_GROUP = 16; // above, the sums of groups of this many, which t
 // with 18); within one L2 waiting first gains nothing
 constexpr int CGP_NAP = 12;
 constexpr long CGP_WAIT = 2000000;  // ticks of the 100 MHz counter: 20 ms
+constexpr int CGP_REST = 16, CGP_REST_MAX = 4096;  // projections without one-launch solves after one that gave up
 constexpr long CGP_LDS = 158 * 1024;  // of the 160 KiB of a CU
 struct CgpBox {
     int k[3], b[3];  // boxes per axis, cells per box and axis (the last box may have fewer, at least 2)
@@ -68,7 +70,8 @@ struct CgpArgs {
     int it;
     int spread, xcd;  // of spread workgroups one takes part, those of blockIdx.x % spread == xcd
     const int *halt;
-    int *fail;
+    int *fail;  // in host memory
+    int *stat;  // in device memory: whether one gave up; how many ran on one XCD
 };
 // a slot of partial sums: 4 words for each workgroup of a group in CGP_COPY copies, then 4 words for each workgroup
 constexpr int CGP_COPY = 16;
@@ -108,6 +111,9 @@ template <int N> __device__ inline void cgp_getn(const cgp_word *p, int i, cgp_w
 #pragma unroll
         for (int j = 0; j < N; ++j) v[j] = __hip_atomic_load(p + i + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+__device__ inline void cgp_count(int *n) {  // no read to wait for
+    (void)__hip_atomic_fetch_add(n, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // the XCD this wavefront runs on (HW_REG_XCC_ID)
 __device__ inline unsigned cgp_xcd() { return __builtin_amdgcn_s_getreg(20 | (3 << 11)); }
@@ -515,7 +521,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
         if (!ok) dead = 1;
         __syncthreads();
         if (dead) {
-            if (tid == 0) *a.fail = 1;
+            if (tid == 0) *a.fail = a.stat[0] = 1;
             break;
         }
         near = !FAR && nears != 0;
@@ -566,6 +572,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
         __syncthreads();
         apply(tag + 1);
     }
+    if (near && wg == 0 && tid == 0) cgp_count(a.stat + 1);
 #pragma unroll
     for (int k = 0; k < C; ++k)
         if (k < cnt)
@@ -599,7 +606,8 @@ struct PcgpArgs {
     double *r2;
     int spread, xcd;  // of spread workgroups one takes part, those of wg % spread == xcd
     const int *halt;
-    int *fail;
+    int *fail;  // in host memory
+    int *stat;  // in device memory: whether one gave up; how many ran on one XCD
 };
 template <int D, int NB, int C, int HC>
 __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
@@ -940,7 +948,8 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
         __syncthreads();
         rho = rho2;
     }
-    if (!ok && tid == 0) *a.fail = 1;
+    if (!ok && tid == 0) *a.fail = a.stat[0] = 1;
+    if (near && wg == 0 && tid == 0) cgp_count(a.stat + 1);
     v = 0;
 #pragma unroll
     for (int k = 0; k < C; ++k)
