@@ -1154,11 +1154,13 @@ template <class T> struct Impl {
             prof_end(c, IA_PROF_LOAD_INC);
             vcycle(c, 0, c->cit_wl, true, true);
             pcg(c, l0, 6, true);
-            hipLaunchKernelGGL(k_ir_accum<T>, B, dim3(NT), 0, c->s, f);
+            hipLaunchKernelGGL(k_ir_accum<T>, B, dim3(NT), 0, c->s, f, c->cgp_stat);
             LAUNCHCHK(c);
             if (int e = true_resid(c, &rr)) return e;
             rel = sqrt(rr) / zn;
             it++;
+            if (cgp_failed(c))
+                if (int e = cgp_give_up(c)) return e;
         }
         // flexible CG, pipelined: the host queues iteration n+1 before it reads
         // iteration n's residual, so the device never waits for the host; the

@@ -1778,9 +1778,12 @@ __global__ void __launch_bounds__(NT) k_fcg_check(FcgV<T> f, const double *part_
         host->halt = halt;
     }
 }
-// plain multigrid refinement: x += s·x_T ; r = z - A x is recomputed by the caller
+// plain multigrid refinement: x += s·x_T ; r = z - A x is recomputed by the
+// caller.  Not if a one-launch solve gave up: its boxes stopped at different
+// iterations, and unlike the flexible CG's α nothing here weighs what they give.
 template <class T>
-__global__ void __launch_bounds__(NT) k_ir_accum(FcgV<T> f) {
+__global__ void __launch_bounds__(NT) k_ir_accum(FcgV<T> f, const int *gave_up) {
+    if (gave_up && *gave_up) return;
     double s = f.S->sload;
     COL_LOOP(f, { f.x[I] += s * (double)f.w[I]; })
 }

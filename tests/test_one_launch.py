@@ -114,3 +114,22 @@ def test_give_up_is_reported_and_tried_again(dims, poisson):
     o = info(s)
     assert o.given_up == 2 and o.rest == 2 * REST
     s.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,perdir", [((192, 136), ()), ((64, 64, 48), (2,)), ((96, 96, 96), ())])
+def test_plain_multigrid_throws_a_cut_short_correction_away(dims, perdir):
+    """Plain multigrid adds each V-cycle's correction as it is: the one whose
+    solve gave up is left out, so one more V-cycle does (one of slack)."""
+    say("plain multigrid, one-launch solve gives up", dims, perdir)
+    s, u = box(dims, perdir, poisson="plain", λρ=0.1)
+    u0, _, st0 = project(s, u)
+    assert info(s).solves > 0 and 0 < st0.rel <= 1e-6
+    info(s, lose=1)
+    u1, _, st1 = project(s, u)
+    o = info(s)
+    print(f"V-cycles {st0.iters} / {st1.iters}, rel {st1.rel:.2e}, {st0.ms:.1f} / {st1.ms:.1f} ms")
+    assert o.given_up == 1 and o.rest == REST
+    assert 0 < st1.rel <= 1e-6 and st0.iters < st1.iters <= st0.iters + 2
+    assert float(abs(u1 - u0).max()) <= 1e-5 * float(abs(u0).max())
+    s.close()
