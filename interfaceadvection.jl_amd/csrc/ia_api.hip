@@ -59,6 +59,20 @@ int noalloc_setup(int dev, const char **why) {
 
 namespace {
 
+// One-launch solves of several contexts of this process on one device.  Each
+// needs its workgroups to run together, so two that hold part of the device
+// each would wait for one another's places until both give up.  While more
+// than one context is in a projection there, such a launch waits (on the
+// device) for those that could stand in its way: one on an XCD of its own for
+// the latest on that XCD and the latest that took them all, any other for all
+// of them.  A context alone, which is the usual case, pays a lock per launch.
+struct Turns {
+    std::mutex mu;
+    std::vector<ia_ctx *> in;            // contexts in a projection
+    ia_ctx *last[CGP_XCDS] = {};         // per XCD, whose launch came last; its cgp_ev stands behind it
+};
+Turns cgp_turns[NOALLOC_MAXDEV];
+
 struct Level {
     Grid g;
     Tiling t;
@@ -120,6 +134,7 @@ struct ia_ctx {
     bool cgp_lose = false;    // the next one-launch solve runs without its last workgroup (ia_one_launch)
     int *cgp_stat = nullptr;  // given up; launches that ran on one XCD
     long cgp_solves = 0, cgp_gave_up = 0;
+    hipEvent_t cgp_ev = nullptr;  // after this context's latest one-launch solve, while contexts take turns (Turns)
     int cg1_nb[MAXLEV];  // workgroup size of the coarse CG step per level (one cell per thread)
     struct Cnn {
         bool ready = false;
@@ -575,8 +590,10 @@ template <class T> struct Impl {
     }
 
     // the levels solved in one launch, by k_cgp (the flexible CG's preconditioner) or k_pcgp (solver!'s pcg!, the
-    // finest level among them): those above the tail whose boxes fit, on a device that holds twice the workgroups at
-    // once (two contexts may run there together)
+    // finest level among them): those above the tail whose boxes fit a device that holds their workgroups at once.  Up
+    // to CGP_ONE of them (2 x 64 on 256 CUs) it has to hold twice as many, which leaves room for what other programs and
+    // streams run meanwhile; more take the device as it is, or 128³ would have no place (16 cells a thread: one
+    // workgroup a CU).  Contexts of one program do not compete (Turns).
     static int cgp_setup(ia_ctx *c) {
         // FP64's sums show the order of their terms in the result, which the launches' tiles set
         if (sizeof(T) != 4 || c->cgp_off || c->P.poisson_mode == IA_POISSON_PCG) return IA_OK;
@@ -614,6 +631,7 @@ template <class T> struct Impl {
             if (int r = alloc_zero(c, (void **)&c->cgp_stat, 2 * sizeof(int))) return r;
             if (int r = alloc_zero(c, (void **)&c->cgp_hw, words * sizeof(unsigned long long))) return r;
             if (int r = alloc_zero(c, (void **)&c->cgp_pw, 2 * CGP_PW * sizeof(unsigned long long))) return r;
+            HIPCHK(c, hipEventCreateWithFlags(&c->cgp_ev, hipEventDisableTiming));
         }
         return IA_OK;
     }
@@ -658,6 +676,46 @@ template <class T> struct Impl {
             c->cgp_lose = false;
         }
         return dim3((unsigned)(n * a.spread));
+    }
+    // around a projection, at whose end its one-launch solves are over: the host has read what they led to
+    struct InTurn {
+        ia_ctx *c;
+        bool ok = false;  // else the projection ended early: wait for them
+        explicit InTurn(ia_ctx *c_) : c(c_) {
+            if (!c->cgp_ev) return;
+            Turns &t = cgp_turns[c->dev];
+            std::lock_guard<std::mutex> lk(t.mu);
+            if (t.in.size() == 1) {  // it was alone and recorded nothing
+                ia_ctx *o = t.in[0];
+                if (hipEventRecord(o->cgp_ev, o->s) == hipSuccess)
+                    for (ia_ctx *&q : t.last) q = o;
+            }
+            t.in.push_back(c);
+        }
+        ~InTurn() {
+            if (!c->cgp_ev) return;
+            if (!ok) (void)hipStreamSynchronize(c->s);
+            Turns &t = cgp_turns[c->dev];
+            std::lock_guard<std::mutex> lk(t.mu);
+            t.in.erase(std::find(t.in.begin(), t.in.end(), c));
+            for (ia_ctx *&q : t.last)
+                if (q == c) q = nullptr;
+        }
+    };
+    template <class F> static void in_turn(ia_ctx *c, bool near, F &&launch) {
+        Turns &t = cgp_turns[c->dev];
+        std::lock_guard<std::mutex> lk(t.mu);
+        if (t.in.size() < 2) {
+            launch();
+            return;
+        }
+        const int x0 = near ? c->xcd : 0, x1 = near ? c->xcd + 1 : CGP_XCDS;
+        for (int x = x0; x < x1; ++x)
+            if (ia_ctx *o = t.last[x]; o && o != c && (x == x0 || o != t.last[x - 1]))
+                (void)hipStreamWaitEvent(c->s, o->cgp_ev, 0);
+        launch();
+        (void)hipEventRecord(c->cgp_ev, c->s);
+        for (int x = x0; x < x1; ++x) t.last[x] = c;
     }
     static size_t cgp_lds(const Level &l, const CgpVariant &v) {
         return sizeof(float) * cgp_words(v.D, v.NB, v.C, l.cgp_box.b);
@@ -731,8 +789,10 @@ template <class T> struct Impl {
         a.gc = prolong ? (&l)[1].g : l.g;
         a.r2 = r2;
         int nv;
-        hipLaunchKernelGGL(pcgp_kernel((int)(l.cgp - cgp_variants(nv))), grid, dim3((unsigned)l.cgp->NB),
-                           cgp_lds(l, *l.cgp), c->s, a);
+        in_turn(c, a.spread > 1, [&] {
+            hipLaunchKernelGGL(pcgp_kernel((int)(l.cgp - cgp_variants(nv))), grid, dim3((unsigned)l.cgp->NB),
+                               cgp_lds(l, *l.cgp), c->s, a);
+        });
     }
     static void pcg(ia_ctx *c, Level &l, int it = 6, bool init_done = false, const FcgV<T> *last = nullptr,
                     int first = 0) {
@@ -816,7 +876,9 @@ template <class T> struct Impl {
             a.xc = prolong && folds(c, l) ? P<float>((&l)[1].x) : nullptr;
             a.gc = a.xc ? (&l)[1].g : l.g;
             if (pc >= 0) prof_begin(c, pc);
-            hipLaunchKernelGGL(l.cgp->k, grid, dim3((unsigned)l.cgp->NB), cgp_lds(l, *l.cgp), c->s, a);
+            in_turn(c, a.spread > 1, [&] {
+                hipLaunchKernelGGL(l.cgp->k, grid, dim3((unsigned)l.cgp->NB), cgp_lds(l, *l.cgp), c->s, a);
+            });
             if (pc >= 0) prof_end(c, pc);
             return;
         }
@@ -1434,10 +1496,12 @@ template <class T> struct Impl {
     static int project(ia_ctx *c, void *u, double dtw, ia_solve_stats *ss, int slot) {
         HIPCHK(c, hipEventRecord(c->ev_solve[slot][0], c->s));
         if (c->cgp_rest > 0) c->cgp_rest--;
+        InTurn turn(c);
         int e = c->P.poisson_mode == IA_POISSON_REFERENCE ? project_ref(c, u, dtw, ss)
                 : c->P.poisson_mode == IA_POISSON_PCG     ? project_pcg(c, u, dtw, ss)
                                                           : project_refined(c, u, dtw, ss);
         if (e) return e;
+        turn.ok = true;
         HIPCHK(c, hipEventRecord(c->ev_solve[slot][1], c->s));
         return IA_OK;
     }
@@ -2068,6 +2132,7 @@ void ia_destroy(ia_ctx *c) {
     }
     for (hipEvent_t e : c->it_ev)
         if (e) (void)hipEventDestroy(e);
+    if (c->cgp_ev) (void)hipEventDestroy(c->cgp_ev);
     if (c->pin) (void)hipHostFree(c->pin);
     if (c->hst) (void)hipHostFree(c->hst);
     if (c->hpart) (void)hipHostFree(c->hpart);

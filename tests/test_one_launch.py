@@ -3,6 +3,7 @@ that runs, and what happens when a launch's workgroups do not run together.  A
 lost workgroup is one that was not launched: the others wait out their bounded
 wait (20 ms) and every kernel ends by itself."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -133,3 +134,39 @@ def test_plain_multigrid_throws_a_cut_short_correction_away(dims, perdir):
     assert 0 < st1.rel <= 1e-6 and st0.iters < st1.iters <= st0.iters + 2
     assert float(abs(u1 - u0).max()) <= 1e-5 * float(abs(u0).max())
     s.close()
+
+
+WIDE = dict(dims=(256, 256, 248), poisson="refined")   # a level of one workgroup per CU
+FLAT = dict(dims=(1024, 640), poisson="reference", poisson_tol=1e-12, poisson_itmx=40)  # 160 workgroups on the finest level
+NEAR = dict(dims=(192, 136), poisson="refined")        # on one XCD
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kinds", [(WIDE, WIDE), (FLAT, FLAT), (WIDE, NEAR, FLAT), (NEAR,) * 10])
+def test_contexts_at_once(kinds):
+    """Contexts that project at the same time from threads of their own: nobody
+    gives up, and everyone's bits are those of its projection alone (the same
+    launches, only later)."""
+    say("one-launch solves of contexts at once", [k["dims"] for k in kinds])
+    sims = [box(perdir=(), seed=3 + i, **k) for i, k in enumerate(kinds)]
+    alone = [project(s, u)[:2] for s, u in sims]
+    gate, wrong = threading.Barrier(len(sims)), []
+
+    def work(i):
+        s, u = sims[i]
+        gate.wait()
+        for _ in range(6):
+            uk, pk, _ = project(s, u)
+            if not ((uk == alone[i][0]).all() and (pk == alone[i][1]).all()):
+                wrong.append(i)
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(len(sims))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    got = [info(s) for s, _ in sims]
+    assert all(o.given_up == 0 and o.solves > 0 for o in got), [o.given_up for o in got]
+    assert not wrong
+    for s, _ in sims:
+        s.close()
