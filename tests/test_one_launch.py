@@ -136,6 +136,56 @@ def test_plain_multigrid_throws_a_cut_short_correction_away(dims, perdir):
     s.close()
 
 
+TAIL, FINEST = 4096, 1 << 20  # cells: the levels below are the tail's; what boxes of 4096 cells hold
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("poisson,dims,perdir", [
+    ("refined", (256, 200), ()), ("refined", (200, 136), (1, 2)), ("refined", (2048, 16), (2,)),
+    ("refined", (16, 2048), (1,)), ("refined", (64, 64, 64), ()), ("refined", (120, 88, 72), (1, 2)),
+    ("refined", (100, 60, 84), (3,)), ("refined", (512, 16, 16), (1, 2, 3)), ("refined", (16, 256, 32), ()),
+    ("refined", (160, 160, 96), (2,)), ("refined", (240, 208, 200), (1,)), ("refined", (256, 256, 248), (3,)),
+    ("reference", (64, 64), (1, 2)), ("reference", (256, 200), ()), ("reference", (1000, 24), (2,)),
+    ("reference", (512, 512), ()), ("reference", (1024, 640), (1,)), ("reference", (48, 32, 40), ()),
+    ("reference", (100, 60, 84), (1, 3)), ("reference", (64, 64, 64), ()), ("reference", (96, 96, 96), (2,)),
+    ("reference", (128, 128, 128), ()),
+])
+def test_every_level_above_the_tail_takes_one_launch(poisson, dims, perdir):
+    """The grids of test_coarse_cg.py: the levels above the tail (and the finest
+    in the default solver), up to 2M cells in 3D and 1M otherwise, are solved in
+    one launch each in every V-cycle, the coarsest of them on one XCD (the XCDs
+    were read on the device), and none gives up."""
+    say("levels in one launch", poisson, dims, perdir)
+    kw = dict(poisson_tol=1e-12, poisson_itmx=3) if poisson == "reference" else {}
+    s, u = box(dims, perdir, poisson=poisson, **kw)
+    _, _, st = project(s, u)
+    o = info(s)
+    want = 0
+    for l in range(s._lib.ia_mg_levels(s._ctx, 0, None)):
+        cells = int(np.prod([n >> l for n in dims]))
+        big = 2 * FINEST if poisson == "refined" and len(dims) == 3 else FINEST
+        if cells <= big and (cells > TAIL or l == 0) and l >= (poisson == "refined"):
+            want |= 1 << l
+    assert o.levels == want and want
+    nl, nn = bin(want).count("1"), bin(o.near_levels).count("1")
+    assert o.near_levels & (1 << (want.bit_length() - 1))
+    assert o.solves in (st.iters * nl, (st.iters + 1) * nl)  # the flexible CG queues one V-cycle ahead
+    assert o.solves_near == st.iters * nn
+    assert o.given_up == 0 and o.rest == 0
+    s.close()
+
+
+@pytest.mark.gpu
+def test_launches_per_iteration_are_none_of_these(monkeypatch):
+    say("no level in one launch with IA_CG1_NB")
+    monkeypatch.setenv("IA_CG1_NB", "256")
+    s, u = box((192, 136), poisson="refined")
+    project(s, u)
+    o = info(s)
+    assert o.levels == 0 and o.solves == 0 and o.solves_near == 0 and o.given_up == 0
+    s.close()
+
+
 WIDE = dict(dims=(256, 256, 248), poisson="refined")   # a level of one workgroup per CU
 FLAT = dict(dims=(1024, 640), poisson="reference", poisson_tol=1e-12, poisson_itmx=40)  # 160 workgroups on the finest level
 NEAR = dict(dims=(192, 136), poisson="refined")        # on one XCD
