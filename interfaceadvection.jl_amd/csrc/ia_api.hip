@@ -502,8 +502,10 @@ template <class T> struct Impl {
         void **l0b[] = {&l0.Dg, &l0.iD, &l0.e, &l0.r};
         for (void **v : l0b)
             if (int r = alloc_zero(c, v, ns * es)) return r;
-        // FP64 pcg! on a small finest level: a launch less per iteration for two more arrays
-        if (es == 8 && interior(g) < (1 << 20))
+        // FP64 pcg! on a small finest level: a launch less per iteration for two more arrays, whose traffic costs more
+        // than the launch on larger ones (20 V-cycles, ms without / with: 64² 2.74 / 2.49, 700² 5.99 / 5.76, 512x1024
+        // 8.38 / 8.18, 900² 8.47 / 8.61; 48³ 4.19 / 3.98, 64³ 5.33 / 5.14, 72³ 6.29 / 6.42, 96³ 8.04 / 8.37)
+        if (es == 8 && interior(g) <= (g.D == 2 ? 1 << 19 : 1 << 18))
             for (void **v : {&l0.e2, &l0.z2})
                 if (int r = alloc_zero(c, v, ns * es)) return r;
         c->nlev = 1;
@@ -594,6 +596,9 @@ template <class T> struct Impl {
     // to CGP_ONE of them (2 x 64 on 256 CUs) it has to hold twice as many, which leaves room for what other programs and
     // streams run meanwhile; more take the device as it is, or 128³ would have no place (16 cells a thread: one
     // workgroup a CU).  Contexts of one program do not compete (Turns).
+    // No level is too large to gain: the default solver in FP32, 20 V-cycles, ms by launches per iteration / here: 64²
+    // 1.68 / 0.95, 256² 2.69 / 1.69, 512² 4.18 / 2.55, 1024x640 4.95 / 2.47, 1024² 6.64 / 3.25, 2048x256 5.06 / 2.42;
+    // 32³ 2.10 / 1.25, 64³ 3.29 / 2.12, 96x96x80 4.54 / 2.97, 96³ 4.54 / 3.16.
     static int cgp_setup(ia_ctx *c) {
         // FP64's sums show the order of their terms in the result, which the launches' tiles set
         if (sizeof(T) != 4 || c->cgp_off || c->P.poisson_mode == IA_POISSON_PCG) return IA_OK;
