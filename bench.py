@@ -67,16 +67,23 @@ BYTES_PER_CELL = {
     # solve in one launch r, iD, L, x -> x
     "cg1_l1": 24 + 4, "cg1_l2": 24 + 4, "cg1_l3": 24 + 4,
 }
-# levels too large for one launch: a step r, w, s, iD, p, x, L -> p, s', x, r', w'
-CG1_STEP, CG1_CELLS = 36 + 20, 2 << 20
-
-
-def bytes_per_cell(k, cells):
-    return CG1_STEP if k.startswith("cg1") and cells > CG1_CELLS else BYTES_PER_CELL[k]
-
-
+# levels solved by one launch per iteration: a step r, w, s, iD, p, x, L -> p, s', x, r', w'
+CG1_STEP = 36 + 20
 # coarse level of a class (its cells are (N >> level)^3); 0 for the fine-level classes
 LEVEL = {"cg1_l1": 1, "cg1_l2": 2, "cg1_l3": 3}
+
+
+def bytes_per_cell(k, one):
+    """Of a launch of class k; `one`: the IAOneLaunchInfo of the context, which
+    says which levels are solved in one launch.  None where a class mixes whole
+    solves and steps (a one-launch solve gave up)."""
+    if not k.startswith("cg1"):
+        return BYTES_PER_CELL[k]
+    if not one.levels >> LEVEL[k] & 1:
+        return CG1_STEP
+    return None if one.given_up else BYTES_PER_CELL[k]
+
+
 # kernel classes timed with HIP events in the timed region; the one with the
 # largest total time is reported as the dominant kernel
 PROFILED = ["load_inc", "prolong_inc", "cheb2_dots", "fcg_Ap", "fcg_update", "vof", "momentum",
@@ -268,8 +275,13 @@ def main():
     classes = [] if args.no_events else (PROFILED if args.profile == "auto" else [args.profile])
     cells = N ** 3
 
+    def one_launch():
+        o = ia.IAOneLaunchInfo()
+        sim._call("ia_one_launch", 0, ia.C.byref(o))
+        return o
+
     def read_classes(names):
-        out = {}
+        out, one = {}, one_launch()
         for k in names:
             nl, ms = ia.C.c_int(), ia.C.c_double()
             sim._call("ia_profile_read", ia.PROFILE[k], ia.C.byref(nl), ia.C.byref(ms))
@@ -277,8 +289,9 @@ def main():
             if nl.value:
                 avg = ms.value / nl.value
                 kc = (N >> LEVEL.get(k, 0)) ** 3
+                b = bytes_per_cell(k, one)
                 out[k] = dict(launches=nl.value, total_ms=round(ms.value, 3), avg_ms=round(avg, 4),
-                              GBps=round(bytes_per_cell(k, kc) * kc / (avg * 1e-3) / 1e9, 1), cells=kc)
+                              GBps=b and round(b * kc / (avg * 1e-3) / 1e9, 1), cells=kc)
         return out
 
     # Every class is timed over the warm-up steps; inside the timed steps only
@@ -329,15 +342,17 @@ def main():
                    "grid": [N, N, N], "poisson": args.poisson, "poisson_rtol": args.rtol,
                    "cg_iterations_per_solve_mean": float(np.mean(iters)),
                    "poisson_time_to_1e-6_ms": round(float(np.mean(solve_ms)), 3),
-                   "poisson_rel_residual_max": float(np.max(rel)) if rel else None},
+                   "poisson_rel_residual_max": float(np.max(rel)) if rel else None,
+                   "one_launch_solves_given_up": one_launch().given_up},
         "kernels": timed if not warm else warm,
         "kernels_timed_over": "the timed steps" if not warm else f"the {args.warmup} warm-up steps "
                               f"(the roofline kernel: the timed steps)",
     }
-    if dom:
+    bpc = bytes_per_cell(dom, one_launch()) if dom else None
+    if bpc:
         traffic, traffic_src = pmc_traffic(dom) if (args.case, N) == ("pool", 256) else (None, None)
         avg_ms = timed[dom]["avg_ms"]
-        bpl = bytes_per_cell(dom, timed[dom]["cells"]) * timed[dom]["cells"]
+        bpl = bpc * timed[dom]["cells"]
         achieved = bpl / (avg_ms * 1e-3) / 1e9
         out["roofline"] = {"kernel": dom, "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK,
                            "unit": "GB/s", "frac": round(achieved / HBM_PEAK, 4),

@@ -58,6 +58,19 @@ def test_info_layout_matches_header(tmp_path):
         assert lay[("ia_one_launch_info", n)] == getattr(ia.IAOneLaunchInfo, n).offset
 
 
+def test_bench_counts_the_path_that_ran():
+    """A coarse level's bytes: of a whole solve where it is one launch, of a step
+    where it is not (whatever its size), of neither where the record mixes both."""
+    import bench
+
+    o = ia.IAOneLaunchInfo()
+    o.levels = 0b1010
+    assert bench.bytes_per_cell("cg1_l1", o) == bench.BYTES_PER_CELL["cg1_l1"] == 28
+    assert bench.bytes_per_cell("cg1_l2", o) == 56 and bench.bytes_per_cell("vof", o) == 21
+    o.given_up = 1
+    assert bench.bytes_per_cell("cg1_l3", o) is None and bench.bytes_per_cell("cg1_l2", o) == 56
+
+
 def div2(u):
     """Σ(div u)² over the interior: what a projection left of the residual."""
     D = u.ndim - 1
