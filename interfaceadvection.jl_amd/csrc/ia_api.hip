@@ -768,10 +768,6 @@ template <class T> struct Impl {
         return v;
     }
     static dim3 cb(const Level &l) { return dim3((unsigned)l.ct.nblk); }
-    static void jacobi(ia_ctx *c, Level &l) {
-        hipLaunchKernelGGL(k_mg_jacobi<T>, cb(l), dim3(NT), 0, c->s, view(l));
-        increment(c, l);
-    }
     static void increment(ia_ctx *c, Level &l) {
         bool f0 = &l == &c->lev[0];
         if (f0) prof_begin(c, IA_PROF_INCREMENT);
@@ -779,9 +775,6 @@ template <class T> struct Impl {
         if (f0) prof_end(c, IA_PROF_INCREMENT);
     }
     static double *pp(ia_ctx *c, int k) { return c->pp + (long)k * c->pp_stride; }
-    // WaterLily pcg!(p; it).  init_done: ϵ = r·iD and the partials of ρ₀ (PP_A)
-    // were produced by the preceding fused prolongate!/increment!.  last: the
-    // final update is fused with the FCG dots of the preconditioned residual.
     // solver!'s pcg! on l in one launch
     static bool one_launch(const ia_ctx *c, const Level &l) { return c->pcgp && l.cgp && cgp_on(c); }
     // r2: also the parts of Σr² (one per workgroup), r, z and the next Jacobi!'s ϵ
@@ -799,6 +792,9 @@ template <class T> struct Impl {
                                cgp_lds(l, *l.cgp), c->s, a);
         });
     }
+    // WaterLily pcg!(p; it).  init_done: ϵ = r·iD and the partials of ρ₀ (PP_A)
+    // were produced by the preceding fused prolongate!/increment!.  last: the
+    // final update is fused with the FCG dots of the preconditioned residual.
     static void pcg(ia_ctx *c, Level &l, int it = 6, bool init_done = false, const FcgV<T> *last = nullptr,
                     int first = 0) {
         if (one_launch(c, l)) {
@@ -860,10 +856,6 @@ template <class T> struct Impl {
         }
         hipLaunchKernelGGL(k_mg_tail<T>, dim3(1), dim3(NT1), c->tail_lds, c->s, a);
     }
-    // Vcycle!(ml; l); the levels from c->tail_level down run in one workgroup.
-    // pre_done: Jacobi! + increment! of level l were fused into the caller's
-    // residual load.  then_pcg: a pcg! on level l follows, so its first
-    // statement is fused into the final prolongate! + increment!.
     // the flexible CG preconditioner's coarse solve: single-reduction CG, in
     // one launch (k_cgp) where the level's boxes fit, else one launch per
     // iteration (k_cg1_init, k_cg1_step).  The final r may sit in r2 or
@@ -924,20 +916,19 @@ template <class T> struct Impl {
         }
         if (pc >= 0) prof_end(c, pc, it);
     }
-    // e_done: Jacobi!'s ϵ = r·iD on level l was written by the restrict! that
-    // produced its r, so only increment! remains.
-    static void vcycle(ia_ctx *c, int l, const int *cit, bool pre_done = false, bool then_pcg = false,
-                       bool e_done = false, int rev = 0) {
+    // Vcycle!(ml; l); the levels from c->tail_level down run in one workgroup.
+    // pre_done: Jacobi! + increment! of level l were fused into the caller's
+    // residual load; else its ϵ = r·iD was written with the r, so that only
+    // increment! remains.  then_pcg: a pcg! on level l follows, so its first
+    // statement is fused into the final prolongate! + increment!.
+    static void vcycle(ia_ctx *c, int l, const int *cit, bool pre_done, bool then_pcg, int rev = 0) {
         Level &fl = c->lev[l], &co = c->lev[l + 1];
         bool rec = l + 2 < c->nlev, co_jacobi = l + 1 < c->tail_level && rec;
-        if (!pre_done && e_done && interior(fl.g) <= 1 << 18) {
+        if (!pre_done && interior(fl.g) <= 1 << 18) {
             auto k = fl.g.D == 3 ? k_mg_inc_restrict<3, T> : k_mg_inc_restrict<2, T>;
             hipLaunchKernelGGL(k, cb(co), dim3(NT), 0, c->s, view(co), view(fl), co_jacobi ? 1 : 0);
         } else {
-            if (!pre_done) {
-                if (e_done) increment(c, fl);
-                else jacobi(c, fl);
-            }
+            if (!pre_done) increment(c, fl);
             hipLaunchKernelGGL(k_mg_restrict<T>, cb(co), dim3(NT), 0, c->s, view(co), fl.g, P<T>(fl.r),
                                co_jacobi ? 1 : 0);
         }
@@ -961,7 +952,7 @@ template <class T> struct Impl {
             a.halt = cur_halt;
             launch_tail(c, a, cit == c->cit_fcg);
         } else {
-            if (rec) vcycle(c, l + 1, cit, false, true, true);
+            if (rec) vcycle(c, l + 1, cit, false, true);
             if (cit == c->cit_fcg) pcg1(c, co, cit[l + 1], rec);
             else pcg(c, co, cit[l + 1], rec);
         }
@@ -1011,7 +1002,7 @@ template <class T> struct Impl {
         if (int e = residual(c, u, &r2)) return e;
         int n = 0;
         while (r2 > tol && n < itmx) {
-            vcycle(c, 0, c->cit_wl, false, true, true);
+            vcycle(c, 0, c->cit_wl, false, true);
             if (one_launch(c, l0)) {
                 pcg_launch(c, l0, 6, true, c->hst->r2);
                 LAUNCHCHK(c);
@@ -1151,7 +1142,7 @@ template <class T> struct Impl {
                            c->fine_cheb ? 0 : 1);
         prof_end(c, IA_PROF_LOAD_INC);
         if (c->fine_cheb) {
-            vcycle(c, 0, c->cit_fcg, true, true, false, !par);
+            vcycle(c, 0, c->cit_fcg, true, true, !par);
             double c0, ca, cb;
             cheb2_coeffs(c0, ca, cb);
             prof_begin(c, IA_PROF_PCG_LAST);

@@ -155,10 +155,6 @@ struct StepOut {
     int pad;
     double r2[256]; // the parts of Σr² of a one-launch pcg!
 };
-struct SolveCtl {
-    double rho, alpha, beta, s, r2, dot;
-    int done, stop, it, pad;
-};
 
 // ---------------------------------------------------------------------------
 // c̄ = f≥½ (advection.jl:40, flow.jl:172) and ρu = u·ρ(f) (VOFutil.jl:208-211);
@@ -1120,12 +1116,6 @@ template <class T> __global__ void __launch_bounds__(MGU_NT) k_coarse_levels(Mgu
         __syncthreads();
     }
 }
-__global__ void __launch_bounds__(NT) k_fin_sum(const double *part, long nblk, double *out) {
-    double v = 0;
-    for (long b = threadIdx.x; b < nblk; b += NT) v += part[b];
-    double s = block_sum(v);
-    if (threadIdx.x == 0) *out = s;
-}
 // myproject!: u -= L ∂x ; BC!(u)  (flow.jl:331-333, :82)
 template <class T>
 __global__ void __launch_bounds__(NT) k_project(Grid g, Tiling t, T *u, const T *L, const T *x, T ubc0, T ubc1, T ubc2) {
@@ -1141,12 +1131,6 @@ __global__ void __launch_bounds__(NT) k_project(Grid g, Tiling t, T *u, const T 
         T xv = i == 0 && g.exitx ? u[I + g.st[0]] : T(0);  // exitBC: the exit face is left alone
         write_row_u<T>(g, u + g.ns * i, p, I, un, true, i, ub[i], xv);
     }
-}
-// f⁰ = (f⁰ + f)/2 over every cell (flow.jl:74)
-template <class T>
-__global__ void k_avg(T *a, const T *b, long n) {
-    long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < n) a[q] = (a[q] + b[q]) / 2;
 }
 // applyVOF! from SDF samples (VOFutil.jl:203-225) + cleanWisp! + BCf!
 template <class T>

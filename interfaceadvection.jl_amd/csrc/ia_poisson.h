@@ -501,19 +501,6 @@ __global__ void __launch_bounds__(NT) k_mg_center_l2(LevV<T> l, const double *pa
     })
     block_partial(v, l.t, part);
 }
-// Jacobi!: ϵ = r·iD
-template <class T>
-__global__ void __launch_bounds__(NT) k_mg_jacobi(LevV<T> l) {
-    HALT_IF(l)
-    const T *__restrict__ r = l.r;
-    const T *__restrict__ iD = l.iD;
-    T *__restrict__ e = l.e;
-    struct V2 {
-        T r, d;
-    };
-    col_pipe(l.g, l.t, [&](const int *, long I) { return V2{r[I], iD[I]}; },
-             [&](const int *, long I, const V2 &v) { e[I] = v.r * v.d; });
-}
 // increment!: r -= Aϵ; x += ϵ
 template <int D, class T> __device__ inline void increment_d(const LevV<T> &l) {
     const T *__restrict__ e = l.e;
@@ -2518,7 +2505,7 @@ __device__ __forceinline__ void f_up(const FLev &l, const FCols<D, C, WAVE> &q, 
         constexpr int NW = NTF / 64;
         double *h = sh + par * 16;
         par ^= 1;
-        if (wv < nw) v = NW <= 4 ? wave_sum_mm(v) : wave_sum1(v);  // the matrix products' rate is too low for more
+        if (wv < nw) v = wave_sum1(v);  // the matrix products' rate is too low for so many wavefronts
         if (lane == 0) h[wv] = wv < nw ? v : 0.0;
         __syncthreads();
         double t[NW];
