@@ -79,9 +79,11 @@ constexpr int CGP_P1 = CGP_COPY * 4 * CGP_ONE;
 constexpr int CGP_PW = CGP_P1 + 5 * CGP_MAXWG;  // the fifth: the XCD (a launch's first sum, if it asked for one)
 typedef unsigned long long cgp_word;
 constexpr int CGP_SC0 = 1, CGP_VOLATILE = (int)0x80000000u;  // of a buffer load's last argument
-// near: all workgroups run on one XCD, so a word need only reach its L2: a store of workgroup scope goes there, and a
-// load with sc0 set reads from there (an atomic load of workgroup scope may be served by the compute unit's own cache:
-// it is compiled without sc0).  Should a load ever take an old word, its tag shows it.
+// near: all workgroups run on one XCD, so a word need only reach its L2.  What makes the difference is the store: of
+// workgroup scope (compiled to sc0) it stays there, of agent scope (sc1) it goes past the L2s.  The loads have to pass
+// the compute unit's own cache: the volatile bit makes them system scope (sc0 sc1), and with sc0 alone they were never
+// shown another unit's words (every solve gave up), nor are atomic loads of workgroup scope.  Such a load still finds the
+// word in its XCD's L2; the far ones are of agent scope (sc1).  Should a load ever take an old word, its tag shows it.
 __device__ inline void cgp_put(cgp_word *p, unsigned v, unsigned tag, bool near) {
     const cgp_word q = ((cgp_word)tag << 32) | v;
     if (near) __hip_atomic_store(p, q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -158,6 +160,73 @@ template <int D, class A> __device__ inline float cgp_mult_parent(const A &a, co
     return mgmult_fc<D>(a.g, P, I, a.L, [&](const int *q) { return cgp_parent<D>(a, q); });
 }
 
+// The exchange, for both kernels.  (Their halo cells' geometry is written out in each: formed by one inlined function it
+// kept its flags in scalar registers that were then spilled in the loops, 0.5% of a step at 64³.)
+// m parts (m <= 64) of a sum, N words each, one part a lane of this wavefront; false: not there in time
+template <int N>
+__device__ __forceinline__ bool cgp_sums(const cgp_word *w, int m, unsigned tag, bool near, int lane, cgp_word (&v)[N]) {
+    const long t0 = wall_clock64();
+    for (int spin = 0;; ++spin) {
+        bool ok = true;
+        if (lane < m) {
+            cgp_getn(w, N * lane, v, near);
+#pragma unroll
+            for (int j = 0; j < N; ++j) ok = ok && (unsigned)(v[j] >> 32) == tag;
+        }
+        if (__all(ok)) break;
+        if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
+    }
+    return true;
+}
+
+// the words of the halo cells, from their owners; false: not there in time
+template <int HC>
+__device__ __forceinline__ bool cgp_words_at(const cgp_word *hw, const bool (&on)[HC], const int (&wo)[HC], unsigned tag,
+                                             bool near, cgp_word (&h)[HC]) {
+    const long t0 = wall_clock64();
+    for (int spin = 0;; ++spin) {
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < HC; ++k) h[k] = cgp_get(hw, wo[k], near);
+#pragma unroll
+        for (int k = 0; k < HC; ++k) ok = ok && (!on[k] || (unsigned)(h[k] >> 32) == tag);
+        if (__all(ok)) break;
+        if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
+    }
+    return true;
+}
+// publishes the values at the box's faces, from their tile
+template <int HC>
+__device__ __forceinline__ void cgp_faces(cgp_word *hw, const float *tile, const bool (&on)[HC], const int (&ti)[HC],
+                                          const int (&wo)[HC], unsigned tag, bool near) {
+    float f[HC];
+#pragma unroll
+    for (int k = 0; k < HC; ++k) f[k] = tile[ti[k]];
+    if (near) {
+#pragma unroll
+        for (int k = 0; k < HC; ++k)
+            if (on[k]) cgp_put(hw + wo[k], __float_as_uint(f[k]), tag, true);
+    } else {
+#pragma unroll
+        for (int k = 0; k < HC; ++k)
+            if (on[k]) cgp_put(hw + wo[k], __float_as_uint(f[k]), tag, false);
+    }
+}
+// the place of workgroup wg's box: its indices, first cell lo (ghost-inclusive), sides n
+template <int D> struct CgpAt {
+    int bi[3], lo[3], n[3];
+    __device__ __forceinline__ CgpAt(const Grid &g, const CgpBox &box, int wg) {
+        bi[0] = wg % box.k[0];
+        bi[1] = wg / box.k[0] % box.k[1];
+        bi[2] = wg / box.k[0] / box.k[1];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = d < D ? 1 + bi[d] * box.b[d] : 0;
+            n[d] = d < D ? min(box.b[d], g.Ng[d] - 1 - lo[d]) : 1;
+        }
+    }
+};
+
 // NB threads; a thread owns a column of C cells along the last axis (so two of a cell's neighbours are mostly its own
 // registers); the halo cells are those of wavefronts 1.. (HC each), while wavefront 0 waits for the sums.
 template <int D, int NB, int C, int HC>
@@ -174,20 +243,8 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     __shared__ int dead, nears;
     const Grid &g = a.g;
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-    // this workgroup's box: first cell lo (ghost-inclusive), sides n
-    int bi[3], lo[3], n[3];
-    {
-        int q = wg;
-        bi[0] = q % a.box.k[0];
-        q /= a.box.k[0];
-        bi[1] = q % a.box.k[1];
-        bi[2] = q / a.box.k[1];
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        lo[d] = d < D ? 1 + bi[d] * a.box.b[d] : 0;
-        n[d] = d < D ? min(a.box.b[d], g.Ng[d] - 1 - lo[d]) : 1;
-    }
+    const CgpAt<D> B(g, a.box, wg);
+    const auto &bi = B.bi, &lo = B.lo, &n = B.n;
     // strides of the u tile, along a column last
     const int zs = BIG ? cgp_zstride(a.box.b[2], C) : 1, t0 = BIG ? zs : 1, t1 = t0 * (a.box.b[0] + 2);
     const int tz = BIG ? 1 : D > 2 ? t1 * (a.box.b[1] + 2) : t1;
@@ -324,18 +381,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     };
     auto faces = [&](unsigned tag) {  // w of the box's faces, from its tile
         cgp_word *hw = a.hw + (tag & 1 ? hslot : 0);
-        float f[HC];
-#pragma unroll
-        for (int k = 0; k < HC; ++k) f[k] = cgp_w[fti[k]];
-        if (near) {
-#pragma unroll
-            for (int k = 0; k < HC; ++k)
-                if (fon[k]) cgp_put(hw + fwo[k], __float_as_uint(f[k]), tag, true);
-        } else {
-#pragma unroll
-            for (int k = 0; k < HC; ++k)
-                if (fon[k]) cgp_put(hw + fwo[k], __float_as_uint(f[k]), tag, false);
-        }
+        cgp_faces(hw, cgp_w, fon, fti, fwo, tag, near);
     };
     auto own = [&](float *tl, const float (&v)[C]) {  // the own cells' values to a tile
         const int t = place();
@@ -440,17 +486,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     // the sums of m pairs (m <= 64) of four words each by this wavefront; false: not there in time
     auto gather = [&](const cgp_word *w4, int m, unsigned tag, double &va, double &vb) {
         cgp_word v[4];
-        const long t0 = wall_clock64();
-        for (int spin = 0;; ++spin) {
-            bool ok = true;
-            if (lane < m) {
-                cgp_getn(w4, 4 * lane, v, near);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) ok = ok && (unsigned)(v[j] >> 32) == tag;
-            }
-            if (__all(ok)) break;
-            if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
-        }
+        if (!cgp_sums(w4, m, tag, near, lane, v)) return false;
         va = lane < m ? __hiloint2double((int)(unsigned)v[1], (int)(unsigned)v[0]) : 0.0;
         vb = lane < m ? __hiloint2double((int)(unsigned)v[3], (int)(unsigned)v[2]) : 0.0;
         wave_sum2(va, vb);
@@ -459,18 +495,7 @@ __global__ void __launch_bounds__(NB) k_cgp(CgpArgs a) {
     // the halo cells' w
     auto halo = [&](const cgp_word *hw, unsigned tag) {
         cgp_word h[HC];
-        const long t0 = wall_clock64();
-        for (int spin = 0;; ++spin) {
-            bool ok = true;
-#pragma unroll
-            for (int k = 0; k < HC; ++k)
-                h[k] = cgp_get(hw, hwo[k], near);
-#pragma unroll
-            for (int k = 0; k < HC; ++k)
-                ok = ok && (!hon[k] || (unsigned)(h[k] >> 32) == tag);
-            if (__all(ok)) break;
-            if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
-        }
+        if (!cgp_words_at(hw, hon, hwo, tag, near, h)) return false;
 #pragma unroll
         for (int k = 0; k < HC; ++k) hv[k] = hon[k] ? __uint_as_float((unsigned)h[k]) : 0.f;
         return true;
@@ -621,20 +646,8 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     __shared__ int dead, nears;
     const Grid &g = a.g;
     const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-    // this workgroup's box: first cell lo (ghost-inclusive), sides n
-    int bi[3], lo[3], n[3];
-    {
-        int q = wg;
-        bi[0] = q % a.box.k[0];
-        q /= a.box.k[0];
-        bi[1] = q % a.box.k[1];
-        bi[2] = q / a.box.k[1];
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        lo[d] = d < D ? 1 + bi[d] * a.box.b[d] : 0;
-        n[d] = d < D ? min(a.box.b[d], g.Ng[d] - 1 - lo[d]) : 1;
-    }
+    const CgpAt<D> B(g, a.box, wg);
+    const auto &bi = B.bi, &lo = B.lo, &n = B.n;
     const int t1 = a.box.b[0] + 2, t2 = t1 * (a.box.b[1] + 2);  // strides of the u tile
     const int tz = D > 2 ? t2 : t1;                            // along a column
     const long sz = g.st[D - 1];
@@ -754,18 +767,7 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     auto half_of = [](double v, int j) { return (unsigned)((j & 1) ? __double2hiint(v) : __double2loint(v)); };
     auto faces = [&](unsigned tag) {  // w of the box's faces, from its tile
         cgp_word *hw = a.hw + (tag & 1 ? hslot : 0);
-        float f[HC];
-#pragma unroll
-        for (int k = 0; k < HC; ++k) f[k] = cgp_w[fti[k]];
-        if (near) {
-#pragma unroll
-            for (int k = 0; k < HC; ++k)
-                if (fon[k]) cgp_put(hw + fwo[k], __float_as_uint(f[k]), tag, true);
-        } else {
-#pragma unroll
-            for (int k = 0; k < HC; ++k)
-                if (fon[k]) cgp_put(hw + fwo[k], __float_as_uint(f[k]), tag, false);
-        }
+        cgp_faces(hw, cgp_w, fon, fti, fwo, tag, near);
     };
     auto tile = [&]() {  // ϵ of the box and its halo
 #pragma unroll
@@ -789,34 +791,14 @@ __global__ void __launch_bounds__(NB) k_pcgp(PcgpArgs a) {
     // the sum of m parts (m <= 64) of two words each by this wavefront; false: not there in time
     auto gather = [&](const cgp_word *w2, int m, unsigned tag, double &v) {
         cgp_word q[2];
-        const long t0 = wall_clock64();
-        for (int spin = 0;; ++spin) {
-            bool ok = true;
-            if (lane < m) {
-                cgp_getn(w2, 2 * lane, q, near);
-                ok = (unsigned)(q[0] >> 32) == tag && (unsigned)(q[1] >> 32) == tag;
-            }
-            if (__all(ok)) break;
-            if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
-        }
+        if (!cgp_sums(w2, m, tag, near, lane, q)) return false;
         v = wave_sum1(lane < m ? __hiloint2double((int)(unsigned)q[1], (int)(unsigned)q[0]) : 0.0);
         return true;
     };
     // the halo cells' z = A ϵ
     auto halo = [&](const cgp_word *hw, unsigned tag) {
         cgp_word h[HC];
-        const long t0 = wall_clock64();
-        for (int spin = 0;; ++spin) {
-            bool ok = true;
-#pragma unroll
-            for (int k = 0; k < HC; ++k)
-                h[k] = cgp_get(hw, hwo[k], near);
-#pragma unroll
-            for (int k = 0; k < HC; ++k)
-                ok = ok && (!hon[k] || (unsigned)(h[k] >> 32) == tag);
-            if (__all(ok)) break;
-            if ((spin & 31) == 31 && wall_clock64() - t0 > CGP_WAIT) return false;
-        }
+        if (!cgp_words_at(hw, hon, hwo, tag, near, h)) return false;
 #pragma unroll
         for (int k = 0; k < HC; ++k) hv[k] = hon[k] ? __uint_as_float((unsigned)h[k]) : 0.f;
         return true;
